@@ -18,13 +18,14 @@
 // cells per edge, where the 27 cells around a cell are distinct (the
 // reference's small-box double counting is not reproduced).
 //
-// g_uu, per origin: displacements of the active particles (k_gu_disp), the
-// running MSD and mean-displacement sums in particle order on one thread
-// (k_gu_sums), then all active pairs i < j on a triangle of 256 x 256 tiles
-// (k_gu_hist) with the histogram of a bin range in LDS.  Bin indices
-// (int)(sqrt(r2)/bin) use correctly rounded sqrt and division, so the pair
-// counts are exact; the two weighted histograms are FP64 sums whose order
-// follows the atomics (agreement with the reference to rounding).
+// g_uu, a batch of origins per launch: displacements of the active particles
+// and their MSD and mean-displacement sums (k_gu_disp), then all active pairs
+// i < j on triangles of 256 x 256 tiles (k_gu_hist, a persistent grid) with
+// the histogram of a bin range in LDS, and the workgroups' histograms summed
+// (k_gu_reduce).  Bin indices are those of correctly rounded sqrt and
+// division (gu_bin), so the pair counts are exact; the two weighted
+// histograms are FP64 sums whose order follows the LDS atomics (agreement
+// with the reference to rounding).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -36,6 +37,7 @@
 #define CG_CAP 64            // neighbours per particle within 1.3 sigma (about 13 at rho = 1.2)
 #define GU_TILE 256
 #define GU_LDS_BINS 6144     // bins per pass: 6144 * 20 B = 120 KB of LDS
+#define GU_BATCH (64u << 20) // bytes of displacements of one launch's origins
 #define PR_TIME_STEP 0.005   // Analysis/global.h:19
 #define PR_DIVIDE_TO 2.0     // Analysis/global.h:21
 #define PR_PI 3.14159265358979
@@ -239,84 +241,116 @@ __global__ void __launch_bounds__(PR_THREADS) k_cg_count(const double *__restric
 
 // ------------------------------------------------------------------- g_uu
 
-// active particles m (ascending index act[m]): displacement to the lag frame
-// (guu.c:151-180) and wrapped origin position (LoadOrigin)
+// active particles m (ascending index act[m]) of each origin of a batch
+// (grid: particle blocks x origins, frame offsets fo[o] = {origin, lag}):
+// displacement to the lag frame (guu.c:151-180) and wrapped origin position
+// (LoadOrigin) to g[o][7][na]; the block's sums of L*L*r2 and r (the terms of
+// MSDtPP and MDtPP, guu.c:172-173) to acc[(o*gridDim.x + block)*2], added up
+// by the host in origin and block order.  (One thread adding them in
+// particle order took 301 us per origin at 5000 active particles, more than
+// twice the pair histogram.)
 __global__ void __launch_bounds__(PR_THREADS) k_gu_disp(const double *__restrict__ X, const double *__restrict__ Y,
-                                                        const double *__restrict__ Z, int n, size_t f0, size_t ft,
-                                                        const int *__restrict__ act, int na, double L, double *g) {
+                                                        const double *__restrict__ Z, int n,
+                                                        const int2 *__restrict__ fo, const int *__restrict__ act,
+                                                        int na, double L, double *gall, double *acc) {
     const int m = blockIdx.x * PR_THREADS + threadIdx.x;
-    if (m >= na) return;
-    const int i = act[m];
-    const double dx = pr_mi(X[ft + i] - X[f0 + i]), dy = pr_mi(Y[ft + i] - Y[f0 + i]),
-                 dz = pr_mi(Z[ft + i] - Z[f0 + i]);
-    const double r2 = (dx * dx + dy * dy + dz * dz);
-    g[0 * (size_t)na + m] = pr_wrap(X[f0 + i]);
-    g[1 * (size_t)na + m] = pr_wrap(Y[f0 + i]);
-    g[2 * (size_t)na + m] = pr_wrap(Z[f0 + i]);
-    g[3 * (size_t)na + m] = L * sqrt(r2);  // drt
-    g[4 * (size_t)na + m] = L * dx;
-    g[5 * (size_t)na + m] = L * dy;
-    g[6 * (size_t)na + m] = L * dz;
-    g[7 * (size_t)na + m] = r2;
-}
-
-// MSDtPP += L*L*r2, MDtPP += r in particle order, carried over origins (guu.c:172-173)
-__global__ void k_gu_sums(const double *__restrict__ g, int na, double L, double *acc) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double msd = acc[0], md = acc[1];
-    for (int m = 0; m < na; m++) {
-        msd += L * L * g[7 * (size_t)na + m];
-        md += g[3 * (size_t)na + m];
+    const size_t f0 = (size_t)fo[blockIdx.y].x * n, ft = (size_t)fo[blockIdx.y].y * n;
+    double *g = gall + (size_t)blockIdx.y * 7 * na;
+    double msd = 0.0, md = 0.0;
+    if (m < na) {
+        const int i = act[m];
+        const double dx = pr_mi(X[ft + i] - X[f0 + i]), dy = pr_mi(Y[ft + i] - Y[f0 + i]),
+                     dz = pr_mi(Z[ft + i] - Z[f0 + i]);
+        const double r2 = (dx * dx + dy * dy + dz * dz);
+        g[0 * (size_t)na + m] = pr_wrap(X[f0 + i]);
+        g[1 * (size_t)na + m] = pr_wrap(Y[f0 + i]);
+        g[2 * (size_t)na + m] = pr_wrap(Z[f0 + i]);
+        md = L * sqrt(r2);  // drt
+        msd = L * L * r2;
+        g[3 * (size_t)na + m] = md;
+        g[4 * (size_t)na + m] = L * dx;
+        g[5 * (size_t)na + m] = L * dy;
+        g[6 * (size_t)na + m] = L * dz;
     }
-    acc[0] = msd;
-    acc[1] = md;
+    __shared__ double s_w[2][PR_THREADS / 64];
+    msd = ac4_wave_sum(msd);
+    md = ac4_wave_sum(md);
+    if ((threadIdx.x & 63) == 0) {
+        s_w[0][threadIdx.x >> 6] = msd;
+        s_w[1][threadIdx.x >> 6] = md;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double t = 0.0;
+        for (int w = 0; w < PR_THREADS / 64; w++) t += s_w[threadIdx.x][w];
+        acc[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 2 + threadIdx.x] = t;
+    }
 }
 
-// pairs (row m1 < column m2) of one tile of the upper triangle; bins [b0, b0+nb)
-__global__ void __launch_bounds__(GU_TILE) k_gu_hist(const double *__restrict__ g, int na, double L, double bin,
-                                                     double maxbin, int b0, int nbins, int ntile,
-                                                     unsigned long long *hc, double *h1, double *h2) {
+// (int)(sqrt(r2) / bin), the bin of guu.c:205-206 with its correctly rounded
+// sqrt and division.  A 32-bit estimate decides wherever it is further from
+// a whole number than its error: r2 rounded to FP32, v_sqrt_f32 (1 ulp) and
+// one product with the rounded 1/bin are together within 3e-7 relative, taken
+// as 1e-6; about one pair in a hundred at 3500 bins takes the exact form.
+__device__ __forceinline__ int gu_bin(double r2, double bin, float rbin) {
+    const float e = __builtin_amdgcn_sqrtf((float)r2) * rbin;
+    const float f = floorf(e), m = 1e-6f * e + 1e-6f;
+    if (e - f > m && f + 1.0f - e > m) return (int)f;
+    return (int)(sqrt(r2) / bin);
+}
+
+// Pairs (row m1 < column m2) of the tiles of the upper triangle of every
+// origin of the batch, bins [b0, b0+nbins), item i = origin i / ntri, tile
+// i % ntri; workgroup w takes items w, w + gridDim.x, ... and keeps one
+// histogram in LDS over all of them, written to its own rows of pc/p1/p2 at
+// the end (k_gu_reduce adds the workgroups in order).  Bound by the FP64
+// pair arithmetic and the LDS atomics.  One launch per origin, a workgroup per
+// tile, each flushed by global atomics: 135 us per origin on 210 workgroups at
+// 5000 active particles; a persistent grid over 20 origins takes 60 us each.
+// Two threads share a row (half of the tile's columns each).
+__global__ void __launch_bounds__(2 * GU_TILE) k_gu_hist(const double *__restrict__ gall, int na, double L, double bin,
+                                                         float rbin, int maxbin, int b0, int nbins, int ntile,
+                                                         int ntri, int nitem, unsigned int *__restrict__ pc,
+                                                         double *__restrict__ p1, double *__restrict__ p2) {
     extern __shared__ unsigned char s_raw[];
     unsigned int *s_c = (unsigned int *)s_raw;
     double *s_1 = (double *)(s_raw + ((sizeof(unsigned int) * nbins + 15) & ~(size_t)15));
     double *s_2 = s_1 + nbins;
     __shared__ double s_col[7][GU_TILE];
-    // tile (tr, tc), tr <= tc, from the linear block index
-    int t = blockIdx.x, tr = 0;
-    while (t >= ntile - tr) {
-        t -= ntile - tr;
-        tr++;
-    }
-    const int tc = tr + t;
-    for (int b = threadIdx.x; b < nbins; b += GU_TILE) {
+    const int t = threadIdx.x, row = t & (GU_TILE - 1), half = t / GU_TILE;
+    for (int b = t; b < nbins; b += 2 * GU_TILE) {
         s_c[b] = 0;
         s_1[b] = 0.0;
         s_2[b] = 0.0;
     }
-    const int cj = tc * GU_TILE + threadIdx.x;
-    if (cj < na) {
-        s_col[0][threadIdx.x] = g[0 * (size_t)na + cj];
-        s_col[1][threadIdx.x] = g[1 * (size_t)na + cj];
-        s_col[2][threadIdx.x] = g[2 * (size_t)na + cj];
-        s_col[3][threadIdx.x] = g[3 * (size_t)na + cj];
-        s_col[4][threadIdx.x] = g[4 * (size_t)na + cj];
-        s_col[5][threadIdx.x] = g[5 * (size_t)na + cj];
-        s_col[6][threadIdx.x] = g[6 * (size_t)na + cj];
-    }
-    __syncthreads();
-    const int mi = tr * GU_TILE + threadIdx.x;
-    if (mi < na) {
+    for (int it = blockIdx.x; it < nitem; it += gridDim.x) {
+        const int o = it / ntri;
+        const double *g = gall + (size_t)o * 7 * na;
+        // tile (tr, tc), tr <= tc, of the triangle
+        int q = it - o * ntri, tr = 0;
+        while (q >= ntile - tr) {
+            q -= ntile - tr;
+            tr++;
+        }
+        const int tc = tr + q;
+        __syncthreads();  // the previous item's columns are read (and the bins cleared)
+        for (int k = t; k < 7 * GU_TILE; k += 2 * GU_TILE) {
+            const int a = k / GU_TILE, c = tc * GU_TILE + k % GU_TILE;
+            if (c < na) s_col[a][k % GU_TILE] = g[(size_t)a * na + c];
+        }
+        __syncthreads();
+        const int mi = tr * GU_TILE + row;
+        if (mi >= na) continue;
         const double xi = g[mi], yi = g[(size_t)na + mi], zi = g[2 * (size_t)na + mi];
         const double ri = g[3 * (size_t)na + mi], ui = g[4 * (size_t)na + mi], vi = g[5 * (size_t)na + mi],
                      wi = g[6 * (size_t)na + mi];
-        const int jn = min(GU_TILE, na - tc * GU_TILE);
-        for (int jj = 0; jj < jn; jj++) {
-            const int mj = tc * GU_TILE + jj;
-            if (mj <= mi) continue;
+        const int j1 = min((half + 1) * (GU_TILE / 2), na - tc * GU_TILE);
+        for (int jj = half * (GU_TILE / 2); jj < j1; jj++) {
+            if (tc * GU_TILE + jj <= mi) continue;
             // guu.c:198-213: x0_j - x0_i, one correction
             const double dx = pr_mi(s_col[0][jj] - xi), dy = pr_mi(s_col[1][jj] - yi), dz = pr_mi(s_col[2][jj] - zi);
             const double r2 = L * L * (dx * dx + dy * dy + dz * dz);
-            const int index = (int)(sqrt(r2) / bin);
+            const int index = gu_bin(r2, bin, rbin);
             if (index < maxbin && index >= b0 && index < b0 + nbins) {
                 const int b = index - b0;
                 atomicAdd(&s_c[b], 1u);
@@ -326,12 +360,41 @@ __global__ void __launch_bounds__(GU_TILE) k_gu_hist(const double *__restrict__ 
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nbins; b += GU_TILE)
-        if (s_c[b]) {
-            atomicAdd(&hc[b0 + b], (unsigned long long)s_c[b]);
-            atomicAdd(&h1[b0 + b], s_1[b]);
-            atomicAdd(&h2[b0 + b], s_2[b]);
+    const size_t w0 = (size_t)blockIdx.x * nbins;
+    for (int b = t; b < nbins; b += 2 * GU_TILE) {
+        pc[w0 + b] = s_c[b];
+        p1[w0 + b] = s_1[b];
+        p2[w0 + b] = s_2[b];
+    }
+}
+
+// the workgroups' histograms added to the totals in workgroup order: 64 bins
+// per workgroup of 256 threads, each quarter of the threads every fourth
+// histogram
+__global__ void __launch_bounds__(256) k_gu_reduce(const unsigned int *__restrict__ pc, const double *__restrict__ p1,
+                                                   const double *__restrict__ p2, int nw, int nbins, int b0,
+                                                   unsigned long long *hc, double *h1, double *h2) {
+    __shared__ unsigned long long s_c[4][64];
+    __shared__ double s_1[4][64], s_2[4][64];
+    const int l = threadIdx.x & 63, q = threadIdx.x >> 6, b = blockIdx.x * 64 + l;
+    unsigned long long c = 0;
+    double a1 = 0.0, a2 = 0.0;
+    if (b < nbins)
+        for (int w = q; w < nw; w += 4) {
+            const size_t k = (size_t)w * nbins + b;
+            c += pc[k];
+            a1 += p1[k];
+            a2 += p2[k];
         }
+    s_c[q][l] = c;
+    s_1[q][l] = a1;
+    s_2[q][l] = a2;
+    __syncthreads();
+    if (q == 0 && b < nbins) {
+        hc[b0 + b] += s_c[0][l] + s_c[1][l] + s_c[2][l] + s_c[3][l];
+        h1[b0 + b] += ((s_1[0][l] + s_1[1][l]) + s_1[2][l]) + s_1[3][l];
+        h2[b0 + b] += ((s_2[0][l] + s_2[1][l]) + s_2[2][l]) + s_2[3][l];
+    }
 }
 
 #define PTRY(e) do { int rc_ = (e); if (rc_ != AC4_OK) return rc_; } while (0)
@@ -483,53 +546,83 @@ extern "C" int ac4_frames_guu(ac4_frames *f, const int *act_tag, int gap, double
     for (int i = 0; i < n; i++)
         if (act_tag[i] == 1) act.push_back(i);
     const int na = (int)act.size();
-    AcDevBuf B;
-    int *d_act;
-    double *d_g, *d_acc, *d_h1, *d_h2;
-    unsigned long long *d_hc;
-    PTRY(B.get(&d_act, std::max(na, 1)));
-    PTRY(B.get(&d_g, (size_t)8 * std::max(na, 1)));
-    PTRY(B.get(&d_acc, 2));
-    PTRY(B.get(&d_hc, std::max(maxbin, 1)));
-    PTRY(B.get(&d_h1, std::max(maxbin, 1)));
-    PTRY(B.get(&d_h2, std::max(maxbin, 1)));
-    hipStream_t s = v.s;
-    if (na) AC4_HIP(hipMemcpyAsync(d_act, act.data(), sizeof(int) * na, hipMemcpyHostToDevice, s));
-    AC4_HIP(hipMemsetAsync(d_acc, 0, sizeof(double) * 2, s));
-    AC4_HIP(hipMemsetAsync(d_hc, 0, sizeof(unsigned long long) * std::max(maxbin, 1), s));
-    AC4_HIP(hipMemsetAsync(d_h1, 0, sizeof(double) * std::max(maxbin, 1), s));
-    AC4_HIP(hipMemsetAsync(d_h2, 0, sizeof(double) * std::max(maxbin, 1), s));
-    const int ntile = (na + GU_TILE - 1) / GU_TILE;
-    const long long ntri = (long long)ntile * (ntile + 1) / 2;
-    const int pass_bins = std::min(maxbin, GU_LDS_BINS);
-    const size_t lds = ((sizeof(unsigned int) * pass_bins + 15) & ~(size_t)15) + sizeof(double) * 2 * pass_bins;
-    AC4_HIP(hipFuncSetAttribute((const void *)k_gu_hist, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    // guu.c:138-231: the origins and their lag frames
+    std::vector<int2> fo;
     int current = 0, on = 0;
-    do {  // guu.c:138-231
+    do {
         const int cf = fidx[current];
         int other = current;
         while (other < nf && fidx[other] != cf + frame_num) other++;
         if (other >= nf) break;
-        if (na) {
-            hipLaunchKernelGGL(k_gu_disp, dim3((na + PR_THREADS - 1) / PR_THREADS), dim3(PR_THREADS), 0, s, v.x, v.y,
-                               v.z, n, (size_t)current * n, (size_t)other * n, d_act, na, L, d_g);
-            hipLaunchKernelGGL(k_gu_sums, dim3(1), dim3(64), 0, s, d_g, na, L, d_acc);
-            for (int b0 = 0; b0 < maxbin && ntri > 0; b0 += pass_bins)
-                hipLaunchKernelGGL(k_gu_hist, dim3((unsigned)ntri), dim3(GU_TILE), lds, s, d_g, na, L, bin, MaxBin,
-                                   b0, std::min(pass_bins, maxbin - b0), ntile, d_hc, d_h1, d_h2);
-            AC4_HIP(hipGetLastError());
-        }
+        fo.push_back(make_int2(current, other));
         on++;
         while (current < nf && fidx[current] != on * gap) current++;
     } while (current < nf);
+    const int ntile = (na + GU_TILE - 1) / GU_TILE;
+    AC4_REQUIRE((long long)ntile * (ntile + 1) / 2 < 2147483647LL, AC4_EARG, "ac4_frames_guu: %d active particles", na);
+    const int ntri = ntile * (ntile + 1) / 2;
+    const int pass_bins = std::min(maxbin, GU_LDS_BINS);
+    const size_t lds = ((sizeof(unsigned int) * pass_bins + 15) & ~(size_t)15) + sizeof(double) * 2 * pass_bins;
+    // origins of one launch: as many as GU_BATCH bytes of displacements hold
+    const size_t per = sizeof(double) * 7 * (size_t)std::max(na, 1);
+    const int batch = (int)std::max<size_t>(1, std::min<size_t>(std::max(on, 1), std::min<size_t>(GU_BATCH / per, 65535)));
+    // the persistent grid: the workgroups that are resident together
+    // (160 KB of LDS per CU, at most four of eight waves)
+    int dev = 0, ncu = 256;
+    (void)hipGetDevice(&dev);
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) ncu = 256;
+    const size_t lds_all = lds + sizeof(double) * 7 * GU_TILE;
+    const int grid = ncu * (int)std::max<size_t>(1, std::min<size_t>(4, 163840 / lds_all));
+    const int dblk = (na + PR_THREADS - 1) / PR_THREADS;
+    AcDevBuf B;
+    int *d_act;
+    int2 *d_fo;
+    double *d_g, *d_acc, *d_h1, *d_h2, *d_p1, *d_p2;
+    unsigned int *d_pc;
+    unsigned long long *d_hc;
+    PTRY(B.get(&d_act, std::max(na, 1)));
+    PTRY(B.get(&d_fo, std::max(on, 1)));
+    PTRY(B.get(&d_g, (size_t)batch * 7 * std::max(na, 1)));
+    PTRY(B.get(&d_acc, (size_t)2 * std::max(on, 1) * std::max(dblk, 1)));
+    PTRY(B.get(&d_hc, std::max(maxbin, 1)));
+    PTRY(B.get(&d_h1, std::max(maxbin, 1)));
+    PTRY(B.get(&d_h2, std::max(maxbin, 1)));
+    PTRY(B.get(&d_pc, (size_t)grid * std::max(pass_bins, 1)));
+    PTRY(B.get(&d_p1, (size_t)grid * std::max(pass_bins, 1)));
+    PTRY(B.get(&d_p2, (size_t)grid * std::max(pass_bins, 1)));
+    hipStream_t s = v.s;
+    if (na) AC4_HIP(hipMemcpyAsync(d_act, act.data(), sizeof(int) * na, hipMemcpyHostToDevice, s));
+    if (on) AC4_HIP(hipMemcpyAsync(d_fo, fo.data(), sizeof(int2) * on, hipMemcpyHostToDevice, s));
+    AC4_HIP(hipMemsetAsync(d_hc, 0, sizeof(unsigned long long) * std::max(maxbin, 1), s));
+    AC4_HIP(hipMemsetAsync(d_h1, 0, sizeof(double) * std::max(maxbin, 1), s));
+    AC4_HIP(hipMemsetAsync(d_h2, 0, sizeof(double) * std::max(maxbin, 1), s));
+    AC4_HIP(hipFuncSetAttribute((const void *)k_gu_hist, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    for (int o0 = 0; na && o0 < on; o0 += batch) {
+        const int no = std::min(batch, on - o0);
+        hipLaunchKernelGGL(k_gu_disp, dim3(dblk, no), dim3(PR_THREADS), 0, s, v.x, v.y, v.z, n, d_fo + o0, d_act, na, L,
+                           d_g, d_acc + (size_t)2 * o0 * dblk);
+        const long long all = (long long)ntri * no;
+        AC4_REQUIRE(all < 2147483647LL - grid, AC4_EARG, "ac4_frames_guu: %d active particles", na);
+        const int nitem = (int)all, gw = std::min(grid, nitem);
+        for (int b0 = 0; b0 < maxbin; b0 += pass_bins) {
+            const int nbins = std::min(pass_bins, maxbin - b0);
+            hipLaunchKernelGGL(k_gu_hist, dim3(gw), dim3(2 * GU_TILE), lds, s, d_g, na, L, bin, (float)(1.0 / bin),
+                               maxbin, b0, nbins, ntile, ntri, nitem, d_pc, d_p1, d_p2);
+            hipLaunchKernelGGL(k_gu_reduce, dim3((nbins + 63) / 64), dim3(256), 0, s, d_pc, d_p1, d_p2, gw, nbins, b0,
+                               d_hc, d_h1, d_h2);
+        }
+        AC4_HIP(hipGetLastError());
+    }
     std::vector<unsigned long long> hc(std::max(maxbin, 1));
-    std::vector<double> h1(std::max(maxbin, 1)), h2(std::max(maxbin, 1));
-    double acc[2];
+    std::vector<double> h1(std::max(maxbin, 1)), h2(std::max(maxbin, 1)), part((size_t)2 * on * dblk);
     AC4_HIP(hipMemcpyAsync(hc.data(), d_hc, sizeof(unsigned long long) * maxbin, hipMemcpyDeviceToHost, s));
     AC4_HIP(hipMemcpyAsync(h1.data(), d_h1, sizeof(double) * maxbin, hipMemcpyDeviceToHost, s));
     AC4_HIP(hipMemcpyAsync(h2.data(), d_h2, sizeof(double) * maxbin, hipMemcpyDeviceToHost, s));
-    AC4_HIP(hipMemcpyAsync(acc, d_acc, sizeof acc, hipMemcpyDeviceToHost, s));
+    if (!part.empty())
+        AC4_HIP(hipMemcpyAsync(part.data(), d_acc, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
     AC4_HIP(hipStreamSynchronize(s));
+    double acc[2] = {0.0, 0.0};
+    for (size_t k = 0; k < part.size(); k++) acc[k & 1] += part[k];
     // guu.c:250-276
     const double MSDt = acc[0] / ((double)n * (double)on);
     const double MDt = acc[1] / ((double)n * (double)on);
