@@ -23,12 +23,15 @@
 //               (<|W(q)|^2> - |<W(q)>|^2)/N),
 // with population variances over the pairs.
 //
-// Kernel: a block stages a tile of particles (weight and wrapped origin
-// position) in LDS; each thread owns one direction and a run of SHELL_RUN
-// consecutive shells and walks the tile: two sincos per particle, then the
-// phase advances from shell to shell by one complex multiplication,
-// exp(i q_{k+1} x) = exp(i q_k x) exp(i dq x), all in FP64.  Per-block partial
-// sums are reduced over blocks in a fixed order, so results are deterministic.
+// Kernel (k_fr_phase): a workgroup stages the overlapping particles of a tile
+// in LDS; each thread owns one direction and NG runs of SHELL_RUN = 27
+// consecutive shells.  A run is taken about its middle shell q_c: with
+// A = exp(i q_c x) and B_m = exp(i m dq x), the products cA cB, sA sB, sA cB
+// and cA sB summed over the particles give both shells q_c +- m dq, so a shell
+// costs two fused multiply-adds where a walk from shell to shell takes six
+// operations, and the chain of B_m is shared by the thread's runs.  All in
+// FP64.  The partial sums of the workgroups are added in a fixed order, so
+// results are deterministic.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -42,9 +45,12 @@ extern "C" int ac4_md_device_xu(ac4_md *md, int r, const double **xu, const doub
 
 #define TRY(e) do { int rc_ = (e); if (rc_ != AC4_OK) return rc_; } while (0)
 #define FR_THREADS 256
-#define FR_TILE 512
-#define SHELL_RUN 27
-#define FR_BLOCKS 240
+#define FR_ROLES 256   // most (direction, run) pairs of a call
+#define SHELL_RUN 27   // shells of a run: the middle one and SHELL_H on either side
+#define SHELL_H 13
+#define PH_THREADS 512 // threads of k_fr_phase and particles of its tile
+#define FR_BLOCKS 256  // its workgroups of one launch: one per CU
+#define FR_PAIRS 32    // pairs of one launch, at most
 
 struct ac4_frames {
     int n = 0, cap = 0, count = 0;
@@ -54,8 +60,6 @@ struct ac4_frames {
     hipStream_t s = nullptr;
     double *part = nullptr;  // [FR_BLOCKS][ndir][nshell][2]
     size_t part_n = 0;
-    double *cs = nullptr;    // [ndir][nshell][2] of one pair
-    size_t cs_n = 0;
     double *dirs = nullptr;
     int dirs_n = 0;
     unsigned int *cnt = nullptr;
@@ -86,69 +90,176 @@ __global__ void __launch_bounds__(FR_THREADS) k_fr_overlap(const double *__restr
     if ((threadIdx.x & 63) == 0 && w) atomicAdd(cnt, (unsigned int)w);
 }
 
-__global__ void __launch_bounds__(FR_THREADS) k_fr_phase(const double *__restrict__ x, const double *__restrict__ y,
-                                                         const double *__restrict__ z, int n, size_t fo, size_t ft,
+// frame offsets (in particles) of the pairs of one launch
+struct FrPairs {
+    size_t o[FR_PAIRS], l[FR_PAIRS];
+};
+
+// exp(2 pi i f), f in turns of any size: whole turns are taken off exactly
+__device__ __forceinline__ void fr_cis(double f, double *c, double *s) { ac4_sincos_turns(f - rint(f), s, c); }
+
+// Phase sums of pair blockIdx.x / bpp over the particles of block
+// blockIdx.x % bpp: part[blockIdx.x][ndir][nshell][2].  Thread t is role
+// t % T of team t / T, T = ndir * ceil(ngroup / NG) roles; the S = PH_THREADS
+// / T teams take every S-th particle of the tile, and their sums are added in
+// team order at the end.
+// Bound by FP64 issue: per particle and role 1 + NG sincos (34 instructions
+// each), 13 products of the B chain (4 each) and 54 sums and products per run
+// (4 per pair of shells).  Two runs per thread (NG = 2, about 230 registers, two
+// waves per SIMD) share the chain; an odd number of runs below five leaves
+// half of the last pair of runs idle, which costs more than the sharing
+// gives, and takes NG = 1.  300000 particles, 64 directions x 108 shells, per
+// pair: walking from shell to shell with the library's sincos 1220 us, this
+// 385 us.
+template <int NG>
+__global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restrict__ x, const double *__restrict__ y,
+                                                         const double *__restrict__ z, int n, FrPairs pr, int bpp,
                                                          double L, double a2, double q0, double dq, int nshell,
                                                          int ndir, int ngroup, const double *__restrict__ dirs,
                                                          double *part) {
-    __shared__ double s_x[FR_TILE], s_y[FR_TILE], s_z[FR_TILE];
-    __shared__ int s_w[FR_TILE];
-    const int t = threadIdx.x, d = t / ngroup, g = t - d * ngroup;
-    const bool active = d < ndir;
-    const int k0 = g * SHELL_RUN, kn = active ? std::min(SHELL_RUN, nshell - k0) : 0;
+    __shared__ double s_x[PH_THREADS], s_y[PH_THREADS], s_z[PH_THREADS];
+    __shared__ int s_n[PH_THREADS / 64 + 1];
+    __shared__ double s_f[PH_THREADS * 4];  // the teams' sums, four values a round
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int nrole = (ngroup + NG - 1) / NG, T = ndir * nrole, S = PH_THREADS / T;
+    const int team = t / T, role = t - team * T, d = role / nrole, g0 = (role - d * nrole) * NG;
+    const bool active = team < S;
+    const int pi = blockIdx.x / bpp, pb = blockIdx.x - pi * bpp;
+    const size_t fo = pr.o[pi], ft = pr.l[pi];
     double nx = 0.0, ny = 0.0, nz = 0.0;
     if (active) { nx = dirs[3 * d]; ny = dirs[3 * d + 1]; nz = dirs[3 * d + 2]; }
-    const double qa = (q0 + (double)k0 * dq) * L, qd = dq * L;  // phases per unit of n.s
-    double ac[SHELL_RUN], as[SHELL_RUN];
+    // phases per unit of n.s in turns: fd of one shell step, fc of the first run's middle shell
+    const double turn = L / 6.283185307179586, fd = dq * turn, fr = (double)SHELL_RUN * fd;
+    const double fc = (q0 + (double)(g0 * SHELL_RUN + SHELL_H) * dq) * turn;
+    double cc[NG][SHELL_H + 1], ss[NG][SHELL_H + 1], sc[NG][SHELL_H + 1], cs[NG][SHELL_H + 1];  // [0]: A alone
 #pragma unroll
-    for (int k = 0; k < SHELL_RUN; k++) { ac[k] = 0.0; as[k] = 0.0; }
-    const int per = (n + gridDim.x - 1) / gridDim.x;
-    const int i0 = blockIdx.x * per, i1 = std::min(n, i0 + per);
-    for (int tb = i0; tb < i1; tb += FR_TILE) {
-        const int m = std::min(FR_TILE, i1 - tb);
-        __syncthreads();
-        for (int j = t; j < m; j += FR_THREADS) {
-            const int i = tb + j;
-            const double ox = x[fo + i], oy = y[fo + i], oz = z[fo + i];
+    for (int u = 0; u < NG; u++)
+#pragma unroll
+        for (int m = 0; m <= SHELL_H; m++) cc[u][m] = ss[u][m] = sc[u][m] = cs[u][m] = 0.0;
+    const int per = (n + bpp - 1) / bpp;
+    const int i0 = min(n, pb * per), i1 = min(n, i0 + per);
+    for (int tb = i0; tb < i1; tb += PH_THREADS) {
+        const int i = tb + t;
+        double ox = 0.0, oy = 0.0, oz = 0.0;
+        bool hit = false;
+        if (i < i1) {
+            ox = x[fo + i]; oy = y[fo + i]; oz = z[fo + i];
             double dx = x[ft + i] - ox, dy = y[ft + i] - oy, dz = z[ft + i] - oz;
             dz = fr_minimg(dz);
             dy = fr_minimg(dy);
             dx = fr_minimg(dx);
-            s_w[j] = L * L * (dx * dx + dy * dy + dz * dz) < a2;
-            s_x[j] = ox - floor(ox);
-            s_y[j] = oy - floor(oy);
-            s_z[j] = oz - floor(oz);
+            hit = L * L * (dx * dx + dy * dy + dz * dz) < a2;
+        }
+        // the overlapping particles of the tile, in order
+        const unsigned long long hm = __ballot(hit);
+        __syncthreads();  // the previous tile is done with
+        if (lane == 0) s_n[wv] = __popcll(hm);
+        __syncthreads();
+        int k = __popcll(hm & ((1ull << lane) - 1ull)), m = 0;
+        for (int w = 0; w < PH_THREADS / 64; w++) {
+            const int c = s_n[w];
+            if (w < wv) k += c;
+            m += c;
+        }
+        if (hit) {
+            s_x[k] = ox - floor(ox);
+            s_y[k] = oy - floor(oy);
+            s_z[k] = oz - floor(oz);
         }
         __syncthreads();
-        if (kn <= 0) continue;
-        for (int j = 0; j < m; j++) {
-            if (!s_w[j]) continue;  // uniform over the block
-            const double p = nx * s_x[j] + ny * s_y[j] + nz * s_z[j];
-            double c, s, cd, sd;
-            sincos(qa * p, &s, &c);
-            sincos(qd * p, &sd, &cd);
+        if (!active) continue;
+        for (int j = team; j < m; j += S) {
+            const double p = fma(nz, s_z[j], fma(ny, s_y[j], nx * s_x[j]));
+            double c1, s1, ca[NG], sa[NG];
+            fr_cis(fd * p, &c1, &s1);
 #pragma unroll
-            for (int k = 0; k < SHELL_RUN; k++) {
-                ac[k] += c;
-                as[k] += s;
-                const double cn = c * cd - s * sd;
-                s = s * cd + c * sd;
-                c = cn;
+            for (int u = 0; u < NG; u++) {
+                fr_cis(u == 0 ? fc * p : fma(fr, p, fc * p), &ca[u], &sa[u]);
+                cc[u][0] += ca[u];
+                ss[u][0] += sa[u];
+            }
+            double cb = c1, sb = s1;
+#pragma unroll
+            for (int h = 1; h <= SHELL_H; h++) {
+#pragma unroll
+                for (int u = 0; u < NG; u++) {
+                    cc[u][h] = fma(ca[u], cb, cc[u][h]);
+                    ss[u][h] = fma(sa[u], sb, ss[u][h]);
+                    sc[u][h] = fma(sa[u], cb, sc[u][h]);
+                    cs[u][h] = fma(ca[u], sb, cs[u][h]);
+                }
+                if (h < SHELL_H) {
+                    const double cn = fma(cb, c1, -(sb * s1));
+                    sb = fma(sb, c1, cb * s1);
+                    cb = cn;
+                }
             }
         }
     }
-    if (!active) return;
-    double *o = part + (size_t)blockIdx.x * ndir * nshell * 2 + ((size_t)d * nshell + k0) * 2;
-    for (int k = 0; k < kn; k++) { o[2 * k] = ac[k]; o[2 * k + 1] = as[k]; }
+    // the shells' sums from the products, folded over the teams in team order
+    double *o = part + (size_t)blockIdx.x * ndir * nshell * 2;
+#pragma unroll
+    for (int u = 0; u < NG; u++) {
+        const int kc = (g0 + u) * SHELL_RUN + SHELL_H;
+#pragma unroll
+        for (int h = 0; h <= SHELL_H; h++) {
+            // shells kc + h and kc - h: {C+, S+, C-, S-} (h = 0: the first two)
+            double v[4];
+            if (h == 0) {
+                v[0] = cc[u][0]; v[1] = ss[u][0]; v[2] = v[3] = 0.0;
+            } else {
+                v[0] = cc[u][h] - ss[u][h];
+                v[1] = sc[u][h] + cs[u][h];
+                v[2] = cc[u][h] + ss[u][h];
+                v[3] = sc[u][h] - cs[u][h];
+            }
+            if (S > 1) {  // uniform over the workgroup
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < 4; q++) s_f[q * PH_THREADS + t] = v[q];
+                __syncthreads();
+                if (team == 0)
+                    for (int w = 1; w < S; w++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) v[q] += s_f[q * PH_THREADS + w * T + role];
+            }
+            if (team == 0) {
+                const int kp = kc + h, km = kc - h;
+                if (kp < nshell) {
+                    o[2 * ((size_t)d * nshell + kp)] = v[0];
+                    o[2 * ((size_t)d * nshell + kp) + 1] = v[1];
+                }
+                if (h > 0 && km < nshell) {
+                    o[2 * ((size_t)d * nshell + km)] = v[2];
+                    o[2 * ((size_t)d * nshell + km) + 1] = v[3];
+                }
+            }
+        }
+    }
 }
 
-// cs[e] = sum over blocks b = 0, 1, ... of part[b][e] (fixed order)
-__global__ void k_fr_reduce(const double *__restrict__ part, int nblk, int ne, double *cs) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ne) return;
+// part[p*bpp][e] = sum over the blocks b of pair p = blockIdx.y of
+// part[p*bpp + b][e]: 64 values per workgroup of 256 threads, wave w the
+// blocks w, w+4, ... with eight loads in flight, the waves added in order
+__global__ void __launch_bounds__(256) k_fr_reduce(double *part, int bpp, int ne) {
+    __shared__ double s_w[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, e = blockIdx.x * 64 + lane;
+    double *p = part + (size_t)blockIdx.y * bpp * ne;
     double a = 0.0;
-    for (int b = 0; b < nblk; b++) a += part[(size_t)b * ne + e];
-    cs[e] = a;
+    if (e < ne) {
+        int b = w;
+        for (; b + 28 < bpp; b += 32) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = p[(size_t)(b + 4 * u) * ne + e];
+#pragma unroll
+            for (int u = 0; u < 8; u++) a += v[u];
+        }
+        for (; b < bpp; b += 4) a += p[(size_t)b * ne + e];
+    }
+    s_w[w][lane] = a;
+    __syncthreads();
+    if (w == 0 && e < ne) p[e] = ((s_w[0][lane] + s_w[1][lane]) + s_w[2][lane]) + s_w[3][lane];
 }
 
 extern "C" int ac4_frames_create(int n, double L, int cap, ac4_frames **out) {
@@ -175,7 +286,7 @@ extern "C" int ac4_frames_create(int n, double L, int cap, ac4_frames **out) {
 extern "C" int ac4_frames_destroy(ac4_frames *f) {
     if (!f) return AC4_OK;
     if (f->s) (void)hipStreamSynchronize(f->s);
-    void *p[] = {f->x, f->y, f->z, f->part, f->cs, f->dirs, f->cnt};
+    void *p[] = {f->x, f->y, f->z, f->part, f->dirs, f->cnt};
     for (void *q : p)
         if (q) (void)hipFree(q);
     if (f->s) (void)hipStreamDestroy(f->s);
@@ -330,11 +441,41 @@ static int s4_check_args(ac4_frames *f, int npairs, const int *orig, const int *
     AC4_REQUIRE(f && npairs > 0 && orig && lagf && a > 0 && nshell > 0 && ndir > 0 && dq >= 0, AC4_EARG,
                 "frames_s4_shells: bad arguments");
     const int ngroup = (nshell + SHELL_RUN - 1) / SHELL_RUN;
-    AC4_REQUIRE(ndir * ngroup <= FR_THREADS, AC4_EARG,
-                "frames_s4_shells: ndir * ceil(nshell/%d) must be <= %d", SHELL_RUN, FR_THREADS);
+    AC4_REQUIRE(ndir * ngroup <= FR_ROLES, AC4_EARG,
+                "frames_s4_shells: ndir * ceil(nshell/%d) must be <= %d", SHELL_RUN, FR_ROLES);
     for (int p = 0; p < npairs; p++)
         AC4_REQUIRE(orig[p] >= 0 && orig[p] < f->count && lagf[p] >= 0 && lagf[p] < f->count, AC4_EARG,
                     "frames_s4_shells: pair %d refers to a frame not in the store", p);
+    return AC4_OK;
+}
+
+// The phase sums of every pair to ph[npairs][ndir][nshell][2] (host) through
+// part (FR_BLOCKS * ndir * nshell * 2 doubles on the device).  The FR_BLOCKS
+// workgroups of a launch are shared by as many pairs as leave each workgroup
+// at least one tile of particles: one pair for boxes of 131072 particles and
+// more, whose workgroups then fill the device alone.
+static int s4_phases(ac4_frames *f, int npairs, const int *orig, const int *lagf, double a, double q0, double dq,
+                     int nshell, int ndir, const double *dirs, double *part, double *ph) {
+    const int ngroup = (nshell + SHELL_RUN - 1) / SHELL_RUN;
+    const size_t ne = (size_t)ndir * nshell * 2;
+    const int bpp = std::max(FR_BLOCKS / FR_PAIRS, std::min(FR_BLOCKS, (f->n + PH_THREADS - 1) / PH_THREADS));
+    const int batch = std::min(FR_PAIRS, FR_BLOCKS / bpp);
+    auto kern = (ngroup % 2 == 0 || ngroup >= 5) ? k_fr_phase<2> : k_fr_phase<1>;
+    for (int p0 = 0; p0 < npairs; p0 += batch) {
+        const int np = std::min(batch, npairs - p0);
+        FrPairs pr = {};
+        for (int k = 0; k < np; k++) {
+            pr.o[k] = (size_t)orig[p0 + k] * f->n;
+            pr.l[k] = (size_t)lagf[p0 + k] * f->n;
+        }
+        hipLaunchKernelGGL(kern, dim3(np * bpp), dim3(PH_THREADS), 0, f->s, f->x, f->y, f->z, f->n, pr, bpp, f->L,
+                           a * a, q0, dq, nshell, ndir, ngroup, dirs, part);
+        hipLaunchKernelGGL(k_fr_reduce, dim3((unsigned)((ne + 63) / 64), np), dim3(256), 0, f->s, part, bpp, (int)ne);
+        AC4_HIP(hipGetLastError());
+        AC4_HIP(hipMemcpy2DAsync(ph + (size_t)p0 * ne, sizeof(double) * ne, part, sizeof(double) * ne * bpp,
+                                 sizeof(double) * ne, np, hipMemcpyDeviceToHost, f->s));
+    }
+    AC4_HIP(hipStreamSynchronize(f->s));
     return AC4_OK;
 }
 
@@ -342,57 +483,45 @@ extern "C" int ac4_frames_s4_shells(ac4_frames *f, int npairs, const int *orig, 
                                     double dq, int nshell, int ndir, uint64_t seed, double *s4_ref, double *s4_dir,
                                     double *phases) {
     TRY(s4_check_args(f, npairs, orig, lagf, a, nshell, ndir, dq));
-    const int ngroup = (nshell + SHELL_RUN - 1) / SHELL_RUN;
     const size_t ne = (size_t)ndir * nshell * 2;
     if (f->part_n < FR_BLOCKS * ne) {
         if (f->part) (void)hipFree(f->part);
         f->part = nullptr;
+        f->part_n = 0;
         AC4_HIP(hipMalloc(&f->part, sizeof(double) * FR_BLOCKS * ne));
         f->part_n = FR_BLOCKS * ne;
-    }
-    if (f->cs_n < ne) {
-        if (f->cs) (void)hipFree(f->cs);
-        f->cs = nullptr;
-        AC4_HIP(hipMalloc(&f->cs, sizeof(double) * ne));
-        f->cs_n = ne;
     }
     if (f->dirs_n < ndir) {
         if (f->dirs) (void)hipFree(f->dirs);
         f->dirs = nullptr;
+        f->dirs_n = 0;
         AC4_HIP(hipMalloc(&f->dirs, sizeof(double) * 3 * ndir));
         f->dirs_n = ndir;
     }
-    std::vector<double> dir(3 * (size_t)ndir), ph((size_t)npairs * ne);
+    std::vector<double> dir(3 * (size_t)ndir), own;
+    if (!phases) {
+        own.resize((size_t)npairs * ne);
+        phases = own.data();
+    }
     TRY(ac4_shell_directions(ndir, seed, dir.data()));
     AC4_HIP(hipMemcpyAsync(f->dirs, dir.data(), sizeof(double) * dir.size(), hipMemcpyHostToDevice, f->s));
-    for (int p = 0; p < npairs; p++) {
-        hipLaunchKernelGGL(k_fr_phase, dim3(FR_BLOCKS), dim3(FR_THREADS), 0, f->s, f->x, f->y, f->z, f->n,
-                           (size_t)orig[p] * f->n, (size_t)lagf[p] * f->n, f->L, a * a, q0, dq, nshell, ndir, ngroup,
-                           f->dirs, f->part);
-        hipLaunchKernelGGL(k_fr_reduce, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, f->s, f->part, FR_BLOCKS,
-                           (int)ne, f->cs);
-        AC4_HIP(hipGetLastError());
-        AC4_HIP(hipMemcpyAsync(ph.data() + (size_t)p * ne, f->cs, sizeof(double) * ne, hipMemcpyDeviceToHost, f->s));
-    }
-    AC4_HIP(hipStreamSynchronize(f->s));
-    if (phases) memcpy(phases, ph.data(), sizeof(double) * ph.size());
-    s4_reduce_host(ph.data(), npairs, ndir, nshell, (double)f->n, s4_ref, s4_dir);
+    TRY(s4_phases(f, npairs, orig, lagf, a, q0, dq, nshell, ndir, f->dirs, f->part, phases));
+    s4_reduce_host(phases, npairs, ndir, nshell, (double)f->n, s4_ref, s4_dir);
     return AC4_OK;
 }
 
 // ---------------------------------------------- S4 on shells, allocating nothing
-// The per-block partial sums, the per-pair sums and the directions live in
-// one file-scope device array instead of buffers of the frame store, so a
+// The per-block partial sums and the directions live in one file-scope device array instead of buffers of the frame store, so a
 // call makes no device or host allocation.  Each GPU holds its own copy of
 // the array until the process ends; its address on the current device is
 // looked up once (hipGetSymbolAddress) and kept per device.  Calls that
 // overlap on one GPU share the array and race.
-// ndir * ceil(nshell / SHELL_RUN) <= FR_THREADS bounds ndir * nshell by
-// FR_THREADS * SHELL_RUN = 6912, so ne = 2 * ndir * nshell <= 13824.
-#define S4_NOALLOC_NE_MAX (2 * FR_THREADS * SHELL_RUN)
-#define S4_NOALLOC_DIR_MAX FR_THREADS
-#define S4_SCRATCH_DOUBLES ((size_t)FR_BLOCKS * S4_NOALLOC_NE_MAX + S4_NOALLOC_NE_MAX + 3 * S4_NOALLOC_DIR_MAX)
-static __device__ __align__(256) double scratch[S4_SCRATCH_DOUBLES];  // 26.7 MB per GPU
+// ndir * ceil(nshell / SHELL_RUN) <= FR_ROLES bounds ndir * nshell by
+// FR_ROLES * SHELL_RUN = 6912, so ne = 2 * ndir * nshell <= 13824.
+#define S4_NOALLOC_NE_MAX (2 * FR_ROLES * SHELL_RUN)
+#define S4_NOALLOC_DIR_MAX FR_ROLES
+#define S4_SCRATCH_DOUBLES ((size_t)FR_BLOCKS * S4_NOALLOC_NE_MAX + 3 * S4_NOALLOC_DIR_MAX)
+static __device__ __align__(256) double scratch[S4_SCRATCH_DOUBLES];  // 28.3 MB per GPU
 #define S4_MAX_DEV 64
 static double *g_scratch_ptr[S4_MAX_DEV];
 
@@ -419,23 +548,13 @@ extern "C" int ac4_frames_s4_shells_noalloc(ac4_frames *f, int npairs, const int
     AC4_REQUIRE(ne <= S4_NOALLOC_NE_MAX, AC4_ECAP,
                 "s4_shells_noalloc: ndir * nshell = %d exceeds the scratch limit of %d", ndir * nshell,
                 S4_NOALLOC_NE_MAX / 2);
-    const int ngroup = (nshell + SHELL_RUN - 1) / SHELL_RUN;
     double *sp = nullptr;
     TRY(scratch_ptr(&sp));
-    double *part = sp, *cs = sp + (size_t)FR_BLOCKS * S4_NOALLOC_NE_MAX, *dirs = cs + S4_NOALLOC_NE_MAX;
-    double dir[3 * S4_NOALLOC_DIR_MAX];  // ndir <= FR_THREADS (checked above)
+    double *part = sp, *dirs = sp + (size_t)FR_BLOCKS * S4_NOALLOC_NE_MAX;
+    double dir[3 * S4_NOALLOC_DIR_MAX];  // ndir <= FR_ROLES (checked above)
     TRY(ac4_shell_directions(ndir, seed, dir));
     AC4_HIP(hipMemcpyAsync(dirs, dir, sizeof(double) * 3 * ndir, hipMemcpyHostToDevice, f->s));
-    for (int p = 0; p < npairs; p++) {
-        hipLaunchKernelGGL(k_fr_phase, dim3(FR_BLOCKS), dim3(FR_THREADS), 0, f->s, f->x, f->y, f->z, f->n,
-                           (size_t)orig[p] * f->n, (size_t)lagf[p] * f->n, f->L, a * a, q0, dq, nshell, ndir, ngroup,
-                           dirs, part);
-        hipLaunchKernelGGL(k_fr_reduce, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, f->s, part, FR_BLOCKS,
-                           (int)ne, cs);
-        AC4_HIP(hipGetLastError());
-        AC4_HIP(hipMemcpyAsync(phases + (size_t)p * ne, cs, sizeof(double) * ne, hipMemcpyDeviceToHost, f->s));
-    }
-    AC4_HIP(hipStreamSynchronize(f->s));
+    TRY(s4_phases(f, npairs, orig, lagf, a, q0, dq, nshell, ndir, dirs, part, phases));
     s4_reduce_host(phases, npairs, ndir, nshell, (double)f->n, s4_ref, s4_dir);
     return AC4_OK;
 }

@@ -203,8 +203,8 @@ int ac4_frames_s4_shells(ac4_frames *f, int npairs, const int *orig, const int *
 /* ac4_frames_s4_shells that allocates nothing, device or host: no reference
  * counterpart.  For callers that cannot allocate (tight analysis loops in a
  * serving process, code that must not call hipMalloc).  Its per-block
- * partials, per-pair sums and directions sit in one file-scope device array
- * of 26.7 MB that each GPU holds until the process ends, sized for the
+ * partials and directions sit in one file-scope device array
+ * of 28.3 MB that each GPU holds until the process ends, sized for the
  * largest shape ac4_frames_s4_shells accepts (ndir * ceil(nshell/27) <= 256,
  * so ndir * nshell <= 6912; larger shapes are refused with AC4_EARG, and a
  * shape over the array with AC4_ECAP); phases is required

@@ -29,3 +29,38 @@ def test_guu_tile_edges(gpu, na, L):
     # a bin sums at most a few thousand FP64 terms: n_terms * 2^-53 of their absolute sum
     scale = max(1.0, np.abs(ho[1]).max())
     assert np.abs(h[1:] - ho[1:]).max() <= 1e-12 * scale
+
+
+# Runs of 27 shells about a middle one: part of a run, one, the odd counts
+# below and from five, even ones; the widest and the smallest teams; one
+# particle, tile remainders, several pairs per launch and more than one batch.
+@pytest.mark.parametrize("n,npairs,nshell,ndir", [(1, 1, 1, 1), (511, 3, 9, 5), (513, 40, 28, 7), (700, 2, 81, 85),
+                                                  (700, 2, 135, 51), (300, 2, 108, 64), (600, 2, 27, 256),
+                                                  (200, 1, 6912, 1), (5000, 20, 54, 3)])
+def test_shell_runs_against_direct_sums(gpu, n, npairs, nshell, ndir):
+    rng = np.random.default_rng(n + nshell)
+    L, a, q0, dq = 9.0, 0.3, 0.11, 0.07
+    X = rng.random((3, npairs + 1, n)) + rng.normal(0, 0.08 / L, (3, npairs + 1, n)) * np.arange(npairs + 1)[:, None]
+    fr = gpu.Frames(n, L, npairs + 1)
+    for k in range(npairs + 1):
+        X[:, k] = X[:, 0] + rng.normal(0, 0.1 / L, (3, n)) if k else X[:, 0]
+        fr.push(*X[:, k], 10 * k)
+    orig, lag = [0] * npairs, list(range(1, npairs + 1))
+    _, s4d, ph = fr.s4_shells(orig, lag, q0, dq, nshell, ndir, 99, a=a, phases=True)
+    fr.close()
+    dirs = gpu.shell_directions(ndir, 99)
+    q = (q0 + dq * np.arange(nshell)) * L
+    pos = X[:, 0] - np.floor(X[:, 0])
+    proj = dirs @ pos
+    for p in range(npairs):
+        d = X[:, lag[p]] - X[:, 0]
+        w = L * L * ((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]) < a * a
+        for k0 in range(0, nshell, 64):
+            f = proj[:, None, w] * q[None, k0:k0 + 64, None]
+            # a term is off by the rounding of its phase and of 13 products
+            tol = (4e-16 * np.abs(f).max() + 4e-14) * max(1, w.sum()) if w.any() else 0.0
+            assert np.abs(ph[p, :, k0:k0 + 64, 0] - np.cos(f).sum(-1)).max() <= tol
+            assert np.abs(ph[p, :, k0:k0 + 64, 1] - np.sin(f).sum(-1)).max() <= tol
+    var = lambda v: (v * v).mean(0) - v.mean(0) ** 2  # noqa: E731
+    want = var(ph).sum(-1).mean(0) / n
+    assert np.allclose(s4d, want, rtol=1e-9, atol=1e-9 * (ph ** 2).max() / n)
