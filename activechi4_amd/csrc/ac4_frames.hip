@@ -95,14 +95,20 @@ struct FrPairs {
     size_t o[FR_PAIRS], l[FR_PAIRS];
 };
 
-// exp(2 pi i f), f in turns of any size: whole turns are taken off exactly
-__device__ __forceinline__ void fr_cis(double f, double *c, double *s) { ac4_sincos_turns(f - rint(f), s, c); }
+// q p in turns, less the whole turns nearest it: the product is not rounded
+// before they are taken off
+__device__ __forceinline__ double fr_turns(double q, double p) { return fma(q, p, -rint(q * p)); }
 
 // Phase sums of pair blockIdx.x / bpp over the particles of block
 // blockIdx.x % bpp: part[blockIdx.x][ndir][nshell][2].  Thread t is role
 // t % T of team t / T, T = ndir * ceil(ngroup / NG) roles; the S = PH_THREADS
 // / T teams take every S-th particle of the tile, and their sums are added in
 // team order at the end.
+// L2 = L * L; f0, fd: the phases of |q| = q0 and of one shell step per unit of
+// n.s, in turns.  The phase of a middle shell is formed from the two reduced
+// phases, so that the step's rounding, multiplied by its number there and by
+// m in B_m, cancels in the shells of small |q|, where the particles' terms
+// add up coherently.
 // Bound by FP64 issue: per particle and role 1 + NG sincos (34 instructions
 // each), 13 products of the B chain (4 each) and 54 sums and products per run
 // (4 per pair of shells).  Two runs per thread (NG = 2, about 230 registers, two
@@ -110,27 +116,31 @@ __device__ __forceinline__ void fr_cis(double f, double *c, double *s) { ac4_sin
 // half of the last pair of runs idle, which costs more than the sharing
 // gives, and takes NG = 1.  300000 particles, 64 directions x 108 shells, per
 // pair: walking from shell to shell with the library's sincos 1220 us, this
-// 385 us.
+// 411 us.
 template <int NG>
 __global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restrict__ x, const double *__restrict__ y,
                                                          const double *__restrict__ z, int n, FrPairs pr, int bpp,
-                                                         double L, double a2, double q0, double dq, int nshell,
+                                                         double L2, double a2, double f0, double fd, int nshell,
                                                          int ndir, int ngroup, const double *__restrict__ dirs,
                                                          double *part) {
     __shared__ double s_x[PH_THREADS], s_y[PH_THREADS], s_z[PH_THREADS];
     __shared__ int s_n[PH_THREADS / 64 + 1];
     __shared__ double s_f[PH_THREADS * 4];  // the teams' sums, four values a round
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nrole = (ngroup + NG - 1) / NG, T = ndir * nrole, S = PH_THREADS / T;
-    const int team = t / T, role = t - team * T, d = role / nrole, g0 = (role - d * nrole) * NG;
+    const int team = t / T;
     const bool active = team < S;
     const int pi = blockIdx.x / bpp, pb = blockIdx.x - pi * bpp;
     const size_t fo = pr.o[pi], ft = pr.l[pi];
-    double nx = 0.0, ny = 0.0, nz = 0.0;
-    if (active) { nx = dirs[3 * d]; ny = dirs[3 * d + 1]; nz = dirs[3 * d + 2]; }
-    // phases per unit of n.s in turns: fd of one shell step, fc of the first run's middle shell
-    const double turn = L / 6.283185307179586, fd = dq * turn, fr = (double)SHELL_RUN * fd;
-    const double fc = (q0 + (double)(g0 * SHELL_RUN + SHELL_H) * dq) * turn;
+    // direction and first middle shell of every role, read from LDS for each
+    // particle (volatile): the registers are the sums'
+    __shared__ double s_role[4][FR_ROLES];
+    if (team == 0) {
+        const int d = t / nrole, g0 = (t - d * nrole) * NG;
+        for (int q = 0; q < 3; q++) s_role[q][t] = dirs[3 * d + q];
+        s_role[3][t] = (double)(g0 * SHELL_RUN + SHELL_H);
+    }
+    const volatile double *vr = &s_role[0][t - team * T];
     double cc[NG][SHELL_H + 1], ss[NG][SHELL_H + 1], sc[NG][SHELL_H + 1], cs[NG][SHELL_H + 1];  // [0]: A alone
 #pragma unroll
     for (int u = 0; u < NG; u++)
@@ -148,14 +158,14 @@ __global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restric
             dz = fr_minimg(dz);
             dy = fr_minimg(dy);
             dx = fr_minimg(dx);
-            hit = L * L * (dx * dx + dy * dy + dz * dz) < a2;
+            hit = L2 * (dx * dx + dy * dy + dz * dz) < a2;
         }
         // the overlapping particles of the tile, in order
         const unsigned long long hm = __ballot(hit);
         __syncthreads();  // the previous tile is done with
-        if (lane == 0) s_n[wv] = __popcll(hm);
+        s_n[wv] = __popcll(hm);  // every lane the same value
         __syncthreads();
-        int k = __popcll(hm & ((1ull << lane) - 1ull)), m = 0;
+        int k = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(hm >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)hm, 0u)), m = 0;
         for (int w = 0; w < PH_THREADS / 64; w++) {
             const int c = s_n[w];
             if (w < wv) k += c;
@@ -169,12 +179,14 @@ __global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restric
         __syncthreads();
         if (!active) continue;
         for (int j = team; j < m; j += S) {
-            const double p = fma(nz, s_z[j], fma(ny, s_y[j], nx * s_x[j]));
+            const double p = fma(vr[2 * FR_ROLES], s_z[j], fma(vr[FR_ROLES], s_y[j], vr[0] * s_x[j]));
             double c1, s1, ca[NG], sa[NG];
-            fr_cis(fd * p, &c1, &s1);
+            const double r0 = fr_turns(f0, p), r1 = fr_turns(fd, p);
+            ac4_sincos_turns(r1, &s1, &c1);
 #pragma unroll
             for (int u = 0; u < NG; u++) {
-                fr_cis(u == 0 ? fc * p : fma(fr, p, fc * p), &ca[u], &sa[u]);
+                const double f = fma(vr[3 * FR_ROLES] + (double)(u * SHELL_RUN), r1, r0);
+                ac4_sincos_turns(f - rint(f), &sa[u], &ca[u]);
                 cc[u][0] += ca[u];
                 ss[u][0] += sa[u];
             }
@@ -198,6 +210,9 @@ __global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restric
     }
     // the shells' sums from the products, folded over the teams in team order
     double *o = part + (size_t)blockIdx.x * ndir * nshell * 2;
+    int te = t;
+    asm volatile("" : "+v"(te));  // the role again, not kept in registers over the loop
+    const int role = te % T, d = role / nrole, g0 = (role - d * nrole) * NG;
 #pragma unroll
     for (int u = 0; u < NG; u++) {
         const int kc = (g0 + u) * SHELL_RUN + SHELL_H;
@@ -460,6 +475,7 @@ static int s4_phases(ac4_frames *f, int npairs, const int *orig, const int *lagf
     const size_t ne = (size_t)ndir * nshell * 2;
     const int bpp = std::max(FR_BLOCKS / FR_PAIRS, std::min(FR_BLOCKS, (f->n + PH_THREADS - 1) / PH_THREADS));
     const int batch = std::min(FR_PAIRS, FR_BLOCKS / bpp);
+    const double turn = f->L / 6.283185307179586;  // phases in turns per unit |q|
     auto kern = (ngroup % 2 == 0 || ngroup >= 5) ? k_fr_phase<2> : k_fr_phase<1>;
     for (int p0 = 0; p0 < npairs; p0 += batch) {
         const int np = std::min(batch, npairs - p0);
@@ -468,8 +484,8 @@ static int s4_phases(ac4_frames *f, int npairs, const int *orig, const int *lagf
             pr.o[k] = (size_t)orig[p0 + k] * f->n;
             pr.l[k] = (size_t)lagf[p0 + k] * f->n;
         }
-        hipLaunchKernelGGL(kern, dim3(np * bpp), dim3(PH_THREADS), 0, f->s, f->x, f->y, f->z, f->n, pr, bpp, f->L,
-                           a * a, q0, dq, nshell, ndir, ngroup, dirs, part);
+        hipLaunchKernelGGL(kern, dim3(np * bpp), dim3(PH_THREADS), 0, f->s, f->x, f->y, f->z, f->n, pr, bpp,
+                           f->L * f->L, a * a, q0 * turn, dq * turn, nshell, ndir, ngroup, dirs, part);
         hipLaunchKernelGGL(k_fr_reduce, dim3((unsigned)((ne + 63) / 64), np), dim3(256), 0, f->s, part, bpp, (int)ne);
         AC4_HIP(hipGetLastError());
         AC4_HIP(hipMemcpy2DAsync(ph + (size_t)p0 * ne, sizeof(double) * ne, part, sizeof(double) * ne * bpp,
