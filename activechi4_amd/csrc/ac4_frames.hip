@@ -111,7 +111,7 @@ __device__ __forceinline__ double fr_turns(double q, double p) { return fma(q, p
 // add up coherently.
 // Bound by FP64 issue: per particle and role 1 + NG sincos (34 instructions
 // each), 13 products of the B chain (4 each) and 54 sums and products per run
-// (4 per pair of shells).  Two runs per thread (NG = 2, about 230 registers, two
+// (4 per pair of shells).  Two runs per thread (NG = 2, 255 registers, two
 // waves per SIMD) share the chain; an odd number of runs below five leaves
 // half of the last pair of runs idle, which costs more than the sharing
 // gives, and takes NG = 1.  300000 particles, 64 directions x 108 shells, per

@@ -95,9 +95,7 @@ struct ChainS {
     double ramp0, ramp1;      // target T = T*(ramp0 + (ramp1-ramp0)*k/(n-1))
 };
 
-// MDcode/cell_list+forces.c:19-20 restricted to the two KA species.
-__device__ __forceinline__ double sig_ab(int a, int b) { return (a + b) == 0 ? 1.00 : ((a + b) == 1 ? 0.80 : 0.88); }
-__device__ __forceinline__ double eps_ab(int a, int b) { return (a + b) == 0 ? 1.0 : ((a + b) == 1 ? 1.5 : 0.50); }
+
 
 __device__ __forceinline__ double minimg_md(double d) {  // cell_list+forces.c:92-97
     if (d < -0.5) d += 1.0;
@@ -1320,33 +1318,65 @@ __global__ void __launch_bounds__(BLK) k_export(const RepC *__restrict__ reps, c
 template <bool FP32>
 struct PairAcc;
 
+// 1/a for a normal positive a: the hardware's estimate (v_rcp_f64) and two
+// Newton steps, within an ulp; a fifth of the instructions of a division.
+__device__ __forceinline__ double rcp_newton(double a) {
+    double r = __builtin_amdgcn_rcp(a);
+    r = fma(fma(-a, r, 1.0), r, r);
+    return fma(fma(-a, r, 1.0), r, r);
+}
+
 template <>
-struct PairAcc<false> {  // FP64: the reference's per-pair arithmetic
+struct PairAcc<false> {
+    // FP64 pair terms of cell_list+forces.c:183-203.  The kernel is bound by
+    // the issue of these instructions and by the gathers: the reference's
+    // three divisions per pair (about 20 instructions each) are one
+    // reciprocal of r^2, the constants of the two possible partner species
+    // are set once per particle (a partner's are picked by one fused
+    // multiply-add with its species, 0.0 or 1.0), the minimum image is d -
+    // rint(d) (the same value as the reference's two tests for differences
+    // of wrapped coordinates), products and sums are fused, and the force is
+    // summed in box units and scaled once.  N=50000, one lane per particle:
+    // 47.6 -> 29.4 us.
     double fx = 0, fy = 0, fz = 0, pe = 0, vir = 0;
+    double L2;
+    double rc[2], s2c[2], e4[2], e8[2], c2i[2];  // value of species 0, difference of species 1
     __device__ __forceinline__ void flush() {}
-    __device__ __forceinline__ PairAcc(int, const RepC &) {}
-    __device__ __forceinline__ void add(const double4 &pi, int ti, const double4 &pj, const RepC &R) {
-        const double L = R.L;
-        double dx = minimg_md(pi.x - pj.x);
-        double dy = minimg_md(pi.y - pj.y);
-        double dz = minimg_md(pi.z - pj.z);
-        double dr2 = (dx * dx + dy * dy + dz * dz) * L * L;  // cell_list+forces.c:183
-        const int tj = (int)pj.w;
-        double eps = eps_ab(ti, tj), sig = sig_ab(ti, tj);
-        double r_over_sig_2 = dr2 / (sig * sig);
-        if (r_over_sig_2 < K_LCUTSQR) {  // :189-203
-            double s2 = 1.0 / r_over_sig_2;
-            double s6 = s2 * s2 * s2;
-            pe += 4.0 * eps * ((s6 * (s6 - 1.0)) + K_C0 + K_C2 * r_over_sig_2);
-            double grad = 8.0 * eps * (6.0 * s6 * (s6 - 0.5) / dr2 - K_C2 / (sig * sig));
-            fx += grad * dx * L;
-            fy += grad * dy * L;
-            fz += grad * dz * L;
-            vir += grad * dr2;
+    __device__ __forceinline__ PairAcc(int ti, const RepC &R) {
+        L2 = R.L * R.L;
+        // (ti, tj) -> ab = ti + tj: sigma {1, 0.8, 0.88}, epsilon {1, 1.5, 0.5} (cell_list+forces.c:19-20)
+        const auto pick = [ti](double v0, double v1, double v2, double (&out)[2]) {
+            const double a = ti ? v1 : v0;
+            out[0] = a;
+            out[1] = (ti ? v2 : v1) - a;
+        };
+        pick(K_LCUTSQR * 1.00 * 1.00, K_LCUTSQR * 0.80 * 0.80, K_LCUTSQR * 0.88 * 0.88, rc);  // (r/sigma)^2 < 6.25 (:189)
+        pick(1.00 * 1.00, 0.80 * 0.80, 0.88 * 0.88, s2c);
+        pick(4.0 * 1.0, 4.0 * 1.5, 4.0 * 0.5, e4);
+        pick(8.0 * 1.0, 8.0 * 1.5, 8.0 * 0.5, e8);
+        pick(K_C2 / (1.00 * 1.00), K_C2 / (0.80 * 0.80), K_C2 / (0.88 * 0.88), c2i);
+    }
+    __device__ __forceinline__ void add(const double4 &pi, int, const double4 &pj, const RepC &) {
+        double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+        dx -= rint(dx);
+        dy -= rint(dy);
+        dz -= rint(dz);
+        const double r2 = fma(dz, dz, fma(dy, dy, dx * dx)) * L2, tj = pj.w;
+        if (r2 < fma(tj, rc[1], rc[0])) {
+            const double inv = rcp_newton(r2);
+            const double s2 = fma(tj, s2c[1], s2c[0]) * inv, c2 = fma(tj, c2i[1], c2i[0]);
+            const double s6 = s2 * s2 * s2;
+            // 4 eps [s6 (s6 - 1) + C0 + C2 (r/sigma)^2], 8 eps [6 s6 (s6 - 1/2) / r^2 - C2 / sigma^2]
+            pe = fma(fma(tj, e4[1], e4[0]), fma(s6, s6 - 1.0, fma(c2, r2, K_C0)), pe);
+            const double grad = fma(tj, e8[1], e8[0]) * fma(6.0 * s6 * inv, s6 - 0.5, -c2);
+            fx = fma(grad, dx, fx);
+            fy = fma(grad, dy, fy);
+            fz = fma(grad, dz, fz);
+            vir = fma(grad, r2, vir);
         }
     }
-    __device__ __forceinline__ void result(double &ox, double &oy, double &oz, const RepC &) const {
-        ox = fx; oy = fy; oz = fz;
+    __device__ __forceinline__ void result(double &ox, double &oy, double &oz, const RepC &R) const {
+        ox = fx * R.L; oy = fy * R.L; oz = fz * R.L;
     }
 };
 
