@@ -58,6 +58,16 @@ struct RepC {
     double skin;    // Verlet skin: list radii 2.5 sigma_ab + skin, rebuild criterion
     float qs2;      // qscale^2 in FP32
     int xcull;      // list teams skip the far x-half of the cells beside along x (configure_rep)
+    int enblk, eblk_off;   // blocks of the energy pass (k_energy), 0 without it
+    float rcq[3], c2i[3];  // species pair ab: cutoff^2 in fixed-point units^2, C2 / sigma^2 (FP32 path)
+};
+
+// One workgroup's particles: replica, first local particle, the replica's
+// first slot and its particle count.  One 16-byte load, after which the
+// particle loads can be issued beside the replica's constants instead of
+// after them.
+struct BlkD {
+    int rep, first, off, n;
 };
 
 // Fixed-point copy of a wrapped position for the FP32 force path and the
@@ -103,9 +113,36 @@ __device__ __forceinline__ double minimg_md(double d) {  // cell_list+forces.c:9
     return d;
 }
 
-// U4 propagator (MDcode/time_evolve.c:578-609) with the p^2 sum supplied.
+// exp(-x) and (1 - exp(-x)) / x.  The chain's x are of order 1e-3: below 1/16
+// both come from one series, phi = sum (-x)^k / (k+1)!, whose remainder there
+// is below 3e-19, and exp(-x) = 1 - x phi: within an ulp, where 1 - exp(-x)
+// loses the digits that cancel.  The chain runs on one lane between two
+// kernels of the step, so the length of its serial chain of operations is
+// what it costs: k_force_end 4.1 -> 3.5 us on one box of N=1000 with this,
+// the reciprocals of q and the start-of-step half kept from k_first_half.
+__host__ __device__ inline double exp_phi(double x, double *phi) {
+    if (fabs(x) < 0.0625) {
+        double p = fma(-x, 1.0 / 3628800.0, 1.0 / 362880.0);
+        p = fma(-x, p, 1.0 / 40320.0);
+        p = fma(-x, p, 1.0 / 5040.0);
+        p = fma(-x, p, 1.0 / 720.0);
+        p = fma(-x, p, 1.0 / 120.0);
+        p = fma(-x, p, 1.0 / 24.0);
+        p = fma(-x, p, 1.0 / 6.0);
+        p = fma(-x, p, 0.5);
+        p = fma(-x, p, 1.0);
+        *phi = p;
+        return fma(-x, p, 1.0);
+    }
+    const double e = exp(-x);
+    *phi = (1.0 - e) / x;
+    return e;
+}
+
+// U4 propagator (MDcode/time_evolve.c:578-609) with the p^2 sum supplied;
+// iq[j] = 1/q[j].
 __host__ __device__ inline void nhc_u4(double t, int jStart, int jEnd, double S, double T, double dof,
-                                       const double *q, double *peta) {
+                                       const double *iq, double *peta) {
     int dj = 1;
     double gj = 0.0;
     if (jStart > jEnd) dj = -1;
@@ -115,13 +152,14 @@ __host__ __device__ inline void nhc_u4(double t, int jStart, int jEnd, double S,
             gj = S;
             gj -= dof * T;
         } else {
-            gj = (peta[j - 1] * peta[j - 1]) / q[j - 1] - T;
+            gj = (peta[j - 1] * peta[j - 1]) * iq[j - 1] - T;
         }
         if (j == 2) {
             peta[j] = peta[j] + t * gj;
         } else {
-            double x = t * peta[j + 1] / q[j + 1];
-            peta[j] = peta[j] * exp(-x) + t * gj * (1.0 - exp(-x)) / x;
+            double phi;
+            const double e = exp_phi(t * peta[j + 1] * iq[j + 1], &phi);
+            peta[j] = peta[j] * e + t * gj * phi;
         }
         j = j + dj;
     } while (j - dj != jEnd);
@@ -131,12 +169,13 @@ __host__ __device__ inline void nhc_u4(double t, int jStart, int jEnd, double S,
 // and :517-519); S = sum p^2 entering; returns the U3 momentum factor.
 __host__ __device__ inline double nhc_half(double S, double T, double dof, const double *q, double *eta,
                                            double *peta, double *S_out) {
-    nhc_u4(K_DT * 0.25, 2, 0, S, T, dof, q, peta);
-    double t = K_DT * 0.50;
-    double s = exp(-t * peta[0] / q[0]);                        // time_evolve.c:571
-    for (int i = 0; i < 3; i++) eta[i] = eta[i] + t * peta[i] / q[i];  // :575
+    const double iq[3] = {1.0 / q[0], 1.0 / q[1], 1.0 / q[2]};
+    nhc_u4(K_DT * 0.25, 2, 0, S, T, dof, iq, peta);
+    double t = K_DT * 0.50, phi;
+    double s = exp_phi(t * peta[0] * iq[0], &phi);                     // time_evolve.c:571
+    for (int i = 0; i < 3; i++) eta[i] = eta[i] + t * peta[i] * iq[i];  // :575
     double S2 = S * s * s;
-    nhc_u4(K_DT * 0.25, 0, 2, S2, T, dof, q, peta);
+    nhc_u4(K_DT * 0.25, 0, 2, S2, T, dof, iq, peta);
     *S_out = S2;
     return s;
 }
@@ -383,7 +422,7 @@ struct ShufArgs {
 };
 
 __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ reps, const ChainS *chain,
-                                                    const int *__restrict__ blk_rep, const int *__restrict__ blk_first,
+                                                    const BlkD *__restrict__ blkd,
                                                     double *x, double *y, double *z, double *xu, double *yu, double *zu,
                                                     double *px, double *py, double *pz, const double *__restrict__ fx,
                                                     const double *__restrict__ fy, const double *__restrict__ fz,
@@ -391,7 +430,7 @@ __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ rep
                                                     const double *__restrict__ zo, const int *__restrict__ type,
                                                     double4 *pos4, QPos *posq, int q32, ChainS *chain_w,
                                                     const int *__restrict__ blk_idx, int *cnt, int *wl_n,
-                                                    ShufArgs sa) {
+                                                    double *__restrict__ mid, ShufArgs sa) {
     __shared__ double s_scale[2];
     __shared__ double s_max[BLK / 64];
     if ((int)blockIdx.x < sa.nblk) {  // the step's shuffle: replica b / 3, component b % 3
@@ -401,7 +440,18 @@ __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ rep
         shuffle_comp(Rs, chain[rs], blockIdx.x % 3, sa.kx, sa.ky, sa.kz, 0, sa.kcap, 0, s_shuf);
         return;
     }
-    const int b = blockIdx.x - sa.nblk, r = blk_rep[b];
+    const int b = blockIdx.x - sa.nblk;
+    const BlkD D = blkd[b];
+    const int r = D.rep, i = D.first + threadIdx.x;
+    const bool valid = i < D.n;
+    const int g = D.off + (valid ? i : 0);
+    // the particle's loads, issued before lane 0's chain half and the
+    // replica's constants are waited for
+    double vx = px[g], vy = py[g], vz = pz[g];
+    const double hx = fx[g], hy = fy[g], hz = fz[g];
+    double sx = x[g], sy = y[g], sz = z[g], ux = xu[g], uy = yu[g], uz = zu[g];
+    const double ox = xo[g], oy = yo[g], oz = zo[g];
+    const int ty = type[g];
     if (b == 0 && threadIdx.x < 3) wl_n[threadIdx.x] = 0;  // rebuild work of this step
     const RepC R = reps[r];
     if (threadIdx.x == 0) {
@@ -409,25 +459,24 @@ __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ rep
         double eta[3] = {c.eta[0], c.eta[1], c.eta[2]}, peta[3] = {c.peta[0], c.peta[1], c.peta[2]}, S2;
         s_scale[0] = c.p_scale;
         s_scale[1] = (c.mode == 0 && R.n > 0) ? nhc_half(c.S_end, R.T, R.dof, c.q, eta, peta, &S2) : 1.0;
+        if (blk_idx[b] == 0)  // the chain at this point of the step, for k_force_end
+            for (int k = 0; k < 3; k++) { mid[6 * r + k] = eta[k]; mid[6 * r + 3 + k] = peta[k]; }
     }
     __syncthreads();
     // clear this replica's cell counts for a possible rebuild later in the step
     for (int c = blk_idx[b] * BLK + threadIdx.x; c < R.ncell; c += R.nblk * BLK) cnt[R.off_cell + c] = 0;
     const double ps = s_scale[0], s1 = s_scale[1];
-    const int i = blk_first[b] + threadIdx.x;
     double d2 = 0.0;
-    if (i < R.n) {
-        const int g = R.off + i;
-        double vx = px[g], vy = py[g], vz = pz[g];
+    if (valid) {
         vx = vx * ps; vy = vy * ps; vz = vz * ps;   // end-of-step U3 of the previous step
         vx = vx * s1; vy = vy * s1; vz = vz * s1;   // U3, time_evolve.c:571-573
-        vx += fx[g] * K_HALF_DT;                    // U2, :562-564
-        vy += fy[g] * K_HALF_DT;
-        vz += fz[g] * K_HALF_DT;
+        vx += hx * K_HALF_DT;                       // U2, :562-564
+        vy += hy * K_HALF_DT;
+        vz += hz * K_HALF_DT;
         px[g] = vx; py[g] = vy; pz[g] = vz;
         double dx = vx * K_DT, dy = vy * K_DT, dz = vz * K_DT;   // U1, :532-540
-        double sx = x[g] + dx * R.invL, sy = y[g] + dy * R.invL, sz = z[g] + dz * R.invL;
-        double ux = xu[g] + dx * R.invL, uy = yu[g] + dy * R.invL, uz = zu[g] + dz * R.invL;
+        sx += dx * R.invL; sy += dy * R.invL; sz += dz * R.invL;
+        ux += dx * R.invL; uy += dy * R.invL; uz += dz * R.invL;
         // applypbc1 (:15-26) loops until the coordinate is in [0,1); a
         // coordinate that is not finite or many boxes away means the run blew
         // up: flag it instead of looping
@@ -444,10 +493,10 @@ __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ rep
         x[g] = sx; y[g] = sy; z[g] = sz;
         xu[g] = ux; yu[g] = uy; zu[g] = uz;
         if (q32)
-            posq[g] = qpos(sx, sy, sz, type[g]);
+            posq[g] = qpos(sx, sy, sz, ty);
         else
-            pos4[g] = make_double4(sx, sy, sz, (double)type[g]);
-        double ex = ux - xo[g], ey = uy - yo[g], ez = uz - zo[g];  // :547-551
+            pos4[g] = make_double4(sx, sy, sz, (double)ty);
+        double ex = ux - ox, ey = uy - oy, ez = uz - oz;  // :547-551
         d2 = ex * ex + ey * ey + ez * ez;
     }
     d2 = ac4_wave_max(d2);
@@ -459,9 +508,11 @@ __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ rep
         // The maximum only grows during this kernel (it was cleared by the
         // previous step's force epilogue), so a block whose maximum is not
         // above the value it reads needs no atomic: same-address atomics are
-        // serialised across the device, one per block of a large replica.
+        // serialised across the device, one per block of a large replica.  A
+        // replica of a few blocks skips the read, whose latency would end the
+        // launch.
         const unsigned long long mb = (unsigned long long)__double_as_longlong(m);
-        if (mb > __hip_atomic_load(&chain_w[r].maxbits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        if (R.nblk <= 64 || mb > __hip_atomic_load(&chain_w[r].maxbits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             atomicMax(&chain_w[r].maxbits, mb);
     }
 }
@@ -1341,7 +1392,6 @@ struct PairAcc<false> {
     double fx = 0, fy = 0, fz = 0, pe = 0, vir = 0;
     double L2;
     double rc[2], s2c[2], e4[2], e8[2], c2i[2];  // value of species 0, difference of species 1
-    __device__ __forceinline__ void flush() {}
     __device__ __forceinline__ PairAcc(int ti, const RepC &R) {
         L2 = R.L * R.L;
         // (ti, tj) -> ab = ti + tj: sigma {1, 0.8, 0.88}, epsilon {1, 1.5, 0.5} (cell_list+forces.c:19-20)
@@ -1356,7 +1406,10 @@ struct PairAcc<false> {
         pick(8.0 * 1.0, 8.0 * 1.5, 8.0 * 0.5, e8);
         pick(K_C2 / (1.00 * 1.00), K_C2 / (0.80 * 0.80), K_C2 / (0.88 * 0.88), c2i);
     }
-    __device__ __forceinline__ void add(const double4 &pi, int, const double4 &pj, const RepC &) {
+    template <bool EN>
+    __device__ __forceinline__ void flush() {}
+    template <bool EN>
+    __device__ __forceinline__ void add(const double4 &pi, const double4 &pj) {
         double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         dx -= rint(dx);
         dy -= rint(dy);
@@ -1367,12 +1420,12 @@ struct PairAcc<false> {
             const double s2 = fma(tj, s2c[1], s2c[0]) * inv, c2 = fma(tj, c2i[1], c2i[0]);
             const double s6 = s2 * s2 * s2;
             // 4 eps [s6 (s6 - 1) + C0 + C2 (r/sigma)^2], 8 eps [6 s6 (s6 - 1/2) / r^2 - C2 / sigma^2]
-            pe = fma(fma(tj, e4[1], e4[0]), fma(s6, s6 - 1.0, fma(c2, r2, K_C0)), pe);
+            if (EN) pe = fma(fma(tj, e4[1], e4[0]), fma(s6, s6 - 1.0, fma(c2, r2, K_C0)), pe);
             const double grad = fma(tj, e8[1], e8[0]) * fma(6.0 * s6 * inv, s6 - 0.5, -c2);
             fx = fma(grad, dx, fx);
             fy = fma(grad, dy, fy);
             fz = fma(grad, dz, fz);
-            vir = fma(grad, r2, vir);
+            if (EN) vir = fma(grad, r2, vir);
         }
     }
     __device__ __forceinline__ void result(double &ox, double &oy, double &oz, const RepC &R) const {
@@ -1403,20 +1456,20 @@ struct PairAcc<true> {
     float sg2[2], e4[2], e8[2], rcq[2], c2i[2], qs2;
     __device__ __forceinline__ PairAcc(int ti, const RepC &R) {
         // (ti, tj) -> ab = ti + tj: sigma {1, 0.8, 0.88}, epsilon {1, 1.5, 0.5}
-        // (cell_list+forces.c:19-20); cutoff (r/sigma)^2 < 6.25 (:189)
+        // (cell_list+forces.c:19-20); what depends on the box comes from RepC
         qs2 = R.qs2;
-        for (int tj = 0; tj < 2; tj++) {
-            const int ab = ti + tj;
-            const double sig = ab == 0 ? 1.00 : (ab == 1 ? 0.80 : 0.88);
-            const double eps = ab == 0 ? 1.00 : (ab == 1 ? 1.50 : 0.50);
-            sg2[tj] = (float)(sig * sig);
-            e4[tj] = (float)(4.0 * eps);
-            e8[tj] = (float)(8.0 * eps);
-            rcq[tj] = (float)(K_LCUTSQR * sig * sig / (double)R.qs2);
-            c2i[tj] = (float)(K_C2 / (sig * sig));  // C2 / sigma^2
-        }
+        const auto pick = [ti](float v0, float v1, float v2, float (&out)[2]) {
+            out[0] = ti ? v1 : v0;
+            out[1] = ti ? v2 : v1;
+        };
+        pick((float)(1.00 * 1.00), (float)(0.80 * 0.80), (float)(0.88 * 0.88), sg2);
+        pick(4.0f * 1.0f, 4.0f * 1.5f, 4.0f * 0.5f, e4);
+        pick(8.0f * 1.0f, 8.0f * 1.5f, 8.0f * 0.5f, e8);
+        pick(R.rcq[0], R.rcq[1], R.rcq[2], rcq);
+        pick(R.c2i[0], R.c2i[1], R.c2i[2], c2i);
     }
-    __device__ __forceinline__ void add(const QPos &pi, int, const QPos &pj, const RepC &) {
+    template <bool EN>
+    __device__ __forceinline__ void add(const QPos &pi, const QPos &pj) {
         const float dx = (float)(int)(pi.x - pj.x);
         const float dy = (float)(int)(pi.y - pj.y);
         const float dz = (float)(int)(pi.z - pj.z);
@@ -1430,187 +1483,261 @@ struct PairAcc<true> {
             const float s6 = s2 * s2 * s2;
             // cell_list+forces.c:194-203: 4 eps [s6 (s6 - 1) + C0 + C2 (r/sigma)^2],
             // 8 eps [6 s6 (s6 - 1/2) / r^2 - C2 / sigma^2]
-            const float pterm = (b ? e4[1] : e4[0]) * __builtin_fmaf(s6, s6 - 1.0f, __builtin_fmaf(c2, r2, (float)K_C0));
             const float grad = (b ? e8[1] : e8[0]) * __builtin_fmaf(6.0f * s6 * inv, s6 - 0.5f, -c2);
             fx += (double)(grad * dx);
             fy += (double)(grad * dy);
             fz += (double)(grad * dz);
-            gpe += pterm;
-            gvir = __builtin_fmaf(grad, r2, gvir);
+            if (EN) {
+                gpe += (b ? e4[1] : e4[0]) * __builtin_fmaf(s6, s6 - 1.0f, __builtin_fmaf(c2, r2, (float)K_C0));
+                gvir = __builtin_fmaf(grad, r2, gvir);
+            }
         }
     }
+    template <bool EN>
     __device__ __forceinline__ void flush() {
-        pe += (double)gpe; vir += (double)gvir;
-        gpe = gvir = 0.f;
+        if (EN) {
+            pe += (double)gpe; vir += (double)gvir;
+            gpe = gvir = 0.f;
+        }
     }
-    __device__ __forceinline__ void result(double &ox, double &oy, double &oz, const RepC &R) {
-        flush();
+    __device__ __forceinline__ void result(double &ox, double &oy, double &oz, const RepC &R) const {
         ox = fx * R.qscale;
         oy = fy * R.qscale;
         oz = fz * R.qscale;
     }
 };
 
-// Four consecutive 16-byte-aligned list entries as one 16-byte load.  (A
-// nontemporal load here measured 79 against 56 us per k_force launch on the
-// 64-replica ensemble: the list stream is better served by the caches.)
-typedef int ac4_v4i __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ int4 ld_list4(const int *p) {
-    const ac4_v4i v = *(const ac4_v4i *)p;
-    return make_int4(v.x, v.y, v.z, v.w);
+// The particle's position at slot j; a 32-bit byte offset for the 12-byte
+// records (a handle of 2^32 / 12 slots does not fit the memory).
+__device__ __forceinline__ QPos ld_pos(const QPos *p, int j) {
+    const unsigned u = (unsigned)j;
+    return *(const QPos *)((const char *)p + (size_t)(u * 12u));
+}
+__device__ __forceinline__ double4 ld_pos(const double4 *p, int j) { return p[j]; }
+
+// Sum over each aligned group of 2^lw lanes (2^lw <= 16), in every lane of it:
+// lane exchanges within a row of 16 (quad permutes, then mirrors of the half
+// row and of the row, whose quads already agree).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double team_sum(double v, int lw) {
+    if (lw > 0) v = dpp_add<0xB1>(v);   // quad_perm 1 0 3 2
+    if (lw > 1) v = dpp_add<0x4E>(v);   // quad_perm 2 3 0 1
+    if (lw > 2) v = dpp_add<0x141>(v);  // row_half_mirror
+    if (lw > 3) v = dpp_add<0x140>(v);  // row_mirror
+    return v;
+}
+// Sum over the wave, the same in every lane, in a fixed order: the rows of
+// 16 lanes, then the four rows.
+__device__ __forceinline__ double wave_sum_rows(double v) {
+    v = team_sum(v, 4);
+    double r[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        r[k] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 16 * k),
+                                __builtin_amdgcn_readlane(__double2loint(v), 16 * k));
+    return (r[0] + r[1]) + (r[2] + r[3]);
 }
 
-// One lane per particle: the list walk in groups of C entries (C/8 list
-// chunks of two 16-byte index loads each), the indices of the next group
-// loaded while this group's positions are gathered; entries at or past m are
-// replaced by the particle itself before they are used as an index.
-template <int C>
-__device__ __forceinline__ void ld_idx(const int *lp, size_t cst, int k, int m, int g, int (&j)[C]) {
+// VEC consecutive list entries in one load.  (A nontemporal load of the list
+// measured 79 against 56 us per k_force launch on the 64-replica ensemble:
+// the list stream is better served by the caches.)
+template <int VEC>
+__device__ __forceinline__ void ld_list(const int *p, int *j) {
+    if (VEC == 1) {
+        j[0] = p[0];
+    } else if (VEC == 2) {
+        const int2 a = *(const int2 *)p;
+        j[0] = a.x; j[1] = a.y;
+    } else {
 #pragma unroll
-    for (int c = 0; c < C / 8; c++) {
-        if (k + 8 * c < m) {  // this list chunk holds entries
-            const int *p = lp + (size_t)(k / 8 + c) * cst;
-            const int4 a = ld_list4(p), b = ld_list4(p + 4);
-            j[8 * c + 0] = a.x; j[8 * c + 1] = a.y; j[8 * c + 2] = a.z; j[8 * c + 3] = a.w;
-            j[8 * c + 4] = b.x; j[8 * c + 5] = b.y; j[8 * c + 6] = b.z; j[8 * c + 7] = b.w;
-        } else {
-#pragma unroll
-            for (int u = 0; u < 8; u++) j[8 * c + u] = g;
+        for (int q = 0; q < VEC; q += 4) {
+            const int4 a = *(const int4 *)(p + q);
+            j[q] = a.x; j[q + 1] = a.y; j[q + 2] = a.z; j[q + 3] = a.w;
         }
     }
 }
-template <int C, class PosT, class Acc>
-__device__ __forceinline__ void walk_list1(const RepC &R, const int *lp, int m, int g, const PosT *__restrict__ pos,
-                                           const PosT &pi, int ti, Acc &acc) {
-    const size_t cst = (size_t)R.n * 8;
-    if (m <= 0) return;
-    int j[C];
-    PosT q[C];
-    ld_idx<C>(lp, cst, 0, m, g, j);
-    for (int k = 0; k < m; k += C) {
+
+// A team's walk of particle g's list of m entries, eight entries per lane and
+// group: the positions of a group are gathered together while the indices of
+// the next are loaded; the last, partial group has its loads issued together
+// too (an entry past m is replaced by g before it is used as an index).
+// VEC = 1: lane t of W takes entries t, t + W, ... (row c of the walk is
+// entries c*W ... c*W + W - 1, cs list words apart); the others read chunks
+// of 8 entries, cs words apart, with W = 8 / |VEC| lanes: VEC > 1 takes VEC
+// consecutive entries of a chunk in one load, VEC < -1 entries t, t + W, ...
+// of it, |VEC| rows per chunk.
+template <int VEC, bool EN, class PosT, class Acc>
+__device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t, int m, int g,
+                                          const PosT *__restrict__ pos, const PosT &pi, Acc &acc) {
+    constexpr int V = VEC > 1 ? VEC : 1;    // entries of a load
+    constexpr int RC = VEC < 0 ? -VEC : 1;  // rows per step of cs
+    constexpr int NR = 8 / V;               // rows of a group
+    const int rl = W * V, full = m / rl;    // entries of a row, whole rows
+    int c = 0, jn[8];
+    if (NR <= full) {
 #pragma unroll
-        for (int u = 0; u < C; u++) q[u] = pos[k + u < m ? j[u] : g];
-        if (k + C < m) ld_idx<C>(lp, cst, k + C, m, g, j);
+        for (int r = 0; r < NR; r++) ld_list<V>(lp + (r / RC) * cs + (r % RC) * W, jn + V * r);
+    }
+    while (c + NR <= full) {
+        PosT q[8];
 #pragma unroll
-        for (int u = 0; u < C; u++)
-            if (k + u < m) acc.add(pi, ti, q[u], R);
-        acc.flush();
+        for (int u = 0; u < 8; u++) q[u] = ld_pos(pos, jn[u]);
+        c += NR;
+        lp += (NR / RC) * cs;
+        if (c + NR <= full) {
+#pragma unroll
+            for (int r = 0; r < NR; r++) ld_list<V>(lp + (r / RC) * cs + (r % RC) * W, jn + V * r);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc.template add<EN>(pi, q[u]);
+        acc.template flush<EN>();
+    }
+    const int k0 = c * rl + t * V;  // this lane's first entry of the last group
+    if (k0 < m) {
+        int jt[8];
+        PosT q[8];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            int *j = jt + V * r;
+            if (k0 + r * rl < m) {
+                ld_list<V>(lp + (r / RC) * cs + (r % RC) * W, j);
+            } else {
+#pragma unroll
+                for (int v = 0; v < V; v++) j[v] = g;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) q[u] = ld_pos(pos, k0 + (u / V) * rl + u % V < m ? jt[u] : g);
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (k0 + (u / V) * rl + u % V < m) acc.template add<EN>(pi, q[u]);
+        acc.template flush<EN>();
     }
 }
 
-// Pair forces: a team of tpp lanes per particle (tpp is fixed per handle at
-// creation, so a replica's results do not depend on what else is loaded) walks the particle's
-// list with stride tpp, 8 independent index/position loads in flight per lane;
-// the team's partial forces are combined by a fixed butterfly.  Each block
-// writes its partial sums of p^2, PE, virial and p_x; k_force_end reduces
-// them per replica.
-template <bool FP32, bool KICK>
-__global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps,
-                                               const int *__restrict__ fblk_rep, const int *__restrict__ fblk_first,
+// Pair forces: a team of W = 2^lw lanes per particle (fixed per handle at
+// creation, so a replica's results do not depend on what else is loaded)
+// walks the particle's list (walk_list); the team's partial forces are
+// combined by a fixed butterfly.  Each block writes its partial sums of p^2
+// and p_x, and with EN of PE and virial; k_force_end reduces them per
+// replica.  A block's loads form a short chain (block table, then position,
+// list length, active index and momentum together, then list, then
+// neighbour positions): on small boxes, a few waves per CU, the launch is as
+// long as that chain.  Each loaded where it was used, with the constants
+// divided out per lane and the sums shuffled through LDS: 7.2 us at N=1000
+// FP64 and 11.0 at N=10000 FP32 (four lanes); this 5.9 and 7.0 (sixteen).
+// EN = false leaves out the pair energy and virial, which every step
+// overwrites and only the call's last one reports: 9 of 55 instructions of
+// an FP32 pair.  (FP32 handles whose team is not the list layout's form them in
+// k_energy.)
+template <bool FP32, bool KICK, bool EN, int VEC>
+__global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, const BlkD *__restrict__ fblk,
                                                const double4 *__restrict__ pos4, const QPos *__restrict__ posq,
                                                const int *__restrict__ nn,
-                                               const int *__restrict__ nl, int cap, const int *__restrict__ act,
+                                               const int *__restrict__ nl, int cap, int lw, int lc,
+                                               const int *__restrict__ act,
                                                const int8_t *__restrict__ kx, const int8_t *__restrict__ ky,
                                                const int8_t *__restrict__ kz, double *fx, double *fy, double *fz,
                                                double *px, double *py, double *pz, double *partial, int nb) {
     __shared__ double s_red[4][BLK / 64];
     const int b = xcd_block(nb);
     if (b < 0) return;
-    const int r = fblk_rep[b];
-    const RepC R = reps[r];
-    const int tpp = R.tpp, t = threadIdx.x & (tpp - 1);
-    const int i = fblk_first[b] + threadIdx.x / tpp;
+    const BlkD D = fblk[b];
+    const int W = 1 << lw, t = threadIdx.x & (W - 1);
+    const int i = D.first + (threadIdx.x >> lw);
     double v_p2 = 0.0, v_pe = 0.0, v_vir = 0.0, v_px = 0.0;
     double Fx = 0.0, Fy = 0.0, Fz = 0.0;
-    const bool valid = i < R.n;
-    const int g = R.off + (valid ? i : 0);
+    const bool valid = i < D.n;
+    const int g = D.off + (valid ? i : 0);
     // FP64: the wrapped box fractions; FP32: their fixed-point copy
     using PosT = typename std::conditional<FP32, QPos, double4>::type;
     const PosT *__restrict__ pos = (const PosT *)(FP32 ? (const void *)posq : (const void *)pos4);
-    if (valid) {
-        const PosT pi = pos[g];
-        const int ti = ptype(pi);
-        PairAcc<FP32> acc(ti, R);
-        const int m = nn[g];
-        if (R.tpp == 1) {
-            walk_list1<8>(R, nl + nl_at(R, cap, 0, i), m, g, pos, pi, ti, acc);
-            acc.result(Fx, Fy, Fz, R);
-            v_pe = acc.pe;
-            v_vir = acc.vir;
-        } else {
-        // entry t + c*tpp of particle i: chunk c of the replica's region
-        const int *lp = nl + nl_at(R, cap, t, i);
-        const size_t cstep = (size_t)R.n << R.ltpp;
-        int k = t;
-        // groups of 8 entries; the indices of the next group are loaded
-        // while the positions of the current one are in flight
-        int jn[8];
-        if (k + 7 * tpp < m) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) jn[u] = lp[u * cstep];
-        }
-        while (k + 7 * tpp < m) {
-            PosT q[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) q[u] = pos[jn[u]];
-            k += 8 * tpp;
-            lp += 8 * cstep;
-            if (k + 7 * tpp < m) {
-#pragma unroll
-                for (int u = 0; u < 8; u++) jn[u] = lp[u * cstep];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc.add(pi, ti, q[u], R);
-            acc.flush();
-        }
-        if (k < m) {  // the last, partial group: its loads issued together, the adds in list order
-            int jt[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) jt[u] = k + u * tpp < m ? lp[u * cstep] : g;
-            PosT q[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) q[u] = pos[jt[u]];
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (k + u * tpp < m) acc.add(pi, ti, q[u], R);
-        }
-        acc.result(Fx, Fy, Fz, R);
-        v_pe = acc.pe;
-        v_vir = acc.vir;
-        }
-    }
-    for (int o = 1; o < tpp; o <<= 1) {  // team butterfly (teams are aligned lane groups)
-        Fx += __shfl_xor(Fx, o, 64);
-        Fy += __shfl_xor(Fy, o, 64);
-        Fz += __shfl_xor(Fz, o, 64);
-    }
+    const PosT pi = ld_pos(pos, g);
+    const int m = valid ? nn[g] : 0;
+    const int a = act[g];
+    double vx = 0.0, vy = 0.0, vz = 0.0;
+    if (KICK) { vx = px[g]; vy = py[g]; vz = pz[g]; }
+    const RepC &R = reps[D.rep];
+    const bool active = a >= 0;
+    const int ka = R.off_act + (active ? a : 0);
+    const double kfx = (double)kx[ka], kfy = (double)ky[ka], kfz = (double)kz[ka];
+    PairAcc<FP32> acc(ptype(pi), R);
+    // entry e of particle i's list (nl_at): VEC = 1, W >= 2^lc, rows of W
+    // entries are W * n words apart; else the chunks of 8 entries, 8 * n
+    const size_t e0 = (size_t)(VEC > 1 ? t * VEC : t);
+    const int *lp = nl + (size_t)D.off * cap + ((((e0 >> lc) * D.n + (g - D.off)) << lc) + (e0 & ((1u << lc) - 1u)));
+    walk_list<VEC, EN>(lp, (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, pos, pi, acc);
+    acc.result(Fx, Fy, Fz, R);
+    v_pe = acc.pe;
+    v_vir = acc.vir;
+    Fx = team_sum(Fx, lw);
+    Fy = team_sum(Fy, lw);
+    Fz = team_sum(Fz, lw);
     if (valid && t == 0) {
-        const int a = act[g];
-        if (a != -1) {  // cell_list+forces.c:207-213
-            Fx += R.f0 * (double)kx[R.off_act + a];
-            Fy += R.f0 * (double)ky[R.off_act + a];
-            Fz += R.f0 * (double)kz[R.off_act + a];
+        if (active) {  // cell_list+forces.c:207-213
+            Fx += R.f0 * kfx;
+            Fy += R.f0 * kfy;
+            Fz += R.f0 * kfz;
         }
         fx[g] = Fx; fy[g] = Fy; fz[g] = Fz;
         if (KICK) {  // U2 after the forces, time_evolve.c:516
-            double vx = px[g] + Fx * K_HALF_DT, vy = py[g] + Fy * K_HALF_DT, vz = pz[g] + Fz * K_HALF_DT;
+            vx += Fx * K_HALF_DT; vy += Fy * K_HALF_DT; vz += Fz * K_HALF_DT;
             px[g] = vx; py[g] = vy; pz[g] = vz;
             v_p2 = vx * vx + vy * vy + vz * vz;
             v_px = vx;
         }
     }
-    double v[4] = {v_p2, v_pe, v_vir, v_px};
+    const double v[4] = {v_p2, v_pe, v_vir, v_px};
+#pragma unroll
     for (int q = 0; q < 4; q++) {
-        double w = ac4_wave_sum(v[q]);
+        if (!EN && (q == 1 || q == 2)) continue;
+        const double w = wave_sum_rows(v[q]);
         if ((threadIdx.x & 63) == 0) s_red[q][threadIdx.x >> 6] = w;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < 4; q++) {
-            double s = 0.0;
-            for (int w = 0; w < BLK / 64; w++) s += s_red[q][w];
-            partial[4 * (size_t)b + q] = s;
-        }
+    if (threadIdx.x < 4 && (EN || threadIdx.x == 0 || threadIdx.x == 3)) {
+        double s = 0.0;
+        for (int w = 0; w < BLK / 64; w++) s += s_red[threadIdx.x][w];
+        partial[4 * (size_t)b + threadIdx.x] = s;
+    }
+}
+
+// Pair energy and virial of FP32 handles whose force team is not the list
+// layout's team of 2^lw lanes: that team walks the list (entries t, t + W, ...;
+// one lane: chunks of 8) and sums the FP32 terms of eight entries before it
+// widens them, so the partial sums, whose rounding shows in the seventh to
+// ninth digit of the energy, do not depend on the force kernel's width.  Runs
+// once per call, after its last step (k_energy_end then completes the step's
+// reported values).
+template <int VEC>
+__global__ void __launch_bounds__(BLK) k_energy(const RepC *__restrict__ reps, const BlkD *__restrict__ eblk,
+                                                const QPos *__restrict__ posq, const int *__restrict__ nn,
+                                                const int *__restrict__ nl, int cap, int lw, double *epart, int nb) {
+    __shared__ double s_red[2][BLK / 64];
+    const int b = xcd_block(nb);
+    if (b < 0) return;
+    const BlkD D = eblk[b];
+    const int W = 1 << lw, t = threadIdx.x & (W - 1), i = D.first + (threadIdx.x >> lw);
+    const bool valid = i < D.n;
+    const int il = valid ? i : 0, g = D.off + il;
+    const QPos pi = ld_pos(posq, g);
+    const int m = valid ? nn[g] : 0;
+    PairAcc<true> acc(ptype(pi), reps[D.rep]);
+    walk_list<VEC, true>(nl + (size_t)D.off * cap + (size_t)il * (VEC == 1 ? W : 8) + t,
+                         (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, posq, pi, acc);
+    const double v[2] = {wave_sum_rows(acc.pe), wave_sum_rows(acc.vir)};
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < 2; q++) s_red[q][threadIdx.x >> 6] = v[q];
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double s = 0.0;
+        for (int w = 0; w < BLK / 64; w++) s += s_red[threadIdx.x][w];
+        epart[2 * (size_t)b + threadIdx.x] = s;
     }
 }
 
@@ -1624,19 +1751,31 @@ __global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps,
 // invalidates the L2 of the block's XCD (buffer_wbl2 / buffer_inv), and the
 // invalidations cost the neighbour gathers of every other block their L2
 // hits (k_force 55.6 -> 42.3 us on the 64-replica ensemble without them).
-template <bool KICK>
+// EN: the pass summed the pair energy and virial (the last step of a call;
+// they are only reported).  apart: k_energy forms them after the call's last
+// step, and Heff is stored without the pair energy for it.
+template <bool KICK, bool EN>
 __global__ void __launch_bounds__(256) k_force_end(const RepC *__restrict__ reps, ChainS *chain,
-                                                   const double *__restrict__ partial) {
+                                                   const double *__restrict__ partial, int apart,
+                                                   const double *__restrict__ mid) {
     __shared__ double s_w[4][4];
     const int r = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, nt = blockDim.x;
     const RepC R = reps[r];
+    ChainS &c = chain[r];
+    ChainS c0;           // loaded beside the partials, not after them
+    double eta[3], peta[3];  // after the start-of-step half (k_first_half)
+    if (KICK && threadIdx.x == 0) {
+        c0 = c;
+        for (int k = 0; k < 3; k++) { eta[k] = mid[6 * r + k]; peta[k] = mid[6 * r + 3 + k]; }
+    }
     double a4[4] = {0.0, 0.0, 0.0, 0.0};
     for (int k = threadIdx.x; k < R.fnblk; k += nt) {  // thread t: blocks t, t+nt, ...
         const double *pp = partial + 4 * (size_t)(R.fblk_off + k);
-        a4[0] += pp[0]; a4[1] += pp[1]; a4[2] += pp[2]; a4[3] += pp[3];
+        a4[0] += pp[0]; a4[3] += pp[3];
+        if (EN) { a4[1] += pp[1]; a4[2] += pp[2]; }
     }
     for (int q = 0; q < 4; q++)
-        for (int o = 1; o < 64; o <<= 1) a4[q] += __shfl_xor(a4[q], o, 64);
+        if (EN || q == 0 || q == 3) a4[q] = wave_sum_rows(a4[q]);
     if (lane == 0)
         for (int q = 0; q < 4; q++) s_w[w][q] = a4[q];
     __syncthreads();
@@ -1645,67 +1784,101 @@ __global__ void __launch_bounds__(256) k_force_end(const RepC *__restrict__ reps
         a4[q] = s_w[0][q];
         for (int k = 1; k < nt / 64; k++) a4[q] += s_w[k][q];
     }
-    ChainS &c = chain[r];
     if (R.n == 0) return;  // idle slot
-    double S = a4[0], pe = a4[1], vir = a4[2], spx = a4[3];
+    double S = a4[0], pe = a4[1], vir = a4[2], spx = a4[3];  // pe, vir: zero without EN
     pe = 0.5 * pe;                  // every pair seen from both sides
     vir = (0.5 * vir) / (3.0e0);   // cell_list+forces.c:220
-    c.pe = pe;
-    c.vir = vir;
+    if (EN) {
+        c.pe = pe;
+        c.vir = vir;
+    }
     if (!KICK) return;
-    const bool rebuilt = need_rebuild(R, c);
-    if (c.mode == 2) {
+    const bool rebuilt = need_rebuild(R, c0);
+    if (c0.mode == 2) {
         // NVE: plain velocity Verlet (AdvanceTimeNVE, MDcode/time_evolve.c:39-171,
         // same U2-U1-F-U2 order as the thermostatted step), Heff = KE + PE
         c.p_scale = 1.0;
         c.S_end = S;
-        c.ke = S * 0.5;
-        c.inst_T = 2.0 * c.ke / R.dof;
+        const double ke = S * 0.5;
+        c.ke = ke;
+        c.inst_T = 2.0 * ke / R.dof;
         c.drift = spx;
-        c.heff = c.ke + pe;
-        if (rebuilt) c.rebuilds += 1;
+        if (EN || apart) c.heff = ke + pe;
+        if (rebuilt) c.rebuilds = c0.rebuilds + 1;
         c.maxbits = 0ull;
         c.force_rebuild = 0;
-        if (R.tau > 0 && c.step % R.tau == 0) c.shuffles += 1;  // k_shuffle ran this step
-        c.step += 1;
+        if (R.tau > 0 && c0.step % R.tau == 0) c.shuffles = c0.shuffles + 1;  // k_shuffle ran this step
+        c.step = c0.step + 1;
         return;
     }
-    if (c.mode == 1) {
+    if (c0.mode == 1) {
         // coldstart/breakxal of MDcode/initialise.c:166-201: momenta rescaled
         // to a ramped target temperature every step, no thermostat chain
-        const double f = c.ramp_n > 1 ? c.ramp0 + (c.ramp1 - c.ramp0) * (double)c.ramp_k / (double)(c.ramp_n - 1)
-                                      : c.ramp1;
+        const double f = c0.ramp_n > 1 ? c0.ramp0 + (c0.ramp1 - c0.ramp0) * (double)c0.ramp_k / (double)(c0.ramp_n - 1)
+                                       : c0.ramp1;
         const double s2 = S > 0.0 ? sqrt(R.T * f * R.dof / S) : 1.0;
         c.p_scale = s2;
-        c.S_end = S * s2 * s2;
-        c.ke = c.S_end * 0.5;
-        c.inst_T = 2.0 * c.ke / R.dof;
+        const double Se = S * s2 * s2, ke = Se * 0.5;
+        c.S_end = Se;
+        c.ke = ke;
+        c.inst_T = 2.0 * ke / R.dof;
         c.drift = spx * s2;
-        c.heff = c.ke + pe;
-        if (++c.ramp_k >= c.ramp_n) c.mode = 0;
-        if (rebuilt) c.rebuilds += 1;
+        if (EN || apart) c.heff = ke + pe;
+        c.ramp_k = c0.ramp_k + 1;
+        if (c0.ramp_k + 1 >= c0.ramp_n) c.mode = 0;
+        if (rebuilt) c.rebuilds = c0.rebuilds + 1;
         c.maxbits = 0ull;
         c.force_rebuild = 0;
         return;
     }
-    double eta[3] = {c.eta[0], c.eta[1], c.eta[2]}, peta[3] = {c.peta[0], c.peta[1], c.peta[2]}, S2;
-    nhc_half(c.S_end, R.T, R.dof, c.q, eta, peta, &S2);   // start of step (same values as k_first_half)
-    double s2 = nhc_half(S, R.T, R.dof, c.q, eta, peta, &S2);  // end of step, time_evolve.c:517-519
+    double S2;
+    const double s2 = nhc_half(S, R.T, R.dof, c0.q, eta, peta, &S2);  // end of step, time_evolve.c:517-519
     for (int k = 0; k < 3; k++) { c.eta[k] = eta[k]; c.peta[k] = peta[k]; }
+    const double ke = S2 * 0.5;      // time_evolve.c:520
     c.S_end = S2;
     c.p_scale = s2;
-    c.ke = S2 * 0.5;                 // time_evolve.c:520
-    c.inst_T = 2.0 * c.ke / R.dof;   // :524
+    c.ke = ke;
+    c.inst_T = 2.0 * ke / R.dof;     // :524
     c.drift = spx * s2;
-    double heff = c.ke + pe + eta[0] * R.T * R.dof;  // print.c:85-87
-    for (int k = 0; k < 3; k++) heff = heff + peta[k] * peta[k] / (2.0 * c.q[k]);
-    for (int k = 1; k < 3; k++) heff = heff + R.T * eta[k];
-    c.heff = heff;
-    if (rebuilt) c.rebuilds += 1;
+    if (EN || apart) {
+        double heff = ke + pe + eta[0] * R.T * R.dof;  // print.c:85-87
+        for (int k = 0; k < 3; k++) heff = heff + peta[k] * peta[k] / (2.0 * c0.q[k]);
+        for (int k = 1; k < 3; k++) heff = heff + R.T * eta[k];
+        c.heff = heff;
+    }
+    if (rebuilt) c.rebuilds = c0.rebuilds + 1;
     c.maxbits = 0ull;
     c.force_rebuild = 0;
-    if (R.tau > 0 && c.step % R.tau == 0) c.shuffles += 1;  // k_shuffle ran this step
-    c.step += 1;
+    if (R.tau > 0 && c0.step % R.tau == 0) c.shuffles = c0.shuffles + 1;  // k_shuffle ran this step
+    c.step = c0.step + 1;
+}
+
+// After k_energy, one workgroup per replica: its energy and virial, and with
+// step the pair energy in Heff (k_force_end stored it without).
+__global__ void __launch_bounds__(256) k_energy_end(const RepC *__restrict__ reps, ChainS *chain,
+                                                    const double *__restrict__ epart, int step) {
+    __shared__ double s_w[2][4];
+    const int r = blockIdx.x, w = threadIdx.x >> 6;
+    const RepC &R = reps[r];
+    if (R.n == 0) return;  // idle slot
+    double pe = 0.0, vir = 0.0;
+    for (int k = threadIdx.x; k < R.enblk; k += 256) {
+        const double *pp = epart + 2 * (size_t)(R.eblk_off + k);
+        pe += pp[0];
+        vir += pp[1];
+    }
+    pe = wave_sum_rows(pe);
+    vir = wave_sum_rows(vir);
+    if ((threadIdx.x & 63) == 0) { s_w[0][w] = pe; s_w[1][w] = vir; }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < 4; k++) { pe += s_w[0][k]; vir += s_w[1][k]; }
+    pe = 0.5 * pe;                 // every pair seen from both sides
+    vir = (0.5 * vir) / (3.0e0);  // cell_list+forces.c:220
+    ChainS &c = chain[r];
+    c.pe = pe;
+    c.vir = vir;
+    if (step) c.heff = c.heff + pe;
 }
 
 // ------------------------------------------------------------- host side
@@ -1715,7 +1888,13 @@ struct ac4_md {
     std::vector<RepC> reps_h;
     RepC *reps = nullptr;
     ChainS *chain = nullptr;
-    int *blk_rep = nullptr, *blk_first = nullptr, *blk_idx = nullptr, *fblk_rep = nullptr, *fblk_first = nullptr;
+    int *blk_rep = nullptr, *blk_first = nullptr, *blk_idx = nullptr;
+    BlkD *blkd = nullptr, *fblk = nullptr;  // particle blocks (k_first_half) and force blocks
+    bool en_apart = false;  // the energy in a pass of its own (k_energy), with the list layout's team:
+    BlkD *eblk = nullptr;   // its block table,
+    double *epart = nullptr;  // its partial sums {pe, virial} per block,
+    int enblk = 0, elw = 0;   // its blocks, log2 of its lanes per particle
+    int lw = 0, lc = 3, vec = 1;  // force teams: log2 lanes, log2 list chunk, list reading (k_force's VEC)
     int *cblk_rep = nullptr, *cblk_cell = nullptr;
     int fnblk = 0, lnblk = 0, ncb = 0;
     int shuf_kcap = 0;     // largest Nact whose directions k_shuffle keeps in LDS
@@ -1729,6 +1908,7 @@ struct ac4_md {
     int *xmid = nullptr;                       // per cell: first slot of its upper x-half
     int *lblk_rep = nullptr, *lblk_first = nullptr;  // list-build block table (LPB particles per block)
     double *partial = nullptr;
+    double *mid = nullptr;  // per replica: the chain's eta, p_eta after the start-of-step half
     PartArrays P{}, A{};  // primary and permutation scratch
     void **ftab = nullptr;  // their pointers on the device (PART_FIELDS of P, then of A)
     double *fx = nullptr, *fy = nullptr, *fz = nullptr, *xo = nullptr, *yo = nullptr, *zo = nullptr;
@@ -1744,7 +1924,7 @@ struct ac4_md {
     long long *ov_step = nullptr;
     // block tables of every slot, in slot order, with each slot's first
     // entry: the launch grids cover only the occupied slots (refresh_tables)
-    std::vector<int> t_brep, t_bfirst, t_bidx, t_frep, t_ffirst, t_lrep, t_lfirst, t_b0, t_f0, t_l0;
+    std::vector<int> t_brep, t_bfirst, t_bidx, t_ffirst, t_lrep, t_lfirst, t_b0, t_f0, t_l0;
     int *ov_list = nullptr;     // replica list of ac4_md_overlap_chi4
     double *ov_out = nullptr;   // its per-lag results
     // frame text on the device (ac4_md_format_frame): 80-byte line slots in
@@ -1802,6 +1982,25 @@ static void free_parts(PartArrays &a) {
 // 0 = one wave per cell, 1 = one thread per particle, 2/3/4 = teams of
 // 16/32/64 lanes per particle.
 #define TPP_LANES 65536.0
+
+// Lanes per particle of the force kernel where they are not pinned, by the
+// handle's total capacity: enough waves to hide the gathers on small handles,
+// few enough that a particle's constants and sums are not paid for by too
+// many lanes.  us per graph-replayed step of one box, at 1 / 2 / 4 / 8 / 16
+// lanes (each with the list layout of that width):
+//   FP32  10000: 32.8 28.7 24.5 23.2 22.6    20000: 41.0 36.3 33.2 32.2 32.5
+//         50000: 49.2 47.7 45.7 45.4 48.4   100000: 64.5 64.9 63.6 64.5 71.9
+//        200000: 92.3 86.7 85.5 91.4  106   500000:  210  200  202  222  270
+//   FP64  10000: 39.9 30.5 25.5 24.5 23.7    20000: 47.8 38.1 35.7 33.7 35.1
+//         50000: 56.6 52.1 51.2 51.9 56.6   100000: 79.7 75.9 72.0 78.3 87.2
+//        200000:  121  113  106  121  143   500000:  288  252  252  292  361
+// On large FP32 handles two lanes reading four entries of a chunk at a time
+// (k_force, VEC = 4) take 194 at 500000; one lane was the rule before.
+static int force_width(double cap_tot, int prec) {
+    if (cap_tot <= 14000.0) return 16;
+    if (cap_tot <= 32768.0) return 8;
+    return prec == AC4_FP32 && cap_tot > 160000.0 ? 2 : 4;
+}
 static int g_tpp = 0, g_nlist_mode = 3;
 static double g_skin = K_SKIN;
 
@@ -1851,6 +2050,11 @@ static const char *configure_rep(RepC &R, const ac4_replica_params &q) {
     if (R.ncell > R.cap_cells) return "density below the slot's cell capacity (0.5)";
     R.qscale = R.L / 4294967296.0;
     R.qs2 = (float)(R.qscale * R.qscale);
+    for (int ab = 0; ab < 3; ab++) {  // cutoff (r/sigma)^2 < 6.25 (cell_list+forces.c:189)
+        const double sig = ab == 0 ? 1.00 : (ab == 1 ? 0.80 : 0.88);
+        R.rcq[ab] = (float)(K_LCUTSQR * sig * sig / (double)R.qs2);
+        R.c2i[ab] = (float)(K_C2 / (sig * sig));
+    }
     R.tau = q.tau_per;
     R.T = q.T;
     R.f0 = q.f0;
@@ -1890,7 +2094,8 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     md->prec = precision;
     md->nlist_mode = g_nlist_mode;
     int off = 0, off_act = 0, off_cell = 0, blk_off = 0, fblk_off = 0;
-    std::vector<int> brep, bfirst, bidx, frep, ffirst, crep, ccell, lrep, lfirst;
+    std::vector<int> brep, bfirst, bidx, ffirst, crep, ccell, lrep, lfirst;
+    std::vector<BlkD> bd, fd;
     int ncb = 0;
     AC4_REQUIRE(nslots < 32768, AC4_EARG, "at most 32767 slots");
     double cap_tot = 0.0;
@@ -1902,6 +2107,20 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         while (tpp < 16 && cap_tot * tpp * 2 <= TPP_LANES) tpp *= 2;
     }
     while ((1 << ltpp) < tpp) ltpp++;
+    // lanes per particle in the force kernel: the pinned width, else by the
+    // handle's total capacity (FORCE_W)
+    const int W = g_tpp ? tpp : std::max(tpp > 1 ? tpp : 1, force_width(cap_tot, precision));
+    while ((1 << md->lw) < W) md->lw++;
+    md->en_apart = precision == AC4_FP32 && W != tpp;
+    md->elw = ltpp;
+    md->lc = tpp == 1 ? 3 : ltpp;
+    // a chunk of 8 entries read by fewer lanes: FP32 teams take consecutive
+    // entries in one load each; FP64 teams (and more than one lane) take
+    // every W-th, so that the lanes of a gather are on neighbouring entries:
+    // the 32-byte records of four are one or two lines (N=100000, four lanes:
+    // 72 against 79 us per step), the 12-byte ones mostly one either way
+    md->vec = W < (1 << md->lc) ? (1 << md->lc) / W : 1;
+    if (precision == AC4_FP64 && W > 1 && md->vec > 1) md->vec = -md->vec;
     for (int r = 0; r < nslots; r++) {
         RepC R;
         memset(&R, 0, sizeof R);
@@ -1922,11 +2141,13 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         R.lc = tpp == 1 ? 3 : ltpp;
         R.nblk = (cn + BLK - 1) / BLK;
         R.blk_off = blk_off;
-        for (int k = 0; k < R.nblk; k++) { brep.push_back(r); bfirst.push_back(k * BLK); bidx.push_back(k); }
-        const int ppb = BLK / R.tpp;  // particles per force block
+        for (int k = 0; k < R.nblk; k++) { brep.push_back(r); bfirst.push_back(k * BLK); bidx.push_back(k); bd.push_back(BlkD{r, k * BLK, off, 0}); }
+        const int ppb = BLK / W;  // particles per force block
         R.fnblk = (cn + ppb - 1) / ppb;
         R.fblk_off = fblk_off;
-        for (int k = 0; k < R.fnblk; k++) { frep.push_back(r); ffirst.push_back(k * ppb); }
+        for (int k = 0; k < R.fnblk; k++) { ffirst.push_back(k * ppb); fd.push_back(BlkD{r, k * ppb, off, 0}); }
+        R.enblk = md->en_apart ? (cn * tpp + BLK - 1) / BLK : 0;
+        md->enblk += R.enblk;
         R.lblk_off = (int)lrep.size();
         R.lnblk = (cn + LPB - 1) / LPB;
         for (int k = 0; k < R.lnblk; k++) { lrep.push_back(r); lfirst.push_back(k * LPB); }
@@ -1943,7 +2164,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         md->reps_h.push_back(R);  // idle: n = 0
     }
     md->t_brep = brep; md->t_bfirst = bfirst; md->t_bidx = bidx;
-    md->t_frep = frep; md->t_ffirst = ffirst; md->t_lrep = lrep; md->t_lfirst = lfirst;
+    md->t_ffirst = ffirst; md->t_lrep = lrep; md->t_lfirst = lfirst;
     for (const RepC &R : md->reps_h) {
         md->t_b0.push_back(R.blk_off);
         md->t_f0.push_back(R.fblk_off);
@@ -1985,8 +2206,9 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         ALLOC(shuf_ent_n, (size_t)nslots * 3 * md->shuf_bmax)
     }
     ALLOC(reps, nslots) ALLOC(chain, nslots) ALLOC(blk_rep, md->nblk) ALLOC(blk_first, md->nblk) ALLOC(blk_idx, md->nblk)
-    ALLOC(fblk_rep, md->fnblk) ALLOC(fblk_first, md->fnblk) ALLOC(lblk_rep, md->lnblk) ALLOC(lblk_first, md->lnblk)
-    ALLOC(wl_item, (size_t)md->nblk + md->lnblk + md->ncb) ALLOC(wl_n, 4) ALLOC(ranges, (size_t)off_cell * NRANGE) ALLOC(xmid, off_cell) ALLOC(cblk_rep, off_cell) ALLOC(cblk_cell, off_cell) ALLOC(partial, 4 * (size_t)md->fnblk)
+    ALLOC(blkd, md->nblk) ALLOC(fblk, md->fnblk) ALLOC(lblk_rep, md->lnblk) ALLOC(lblk_first, md->lnblk)
+    ALLOC(wl_item, (size_t)md->nblk + md->lnblk + md->ncb) ALLOC(wl_n, 4) ALLOC(ranges, (size_t)off_cell * NRANGE) ALLOC(xmid, off_cell) ALLOC(cblk_rep, off_cell) ALLOC(cblk_cell, off_cell) ALLOC(partial, 4 * (size_t)md->fnblk) ALLOC(mid, 6 * (size_t)nslots)
+    if (md->en_apart) { ALLOC(eblk, md->enblk) ALLOC(epart, 2 * (size_t)md->enblk) }
     ALLOC(fx, off) ALLOC(fy, off) ALLOC(fz, off) ALLOC(xo, off) ALLOC(yo, off) ALLOC(zo, off) ALLOC(pos4, off) ALLOC(posq, off)
     ALLOC(cell_mem, (size_t)off_cell * CELL_CAP) ALLOC(nn, off) ALLOC(nn_ref, off) ALLOC(nl, (size_t)md->cap * off) ALLOC(cnt, off_cell) ALLOC(start, off_cell)
     ALLOC(members, off) ALLOC(kx, off_act) ALLOC(ky, off_act) ALLOC(kz, off_act)
@@ -2016,8 +2238,8 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     AC4_HIP(hipMemcpy(md->blk_rep, brep.data(), sizeof(int) * md->nblk, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->blk_first, bfirst.data(), sizeof(int) * md->nblk, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->blk_idx, bidx.data(), sizeof(int) * md->nblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->fblk_rep, frep.data(), sizeof(int) * md->fnblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->fblk_first, ffirst.data(), sizeof(int) * md->fnblk, hipMemcpyHostToDevice));
+    AC4_HIP(hipMemcpy(md->blkd, bd.data(), sizeof(BlkD) * md->nblk, hipMemcpyHostToDevice));
+    AC4_HIP(hipMemcpy(md->fblk, fd.data(), sizeof(BlkD) * md->fnblk, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->lblk_rep, lrep.data(), sizeof(int) * md->lnblk, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->lblk_first, lfirst.data(), sizeof(int) * md->lnblk, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->cblk_rep, crep.data(), sizeof(int) * off_cell, hipMemcpyHostToDevice));
@@ -2053,7 +2275,8 @@ static void drop_graphs(ac4_md *md) {
 static int refresh_tables(ac4_md *md) {
     bool any = false;
     for (const RepC &R : md->reps_h) any |= R.n > 0;
-    std::vector<int> br, bf, bi, fr, ff, lr, lf;
+    std::vector<int> br, bf, bi, lr, lf;
+    std::vector<BlkD> bd, fd, ed;
     for (int r = 0; r < md->R; r++) {
         RepC &R = md->reps_h[r];
         if (any && R.n == 0) continue;
@@ -2061,9 +2284,11 @@ static int refresh_tables(ac4_md *md) {
         br.insert(br.end(), md->t_brep.begin() + md->t_b0[r], md->t_brep.begin() + md->t_b0[r] + R.nblk);
         bf.insert(bf.end(), md->t_bfirst.begin() + md->t_b0[r], md->t_bfirst.begin() + md->t_b0[r] + R.nblk);
         bi.insert(bi.end(), md->t_bidx.begin() + md->t_b0[r], md->t_bidx.begin() + md->t_b0[r] + R.nblk);
-        R.fblk_off = (int)fr.size();
-        fr.insert(fr.end(), md->t_frep.begin() + md->t_f0[r], md->t_frep.begin() + md->t_f0[r] + R.fnblk);
-        ff.insert(ff.end(), md->t_ffirst.begin() + md->t_f0[r], md->t_ffirst.begin() + md->t_f0[r] + R.fnblk);
+        for (int k = 0; k < R.nblk; k++) bd.push_back(BlkD{r, md->t_bfirst[md->t_b0[r] + k], R.off, R.n});
+        R.fblk_off = (int)fd.size();
+        for (int k = 0; k < R.fnblk; k++) fd.push_back(BlkD{r, md->t_ffirst[md->t_f0[r] + k], R.off, R.n});
+        R.eblk_off = (int)ed.size();
+        for (int k = 0; k < R.enblk; k++) ed.push_back(BlkD{r, k * (BLK >> md->elw), R.off, R.n});
         R.lblk_off = (int)lr.size();
         lr.insert(lr.end(), md->t_lrep.begin() + md->t_l0[r], md->t_lrep.begin() + md->t_l0[r] + R.lnblk);
         lf.insert(lf.end(), md->t_lfirst.begin() + md->t_l0[r], md->t_lfirst.begin() + md->t_l0[r] + R.lnblk);
@@ -2073,12 +2298,14 @@ static int refresh_tables(ac4_md *md) {
     drop_graphs(md);
     TRY(h2d(md->blk_rep, br.data(), br.size(), s)); TRY(h2d(md->blk_first, bf.data(), bf.size(), s));
     TRY(h2d(md->blk_idx, bi.data(), bi.size(), s));
-    TRY(h2d(md->fblk_rep, fr.data(), fr.size(), s)); TRY(h2d(md->fblk_first, ff.data(), ff.size(), s));
+    TRY(h2d(md->blkd, bd.data(), bd.size(), s)); TRY(h2d(md->fblk, fd.data(), fd.size(), s));
+    if (!ed.empty()) TRY(h2d(md->eblk, ed.data(), ed.size(), s));
     TRY(h2d(md->lblk_rep, lr.data(), lr.size(), s)); TRY(h2d(md->lblk_first, lf.data(), lf.size(), s));
     TRY(h2d(md->reps, md->reps_h.data(), md->reps_h.size(), s));
     AC4_HIP(hipStreamSynchronize(s));
     md->nblk = (int)br.size();
-    md->fnblk = (int)fr.size();
+    md->fnblk = (int)fd.size();
+    md->enblk = (int)ed.size();
     md->lnblk = (int)lr.size();
     return AC4_OK;
 }
@@ -2088,14 +2315,13 @@ extern "C" int ac4_md_assign(ac4_md *md, int slot, const ac4_replica_params *p) 
     RepC R = md->reps_h[slot];
     const char *why = configure_rep(R, *p);
     AC4_REQUIRE(!why, AC4_EARG, "slot %d: %s", slot, why ? why : "");
-    const bool was_idle = md->reps_h[slot].n == 0;
     md->reps_h[slot] = R;
     ChainS c;
     fresh_chain(c, R);
     AC4_HIP(hipMemcpyAsync(md->reps + slot, &md->reps_h[slot], sizeof(RepC), hipMemcpyHostToDevice, md->stream));
     AC4_HIP(hipMemcpyAsync(md->chain + slot, &c, sizeof(ChainS), hipMemcpyHostToDevice, md->stream));
     AC4_HIP(hipStreamSynchronize(md->stream));
-    return was_idle ? refresh_tables(md) : AC4_OK;
+    return refresh_tables(md);  // the block tables hold the replica's n
 }
 
 extern "C" int ac4_md_release(ac4_md *md, int slot) {
@@ -2133,11 +2359,11 @@ extern "C" int ac4_md_destroy(ac4_md *md) {
     if (!md) return AC4_OK;
     if (md->stream) (void)hipStreamSynchronize(md->stream);
     drop_graphs(md);
-    void *ptrs[] = {md->reps, md->chain, md->blk_rep, md->blk_first, md->blk_idx, md->fblk_rep, md->fblk_first,
+    void *ptrs[] = {md->reps, md->chain, md->blk_rep, md->blk_first, md->blk_idx, md->blkd, md->fblk, md->eblk, md->epart,
                     md->lblk_rep, md->lblk_first, md->wl_item, md->wl_n, md->ranges, md->xmid,
                     md->cblk_rep, md->cblk_cell, md->ox, md->oy, md->oz, md->ov_q, md->ov_q2,
                     md->ov_step, md->ov_cnt, md->ov_n, md->ov_list, md->ov_out,
-                    md->partial, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo, md->pos4, md->posq, md->cell_mem, md->shuf_ent, md->shuf_ent_n, md->nn,
+                    md->partial, md->mid, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo, md->pos4, md->posq, md->cell_mem, md->shuf_ent, md->shuf_ent_n, md->nn,
                     md->nn_ref, md->nl,
                     md->cnt, md->start, md->members, md->kx, md->ky, md->kz, md->ex, md->ey, md->ez, md->et};
     for (void *q : ptrs)
@@ -2171,9 +2397,9 @@ extern "C" long long ac4_md_slot_bytes(int cap_n, int n_origin, int n_lags) {
     b += 2 * n * (9 * 8 + 5 * 4);                                    // particle arrays and their scratch copy
     b += n * (3 * 8 + 4);                                            // reference-order export
     b += cells * ((long long)NRANGE * 8 + 3 * 4 + (long long)CELL_CAP * 8 + 2 * 4);
-    b += nblk * 3 * 4 + fnb * 2 * 4 + lnblk * 2 * 4;                // block tables
+    b += nblk * (3 * 4 + 16) + fnb * (2 * 16 + 16) + lnblk * 2 * 4;  // block tables, energy partials
     b += (nblk + lnblk + ncb) * 4 + fnb * 4 * 8;                     // work list, force partials
-    b += (long long)sizeof(RepC) + (long long)sizeof(ChainS);
+    b += (long long)sizeof(RepC) + (long long)sizeof(ChainS) + 6 * 8;
     if (cap_n > SHUF_PAR_MIN) b += 3LL * 2 * ((n + SHUF_M - 1) / SHUF_M) * SHUF_M * 4 + 3LL * ((n + SHUF_M - 1) / SHUF_M) * 4;
     if (n_origin > 0) b += n * 24LL * n_origin + (long long)n_origin * 12 + (long long)(n_lags + 1) * 20;
     return b;
@@ -2752,33 +2978,53 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
     return AC4_OK;
 }
 
-template <bool KICK>
+template <bool FP32, bool KICK, bool EN>
+static int launch_force_kernel(ac4_md *md) {
+    // FP32 teams read consecutive entries of a chunk, FP64 ones (four lanes)
+    // strided ones; en_apart: no energy in this kernel
+    auto kern = md->vec == 8 ? k_force<FP32, KICK, EN, 8>
+                : md->vec == 1 ? k_force<FP32, KICK, EN, 1>
+                : md->vec == 4 ? k_force<true, KICK, false, 4>
+                : md->vec == 2 ? k_force<true, KICK, false, 2>
+                               : k_force<false, KICK, EN, -2>;
+    hipLaunchKernelGGL(kern, dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, md->stream, md->reps, md->fblk, md->pos4,
+                       md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->P.act, md->kx, md->ky, md->kz, md->fx,
+                       md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk);
+    AC4_HIP(hipGetLastError());
+    return AC4_OK;
+}
+// The energy of en_apart handles, after the last of the call's steps (step)
+// or after calculate_forces' pass.
+static int launch_energy(ac4_md *md, bool step) {
+    if (!md->en_apart) return AC4_OK;
+    hipLaunchKernelGGL((md->elw ? k_energy<1> : k_energy<8>), dim3(xcd_grid(md->enblk)), dim3(BLK), 0, md->stream,
+                       md->reps, md->eblk, md->posq, md->nn, md->nl, md->cap, md->elw, md->epart, md->enblk);
+    hipLaunchKernelGGL(k_energy_end, dim3(md->R), dim3(256), 0, md->stream, md->reps, md->chain, md->epart,
+                       step ? 1 : 0);
+    AC4_HIP(hipGetLastError());
+    return AC4_OK;
+}
+template <bool KICK, bool EN>
 static int launch_force_pass(ac4_md *md) {
-    hipStream_t s = md->stream;
-    if (md->prec == AC4_FP32)
-        hipLaunchKernelGGL((k_force<true, KICK>), dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, s, md->reps,
-                           md->fblk_rep, md->fblk_first, md->pos4, md->posq, md->nn, md->nl, md->cap, md->P.act, md->kx,
-                           md->ky, md->kz, md->fx, md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial,
-                           md->fnblk);
-    else
-        hipLaunchKernelGGL((k_force<false, KICK>), dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, s, md->reps,
-                           md->fblk_rep, md->fblk_first, md->pos4, md->posq, md->nn, md->nl, md->cap, md->P.act, md->kx,
-                           md->ky, md->kz, md->fx, md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial,
-                           md->fnblk);
-    AC4_HIP(hipGetLastError());
-    return AC4_OK;
+    return md->prec == AC4_FP32 ? launch_force_kernel<true, KICK, EN>(md) : launch_force_kernel<false, KICK, EN>(md);
 }
-template <bool KICK>
+template <bool KICK, bool EN>
 static int launch_force_end(ac4_md *md) {
-    hipLaunchKernelGGL(k_force_end<KICK>, dim3(md->R), dim3(md->max_fnblk > 64 ? 256 : 64), 0, md->stream, md->reps,
-                       md->chain, md->partial);
+    auto kern = k_force_end<KICK, EN>;
+    hipLaunchKernelGGL(kern, dim3(md->R), dim3(md->max_fnblk > 64 ? 256 : 64), 0, md->stream, md->reps, md->chain,
+                       md->partial, md->en_apart ? 1 : 0, md->mid);
     AC4_HIP(hipGetLastError());
     return AC4_OK;
 }
+// energy: form the pair energy and virial in this pass
 template <bool KICK>
-static int launch_force(ac4_md *md) {
-    TRY(launch_force_pass<KICK>(md));
-    return launch_force_end<KICK>(md);
+static int launch_force(ac4_md *md, bool energy) {
+    if (energy && !md->en_apart) {
+        TRY((launch_force_pass<KICK, true>(md)));
+        return launch_force_end<KICK, true>(md);
+    }
+    TRY((launch_force_pass<KICK, false>(md)));
+    return launch_force_end<KICK, false>(md);
 }
 
 static void launch_shuffle(ac4_md *md, int force, hipStream_t s) {
@@ -2797,10 +3043,10 @@ static void launch_shuffle(ac4_md *md, int force, hipStream_t s) {
 static void launch_first_half(ac4_md *md, bool with_shuffle) {
     const ShufArgs sa{md->kx, md->ky, md->kz, md->shuf_kcap, with_shuffle ? 3 * md->R : 0};
     hipLaunchKernelGGL(k_first_half, dim3(md->nblk + sa.nblk), dim3(BLK), with_shuffle ? md->shuf_lds : 0, md->stream,
-                       md->reps, md->chain, md->blk_rep, md->blk_first, md->P.x, md->P.y, md->P.z, md->P.xu, md->P.yu,
+                       md->reps, md->chain, md->blkd, md->P.x, md->P.y, md->P.z, md->P.xu, md->P.yu,
                        md->P.zu, md->P.px, md->P.py, md->P.pz, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo,
                        md->P.type, md->pos4, md->posq, md->prec == AC4_FP32 ? 1 : 0, md->chain, md->blk_idx, md->cnt,
-                       md->wl_n, sa);
+                       md->wl_n, md->mid, sa);
 }
 
 // One MD step, one chain of launches on the handle's stream (also when
@@ -2808,7 +3054,10 @@ static void launch_first_half(ac4_md *md, bool with_shuffle) {
 // ran on a second graph branch beside the half kick and the rebuild: the
 // fork and join cost more than the overlap gave (about 9 us per step).  It
 // now runs inside k_first_half where its LDS allows, else as k_shuffle first.
-static int launch_step(ac4_md *md) {
+// last: the call's last step, whose pair energy and virial a caller can read
+// (each step overwrites them, so the steps before it do not form them; the
+// callers follow it with launch_energy).
+static int launch_step(ac4_md *md, bool last) {
     if (md->shuf_fused) {
         launch_first_half(md, true);
     } else {
@@ -2817,7 +3066,7 @@ static int launch_step(ac4_md *md) {
     }
     AC4_HIP(hipGetLastError());
     TRY(launch_rebuild(md));
-    return launch_force<true>(md);
+    return launch_force<true>(md, last);
 }
 
 static int check_err(ac4_md *md) {
@@ -2860,7 +3109,8 @@ extern "C" int ac4_md_calculate_forces(ac4_md *md, double *out2) {
     bool stale = false;
     for (auto &e : c) stale |= e.force_rebuild != 0;
     if (stale) TRY(force_rebuild_all(md));
-    TRY(launch_force<false>(md));
+    TRY(launch_force<false>(md, true));
+    TRY(launch_energy(md, false));
     TRY(get_chains(md, c));
     if (out2)
         for (int r = 0; r < md->R; r++) { out2[2 * r] = c[r].pe; out2[2 * r + 1] = c[r].vir; }
@@ -2871,8 +3121,8 @@ extern "C" int ac4_md_calculate_forces(ac4_md *md, double *out2) {
 extern "C" int ac4_md_step(ac4_md *md, int nsteps) {
     AC4_REQUIRE(md && nsteps >= 0, AC4_EARG, "bad arguments");
     if (!md->have_forces) TRY(ac4_md_calculate_forces(md, nullptr));
-    for (int k = 0; k < nsteps; k++) TRY(launch_step(md));
-    return AC4_OK;
+    for (int k = 0; k < nsteps; k++) TRY(launch_step(md, k == nsteps - 1));
+    return nsteps > 0 ? launch_energy(md, true) : AC4_OK;
 }
 
 // Steps are replayed from captured graphs: GRAPH_CHUNK steps per launch (one
@@ -2886,7 +3136,7 @@ static int capture_steps(ac4_md *md, int k) {
     const int m = k ? GRAPH_CHUNK : 1;
     AC4_HIP(hipStreamBeginCapture(md->stream, hipStreamCaptureModeThreadLocal));
     int rc = AC4_OK;
-    for (int q = 0; q < m && rc == AC4_OK; q++) rc = launch_step(md);
+    for (int q = 0; q < m && rc == AC4_OK; q++) rc = launch_step(md, q == m - 1);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(md->stream, &g);
     if (rc != AC4_OK || e != hipSuccess) {  // nothing of a failed capture is kept
@@ -2917,7 +3167,7 @@ extern "C" int ac4_md_step_graph(ac4_md *md, int nsteps) {
     TRY(ready_graphs(md));
     for (int k = 0; k < nsteps / GRAPH_CHUNK; k++) AC4_HIP(hipGraphLaunch(md->gexec[1], md->stream));
     for (int k = 0; k < nsteps % GRAPH_CHUNK; k++) AC4_HIP(hipGraphLaunch(md->gexec[0], md->stream));
-    return AC4_OK;
+    return nsteps > 0 ? launch_energy(md, true) : AC4_OK;
 }
 
 // Several handles stepped together: each on its own stream, the graph
@@ -2936,6 +3186,7 @@ extern "C" int ac4_md_step_graph_multi(ac4_md *const *mds, int nh, int nsteps) {
         for (int h = 0; h < nh; h++) AC4_HIP(hipGraphLaunch(mds[h]->gexec[1], mds[h]->stream));
     for (int k = 0; k < nsteps % GRAPH_CHUNK; k++)
         for (int h = 0; h < nh; h++) AC4_HIP(hipGraphLaunch(mds[h]->gexec[0], mds[h]->stream));
+    for (int h = 0; h < nh && nsteps > 0; h++) TRY(launch_energy(mds[h], true));
     return AC4_OK;
 }
 
@@ -2946,7 +3197,8 @@ extern "C" int ac4_md_relax(ac4_md *md, int nsteps, double f_start, double f_end
     TRY(get_chains(md, c));
     for (auto &e : c) { e.mode = 1; e.ramp_n = nsteps; e.ramp_k = 0; e.ramp0 = f_start; e.ramp1 = f_end; }
     TRY(put_chains(md, c));
-    for (int k = 0; k < nsteps; k++) TRY(launch_step(md));
+    for (int k = 0; k < nsteps; k++) TRY(launch_step(md, k == nsteps - 1));
+    TRY(launch_energy(md, true));
     return check_err(md);
 }
 
@@ -2970,9 +3222,10 @@ extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
         AC4_HIP(hipEventRecord(ev[2], s));
         TRY(launch_rebuild(md));
         AC4_HIP(hipEventRecord(ev[3], s));
-        TRY(launch_force_pass<true>(md));
+        const bool en = k == nsteps - 1 && !md->en_apart;
+        TRY((en ? launch_force_pass<true, true>(md) : launch_force_pass<true, false>(md)));
         AC4_HIP(hipEventRecord(ev[4], s));
-        TRY(launch_force_end<true>(md));
+        TRY((en ? launch_force_end<true, true>(md) : launch_force_end<true, false>(md)));
         AC4_HIP(hipEventRecord(ev[5], s));
         AC4_HIP(hipEventSynchronize(ev[5]));
         float t[5];
@@ -2981,6 +3234,7 @@ extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
     }
     for (auto &e : ev) (void)hipEventDestroy(e);
     for (int q = 0; q < 5; q++) ms[q] = acc[q] / nsteps;
+    TRY(launch_energy(md, true));
     return check_err(md);
 }
 

@@ -64,3 +64,30 @@ def test_shell_runs_against_direct_sums(gpu, n, npairs, nshell, ndir):
     var = lambda v: (v * v).mean(0) - v.mean(0) ** 2  # noqa: E731
     want = var(ph).sum(-1).mean(0) / n
     assert np.allclose(s4d, want, rtol=1e-9, atol=1e-9 * (ph ** 2).max() / n)
+
+
+# One size in each range of the automatic force team (16, 8, 4 and 2 lanes,
+# with the list layouts of 16, 8, 4, 2 and one nominal lanes) against one
+# pinned lane: the same pair terms, summed in FP64 in another order.
+@pytest.mark.parametrize("prec,n", [(0, 700), (0, 6000), (0, 9001), (0, 14001), (0, 33001), (1, 700), (1, 6000),
+                                    (1, 9001), (1, 14001), (1, 33001), (1, 160001)])
+def test_force_team_widths(gpu, prec, n):
+    s = gpu.init_lattice(n, 0.5, n)
+    rng = np.random.default_rng(n)
+    x = [(s[k] + rng.normal(0, 0.02 / n ** (1 / 3), n)) % 1.0 for k in ("x", "y", "z")]
+    out = []
+    for tpp in (0, 1):
+        gpu.set_tuning(tpp)
+        try:
+            md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 200, 3)], precision=prec)
+        finally:
+            gpu.set_tuning()
+        md.set_state(0, *x, *x, s["px"], s["py"], s["pz"], s["type"], s["act_tag"], s["kx"], s["ky"], s["kz"])
+        pv = md.calculate_forces()[0]
+        out.append((np.stack(md.forces(0)), pv))
+        md.close()
+    (fa, pa), (fb, pb) = out
+    # about 100 terms of up to a few hundred times the rms force cancel: 100 * 300 * 2^-53
+    assert np.abs(fa - fb).max() <= 4e-12 * np.sqrt((fb ** 2).mean())
+    # energy and virial: FP32 partial sums of eight pairs in FP32 mode
+    assert np.allclose(pa, pb, rtol=1e-11 if prec == 0 else 1e-6)
