@@ -5,10 +5,13 @@
 // and walks (origin, lag) pairs with one MPI_Reduce per pair; here frames are
 // pushed once in file order, origin frames stay resident in HBM, and each
 // pushed frame is compared with all origins whose walk it completes in one
-// launch (grid = particle blocks x pairs, x q groups for Fs); S4's phase sums
-// are formed once per origin over all of its lags on the FP64 matrix cores.
-// Per-pair results are reduced in a fixed order and accumulated into lag
-// slots in the reference's origin order on the device, so integer
+// launch (k_frame: MSD sums, overlap counts and S4 masks of every pair, and
+// the copy of an origin frame to its resident place), with a second one for
+// Fs (k_fs).  The walk is known when the handle is made, so the pairs of every
+// frame and the origins' places are laid out on the device then.  S4's phase
+// sums are formed once per origin over all of its lags on the FP64 matrix
+// cores.  Per-pair results are reduced in a fixed order and accumulated into
+// lag slots in the reference's origin order on the device, so integer
 // observables (overlap counts) reproduce the reference's output bit for
 // bit.
 #include <hip/hip_runtime.h>
@@ -19,15 +22,20 @@
 #include "ac4_internal.h"
 
 #define ABLK 256
-#define QG 18                 // q vectors per thread group
-#define NQG (AC4_NQ / QG)     // 9 groups
 #define A_PI 3.14159265358979 // Analysis/global.h:14
 
 __constant__ int c_vx[AC4_NQ], c_vy[AC4_NQ], c_vz[AC4_NQ], c_dg[AC4_NQ];
 
-struct Job {  // one (origin, lag) pair evaluated against the pushed frame
-    const double *x0, *y0, *z0;
-    int pair, slot;
+struct Job {       // one (origin, lag) pair evaluated against the pushed frame
+    int org;       // the origin's place among the resident frames
+    int p0, p1;    // pair of the MSD walk and of the overlap/S4/Fs walk, -1 where it is none (or not asked for)
+    int slot;      // lag slot, the number of wraps S4 and Fs apply to the origin
+};
+// resident origin frames: x, y, z of place k at f + (3*k + {0,1,2})*n
+struct Origins {
+    double *f;
+    size_t n;
+    __host__ __device__ double *at(int k, int c) const { return f + ((size_t)3 * k + c) * n; }
 };
 
 __device__ __forceinline__ double minimg_ana(double d) {  // overlap.c:67-78
@@ -68,47 +76,106 @@ __device__ __forceinline__ void block_sum_store(double (&v)[NV], double *out) {
     }
 }
 
-// MSD sums (msd_pos.c:64-76): grid (blocks, jobs); partial[(job*nb+blk)*3+v]
-__global__ void __launch_bounds__(ABLK) k_msd(const Job *__restrict__ jobs, int n, double L,
-                                              const double *__restrict__ x, const double *__restrict__ y,
-                                              const double *__restrict__ z, const int *__restrict__ ty, int flag,
-                                              double *partial) {
-    const Job J = jobs[blockIdx.y];
-    const int i = blockIdx.x * ABLK + threadIdx.x;
-    double v[3] = {0.0, 0.0, 0.0};
-    if (i < n && (ty[i] != 1 || flag == 0)) {
-        double dx = x[i] - J.x0[i];
-        double dy = y[i] - J.y0[i];
-        double dz = z[i] - J.z0[i];
-        double r2 = L * L * (dx * dx + dy * dy + dz * dz);
-        double r3 = r2 * r2;
-        double r4 = L * L * L * L * (dx * dx * dx * dx + dy * dy * dy * dy + dz * dz * dz * dz);
-        v[0] = r2;  // sum
-        v[1] = r4;  // sumSq
-        v[2] = r3;  // sumCube
+// One pushed frame against the origins of its jobs: grid (blocks, jobs, plus
+// one row copying the frame to place `keep` when keep >= 0).  Block b takes
+// particles [b*ppb, (b+1)*ppb), ppb a multiple of ABLK.  Per job:
+//  MSD sums (msd_pos.c:64-76) to msdp[(p0*gridDim.x + b)*3 + v];
+//  overlap count (overlap.c:61-84) to ovp[p1*gridDim.x + b];
+//  S4's overlap mask (S4Qt.c:125-133): bit i of mask[p1*nwords + i/32], count
+//  to s4p[p1*gridDim.x + b]; its coordinates take the reference's per-lag
+//  single-if wraps (wrapn) exactly as it applies them.
+// k_msd_pairs and k_counts add the blocks up, for all pairs at once.  A
+// frame has about one job, so each launch is a latency of a few
+// microseconds whatever it does: three kernels, each with a reduction kernel
+// of its own, the jobs copied from the host and a synchronisation per walk
+// took 83 us per frame of 50000 particles (MSD, overlap, S4 masks); one
+// launch and one synchronisation take 18.
+__global__ void __launch_bounds__(ABLK) k_frame(const Job *__restrict__ jobs, int nj, int n, int ppb, double L,
+                                                double param, const double *__restrict__ x,
+                                                const double *__restrict__ y, const double *__restrict__ z,
+                                                const int *__restrict__ ty, int flag, int obs, Origins org, int keep,
+                                                double *msdp, int *ovp, int *s4p, int nwords,
+                                                unsigned *mask) {
+    const int b = blockIdx.x, i0 = b * ppb, i1 = min(n, i0 + ppb), lane = threadIdx.x & 63;
+    if ((int)blockIdx.y >= nj) {  // the frame is an origin: keep it
+        double *ox = org.at(keep, 0), *oy = org.at(keep, 1), *oz = org.at(keep, 2);
+        for (int i = i0 + threadIdx.x; i < i1; i += ABLK) {
+            ox[i] = x[i];
+            oy[i] = y[i];
+            oz[i] = z[i];
+        }
+        return;
     }
-    block_sum_store<3>(v, partial + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3);
+    const Job J = jobs[blockIdx.y];
+    const double *ox = org.at(J.org, 0), *oy = org.at(J.org, 1), *oz = org.at(J.org, 2);
+    double v[3] = {0.0, 0.0, 0.0};
+    int nov = 0, ns4 = 0;
+    for (int t = i0; t < i1; t += ABLK) {
+        const int i = t + threadIdx.x;
+        bool ov = false, s4 = false;
+        if (i < i1) {
+            const double xa = x[i], ya = y[i], za = z[i], xb = ox[i], yb = oy[i], zb = oz[i];
+            const bool use = ty[i] != 1 || flag == 0;
+            double dx = xa - xb, dy = ya - yb, dz = za - zb;
+            if (J.p0 >= 0 && use) {
+                double r2 = L * L * (dx * dx + dy * dy + dz * dz);
+                double r3 = r2 * r2;
+                double r4 = L * L * L * L * (dx * dx * dx * dx + dy * dy * dy * dy + dz * dz * dz * dz);
+                v[0] += r2;  // sum
+                v[1] += r4;  // sumSq
+                v[2] += r3;  // sumCube
+            }
+            if (J.p1 >= 0 && (obs & AC4_OBS_OVERLAP)) {
+                dz = minimg_ana(dz);
+                dy = minimg_ana(dy);
+                dx = minimg_ana(dx);
+                ov = use && L * L * (dx * dx + dy * dy + dz * dz) < param;
+            }
+            if (J.p1 >= 0 && (obs & AC4_OBS_S4)) {
+                const double x0 = wrapn(xb, J.slot), y0 = wrapn(yb, J.slot), z0 = wrapn(zb, J.slot);
+                double ex = wrap1(xa) - x0, ey = wrap1(ya) - y0, ez = wrap1(za) - z0;
+                ez = minimg_ana(ez);
+                ey = minimg_ana(ey);
+                ex = minimg_ana(ex);
+                s4 = L * L * (ex * ex + ey * ey + ez * ez) < param;  // S4Qt.c:131-132
+            }
+        }
+        nov += __popcll(__ballot(ov));
+        if (J.p1 >= 0 && (obs & AC4_OBS_S4)) {
+            const unsigned long long m = __ballot(s4);
+            const int w = (t + (threadIdx.x & ~63)) >> 5;  // first of the wave's two words
+            unsigned *row = mask + (size_t)J.p1 * nwords;
+            if (lane == 0 && w < nwords) row[w] = (unsigned)m;
+            if (lane == 1 && w + 1 < nwords) row[w + 1] = (unsigned)(m >> 32);
+            ns4 += __popcll(m);
+        }
+    }
+    __shared__ int s_c[2][ABLK / 64];
+    if (lane == 0) { s_c[0][threadIdx.x >> 6] = nov; s_c[1][threadIdx.x >> 6] = ns4; }
+    if (J.p0 >= 0) block_sum_store<3>(v, msdp + ((size_t)J.p0 * gridDim.x + b) * 3);
+    __syncthreads();
+    if (J.p1 >= 0 && threadIdx.x < 2 && (obs & (threadIdx.x == 0 ? AC4_OBS_OVERLAP : AC4_OBS_S4))) {
+        int c = 0;
+        for (int w = 0; w < ABLK / 64; w++) c += s_c[threadIdx.x][w];
+        (threadIdx.x == 0 ? ovp : s4p)[(size_t)J.p1 * gridDim.x + b] = c;
+    }
 }
 
-// overlap count (overlap.c:61-84): partial[(job*nb+blk)]
-__global__ void __launch_bounds__(ABLK) k_overlap(const Job *__restrict__ jobs, int n, double L, double param,
-                                                  const double *__restrict__ x, const double *__restrict__ y,
-                                                  const double *__restrict__ z, const int *__restrict__ ty, int flag,
-                                                  double *partial) {
-    const Job J = jobs[blockIdx.y];
-    const int i = blockIdx.x * ABLK + threadIdx.x;
-    double v[1] = {0.0};
-    if (i < n && (ty[i] != 1 || flag == 0)) {
-        double dx = x[i] - J.x0[i];
-        double dy = y[i] - J.y0[i];
-        double dz = z[i] - J.z0[i];
-        dz = minimg_ana(dz);
-        dy = minimg_ana(dy);
-        dx = minimg_ana(dx);
-        double r2 = L * L * (dx * dx + dy * dy + dz * dz);
-        if (r2 < param) v[0] = 1.0;
-    }
-    block_sum_store<1>(v, partial + ((size_t)blockIdx.y * gridDim.x + blockIdx.x));
+// out[p*3 + v] = the MSD sums of pair p over its nb blocks, in a fixed order;
+// one workgroup per pair
+__global__ void __launch_bounds__(ABLK) k_msd_pairs(const double *__restrict__ msdp, int nb, double *out) {
+    double v[3] = {0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < nb; b += ABLK)
+        for (int k = 0; k < 3; k++) v[k] += msdp[((size_t)blockIdx.x * nb + b) * 3 + k];
+    block_sum_store<3>(v, out + (size_t)blockIdx.x * 3);
+}
+
+// out[p] = count of pair p over its nb blocks; one wave per pair
+__global__ void __launch_bounds__(64) k_counts(const int *__restrict__ c, int nb, double *out) {
+    int v = 0;
+    for (int b = threadIdx.x; b < nb; b += 64) v += c[(size_t)blockIdx.x * nb + b];
+    v = ac4_wave_sum_i(v);
+    if (threadIdx.x == 0) out[blockIdx.x] = (double)v;
 }
 
 // Permutation s of a degeneracy-d vector in the order of S4Qt.c:133-214.
@@ -127,58 +194,205 @@ __host__ __device__ __forceinline__ void perm_q(int d, int s, int a, int b, int 
     }
 }
 
-// Fs (Fsqt.c:103-222): grid (blocks, NQG, jobs).  The phase is that of each
-// particle's displacement, so every (origin, lag) pair takes its own 573
-// sincos per particle.
-// partial[((job*nb+blk)*AC4_NQ*2) + n] = cos sum, + AC4_NQ + n = sin sum.
-__global__ void __launch_bounds__(ABLK) k_phase(const Job *__restrict__ jobs, int n, const double *__restrict__ x,
-                                                const double *__restrict__ y, const double *__restrict__ z,
-                                                const int *__restrict__ ty, int flag, double *partial) {
-    const Job J = jobs[blockIdx.z];
-    const int i = blockIdx.x * ABLK + threadIdx.x;
-    const int qg = blockIdx.y;
-    double v[2 * QG];
-    for (int k = 0; k < 2 * QG; k++) v[k] = 0.0;
-    if (i < n && (ty[i] != 1 || flag == 0)) {
-        const double x0 = wrapn(J.x0[i], J.slot), y0 = wrapn(J.y0[i], J.slot), z0 = wrapn(J.z0[i], J.slot);
-        const double xs = wrap1(x[i]), ys = wrap1(y[i]), zs = wrap1(z[i]);
-        // phases of the displacement (Fsqt.c:145-146)
-        const double p0 = minimg_ana(xs - x0), p1 = minimg_ana(ys - y0), p2 = minimg_ana(zs - z0);
-        for (int k = 0; k < QG; k++) {
-            const int nq = qg * QG + k;
-            const int d = c_dg[nq];
-            double cs = 0.0, sn = 0.0;
-            for (int s = 0; s < d; s++) {
-                int o0, o1, o2;
-                perm_q(d, s, c_vx[nq], c_vy[nq], c_vz[nq], o0, o1, o2);
-                // Fsqt.c:147-213 forms arg = q.L.p with q = 2*A_PI/L*(o0,o1,o2):
-                // arg = 2 pi f with f = o.p turns, evaluated in turns.  The
-                // reference's A_PI and its invL*L differ from pi and 1 in the
-                // 15th digit: below 1e-12 in the phase for |f| <= 63.
-                double sa, ca;
-                ac4_sincos_turns((double)o0 * p0 + (double)o1 * p1 + (double)o2 * p2, &sa, &ca);
-                cs += ca;
-                sn += sa;
-            }
-            if (d == 3) { cs = cs / 3.0; sn = sn / 3.0; }
-            else if (d == 6) { cs = cs / 6.0; sn = sn / 6.0; }
-            v[k] = cs;
-            v[QG + k] = sn;
-        }
+// The permuted GetQ vectors as columns (S4 and Fs)
+#define S4_NCOL 576           // the 573 permuted vectors, padded to whole 16-column tiles
+__constant__ int c_pv[3 * S4_NCOL];  // permuted vector (o0, o1, o2) per column; zero in the padding
+__constant__ int c_pcol[AC4_NQ];     // first column of each GetQ vector
+
+// ---------------------------------------------------------------- Fs
+// Fsqt.c:103-222: for each (origin, lag) pair the sums over particles of
+// exp(i q.p), p the particle's displacement, for the 573 permutations of the
+// GetQ vectors.  q is a lattice vector (o0, o1, o2) of the box, so the phase
+// factorises: exp(i q.p) = X[o0] Y[o1] Z[o2] with X[m] = exp(2 pi i m p_x).
+// The sum over particles of products of two factors is a matrix product with
+// the particles as the inner dimension, and every permuted vector is one
+// entry of it: (i, j, j) is X[i] (YZ)[j] (and the same for the other axes:
+// three products of 15 x 15), (0, k, i) with k = 1, 2 one factor of each of
+// two axes (a product of 6 rows with 3 x 21 columns), (1, 0, 0) a row with a
+// column of ones.  v_mfma_f64_16x16x4f64 takes 20 products of 16 x 16 per four
+// particles, where forming each of the 573 phases took 573 sincos per
+// particle (34 instructions each).  Per workgroup and tile of FS_P particles:
+// the factors of the three axes, m = 1 ... 21, by sincos of the exactly
+// reduced m p (63 per particle), the 45 products of two axes, both in LDS;
+// then in each set of four waves wave w < 3 takes the product of axis w with
+// the other two (real and imaginary parts, four MFMAs) and one of the eight
+// tiles of the (0, k, i) group, wave 3 the other five.  The FS_SETS sets
+// take every FS_SETS-th MFMA step and are added in order at the end: a frame
+// has about one pair, so the launch is as long as one workgroup's tiles, and
+// four waves per SIMD make them shorter.  1000 and 20011 particles, per pair:
+// one sincos per vector and particle 33.6 and 59.5 us, this 9.5 and 17.6 (one
+// set of waves, the displacements loaded per tile: 13.3 and 27.5).
+#define FS_P 32        // particles of a tile
+#define FS_M 21        // largest component of a GetQ vector
+#define FS_J 15        // largest j of the (i, j, j) vectors
+#define FS_RL (FS_P + 1)  // row of a table: FS_P values, padded against bank conflicts
+#define FS_TILES 14    // accumulated 16 x 16 tiles: 3 x {cos, sin}, then the (0, k, i) group's 8
+#define FS_LOAD 256    // particles whose displacements are loaded together
+#define FS_NBLK 256    // workgroups per pair, at most
+#define FS_SETS 4      // sets of four waves per workgroup
+#define FS_T (256 * FS_SETS)
+
+typedef double ac4_d4 __attribute__((ext_vector_type(4)));
+
+// rows of the axis table (axis a, component m = 0 ... 21, c = 0 cos, 1 sin) and of the product table (j = 1 ... 15)
+__device__ __forceinline__ int fs_ax(int a, int m, int c) { return ((a * (FS_M + 1) + m) * 2 + c) * FS_RL; }
+__device__ __forceinline__ int fs_pr(int a, int j, int c) {
+    return (3 * (FS_M + 1) * 2 + (a * FS_J + j - 1) * 2 + c) * FS_RL;
+}
+#define FS_LDS ((3 * (FS_M + 1) * 2 + 3 * FS_J * 2) * FS_RL)  // doubles; the accumulated tiles reuse it
+
+// cos and sin sums of the permuted vector (o0, o1, o2) from the accumulated tiles s_t[tile][row][column]
+__device__ __forceinline__ void fs_entry(const double *s_t, int o0, int o1, int o2, double &c, double &s) {
+    const int o[3] = {o0, o1, o2};
+    const int nz = (o0 != 0) + (o1 != 0) + (o2 != 0);
+    if (nz == 3) {
+        const int a = o1 == o2 ? 0 : (o0 == o2 ? 1 : 2), j = a == 0 ? o1 : o0;  // axis of the odd component
+        const int e = (o[a] - 1) * 16 + j - 1;
+        c = s_t[(2 * a) * 256 + e];
+        s = s_t[(2 * a + 1) * 256 + e];
+        return;
     }
-    double *out = partial + ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * (AC4_NQ * 2);
-    __shared__ double s_red[2 * QG][ABLK / 64];
-    for (int k = 0; k < 2 * QG; k++) {
-        double w = ac4_wave_sum(v[k]);
-        if ((threadIdx.x & 63) == 0) s_red[k][threadIdx.x >> 6] = w;
+    // row axis: a component of 1 or 2; column axis: the other one, or the column of ones
+    int ra = o0 != 0 ? 0 : (o1 != 0 ? 1 : 2), ca = o2 != 0 ? 2 : (o1 != 0 ? 1 : 0);
+    if (o[ra] > 2) { const int t = ra; ra = ca; ca = t; }
+    const int r = 2 * ra + o[ra] - 1, q = nz == 2 ? ca * FS_M + o[ca] - 1 : 63;
+    const double *t0 = s_t + (6 + 2 * (q >> 4)) * 256 + (q & 15), *t1 = t0 + 256;
+    c = t0[r * 16] - t1[(r + 6) * 16];
+    s = t0[(r + 6) * 16] + t1[r * 16];
+}
+
+// grid (blocks of ppb particles, jobs), ppb a multiple of FS_P;
+// partial[((job*gridDim.x+blk)*AC4_NQ*2) + n] = cos sum, + AC4_NQ + n = sin
+// sum, averaged over the vector's permutations.
+__global__ void __launch_bounds__(FS_T) k_fs(const Job *__restrict__ jobs, int n, int ppb,
+                                            const double *__restrict__ x, const double *__restrict__ y,
+                                            const double *__restrict__ z, const int *__restrict__ ty, int flag,
+                                            Origins org, double *partial) {
+    __shared__ double s_t[FS_LDS];
+    __shared__ double s_p[3][FS_LOAD];
+    __shared__ double s_use[FS_LOAD];
+    const Job J = jobs[blockIdx.y];
+    if (J.p1 < 0) return;
+    const int t = threadIdx.x, lane = t & 63, set = t >> 8, wv = (t >> 6) & 3, i16 = lane & 15, k4 = lane >> 4;
+    const double *ox = org.at(J.org, 0), *oy = org.at(J.org, 1), *oz = org.at(J.org, 2);
+    // for the end: this thread's permuted vector, and of its output value the columns
+    const int pc = min(t, S4_NCOL - 1), o0 = c_pv[3 * pc], o1 = c_pv[3 * pc + 1], o2 = c_pv[3 * pc + 2];
+    const int oq = t < 2 * AC4_NQ ? t % AC4_NQ : 0, od = c_dg[oq], oc = c_pcol[oq];
+    ac4_d4 acc[5];
+    for (int q = 0; q < 5; q++) acc[q] = ac4_d4{0.0, 0.0, 0.0, 0.0};
+    // operand rows of this lane (in the tables, without the particle): the
+    // axis row i16 + 1 and product column i16 + 1 of waves 0-2; the (0, k, i)
+    // group's row and its four columns
+    const int oth = wv < 3 ? wv : 0;
+    const int xa = fs_ax(oth, i16 + 1, 0), pb = fs_pr(oth, min(i16 + 1, FS_J), 0);
+    const int kr = min(i16, 11), ka = fs_ax((kr % 6) >> 1, (kr & 1) + 1, kr / 6);
+    int kb[4];
+    for (int q = 0; q < 4; q++) {
+        const int cq = 16 * q + i16;
+        kb[q] = cq < 3 * FS_M ? fs_ax(cq / FS_M, cq % FS_M + 1, 0) : fs_ax(0, 0, 0);
+    }
+    const int i0 = blockIdx.x * ppb, i1 = min(n, i0 + ppb);
+    for (int tb = i0; tb < i1; tb += FS_P) {
+        const int lb = (tb - i0) & (FS_LOAD - 1);  // the tile among the loaded particles
+        if (lb == 0 && t < FS_LOAD) {
+            const int i = tb + t;
+            double p0 = 0.0, p1 = 0.0, p2 = 0.0, use = 0.0;
+            if (i < i1) {
+                const int ti = ty[i];
+                const double xb = ox[i], yb = oy[i], zb = oz[i], xc = x[i], yc = y[i], zc = z[i];
+                if (ti != 1 || flag == 0) {
+                    // phases of the displacement (Fsqt.c:145-146)
+                    p0 = minimg_ana(wrap1(xc) - wrapn(xb, J.slot));
+                    p1 = minimg_ana(wrap1(yc) - wrapn(yb, J.slot));
+                    p2 = minimg_ana(wrap1(zc) - wrapn(zb, J.slot));
+                    use = 1.0;
+                }
+            }
+            s_p[0][t] = p0; s_p[1][t] = p1; s_p[2][t] = p2;
+            s_use[t] = use;
+        }
+        if (lb == 0) __syncthreads();
+        if (t < FS_P) {
+            s_t[fs_ax(0, 0, 0) + t] = s_use[lb + t];  // the column of ones
+            s_t[fs_ax(0, 0, 1) + t] = 0.0;
+        }
+        const int pp = t & (FS_P - 1);
+        const bool use = s_use[lb + pp] != 0.0;
+        for (int e = t / FS_P; e < 3 * FS_M; e += FS_T / FS_P) {
+            const int a = e / FS_M, m = e - a * FS_M + 1;
+            // Fsqt.c:147-213 forms arg = q.L.p with q = 2*A_PI/L*(o0,o1,o2);
+            // in turns the component's part is m p, its whole turns taken off
+            // the unrounded product.  The reference's A_PI and its invL*L
+            // differ from pi and 1 in the 15th digit: below 1e-12 in the phase.
+            const double p = s_p[a][lb + pp], f = fma((double)m, p, -rint((double)m * p));
+            double sn, cs;
+            ac4_sincos_turns(f, &sn, &cs);
+            s_t[fs_ax(a, m, 0) + pp] = use ? cs : 0.0;
+            s_t[fs_ax(a, m, 1) + pp] = use ? sn : 0.0;
+        }
+        __syncthreads();
+        for (int e = t / FS_P; e < 3 * FS_J; e += FS_T / FS_P) {
+            const int a = e / FS_J, j = e - a * FS_J + 1, b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+            const double cb = s_t[fs_ax(b, j, 0) + pp], sb = s_t[fs_ax(b, j, 1) + pp], cc = s_t[fs_ax(c, j, 0) + pp],
+                         sc = s_t[fs_ax(c, j, 1) + pp];
+            s_t[fs_pr(a, j, 0) + pp] = fma(cb, cc, -(sb * sc));
+            s_t[fs_pr(a, j, 1) + pp] = fma(sb, cc, cb * sc);
+        }
+        __syncthreads();
+        if (wv < 3) {
+            const int kq = kb[0] * (wv == 0 || wv == 1) + kb[1] * (wv == 2) + (wv == 1 ? FS_RL : 0);  // tiles 0, 1, 2
+#pragma unroll
+            for (int st = set; st < FS_P / 4; st += FS_SETS) {
+                const int q = 4 * st + k4;
+                const double ac = s_t[xa + q], as = s_t[xa + FS_RL + q], bc = s_t[pb + q], bs = s_t[pb + FS_RL + q];
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac, bc, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(as, bc, acc[1], 0, 0, 0);
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(-as, bs, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac, bs, acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(s_t[ka + q], s_t[kq + q], acc[2], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int st = set; st < FS_P / 4; st += FS_SETS) {
+                const int q = 4 * st + k4;
+                const double a = s_t[ka + q];  // tiles 3 ... 7: columns 16..31 sin, 32..47 and 48..63 cos and sin
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, s_t[kb[1] + FS_RL + q], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, s_t[kb[2] + q], acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, s_t[kb[2] + FS_RL + q], acc[2], 0, 0, 0);
+                acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, s_t[kb[3] + q], acc[3], 0, 0, 0);
+                acc[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, s_t[kb[3] + FS_RL + q], acc[4], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    // the accumulated tiles to LDS (element e of lane l: row l/16 + 4*e, column l%16)
+    for (int w = 0; w < FS_SETS; w++) {
+        if (set == w)
+#pragma unroll
+            for (int q = 0; q < 5; q++) {
+                if (wv < 3 && q >= 3) continue;
+                const int tile = wv < 3 ? (q < 2 ? 2 * wv + q : 6 + wv) : 9 + q;
+                for (int e = 0; e < 4; e++) {
+                    double *d = &s_t[tile * 256 + (k4 + 4 * e) * 16 + i16];
+                    *d = w == 0 ? acc[q][e] : *d + acc[q][e];
+                }
+            }
+        __syncthreads();
+    }
+    // the permuted vectors' sums, then each vector's average over its permutations
+    double c = 0.0, sn = 0.0;
+    if (t < S4_NCOL - 3) fs_entry(s_t, o0, o1, o2, c, sn);
+    __syncthreads();
+    if (t < S4_NCOL) {
+        s_t[t] = c;
+        s_t[S4_NCOL + t] = sn;
     }
     __syncthreads();
-    if (threadIdx.x < 2 * QG) {
-        double s = 0.0;
-        for (int w = 0; w < ABLK / 64; w++) s += s_red[threadIdx.x][w];
-        const int k = threadIdx.x;
-        if (k < QG) out[qg * QG + k] = s;
-        else out[AC4_NQ + qg * QG + (k - QG)] = s;
+    if (t < 2 * AC4_NQ) {
+        const double *src = s_t + (t < AC4_NQ ? 0 : S4_NCOL) + oc;
+        double v = 0.0;
+        for (int k = 0; k < od; k++) v += src[k];
+        partial[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * (AC4_NQ * 2) + t] = od == 1 ? v : v / (double)od;
     }
 }
 
@@ -188,7 +402,7 @@ __global__ void __launch_bounds__(ABLK) k_phase(const Job *__restrict__ jobs, in
 // position at the lag (|r(t) - r0| < a), averaged over q's permutations.
 // The phase depends on the origin frame alone, so it is evaluated once per
 // origin and shared by all of that origin's lags:
-//   k_s4_mask   at each lag frame: the overlap mask of the pair, one bit per
+//   k_frame     at each lag frame: the overlap mask of the pair, one bit per
 //               particle (and the overlap count of the pair);
 //   k_s4_origin when the origin's last lag has been masked: the phase matrix
 //               P[particle][573 permuted vectors] times the mask matrix
@@ -197,46 +411,9 @@ __global__ void __launch_bounds__(ABLK) k_phase(const Job *__restrict__ jobs, in
 //   k_s4_reduce sums the chunk partials in a fixed order and averages each
 //               vector's permutations.
 // This evaluates 573 sincos per particle per origin instead of per pair.
-#define S4_NCOL 576           // the 573 permuted vectors, padded to whole 16-column tiles
 #define S4_NCT (S4_NCOL / 16) // column tiles
 #define S4_RT_MAX 4           // lag rows of one pass: up to 64 lags
 #define S4_CHUNKS 64          // particle chunks a pass is split into (at most)
-
-__constant__ int c_pv[3 * S4_NCOL];  // permuted vector (o0, o1, o2) per column; zero in the padding
-__constant__ int c_pcol[AC4_NQ];     // first column of each GetQ vector
-
-typedef double ac4_d4 __attribute__((ext_vector_type(4)));
-
-// Overlap mask of S4Qt.c:125-133 for each pair: grid (blocks, jobs).  Bit i
-// of mask[pair*nwords + i/32] is set when particle i overlaps; the count per
-// block goes to mpartial[job*nb+blk].  The origin coordinates take the
-// reference's per-lag single-if wraps (wrapn) exactly as it applies them.
-__global__ void __launch_bounds__(ABLK) k_s4_mask(const Job *__restrict__ jobs, int n, double L, double param,
-                                                  const double *__restrict__ x, const double *__restrict__ y,
-                                                  const double *__restrict__ z, int nwords, unsigned *mask,
-                                                  double *mpartial) {
-    const Job J = jobs[blockIdx.y];
-    const int i = blockIdx.x * ABLK + threadIdx.x;
-    bool use = false;
-    if (i < n) {
-        const double x0 = wrapn(J.x0[i], J.slot), y0 = wrapn(J.y0[i], J.slot), z0 = wrapn(J.z0[i], J.slot);
-        const double xs = wrap1(x[i]), ys = wrap1(y[i]), zs = wrap1(z[i]);
-        double dx = (xs - x0), dy = (ys - y0), dz = (zs - z0);
-        dz = minimg_ana(dz);
-        dy = minimg_ana(dy);
-        dx = minimg_ana(dx);
-        const double r2 = L * L * (dx * dx + dy * dy + dz * dz);  // S4Qt.c:131-132
-        use = r2 < param;
-    }
-    const unsigned long long b = __ballot(use);
-    const int lane = threadIdx.x & 63;
-    const int w = (blockIdx.x * ABLK + (threadIdx.x & ~63)) >> 5;  // first of the wave's two words
-    unsigned *row = mask + (size_t)J.pair * nwords;
-    if (lane == 0 && w < nwords) row[w] = (unsigned)b;
-    if (lane == 1 && w + 1 < nwords) row[w + 1] = (unsigned)(b >> 32);
-    double m[1] = {use ? 1.0 : 0.0};
-    block_sum_store<1>(m, mpartial + ((size_t)blockIdx.y * gridDim.x + blockIdx.x));
-}
 
 // One origin, one pass of up to RT*16 of its lags: grid (chunks, S4_NCT),
 // 256 threads.  Wave w of block (c, ct) takes the mask words
@@ -341,7 +518,7 @@ __global__ void __launch_bounds__(256) k_s4_reduce(const double *__restrict__ pa
     }
 }
 
-// Fixed-order sum over blocks: out[pair*nv + v] = sum_b partial[(job*nb+b)*nv + v].
+// Fixed-order sum over blocks of Fs's partials: out[p1*nv + v] = sum_b partial[(job*nb+b)*nv + v].
 // Grid (jobs, ceil(nv/64)), 256 threads: lane l of wave w takes value
 // v = 64*blockIdx.y + l (consecutive values, coalesced loads) and the blocks
 // b = w, w+4, w+8, ... with 8 loads in flight; the four wave sums are added
@@ -350,6 +527,7 @@ __global__ void __launch_bounds__(256) k_reduce_jobs(const Job *__restrict__ job
                                                      const double *__restrict__ partial, double *out) {
     __shared__ double s_w[4][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, v = blockIdx.y * 64 + lane;
+    if (jobs[blockIdx.x].p1 < 0) return;  // uniform over the workgroup
     double acc = 0.0;
     if (v < nv) {
         const double *p = partial + (size_t)blockIdx.x * nb * nv + v;
@@ -366,8 +544,7 @@ __global__ void __launch_bounds__(256) k_reduce_jobs(const Job *__restrict__ job
     s_w[w][lane] = acc;
     __syncthreads();
     if (w == 0 && v < nv) {
-        const Job J = jobs[blockIdx.x];
-        out[(size_t)J.pair * nv + v] = ((s_w[0][lane] + s_w[1][lane]) + s_w[2][lane]) + s_w[3][lane];
+        out[(size_t)jobs[blockIdx.x].p1 * nv + v] = ((s_w[0][lane] + s_w[1][lane]) + s_w[2][lane]) + s_w[3][lane];
     }
 }
 
@@ -391,14 +568,8 @@ __global__ void k_slots(const double *__restrict__ vals, int nv, const int *__re
 }
 
 // ------------------------------------------------------------------ host
-struct Frame {
-    double *x = nullptr, *y = nullptr, *z = nullptr;
-    int *t = nullptr;
-};
-
 struct WalkInfo {
     ac4_walk_t w;
-    std::vector<std::vector<int>> by_oth;  // pair ids completed by frame pos
     std::vector<int> last_use;             // per origin pos: last frame pos needing it
     std::vector<int> slot_ptr, slot_pairs; // CSR of pairs per slot (walk order)
     int nslots = 0;
@@ -409,12 +580,22 @@ struct ac4_ana {
     double L = 0, invL = 0, factor = 1.4, a = 0.3, param = 0.09;
     std::vector<int> fidx;
     WalkInfo W[2];
-    std::vector<Frame> store;   // resident origin frames by pos
-    Frame cur;                  // staging for the pushed frame
+    // the plan: each frame's jobs (CSR by frame position) and their origin
+    // frames, each origin's place among the resident frames (-1: no origin),
+    // the origins by the frame of their last lag; which origins are resident
+    std::vector<Job> jobs;
+    std::vector<int> jorg, jptr, place;
+    std::vector<std::vector<int>> ends;
+    std::vector<char> resident;
+    Origins org{nullptr, 0};    // the resident frames
+    double *cur = nullptr;      // a frame pushed from the host that is no origin: x, y, z
+    int *cur_t = nullptr;       // types of a frame pushed from the host
     int last_pos = -1;
     double *d_msd = nullptr, *d_ov = nullptr, *d_s4 = nullptr, *d_s4m = nullptr, *d_fs = nullptr;
-    double *d_part = nullptr, *d_mpart = nullptr;
+    double *d_part = nullptr, *d_msdp = nullptr;
+    int *d_ovp = nullptr, *d_s4p = nullptr;  // per block: overlap counts of the overlap and the S4 rule
     Job *d_jobs = nullptr;
+    bool stale = false;         // frames came in since d_msd, d_ov and d_s4m were formed from the blocks' values
     // S4 by origin: pair ids per origin (CSR, walk order), origins whose
     // last lag is frame pos, the pairs' overlap masks and the chunk partials
     std::vector<int> s4_optr, s4_opairs;
@@ -424,7 +605,7 @@ struct ac4_ana {
     unsigned *d_s4mask = nullptr;
     double *d_s4part = nullptr;
     int nwords = 0, s4_wpw = 1, s4_nchunk = 1;
-    int max_jobs = 0, nb = 0;
+    int max_jobs = 0, ppb = ABLK, nb = 0, fs_ppb = FS_P, fs_nb = 0;
     std::vector<int> vx, vy, vz, qsq;
     std::vector<double> qval;
     hipStream_t stream = nullptr;
@@ -436,31 +617,69 @@ struct ac4_ana {
     int noi_msd = 0, noi_ov = 0;
 };
 
-static int frame_alloc(Frame &f, int n) {
-    AC4_HIP(hipMalloc(&f.x, sizeof(double) * n));
-    AC4_HIP(hipMalloc(&f.y, sizeof(double) * n));
-    AC4_HIP(hipMalloc(&f.z, sizeof(double) * n));
-    AC4_HIP(hipMalloc(&f.t, sizeof(int) * n));
-    return AC4_OK;
-}
-static void frame_free(Frame &f) {
-    if (f.x) (void)hipFree(f.x);
-    if (f.y) (void)hipFree(f.y);
-    if (f.z) (void)hipFree(f.z);
-    if (f.t) (void)hipFree(f.t);
-    f = Frame();
-}
-
 #define TRY(e) do { int rc_ = (e); if (rc_ != AC4_OK) return rc_; } while (0)
 
 static void build_walk_info(ac4_ana *an, WalkInfo &W, int rule) {
     ac4_walk(an->fidx.data(), an->nframes, an->gap, an->factor, rule, &W.w);
-    W.by_oth.assign(an->nframes, {});
     W.last_use.assign(an->nframes, -1);
-    for (int p = 0; p < W.w.np; p++) {
-        W.by_oth[W.w.oth[p]].push_back(p);
-        W.last_use[W.w.cur[p]] = std::max(W.last_use[W.w.cur[p]], W.w.oth[p]);
+    for (int p = 0; p < W.w.np; p++) W.last_use[W.w.cur[p]] = std::max(W.last_use[W.w.cur[p]], W.w.oth[p]);
+}
+
+// The jobs of every frame and the origins' places.  The two walks visit the
+// same origins and lags up to their longest lag, so their pairs are matched:
+// one job reads an origin for both.  An origin holds its place from its own
+// frame to its last lag's; a place is taken over by the first origin after
+// that (a frame that is both a last lag and an origin takes another place:
+// both are in use in its launch).  Returns the number of places.
+static int build_plan(ac4_ana *an) {
+    const bool want0 = (an->obs & AC4_OBS_MSD) != 0,
+               want1 = (an->obs & (AC4_OBS_OVERLAP | AC4_OBS_S4 | AC4_OBS_FS)) != 0;
+    const int nf = an->nframes;
+    std::vector<int> last(nf, -1);
+    for (int o = 0; o < nf; o++) last[o] = std::max(an->W[0].last_use[o], an->W[1].last_use[o]);
+    an->place.assign(nf, -1);
+    an->resident.assign(nf, 0);
+    an->ends.assign(nf, {});
+    int places = 0;
+    std::vector<int> avail;
+    for (int f = 0; f < nf; f++) {
+        if (last[f] >= 0) {
+            if (avail.empty()) avail.push_back(places++);
+            an->place[f] = avail.back();
+            avail.pop_back();
+            an->ends[last[f]].push_back(f);  // a lag frame comes after its origin
+        }
+        for (int o : an->ends[f]) avail.push_back(an->place[o]);
     }
+    std::vector<std::vector<std::pair<int, Job>>> by(nf);  // (origin frame, job) per lag frame
+    for (int w = 0; w < 2; w++) {
+        if (!(w == 0 ? want0 : want1)) continue;
+        const ac4_walk_t &k = an->W[w].w;
+        for (int p = 0; p < k.np; p++) {
+            auto &v = by[k.oth[p]];
+            Job *j = nullptr;
+            for (auto &e : v)
+                if (e.first == k.cur[p] && e.second.slot == k.slot[p] && (w == 0 ? e.second.p0 : e.second.p1) < 0) {
+                    j = &e.second;
+                    break;
+                }
+            if (!j) {
+                v.push_back({k.cur[p], Job{an->place[k.cur[p]], -1, -1, k.slot[p]}});
+                j = &v.back().second;
+            }
+            (w == 0 ? j->p0 : j->p1) = p;
+        }
+    }
+    an->jptr.assign(nf + 1, 0);
+    for (int f = 0; f < nf; f++) {
+        for (auto &e : by[f]) {
+            an->jorg.push_back(e.first);
+            an->jobs.push_back(e.second);
+        }
+        an->jptr[f + 1] = (int)an->jobs.size();
+        an->max_jobs = std::max(an->max_jobs, (int)by[f].size());
+    }
+    return places;
 }
 
 static void build_slots(WalkInfo &W, int nslots) {
@@ -473,10 +692,8 @@ static void build_slots(WalkInfo &W, int nslots) {
     for (int p = 0; p < W.w.np; p++) W.slot_pairs[fill[W.w.slot[p]]++] = p;  // walk order kept
 }
 
-// S4 by origin: the permuted-vector columns, the per-origin pair lists and
-// the device buffers.  Masks and sums start at zero, so a pair whose lag
-// frame never arrives contributes nothing.
-static int s4_setup(ac4_ana *an, const std::vector<int> &dg) {
+// the permuted-vector columns of S4 and Fs
+static int set_columns(ac4_ana *an, const std::vector<int> &dg) {
     std::vector<int> pv(3 * S4_NCOL, 0), pcol(AC4_NQ, 0);
     int col = 0;
     for (int q = 0; q < AC4_NQ; q++) {
@@ -487,6 +704,12 @@ static int s4_setup(ac4_ana *an, const std::vector<int> &dg) {
     AC4_REQUIRE(col <= S4_NCOL, AC4_EARG, "S4: %d permuted vectors exceed %d columns", col, S4_NCOL);
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_pv), pv.data(), sizeof(int) * 3 * S4_NCOL));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_pcol), pcol.data(), sizeof(int) * AC4_NQ));
+    return AC4_OK;
+}
+
+// S4 by origin: the per-origin pair lists and the device buffers.  Masks and sums start at zero, so a pair whose lag
+// frame never arrives contributes nothing.
+static int s4_setup(ac4_ana *an) {
     const ac4_walk_t &w = an->W[1].w;
     an->s4_optr.assign(an->nframes + 1, 0);
     for (int p = 0; p < w.np; p++) an->s4_optr[w.cur[p] + 1]++;
@@ -508,15 +731,14 @@ static int s4_setup(ac4_ana *an, const std::vector<int> &dg) {
     AC4_HIP(hipMalloc(&an->d_s4part, sizeof(double) * (size_t)an->s4_nchunk * 16 * S4_RT_MAX * 2 * S4_NCOL));
     AC4_HIP(hipMemset(an->d_s4mask, 0, sizeof(unsigned) * np1 * an->nwords));
     AC4_HIP(hipMemset(an->d_s4, 0, sizeof(double) * 2 * AC4_NQ * np1));
-    AC4_HIP(hipMemset(an->d_s4m, 0, sizeof(double) * np1));
     return AC4_OK;
 }
 
 // The S4 sums of every pair of origin o, from its resident frame and the
 // masks its lags left; passes of up to 16*S4_RT_MAX lags.
 static int s4_origin(ac4_ana *an, int o) {
-    const Frame &F = an->store[o];
-    AC4_REQUIRE(F.x, AC4_ESTATE, "S4: origin frame %d is not resident", o);
+    AC4_REQUIRE(an->resident[o], AC4_ESTATE, "S4: origin frame %d is not resident", o);
+    const double *ox = an->org.at(an->place[o], 0), *oy = an->org.at(an->place[o], 1), *oz = an->org.at(an->place[o], 2);
     hipStream_t s = an->stream;
     const int b = an->s4_optr[o], e = an->s4_optr[o + 1];
     for (int p0 = b; p0 < e; p0 += 16 * S4_RT_MAX) {
@@ -524,13 +746,13 @@ static int s4_origin(ac4_ana *an, int o) {
         const int *lags = an->d_s4_opairs + p0;
         const dim3 g(an->s4_nchunk, S4_NCT);
         switch (rt) {
-            case 1: hipLaunchKernelGGL(k_s4_origin<1>, g, dim3(256), 0, s, F.x, F.y, F.z, an->n, an->nwords,
+            case 1: hipLaunchKernelGGL(k_s4_origin<1>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
                                        an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
-            case 2: hipLaunchKernelGGL(k_s4_origin<2>, g, dim3(256), 0, s, F.x, F.y, F.z, an->n, an->nwords,
+            case 2: hipLaunchKernelGGL(k_s4_origin<2>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
                                        an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
-            case 3: hipLaunchKernelGGL(k_s4_origin<3>, g, dim3(256), 0, s, F.x, F.y, F.z, an->n, an->nwords,
+            case 3: hipLaunchKernelGGL(k_s4_origin<3>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
                                        an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
-            default: hipLaunchKernelGGL(k_s4_origin<4>, g, dim3(256), 0, s, F.x, F.y, F.z, an->n, an->nwords,
+            default: hipLaunchKernelGGL(k_s4_origin<4>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
                                         an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
         }
         hipLaunchKernelGGL(k_s4_reduce, dim3(nl, (2 * AC4_NQ + 63) / 64), dim3(256), 0, s, an->d_s4part,
@@ -565,7 +787,7 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     an->noi_ov = 10 + (int)(log((double)an->W[1].w.maximal_interval) / lf);
     build_slots(an->W[0], std::max(an->noi_msd, an->W[0].w.max_slot + 1));
     build_slots(an->W[1], std::max(std::max(an->noi_ov, nframes), an->W[1].w.max_slot + 1));
-    an->store.assign(nframes, Frame());
+    const int places = build_plan(an);
     an->vx.resize(AC4_NQ); an->vy.resize(AC4_NQ); an->vz.resize(AC4_NQ); an->qsq.resize(AC4_NQ + 8);
     ac4_getq(an->vx.data(), an->vy.data(), an->vz.data(), an->qsq.data());
     std::vector<int> dg(AC4_NQ);
@@ -586,23 +808,36 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vy), an->vy.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vz), an->vz.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_dg), dg.data(), sizeof(int) * AC4_NQ));
-    an->nb = (n + ABLK - 1) / ABLK;
-    for (int w = 0; w < 2; w++)
-        for (int f = 0; f < nframes; f++) an->max_jobs = std::max(an->max_jobs, (int)an->W[w].by_oth[f].size());
+    if ((rc = set_columns(an, dg)) != AC4_OK) return fail(rc);
+    // blocks of k_frame: one tile of ABLK particles each up to 256 of them, then more tiles per block
+    an->ppb = ABLK * ((n + 256 * ABLK - 1) / (256 * ABLK));
+    an->nb = (n + an->ppb - 1) / an->ppb;
+    an->fs_ppb = FS_P * ((n + FS_NBLK * FS_P - 1) / (FS_NBLK * FS_P));
+    an->fs_nb = (n + an->fs_ppb - 1) / an->fs_ppb;
     an->max_jobs = std::max(an->max_jobs, 1);
-    const int np0 = std::max(an->W[0].w.np, 1), np1 = std::max(an->W[1].w.np, 1);
-    if (hipMalloc(&an->d_jobs, sizeof(Job) * an->max_jobs) != hipSuccess) return fail(AC4_EHIP);
-    if (hipMalloc(&an->d_part, sizeof(double) * (size_t)an->max_jobs * an->nb * AC4_NQ * 2) != hipSuccess) return fail(AC4_EHIP);
-    if (hipMalloc(&an->d_mpart, sizeof(double) * (size_t)an->max_jobs * an->nb) != hipSuccess) return fail(AC4_EHIP);
-    if (obs & AC4_OBS_MSD) if (hipMalloc(&an->d_msd, sizeof(double) * 3 * (size_t)np0) != hipSuccess) return fail(AC4_EHIP);
-    if (obs & AC4_OBS_OVERLAP) if (hipMalloc(&an->d_ov, sizeof(double) * (size_t)np1) != hipSuccess) return fail(AC4_EHIP);
+    const size_t np0 = std::max(an->W[0].w.np, 1), np1 = std::max(an->W[1].w.np, 1);
+    auto get = [&](auto **p, size_t count, bool zero) {
+        if (hipMalloc((void **)p, sizeof(**p) * count) != hipSuccess) return false;
+        return !zero || hipMemset(*p, 0, sizeof(**p) * count) == hipSuccess;
+    };
+    an->org.n = (size_t)n;
+    if (!get(&an->d_jobs, std::max<size_t>(an->jobs.size(), 1), false)) return fail(AC4_EHIP);
+    if (!an->jobs.empty() && hipMemcpy(an->d_jobs, an->jobs.data(), sizeof(Job) * an->jobs.size(),
+                                       hipMemcpyHostToDevice) != hipSuccess) return fail(AC4_EHIP);
+    if (!get(&an->org.f, (size_t)3 * n * std::max(places, 1), false)) return fail(AC4_EHIP);
+    if (!get(&an->cur, (size_t)3 * n, false) || !get(&an->cur_t, n, false)) return fail(AC4_EHIP);
+    if (obs & AC4_OBS_MSD)
+        if (!get(&an->d_msd, 3 * np0, true) || !get(&an->d_msdp, 3 * np0 * an->nb, true)) return fail(AC4_EHIP);
+    if (obs & AC4_OBS_OVERLAP)
+        if (!get(&an->d_ov, np1, true) || !get(&an->d_ovp, np1 * an->nb, true)) return fail(AC4_EHIP);
+    if (obs & AC4_OBS_FS)
+        if (!get(&an->d_fs, 2 * AC4_NQ * np1, true) ||
+            !get(&an->d_part, (size_t)an->max_jobs * an->fs_nb * AC4_NQ * 2, false)) return fail(AC4_EHIP);
     if (obs & AC4_OBS_S4) {
         if (hipMalloc(&an->d_s4, sizeof(double) * 2 * AC4_NQ * (size_t)np1) != hipSuccess) return fail(AC4_EHIP);
-        if (hipMalloc(&an->d_s4m, sizeof(double) * (size_t)np1) != hipSuccess) return fail(AC4_EHIP);
-        if ((rc = s4_setup(an, dg)) != AC4_OK) return fail(rc);
+        if (!get(&an->d_s4m, np1, true) || !get(&an->d_s4p, np1 * an->nb, true)) return fail(AC4_EHIP);
+        if ((rc = s4_setup(an)) != AC4_OK) return fail(rc);
     }
-    if (obs & AC4_OBS_FS) if (hipMalloc(&an->d_fs, sizeof(double) * 2 * AC4_NQ * (size_t)np1) != hipSuccess) return fail(AC4_EHIP);
-    if ((rc = frame_alloc(an->cur, n)) != AC4_OK) return fail(rc);
     *out = an;
     return AC4_OK;
 }
@@ -610,9 +845,8 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
 extern "C" int ac4_ana_destroy(ac4_ana *an) {
     if (!an) return AC4_OK;
     if (an->stream) (void)hipStreamSynchronize(an->stream);
-    for (auto &f : an->store) frame_free(f);
-    frame_free(an->cur);
-    void *ptrs[] = {an->d_msd, an->d_ov, an->d_s4, an->d_s4m, an->d_fs, an->d_part, an->d_mpart, an->d_jobs,
+    void *ptrs[] = {an->org.f, an->cur, an->cur_t, an->d_msd, an->d_msdp, an->d_ov, an->d_ovp, an->d_s4, an->d_s4m, an->d_s4p,
+                    an->d_fs, an->d_part, an->d_jobs,
                     an->d_s4_opairs, an->d_s4mask, an->d_s4part};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -624,98 +858,73 @@ extern "C" int ac4_ana_destroy(ac4_ana *an) {
 
 extern "C" int ac4_ana_gap(const ac4_ana *an) { return an ? an->gap : AC4_EARG; }
 
-static bool is_origin(const ac4_ana *an, int pos) {
-    return an->W[0].last_use[pos] >= 0 || an->W[1].last_use[pos] >= 0;
-}
-
-// Runs every pair completed by the frame now in `f` (device arrays).
-static int process_frame(ac4_ana *an, int pos, const double *x, const double *y, const double *z, const int *t) {
+// Runs every job of the frame whose arrays (device) are x, y, z, t; keep: the
+// origin place the frame is copied to, or -1.
+static int process_frame(ac4_ana *an, int pos, const double *x, const double *y, const double *z, const int *t,
+                         int keep) {
     hipStream_t s = an->stream;
-    const int nb = an->nb;
-    for (int w = 0; w < 2; w++) {
-        const std::vector<int> &ps = an->W[w].by_oth[pos];
-        if (ps.empty()) continue;
-        const bool want = w == 0 ? (an->obs & AC4_OBS_MSD) != 0
-                                 : (an->obs & (AC4_OBS_OVERLAP | AC4_OBS_S4 | AC4_OBS_FS)) != 0;
-        if (!want) continue;
-        std::vector<Job> jobs(ps.size());
-        for (size_t k = 0; k < ps.size(); k++) {
-            const int p = ps[k], o = an->W[w].w.cur[p];
-            const Frame &F = an->store[o];
-            AC4_REQUIRE(F.x, AC4_ESTATE, "origin frame %d of pair %d was not pushed", o, p);
-            jobs[k] = Job{F.x, F.y, F.z, p, an->W[w].w.slot[p]};
-        }
-        const int nj = (int)jobs.size();
-        AC4_HIP(hipMemcpyAsync(an->d_jobs, jobs.data(), sizeof(Job) * nj, hipMemcpyHostToDevice, s));
-        if (w == 0) {
-            hipLaunchKernelGGL(k_msd, dim3(nb, nj), dim3(ABLK), 0, s, an->d_jobs, an->n, an->L, x, y, z, t, an->flag,
-                               an->d_part);
-            hipLaunchKernelGGL(k_reduce_jobs, dim3(nj, 1), dim3(256), 0, s, an->d_jobs, nb, 3, an->d_part, an->d_msd);
-        } else {
-            if (an->obs & AC4_OBS_OVERLAP) {
-                hipLaunchKernelGGL(k_overlap, dim3(nb, nj), dim3(ABLK), 0, s, an->d_jobs, an->n, an->L, an->param, x,
-                                   y, z, t, an->flag, an->d_part);
-                hipLaunchKernelGGL(k_reduce_jobs, dim3(nj, 1), dim3(256), 0, s, an->d_jobs, nb, 1, an->d_part, an->d_ov);
-            }
-            if (an->obs & AC4_OBS_S4) {
-                hipLaunchKernelGGL(k_s4_mask, dim3(nb, nj), dim3(ABLK), 0, s, an->d_jobs, an->n, an->L, an->param, x,
-                                   y, z, an->nwords, an->d_s4mask, an->d_mpart);
-                hipLaunchKernelGGL(k_reduce_jobs, dim3(nj, 1), dim3(256), 0, s, an->d_jobs, nb, 1, an->d_mpart, an->d_s4m);
-            }
-            if (an->obs & AC4_OBS_FS) {
-                hipLaunchKernelGGL(k_phase, dim3(nb, NQG, nj), dim3(ABLK), 0, s, an->d_jobs, an->n, x, y, z, t,
-                                   an->flag, an->d_part);
-                hipLaunchKernelGGL(k_reduce_jobs, dim3(nj, (2 * AC4_NQ + 63) / 64), dim3(256), 0, s, an->d_jobs, nb, 2 * AC4_NQ, an->d_part,
-                                   an->d_fs);
-            }
-        }
-        AC4_HIP(hipGetLastError());
-        // jobs[] is a pageable host vector: the copy must finish before it dies
-        AC4_HIP(hipStreamSynchronize(s));
+    const int j0 = an->jptr[pos], nj = an->jptr[pos + 1] - j0;
+    const int nf = an->obs & (AC4_OBS_MSD | AC4_OBS_OVERLAP | AC4_OBS_S4) ? nj : 0;  // Fs has its own kernel
+    if (nf > 0 || keep >= 0) {
+        hipLaunchKernelGGL(k_frame, dim3(an->nb, nf + (keep >= 0 ? 1 : 0)), dim3(ABLK), 0, s, an->d_jobs + j0, nf, an->n,
+                           an->ppb, an->L, an->param, x, y, z, t, an->flag, an->obs, an->org, keep, an->d_msdp,
+                           an->d_ovp, an->d_s4p, an->nwords, an->d_s4mask);
+        an->stale = true;
     }
-    // origins whose last lag this frame was: their S4 sums, before the
-    // origin frames are released
-    if ((an->obs & AC4_OBS_S4) && !an->s4_end[pos].empty()) {
+    if (nj > 0 && (an->obs & AC4_OBS_FS)) {
+        hipLaunchKernelGGL(k_fs, dim3(an->fs_nb, nj), dim3(FS_T), 0, s, an->d_jobs + j0, an->n, an->fs_ppb, x, y, z, t,
+                           an->flag, an->org, an->d_part);
+        hipLaunchKernelGGL(k_reduce_jobs, dim3(nj, (2 * AC4_NQ + 63) / 64), dim3(256), 0, s, an->d_jobs + j0, an->fs_nb,
+                           2 * AC4_NQ, an->d_part, an->d_fs);
+    }
+    AC4_HIP(hipGetLastError());
+    // origins whose last lag this frame was: their S4 sums, before another
+    // origin takes their place
+    if (an->obs & AC4_OBS_S4)
         for (int o : an->s4_end[pos]) TRY(s4_origin(an, o));
-        AC4_HIP(hipStreamSynchronize(s));
-    }
     return AC4_OK;
 }
 
 static int push_common(ac4_ana *an, int pos, const double *x, const double *y, const double *z, const int *t,
-                       hipMemcpyKind kind) {
+                       bool host) {
     AC4_REQUIRE(an && pos >= 0 && pos < an->nframes && x && y && z && t, AC4_EARG, "push_frame: bad arguments");
     AC4_REQUIRE(pos > an->last_pos, AC4_ESTATE, "push_frame: frame %d after %d (frames must increase)", pos,
                 an->last_pos);
     AC4_REQUIRE(!an->finalized, AC4_ESTATE, "push_frame after finalize");
+    for (int j = an->jptr[pos]; j < an->jptr[pos + 1]; j++)
+        AC4_REQUIRE(an->resident[an->jorg[j]], AC4_ESTATE, "origin frame %d of pair %d was not pushed", an->jorg[j],
+                    an->jobs[j].p0 >= 0 ? an->jobs[j].p0 : an->jobs[j].p1);
     hipStream_t s = an->stream;
-    const size_t n = an->n;
-    Frame dst = an->cur;
-    if (is_origin(an, pos)) {
-        TRY(frame_alloc(an->store[pos], an->n));
-        dst = an->store[pos];
+    const size_t n = an->n, b = sizeof(double) * n;
+    int keep = an->place[pos];
+    if (host) {  // an origin frame straight to its place
+        double *dx = an->cur, *dy = dx + n, *dz = dy + n;
+        if (keep >= 0) { dx = an->org.at(keep, 0); dy = an->org.at(keep, 1); dz = an->org.at(keep, 2); }
+        AC4_HIP(hipMemcpyAsync(dx, x, b, hipMemcpyHostToDevice, s));
+        AC4_HIP(hipMemcpyAsync(dy, y, b, hipMemcpyHostToDevice, s));
+        AC4_HIP(hipMemcpyAsync(dz, z, b, hipMemcpyHostToDevice, s));
+        AC4_HIP(hipMemcpyAsync(an->cur_t, t, sizeof(int) * n, hipMemcpyHostToDevice, s));
+        x = dx; y = dy; z = dz; t = an->cur_t;
+        keep = -1;
     }
-    AC4_HIP(hipMemcpyAsync(dst.x, x, sizeof(double) * n, kind, s));
-    AC4_HIP(hipMemcpyAsync(dst.y, y, sizeof(double) * n, kind, s));
-    AC4_HIP(hipMemcpyAsync(dst.z, z, sizeof(double) * n, kind, s));
-    AC4_HIP(hipMemcpyAsync(dst.t, t, sizeof(int) * n, kind, s));
-    AC4_HIP(hipStreamSynchronize(s));
-    TRY(process_frame(an, pos, dst.x, dst.y, dst.z, dst.t));
+    an->resident[pos] = an->place[pos] >= 0;
+    TRY(process_frame(an, pos, x, y, z, t, keep));
+    AC4_HIP(hipStreamSynchronize(s));  // the caller may reuse its arrays
+    // origins no pair needs any more (their places may be taken from now on)
+    for (int f = an->last_pos + 1; f <= pos; f++)
+        for (int o : an->ends[f]) an->resident[o] = 0;
     an->last_pos = pos;
-    // release origins no pair needs any more
-    for (int o = 0; o <= pos; o++)
-        if (an->store[o].x && an->W[0].last_use[o] <= pos && an->W[1].last_use[o] <= pos) frame_free(an->store[o]);
     return AC4_OK;
 }
 
 extern "C" int ac4_ana_push_frame(ac4_ana *an, int pos, const double *x, const double *y, const double *z,
                                   const int *type) {
-    return push_common(an, pos, x, y, z, type, hipMemcpyHostToDevice);
+    return push_common(an, pos, x, y, z, type, true);
 }
 
 extern "C" int ac4_ana_push_frame_device(ac4_ana *an, int pos, const double *x, const double *y, const double *z,
                                          const int *type) {
-    return push_common(an, pos, x, y, z, type, hipMemcpyDeviceToDevice);
+    return push_common(an, pos, x, y, z, type, false);
 }
 
 extern "C" int ac4_md_device_xu(ac4_md *md, int r, const double **xu, const double **yu, const double **zu,
@@ -727,7 +936,7 @@ extern "C" int ac4_ana_push_md(ac4_ana *an, int pos, ac4_md *md, int r) {
     TRY(ac4_md_device_xu(md, r, &x, &y, &z, &t, &n));
     AC4_REQUIRE(an && n == an->n, AC4_EARG, "push_md: replica has %d particles, analysis expects %d", n,
                 an ? an->n : -1);
-    return push_common(an, pos, x, y, z, t, hipMemcpyDeviceToDevice);
+    return push_common(an, pos, x, y, z, t, false);
 }
 
 static int slots_run(ac4_ana *an, int w, const double *dvals, int nv, int mode, double div, std::vector<double> &sum,
@@ -765,12 +974,28 @@ static void split_phase(const std::vector<double> &in, int ns, std::vector<doubl
         }
 }
 
+// Every pair's MSD sums and overlap counts from its blocks' values
+static int sum_blocks(ac4_ana *an) {
+    if (!an->stale) return AC4_OK;
+    const int np0 = an->W[0].w.np, np1 = an->W[1].w.np;
+    if ((an->obs & AC4_OBS_MSD) && np0 > 0)
+        hipLaunchKernelGGL(k_msd_pairs, dim3(np0), dim3(ABLK), 0, an->stream, an->d_msdp, an->nb, an->d_msd);
+    if ((an->obs & AC4_OBS_OVERLAP) && np1 > 0)
+        hipLaunchKernelGGL(k_counts, dim3(np1), dim3(64), 0, an->stream, an->d_ovp, an->nb, an->d_ov);
+    if ((an->obs & AC4_OBS_S4) && np1 > 0)
+        hipLaunchKernelGGL(k_counts, dim3(np1), dim3(64), 0, an->stream, an->d_s4p, an->nb, an->d_s4m);
+    AC4_HIP(hipGetLastError());
+    an->stale = false;
+    return AC4_OK;
+}
+
 extern "C" int ac4_ana_finalize(ac4_ana *an) {
     AC4_REQUIRE(an, AC4_EARG, "NULL handle");
     if (an->finalized) return AC4_OK;
     if (an->obs & AC4_OBS_S4)  // origins whose last lag frame was never pushed
         for (int o = 0; o < an->nframes; o++)
-            if (!an->s4_done[o] && an->store[o].x && an->s4_optr[o + 1] > an->s4_optr[o]) TRY(s4_origin(an, o));
+            if (!an->s4_done[o] && an->resident[o] && an->s4_optr[o + 1] > an->s4_optr[o]) TRY(s4_origin(an, o));
+    TRY(sum_blocks(an));
     AC4_HIP(hipStreamSynchronize(an->stream));
     const double tot = an->flag == 1 ? 0.8 * an->n : (double)an->n;  // msd_pos.c:26-27
     for (int w = 0; w < 2; w++) {  // counters and delta_t (msd_pos.c:90-92)
@@ -868,23 +1093,19 @@ extern "C" int ac4_ana_npairs(const ac4_ana *an, int obs) {
 
 extern "C" int ac4_ana_get_pairs(ac4_ana *an, int obs, double *vals, int *ivals) {
     AC4_REQUIRE(an && (an->obs & obs), AC4_ESTATE, "get_pairs: observable not requested");
+    TRY(sum_blocks(an));
     AC4_HIP(hipStreamSynchronize(an->stream));
     const size_t np = obs == AC4_OBS_MSD ? an->W[0].w.np : an->W[1].w.np;
     if (np == 0) return AC4_OK;
     if (obs == AC4_OBS_MSD && vals) AC4_HIP(hipMemcpy(vals, an->d_msd, sizeof(double) * 3 * np, hipMemcpyDeviceToHost));
-    if (obs == AC4_OBS_OVERLAP && ivals) {
+    const double *cnt = obs == AC4_OBS_OVERLAP ? an->d_ov : (obs == AC4_OBS_S4 ? an->d_s4m : nullptr);
+    if (cnt && ivals) {
         std::vector<double> v(np);
-        AC4_HIP(hipMemcpy(v.data(), an->d_ov, sizeof(double) * np, hipMemcpyDeviceToHost));
+        AC4_HIP(hipMemcpy(v.data(), cnt, sizeof(double) * np, hipMemcpyDeviceToHost));
         for (size_t p = 0; p < np; p++) ivals[p] = (int)v[p];
     }
-    if (obs == AC4_OBS_S4) {
-        if (vals) AC4_HIP(hipMemcpy(vals, an->d_s4, sizeof(double) * 2 * AC4_NQ * np, hipMemcpyDeviceToHost));
-        if (ivals) {
-            std::vector<double> v(np);
-            AC4_HIP(hipMemcpy(v.data(), an->d_s4m, sizeof(double) * np, hipMemcpyDeviceToHost));
-            for (size_t p = 0; p < np; p++) ivals[p] = (int)v[p];
-        }
-    }
+    if (obs == AC4_OBS_S4 && vals)
+        AC4_HIP(hipMemcpy(vals, an->d_s4, sizeof(double) * 2 * AC4_NQ * np, hipMemcpyDeviceToHost));
     if (obs == AC4_OBS_FS && vals) AC4_HIP(hipMemcpy(vals, an->d_fs, sizeof(double) * 2 * AC4_NQ * np, hipMemcpyDeviceToHost));
     return AC4_OK;
 }

@@ -91,3 +91,68 @@ def test_force_team_widths(gpu, prec, n):
     assert np.abs(fa - fb).max() <= 4e-12 * np.sqrt((fb ** 2).mean())
     # energy and virial: FP32 partial sums of eight pairs in FP32 mode
     assert np.allclose(pa, pb, rtol=1e-11 if prec == 0 else 1e-6)
+
+
+# Particle counts around the tiles of the frame kernel (256) and of the Fs
+# kernel (32, loads of 256), and one large enough for several of each per
+# workgroup; with and without the B particles.
+@pytest.mark.parametrize("n,flag", [(1, 0), (31, 0), (32, 1), (33, 0), (255, 1), (257, 0), (513, 0), (70001, 1)])
+def test_frame_and_fs_tile_edges(gpu, n, flag):
+    frames = [0, 1, 2, 3, 10, 11]
+    X, Y, Z, T = trajgen.make_frames(n, frames, 7 + n, 0.08, 1.0)
+    L = max(4.0, (n / 1.2) ** (1.0 / 3.0))
+    an = gpu.Analysis(n, L, frames, gap=10, obs=11 if n > 1000 else 15, type_flag=flag)
+    for f in range(len(frames)):
+        an.push(f, X[f], Y[f], Z[f], T[f])
+    om = OL.msd(n, L, X, Y, Z, T, frames, 10, flag=flag)
+    assert np.allclose(an.pairs(gpu.OBS_MSD), om["pairs"], rtol=1e-12, atol=0)
+    oo = OL.overlap(n, L, X, Y, Z, T, frames, 10, flag=flag)
+    assert len(oo["pairs"]) == 4 and np.array_equal(an.pairs(gpu.OBS_OVERLAP), oo["pairs"])
+    an.finalize()
+    ofs = OL.phase("fs", n, L, X, Y, Z, T, frames, 10, flag=flag)
+    assert np.abs(an.pairs(gpu.OBS_FS) - ofs["pairs"]).max() < 1e-12 * n  # a term is off by at most a few 1e-14
+    if n <= 1000:
+        os4 = OL.phase("s4", n, L, X, Y, Z, T, frames, 10)
+        v, m = an.pairs(gpu.OBS_S4)
+        assert np.array_equal(m, os4["mask"]) and np.abs(v - os4["pairs"]).max() < 1e-12 * n
+
+
+def test_frames_that_never_arrive(gpu):
+    """A lag frame whose origin was left out is refused, an origin's lag frame
+    may be left out: the pairs that arrived are those of the full walk."""
+    n, frames = 300, trajgen.case_frames(3, 30)
+    X, Y, Z, T = trajgen.make_frames(n, frames, 5, 0.08, 1.0)
+    L = (n / 1.2) ** (1.0 / 3.0)
+    an = gpu.Analysis(n, L, frames, gap=30)
+    with pytest.raises(gpu.AC4Error, match="origin frame 0 of pair 0 was not pushed"):
+        an.push(1, X[1], Y[1], Z[1], T[1])
+    oo = OL.overlap(n, L, X, Y, Z, T, frames, 30)
+    om = OL.msd(n, L, X, Y, Z, T, frames, 30)
+    an = gpu.Analysis(n, L, frames, gap=30)
+    left_out = [k for k in range(len(frames)) if frames[k] % 30 and k % 4 == 1]
+    for f in range(len(frames)):
+        if f not in left_out:
+            an.push(f, X[f], Y[f], Z[f], T[f])
+    an.finalize()
+    got, want = an.pairs(gpu.OBS_OVERLAP), oo["pairs"]
+    lag = np.array([frames.index(o + l) for o, l in _walk(frames, 30)])
+    here = ~np.isin(lag, left_out)
+    assert 0 < here.sum() < len(want)
+    assert np.array_equal(got[here], want[here]) and not got[~here].any()
+    assert np.allclose(an.pairs(gpu.OBS_MSD)[:len(here)][here[:len(om["pairs"])]], om["pairs"][here[:len(om["pairs"])]],
+                       rtol=1e-12, atol=0)
+
+
+def _walk(frames, gap):
+    """(origin step, lag) of every pair of the overlap walk, in its order."""
+    pos, on = set(frames), 0
+    while on * gap + 1 in pos:
+        on += 1
+    out, k = [], 0
+    while k * gap in pos:
+        off = 1
+        while off < int(on * gap / 2.0) and k * gap + off in pos:
+            out.append((k * gap, off))
+            off = off + 1 if int(off * 1.4) == off else int(off * 1.4)
+        k += 1
+    return out
