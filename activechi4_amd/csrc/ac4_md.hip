@@ -16,10 +16,8 @@
 //   k_bin .. k_nlist_team   counting-sort cell build + neighbour lists,
 //                  executed only for replicas whose displacement criterion
 //                  fired (flag read on device, so the sequence is graphable)
-//   k_force        pair forces + active force + second U2 kick + block
-//                  partial sums
-//   k_force_end    per replica: the partials summed in block order, U4 U3 U4
-//                  (chain end).
+//   k_force        pair forces + active force + second U2 kick; in the last
+//                  workgroups the sums per replica and U4 U3 U4 (chain end)
 // The momentum factor of the last U3 is kept pending (p_scale) and applied at
 // the next first half, so a step needs one sum of p^2 instead of four.
 #include <hip/hip_runtime.h>
@@ -118,7 +116,7 @@ __device__ __forceinline__ double minimg_md(double d) {  // cell_list+forces.c:9
 // is below 3e-19, and exp(-x) = 1 - x phi: within an ulp, where 1 - exp(-x)
 // loses the digits that cancel.  The chain runs on one lane between two
 // kernels of the step, so the length of its serial chain of operations is
-// what it costs: k_force_end 4.1 -> 3.5 us on one box of N=1000 with this,
+// what it costs: 4.1 -> 3.5 us (with the sums) on one box of N=1000 with this,
 // the reciprocals of q and the start-of-step half kept from k_first_half.
 __host__ __device__ inline double exp_phi(double x, double *phi) {
     if (fabs(x) < 0.0625) {
@@ -187,6 +185,40 @@ __device__ __forceinline__ bool need_rebuild(const RepC &R, const ChainS &c) {
     return (c.crit == 1 ? 3.0 : 4.0) * maxD > R.skin * R.skin;  // :508 (crit 1, skin 0.35 there)
 }
 
+// The last workgroup of a replica to finish a kernel does what follows it for
+// the whole replica (k_force: sums and chain update; k_bin: scan of the cell
+// counts).  What the workgroups hand over goes through agent-scope relaxed
+// stores and loads, which are coherent between the XCDs' L2s by themselves:
+// the giver waits for its stores to arrive (wait_stores) before it counts
+// itself done, and the last one, told by the count, reads.  An agent-scope
+// release or acquire fence instead writes back and invalidates the L2 of the
+// workgroup's XCD (buffer_wbl2, buffer_inv) and costs every other workgroup
+// its gathers' L2 hits (k_force 42.3 -> 55.6 us on the 64-replica ensemble).
+// Nothing waits for another workgroup.
+__device__ __forceinline__ void st_agent(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ld_agent(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int ld_agent(const int *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Counts that several parties reach at once lie a line (DONE_PAD ints) apart:
+// atomics on one line are done one after the other across the device (about
+// 8 ns each; with the groups' counts side by side k_force at N=10000 was 4 us
+// longer).
+#define DONE_PAD 32
+// one more of the `of` parties is done; true for the last, whose count starts the next launch at zero
+__device__ __forceinline__ bool last_done(unsigned *count, int of) {
+    const unsigned k = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (k + 1u != (unsigned)of) return false;
+    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::: "memory");  // what the others handed over is read after this
+    return true;
+}
+
 // Rebuild work of one step: the blocks of the replicas due for a rebuild,
 // appended by k_bin_end for each such replica, so the kernels after
 // k_bin run a fixed grid over this list instead of one workgroup per block of
@@ -219,7 +251,7 @@ static inline int xcd_grid(int nb) { return ((nb + N_XCD - 1) / N_XCD) * N_XCD; 
 // on the array, so the 256 lanes draw them SHUF_CH at a time into LDS and one
 // lane applies the swaps in order.  The component lives in dynamic LDS when
 // it fits (kcap bytes, sized from the device's LDS per workgroup), else in
-// global memory.  The shuffle counter is advanced by k_force_end (or
+// global memory.  The shuffle counter is advanced by force_end (or
 // the host for an explicit shuffle), after every component has read it.
 #define SHUF_CH 4096
 #define SHUF_PAR_MIN 16384  // active sets above this take the parallel path (k_shuf_part, k_shuf_apply)
@@ -459,7 +491,7 @@ __global__ void __launch_bounds__(BLK) k_first_half(const RepC *__restrict__ rep
         double eta[3] = {c.eta[0], c.eta[1], c.eta[2]}, peta[3] = {c.peta[0], c.peta[1], c.peta[2]}, S2;
         s_scale[0] = c.p_scale;
         s_scale[1] = (c.mode == 0 && R.n > 0) ? nhc_half(c.S_end, R.T, R.dof, c.q, eta, peta, &S2) : 1.0;
-        if (blk_idx[b] == 0)  // the chain at this point of the step, for k_force_end
+        if (blk_idx[b] == 0)  // the chain at this point of the step, for force_end
             for (int k = 0; k < 3; k++) { mid[6 * r + k] = eta[k]; mid[6 * r + 3 + k] = peta[k]; }
     }
     __syncthreads();
@@ -540,14 +572,69 @@ __device__ __forceinline__ int clampc(int c, int n) { return min(max(c, 0), n - 
 // InCell[cell][MaxPartInCell], MDcode/global.h:20,85; a fuller cell sets the
 // capacity error).  key: the octant of the cell the particle is in (x bit
 // highest where the list teams cull, else z), then its id, the order
-// k_cell_sort puts the cell in.  k_bin_end
-// then turns the cell counts into start offsets.
+// k_cell_sort puts the cell in.  The replica's last workgroup (fuse; else
+// k_bin_end) then turns the cell counts into start offsets.
+// The cell counts of a replica due for a rebuild turned into start offsets
+// (exclusive scan) and the replica's share of the step's rebuild work appended
+// to the work list, by one workgroup of nt threads.
+#define BIN_END_T 1024
+template <bool AGENT>
+__device__ __forceinline__ void bin_end(const RepC &R, int r, const int *cnt, int *start, WorkList wl, int nt, int *s_w,
+                                        int *s_base) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int *vc = cnt + R.off_cell;
+    const int per = (R.ncell + nt - 1) / nt;
+    const int c0 = min((int)threadIdx.x * per, R.ncell), c1 = min(c0 + per, R.ncell);
+    int own = 0;
+    for (int q = c0; q < c1; q++) own += AGENT ? ld_agent(vc + q) : vc[q];
+    int v = own;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(v, o, 64);
+        if (lane >= o) v += t;
+    }
+    if (lane == 63) s_w[w] = v;
+    __syncthreads();
+    int acc = v - own;
+    for (int k = 0; k < w; k++) acc += s_w[k];
+    for (int q = c0; q < c1; q++) {
+        start[R.off_cell + q] = acc;
+        acc += AGENT ? ld_agent(vc + q) : vc[q];
+    }
+    // this replica's share of the step's rebuild work
+    const int nb = (R.n + BLK - 1) / BLK, nl = (R.n + LPB - 1) / LPB, ncb = (R.ncell + BLK / 64 - 1) / (BLK / 64);
+    if (threadIdx.x == 0) {
+        s_base[0] = atomicAdd(&wl.n[0], nb);
+        s_base[1] = atomicAdd(&wl.n[1], nl);
+        s_base[2] = atomicAdd(&wl.n[2], ncb);
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < nb; q += nt) wl.item[s_base[0] + q] = R.blk_off + q;
+    for (int q = threadIdx.x; q < nl; q += nt) wl.item[wl.off_l + s_base[1] + q] = R.lblk_off + q;
+    for (int q = threadIdx.x; q < ncb; q += nt) wl.item[wl.off_c + s_base[2] + q] = (r << 16) | q;
+}
+
+// The same as a kernel of its own, one workgroup per replica, for handles
+// with a slot of more than BIN_FUSE_CELLS cells, whose scan would be long for
+// a k_bin workgroup (BIN_END_T threads there).
+#define BIN_FUSE_CELLS 4096
+__global__ void __launch_bounds__(BIN_END_T) k_bin_end(const RepC *__restrict__ reps,
+                                                       const ChainS *__restrict__ chain, const int *__restrict__ cnt,
+                                                       int *start, WorkList wl) {
+    __shared__ int s_w[BIN_END_T / 64], s_base[3];
+    const int r = blockIdx.x;
+    const RepC R = reps[r];
+    if (!need_rebuild(R, chain[r])) return;  // uniform over the workgroup
+    bin_end<false>(R, r, cnt, start, wl, blockDim.x, s_w, s_base);
+}
+
 #define CELL_CAP 600
 __global__ void __launch_bounds__(BLK) k_bin(const RepC *__restrict__ reps, ChainS *chain,
                                              const int *__restrict__ blk_rep, const int *__restrict__ blk_first,
                                              const double *__restrict__ x, const double *__restrict__ y,
                                              const double *__restrict__ z, const int *__restrict__ id, int *cnt,
-                                             int *cell_of, int2 *cell_mem, int *cell_ref) {
+                                             int *cell_of, int2 *cell_mem, int *cell_ref, int fuse, unsigned *done,
+                                             int *start, WorkList wl) {
+    __shared__ int s_w[BLK / 64], s_base[3], s_last;
     const int b = blockIdx.x, r = blk_rep[b];
     const RepC R = reps[r];
     if (!need_rebuild(R, chain[r])) return;  // uniform over the replica's blocks
@@ -606,52 +693,13 @@ __global__ void __launch_bounds__(BLK) k_bin(const RepC *__restrict__ reps, Chai
         if (my_rank < CELL_CAP) cell_mem[(size_t)(R.off_cell + c) * CELL_CAP + my_rank] = make_int2(i, key);
         else atomicOr(&chain[r].err, 1);
     }
-}
-
-// After k_bin, one workgroup per replica due for a rebuild: the cell counts
-// turned into start offsets (exclusive scan) and the replica's share of the
-// step's rebuild work appended to the work list.  A kernel of its own rather
-// than the last k_bin block of each replica, which needs an agent-scope
-// fence per block (on gfx950 a write-back and invalidation of the XCD's L2).
-// BIN_END_T threads per replica where a slot holds more than BIN_END_T cells
-// (fixed per handle at creation), else BLK.
-#define BIN_END_T 1024
-__global__ void __launch_bounds__(BIN_END_T) k_bin_end(const RepC *__restrict__ reps,
-                                                       const ChainS *__restrict__ chain, const int *__restrict__ cnt,
-                                                       int *start, WorkList wl) {
-    __shared__ int s_w[BIN_END_T / 64], s_base[3];
-    const int r = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, nt = blockDim.x;
-    const RepC R = reps[r];
-    if (!need_rebuild(R, chain[r])) return;  // uniform over the workgroup
-    const int *vc = cnt + R.off_cell;
-    const int per = (R.ncell + nt - 1) / nt;
-    const int c0 = min((int)threadIdx.x * per, R.ncell), c1 = min(c0 + per, R.ncell);
-    int own = 0;
-    for (int q = c0; q < c1; q++) own += vc[q];
-    int v = own;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(v, o, 64);
-        if (lane >= o) v += t;
-    }
-    if (lane == 63) s_w[w] = v;
+    if (!fuse) return;
+    wait_stores();  // this wave's counts are in
     __syncthreads();
-    int acc = v - own;
-    for (int k = 0; k < w; k++) acc += s_w[k];
-    for (int q = c0; q < c1; q++) {
-        start[R.off_cell + q] = acc;
-        acc += vc[q];
-    }
-    // this replica's share of the step's rebuild work
-    const int nb = (R.n + BLK - 1) / BLK, nl = (R.n + LPB - 1) / LPB, ncb = (R.ncell + BLK / 64 - 1) / (BLK / 64);
-    if (threadIdx.x == 0) {
-        s_base[0] = atomicAdd(&wl.n[0], nb);
-        s_base[1] = atomicAdd(&wl.n[1], nl);
-        s_base[2] = atomicAdd(&wl.n[2], ncb);
-    }
+    if (threadIdx.x == 0) s_last = last_done(done + r * DONE_PAD, R.nblk);
     __syncthreads();
-    for (int q = threadIdx.x; q < nb; q += nt) wl.item[s_base[0] + q] = R.blk_off + q;
-    for (int q = threadIdx.x; q < nl; q += nt) wl.item[wl.off_l + s_base[1] + q] = R.lblk_off + q;
-    for (int q = threadIdx.x; q < ncb; q += nt) wl.item[wl.off_c + s_base[2] + q] = (r << 16) | q;
+    if (!s_last) return;
+    bin_end<true>(R, r, cnt, start, wl, BLK, s_w, s_base);
 }
 
 // Distinct neighbour-cell coordinates along one axis (cells are at least one
@@ -1570,23 +1618,28 @@ __device__ __forceinline__ void ld_list(const int *p, int *j) {
 // entries c*W ... c*W + W - 1, cs list words apart); the others read chunks
 // of 8 entries, cs words apart, with W = 8 / |VEC| lanes: VEC > 1 takes VEC
 // consecutive entries of a chunk in one load, VEC < -1 entries t, t + W, ...
-// of it, |VEC| rows per chunk.
+// of it, |VEC| rows per chunk, and six entries per group (FP64 only: 128
+// vector registers in k_force instead of 148, four waves per SIMD instead of
+// three; us per step at N=50000 50.7 -> 50.1, 80000 63.5 -> 61.4, 200000
+// 104 -> 99.5.  Teams of 8 and 16 lanes, whose lists are one or two groups,
+// keep eight: 22.0 against 22.8 at N=10000).
 template <int VEC, bool EN, class PosT, class Acc>
 __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t, int m, int g,
                                           const PosT *__restrict__ pos, const PosT &pi, Acc &acc) {
     constexpr int V = VEC > 1 ? VEC : 1;    // entries of a load
     constexpr int RC = VEC < 0 ? -VEC : 1;  // rows per step of cs
-    constexpr int NR = 8 / V;               // rows of a group
+    constexpr int G = VEC < 0 ? 6 : 8;      // entries of a group
+    constexpr int NR = G / V;               // rows of a group
     const int rl = W * V, full = m / rl;    // entries of a row, whole rows
-    int c = 0, jn[8];
+    int c = 0, jn[G];
     if (NR <= full) {
 #pragma unroll
         for (int r = 0; r < NR; r++) ld_list<V>(lp + (r / RC) * cs + (r % RC) * W, jn + V * r);
     }
     while (c + NR <= full) {
-        PosT q[8];
+        PosT q[G];
 #pragma unroll
-        for (int u = 0; u < 8; u++) q[u] = ld_pos(pos, jn[u]);
+        for (int u = 0; u < G; u++) q[u] = ld_pos(pos, jn[u]);
         c += NR;
         lp += (NR / RC) * cs;
         if (c + NR <= full) {
@@ -1594,13 +1647,13 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
             for (int r = 0; r < NR; r++) ld_list<V>(lp + (r / RC) * cs + (r % RC) * W, jn + V * r);
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) acc.template add<EN>(pi, q[u]);
+        for (int u = 0; u < G; u++) acc.template add<EN>(pi, q[u]);
         acc.template flush<EN>();
     }
     const int k0 = c * rl + t * V;  // this lane's first entry of the last group
     if (k0 < m) {
-        int jt[8];
-        PosT q[8];
+        int jt[G];
+        PosT q[G];
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             int *j = jt + V * r;
@@ -1612,179 +1665,23 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
             }
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) q[u] = ld_pos(pos, k0 + (u / V) * rl + u % V < m ? jt[u] : g);
+        for (int u = 0; u < G; u++) q[u] = ld_pos(pos, k0 + (u / V) * rl + u % V < m ? jt[u] : g);
 #pragma unroll
-        for (int u = 0; u < 8; u++)
+        for (int u = 0; u < G; u++)
             if (k0 + (u / V) * rl + u % V < m) acc.template add<EN>(pi, q[u]);
         acc.template flush<EN>();
     }
 }
 
-// Pair forces: a team of W = 2^lw lanes per particle (fixed per handle at
-// creation, so a replica's results do not depend on what else is loaded)
-// walks the particle's list (walk_list); the team's partial forces are
-// combined by a fixed butterfly.  Each block writes its partial sums of p^2
-// and p_x, and with EN of PE and virial; k_force_end reduces them per
-// replica.  A block's loads form a short chain (block table, then position,
-// list length, active index and momentum together, then list, then
-// neighbour positions): on small boxes, a few waves per CU, the launch is as
-// long as that chain.  Each loaded where it was used, with the constants
-// divided out per lane and the sums shuffled through LDS: 7.2 us at N=1000
-// FP64 and 11.0 at N=10000 FP32 (four lanes); this 5.9 and 7.0 (sixteen).
-// EN = false leaves out the pair energy and virial, which every step
-// overwrites and only the call's last one reports: 9 of 55 instructions of
-// an FP32 pair.  (FP32 handles whose team is not the list layout's form them in
-// k_energy.)
-template <bool FP32, bool KICK, bool EN, int VEC>
-__global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, const BlkD *__restrict__ fblk,
-                                               const double4 *__restrict__ pos4, const QPos *__restrict__ posq,
-                                               const int *__restrict__ nn,
-                                               const int *__restrict__ nl, int cap, int lw, int lc,
-                                               const int *__restrict__ act,
-                                               const int8_t *__restrict__ kx, const int8_t *__restrict__ ky,
-                                               const int8_t *__restrict__ kz, double *fx, double *fy, double *fz,
-                                               double *px, double *py, double *pz, double *partial, int nb) {
-    __shared__ double s_red[4][BLK / 64];
-    const int b = xcd_block(nb);
-    if (b < 0) return;
-    const BlkD D = fblk[b];
-    const int W = 1 << lw, t = threadIdx.x & (W - 1);
-    const int i = D.first + (threadIdx.x >> lw);
-    double v_p2 = 0.0, v_pe = 0.0, v_vir = 0.0, v_px = 0.0;
-    double Fx = 0.0, Fy = 0.0, Fz = 0.0;
-    const bool valid = i < D.n;
-    const int g = D.off + (valid ? i : 0);
-    // FP64: the wrapped box fractions; FP32: their fixed-point copy
-    using PosT = typename std::conditional<FP32, QPos, double4>::type;
-    const PosT *__restrict__ pos = (const PosT *)(FP32 ? (const void *)posq : (const void *)pos4);
-    const PosT pi = ld_pos(pos, g);
-    const int m = valid ? nn[g] : 0;
-    const int a = act[g];
-    double vx = 0.0, vy = 0.0, vz = 0.0;
-    if (KICK) { vx = px[g]; vy = py[g]; vz = pz[g]; }
-    const RepC &R = reps[D.rep];
-    const bool active = a >= 0;
-    const int ka = R.off_act + (active ? a : 0);
-    const double kfx = (double)kx[ka], kfy = (double)ky[ka], kfz = (double)kz[ka];
-    PairAcc<FP32> acc(ptype(pi), R);
-    // entry e of particle i's list (nl_at): VEC = 1, W >= 2^lc, rows of W
-    // entries are W * n words apart; else the chunks of 8 entries, 8 * n
-    const size_t e0 = (size_t)(VEC > 1 ? t * VEC : t);
-    const int *lp = nl + (size_t)D.off * cap + ((((e0 >> lc) * D.n + (g - D.off)) << lc) + (e0 & ((1u << lc) - 1u)));
-    walk_list<VEC, EN>(lp, (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, pos, pi, acc);
-    acc.result(Fx, Fy, Fz, R);
-    v_pe = acc.pe;
-    v_vir = acc.vir;
-    Fx = team_sum(Fx, lw);
-    Fy = team_sum(Fy, lw);
-    Fz = team_sum(Fz, lw);
-    if (valid && t == 0) {
-        if (active) {  // cell_list+forces.c:207-213
-            Fx += R.f0 * kfx;
-            Fy += R.f0 * kfy;
-            Fz += R.f0 * kfz;
-        }
-        fx[g] = Fx; fy[g] = Fy; fz[g] = Fz;
-        if (KICK) {  // U2 after the forces, time_evolve.c:516
-            vx += Fx * K_HALF_DT; vy += Fy * K_HALF_DT; vz += Fz * K_HALF_DT;
-            px[g] = vx; py[g] = vy; pz[g] = vz;
-            v_p2 = vx * vx + vy * vy + vz * vz;
-            v_px = vx;
-        }
-    }
-    const double v[4] = {v_p2, v_pe, v_vir, v_px};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (!EN && (q == 1 || q == 2)) continue;
-        const double w = wave_sum_rows(v[q]);
-        if ((threadIdx.x & 63) == 0) s_red[q][threadIdx.x >> 6] = w;
-    }
-    __syncthreads();
-    if (threadIdx.x < 4 && (EN || threadIdx.x == 0 || threadIdx.x == 3)) {
-        double s = 0.0;
-        for (int w = 0; w < BLK / 64; w++) s += s_red[threadIdx.x][w];
-        partial[4 * (size_t)b + threadIdx.x] = s;
-    }
-}
-
-// Pair energy and virial of FP32 handles whose force team is not the list
-// layout's team of 2^lw lanes: that team walks the list (entries t, t + W, ...;
-// one lane: chunks of 8) and sums the FP32 terms of eight entries before it
-// widens them, so the partial sums, whose rounding shows in the seventh to
-// ninth digit of the energy, do not depend on the force kernel's width.  Runs
-// once per call, after its last step (k_energy_end then completes the step's
-// reported values).
-template <int VEC>
-__global__ void __launch_bounds__(BLK) k_energy(const RepC *__restrict__ reps, const BlkD *__restrict__ eblk,
-                                                const QPos *__restrict__ posq, const int *__restrict__ nn,
-                                                const int *__restrict__ nl, int cap, int lw, double *epart, int nb) {
-    __shared__ double s_red[2][BLK / 64];
-    const int b = xcd_block(nb);
-    if (b < 0) return;
-    const BlkD D = eblk[b];
-    const int W = 1 << lw, t = threadIdx.x & (W - 1), i = D.first + (threadIdx.x >> lw);
-    const bool valid = i < D.n;
-    const int il = valid ? i : 0, g = D.off + il;
-    const QPos pi = ld_pos(posq, g);
-    const int m = valid ? nn[g] : 0;
-    PairAcc<true> acc(ptype(pi), reps[D.rep]);
-    walk_list<VEC, true>(nl + (size_t)D.off * cap + (size_t)il * (VEC == 1 ? W : 8) + t,
-                         (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, posq, pi, acc);
-    const double v[2] = {wave_sum_rows(acc.pe), wave_sum_rows(acc.vir)};
-    if ((threadIdx.x & 63) == 0)
-        for (int q = 0; q < 2; q++) s_red[q][threadIdx.x >> 6] = v[q];
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        double s = 0.0;
-        for (int w = 0; w < BLK / 64; w++) s += s_red[threadIdx.x][w];
-        epart[2 * (size_t)b + threadIdx.x] = s;
-    }
-}
-
-// End of the force pass, one workgroup per replica after k_force: the block
-// partials summed in a fixed order (thread t of nt takes blocks t, t+nt, ...;
-// a fixed butterfly per wave; the waves in order), then the end-of-step chain
-// update.  nt = 64, or 256 where a replica has more than 64 force blocks
-// (fixed per handle at creation).  A kernel of its own
-// rather than the last force block of each replica: that pattern needs an
-// agent-scope release fence in every block, which on gfx950 writes back and
-// invalidates the L2 of the block's XCD (buffer_wbl2 / buffer_inv), and the
-// invalidations cost the neighbour gathers of every other block their L2
-// hits (k_force 55.6 -> 42.3 us on the 64-replica ensemble without them).
-// EN: the pass summed the pair energy and virial (the last step of a call;
-// they are only reported).  apart: k_energy forms them after the call's last
-// step, and Heff is stored without the pair energy for it.
+// End of the force pass for one replica, on one lane: the sums a4 = {p^2, PE,
+// virial, p_x} (PE and virial with EN only) to the end-of-step chain update.
+// c0: the chain as it is; eta, peta: after the start-of-step half
+// (k_first_half).  EN: the pass summed the pair energy and virial (the last
+// step of a call; they are only reported).  apart: k_energy forms them after
+// the call's last step, and Heff is stored without the pair energy for it.
 template <bool KICK, bool EN>
-__global__ void __launch_bounds__(256) k_force_end(const RepC *__restrict__ reps, ChainS *chain,
-                                                   const double *__restrict__ partial, int apart,
-                                                   const double *__restrict__ mid) {
-    __shared__ double s_w[4][4];
-    const int r = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, nt = blockDim.x;
-    const RepC R = reps[r];
-    ChainS &c = chain[r];
-    ChainS c0;           // loaded beside the partials, not after them
-    double eta[3], peta[3];  // after the start-of-step half (k_first_half)
-    if (KICK && threadIdx.x == 0) {
-        c0 = c;
-        for (int k = 0; k < 3; k++) { eta[k] = mid[6 * r + k]; peta[k] = mid[6 * r + 3 + k]; }
-    }
-    double a4[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int k = threadIdx.x; k < R.fnblk; k += nt) {  // thread t: blocks t, t+nt, ...
-        const double *pp = partial + 4 * (size_t)(R.fblk_off + k);
-        a4[0] += pp[0]; a4[3] += pp[3];
-        if (EN) { a4[1] += pp[1]; a4[2] += pp[2]; }
-    }
-    for (int q = 0; q < 4; q++)
-        if (EN || q == 0 || q == 3) a4[q] = wave_sum_rows(a4[q]);
-    if (lane == 0)
-        for (int q = 0; q < 4; q++) s_w[w][q] = a4[q];
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int q = 0; q < 4; q++) {
-        a4[q] = s_w[0][q];
-        for (int k = 1; k < nt / 64; k++) a4[q] += s_w[k][q];
-    }
-    if (R.n == 0) return;  // idle slot
+__device__ __forceinline__ void force_end(const RepC &R, ChainS &c, const ChainS &c0, double *eta, double *peta,
+                                          const double *a4, int apart) {
     double S = a4[0], pe = a4[1], vir = a4[2], spx = a4[3];  // pe, vir: zero without EN
     pe = 0.5 * pe;                  // every pair seen from both sides
     vir = (0.5 * vir) / (3.0e0);   // cell_list+forces.c:220
@@ -1853,8 +1750,188 @@ __global__ void __launch_bounds__(256) k_force_end(const RepC *__restrict__ reps
     c.step = c0.step + 1;
 }
 
+// What k_force's last workgroups need: the chains, the chain variables after
+// the start-of-step half, the partial sums of groups of FORCE_GRP blocks and
+// the counts of finished blocks of each group and groups of each replica.
+#define FORCE_GRP 64
+struct EndArgs {
+    ChainS *chain;
+    const double *mid;
+    double *gpart;
+    unsigned *gdone, *rdone;
+    int apart;
+};
+
+// Pair forces: a team of W = 2^lw lanes per particle (fixed per handle at
+// creation, so a replica's results do not depend on what else is loaded)
+// walks the particle's list (walk_list); the team's partial forces are
+// combined by a fixed butterfly.  Each block hands over its partial sums of
+// p^2 and p_x, and with EN of PE and virial; the last block of each FORCE_GRP
+// adds theirs up (lane k block k, a fixed butterfly), the replica's last group
+// adds the groups' in a fixed order and updates the chain (force_end).  Two levels: atomics on one line are done one after the other.
+// As a kernel of their own after this
+// one, sums and update took 3.5 us of N=1000's step, 5.1 of N=50000's and
+// 11.4 of N=1e6's.  A block's loads form a short chain (block table, then position,
+// list length, active index and momentum together, then list, then
+// neighbour positions): on small boxes, a few waves per CU, the launch is as
+// long as that chain.  Each loaded where it was used, with the constants
+// divided out per lane and the sums shuffled through LDS: 7.2 us at N=1000
+// FP64 and 11.0 at N=10000 FP32 (four lanes); this 5.9 and 7.0 (sixteen).
+// EN = false leaves out the pair energy and virial, which every step
+// overwrites and only the call's last one reports: 9 of 55 instructions of
+// an FP32 pair.  (FP32 handles whose team is not the list layout's form them in
+// k_energy.)
+template <bool FP32, bool KICK, bool EN, int VEC>
+__global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, const BlkD *__restrict__ fblk,
+                                               const double4 *__restrict__ pos4, const QPos *__restrict__ posq,
+                                               const int *__restrict__ nn,
+                                               const int *__restrict__ nl, int cap, int lw, int lc,
+                                               const int *__restrict__ act,
+                                               const int8_t *__restrict__ kx, const int8_t *__restrict__ ky,
+                                               const int8_t *__restrict__ kz, double *fx, double *fy, double *fz,
+                                               double *px, double *py, double *pz, double *partial, int nb,
+                                               EndArgs E) {
+    static_assert(BLK == 256, "four waves per block");
+    __shared__ double s_red[4][BLK / 64];
+    const int b = xcd_block(nb);
+    if (b < 0) return;
+    const BlkD D = fblk[b];
+    const int W = 1 << lw, t = threadIdx.x & (W - 1);
+    const int i = D.first + (threadIdx.x >> lw);
+    double v_p2 = 0.0, v_pe = 0.0, v_vir = 0.0, v_px = 0.0;
+    double Fx = 0.0, Fy = 0.0, Fz = 0.0;
+    const bool valid = i < D.n;
+    const int g = D.off + (valid ? i : 0);
+    // FP64: the wrapped box fractions; FP32: their fixed-point copy
+    using PosT = typename std::conditional<FP32, QPos, double4>::type;
+    const PosT *__restrict__ pos = (const PosT *)(FP32 ? (const void *)posq : (const void *)pos4);
+    const PosT pi = ld_pos(pos, g);
+    const int m = valid ? nn[g] : 0;
+    const int a = act[g];
+    double vx = 0.0, vy = 0.0, vz = 0.0;
+    if (KICK) { vx = px[g]; vy = py[g]; vz = pz[g]; }
+    const RepC &R = reps[D.rep];
+    const bool active = a >= 0;
+    const int ka = R.off_act + (active ? a : 0);
+    const double kfx = (double)kx[ka], kfy = (double)ky[ka], kfz = (double)kz[ka];
+    PairAcc<FP32> acc(ptype(pi), R);
+    // entry e of particle i's list (nl_at): VEC = 1, W >= 2^lc, rows of W
+    // entries are W * n words apart; else the chunks of 8 entries, 8 * n
+    const size_t e0 = (size_t)(VEC > 1 ? t * VEC : t);
+    const int *lp = nl + (size_t)D.off * cap + ((((e0 >> lc) * D.n + (g - D.off)) << lc) + (e0 & ((1u << lc) - 1u)));
+    walk_list<VEC, EN>(lp, (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, pos, pi, acc);
+    acc.result(Fx, Fy, Fz, R);
+    v_pe = acc.pe;
+    v_vir = acc.vir;
+    Fx = team_sum(Fx, lw);
+    Fy = team_sum(Fy, lw);
+    Fz = team_sum(Fz, lw);
+    if (valid && t == 0) {
+        if (active) {  // cell_list+forces.c:207-213
+            Fx += R.f0 * kfx;
+            Fy += R.f0 * kfy;
+            Fz += R.f0 * kfz;
+        }
+        fx[g] = Fx; fy[g] = Fy; fz[g] = Fz;
+        if (KICK) {  // U2 after the forces, time_evolve.c:516
+            vx += Fx * K_HALF_DT; vy += Fy * K_HALF_DT; vz += Fz * K_HALF_DT;
+            px[g] = vx; py[g] = vy; pz[g] = vz;
+            v_p2 = vx * vx + vy * vy + vz * vz;
+            v_px = vx;
+        }
+    }
+    const double v[4] = {v_p2, v_pe, v_vir, v_px};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (!EN && (q == 1 || q == 2)) continue;
+        const double w = wave_sum_rows(v[q]);
+        if ((threadIdx.x & 63) == 0) s_red[q][threadIdx.x >> 6] = w;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x, fb = b - R.fblk_off, gr = fb / FORCE_GRP;
+    const int ngr = (R.fnblk + FORCE_GRP - 1) / FORCE_GRP, gsz = min(FORCE_GRP, R.fnblk - gr * FORCE_GRP);
+    const bool mine = lane < 4 && (EN || lane == 0 || lane == 3);  // lane q: sum q
+    if (mine) {
+        const double *w = s_red[lane];
+        st_agent(partial + 4 * (size_t)b + lane, (w[0] + w[1]) + (w[2] + w[3]));
+    }
+    wait_stores();
+    int last = 0;
+    if (lane == 0) last = last_done(E.gdone + R.fblk_off + gr * FORCE_GRP, gsz);
+    if (!__builtin_amdgcn_readfirstlane(last)) return;
+    double a4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (EN || q == 0 || q == 3)
+            a4[q] = lane < gsz ? ld_agent(partial + 4 * (size_t)(R.fblk_off + gr * FORCE_GRP + lane) + q) : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (EN || q == 0 || q == 3) a4[q] = wave_sum_rows(a4[q]);
+    if (ngr > 1) {
+        double *gp = E.gpart + 4 * (size_t)R.fblk_off;
+        if (mine) st_agent(gp + 4 * gr + lane, lane == 0 ? a4[0] : (lane == 1 ? a4[1] : (lane == 2 ? a4[2] : a4[3])));
+        wait_stores();
+        last = 0;
+        if (lane == 0) last = last_done(E.rdone + D.rep * DONE_PAD, ngr);
+        if (!__builtin_amdgcn_readfirstlane(last)) return;
+        const bool few = ngr <= 4;  // one after the other, else lane k groups k, k + 64, ...
+        for (int q = 0; q < 4; q++) a4[q] = 0.0;
+        for (int k = few ? 0 : lane; k < ngr; k += few ? 1 : 64)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (EN || q == 0 || q == 3) a4[q] += ld_agent(gp + 4 * k + q);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (!few && (EN || q == 0 || q == 3)) a4[q] = wave_sum_rows(a4[q]);
+    }
+    if (lane == 0) {
+        ChainS c0;
+        double eta[3], peta[3];
+        if (KICK) {
+            c0 = E.chain[D.rep];
+            for (int k = 0; k < 3; k++) { eta[k] = E.mid[6 * D.rep + k]; peta[k] = E.mid[6 * D.rep + 3 + k]; }
+        }
+        force_end<KICK, EN>(R, E.chain[D.rep], c0, eta, peta, a4, E.apart);
+    }
+}
+
+// Pair energy and virial of FP32 handles whose force team is not the list
+// layout's team of 2^lw lanes: that team walks the list (entries t, t + W, ...;
+// one lane: chunks of 8) and sums the FP32 terms of eight entries before it
+// widens them, so the partial sums, whose rounding shows in the seventh to
+// ninth digit of the energy, do not depend on the force kernel's width.  Runs
+// once per call, after its last step (k_energy_end then completes the step's
+// reported values).
+template <int VEC>
+__global__ void __launch_bounds__(BLK) k_energy(const RepC *__restrict__ reps, const BlkD *__restrict__ eblk,
+                                                const QPos *__restrict__ posq, const int *__restrict__ nn,
+                                                const int *__restrict__ nl, int cap, int lw, double *epart, int nb) {
+    __shared__ double s_red[2][BLK / 64];
+    const int b = xcd_block(nb);
+    if (b < 0) return;
+    const BlkD D = eblk[b];
+    const int W = 1 << lw, t = threadIdx.x & (W - 1), i = D.first + (threadIdx.x >> lw);
+    const bool valid = i < D.n;
+    const int il = valid ? i : 0, g = D.off + il;
+    const QPos pi = ld_pos(posq, g);
+    const int m = valid ? nn[g] : 0;
+    PairAcc<true> acc(ptype(pi), reps[D.rep]);
+    walk_list<VEC, true>(nl + (size_t)D.off * cap + (size_t)il * (VEC == 1 ? W : 8) + t,
+                         (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, posq, pi, acc);
+    const double v[2] = {wave_sum_rows(acc.pe), wave_sum_rows(acc.vir)};
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < 2; q++) s_red[q][threadIdx.x >> 6] = v[q];
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double s = 0.0;
+        for (int w = 0; w < BLK / 64; w++) s += s_red[threadIdx.x][w];
+        epart[2 * (size_t)b + threadIdx.x] = s;
+    }
+}
+
 // After k_energy, one workgroup per replica: its energy and virial, and with
-// step the pair energy in Heff (k_force_end stored it without).
+// step the pair energy in Heff (force_end stored it without).
 __global__ void __launch_bounds__(256) k_energy_end(const RepC *__restrict__ reps, ChainS *chain,
                                                     const double *__restrict__ epart, int step) {
     __shared__ double s_w[2][4];
@@ -1884,7 +1961,6 @@ __global__ void __launch_bounds__(256) k_energy_end(const RepC *__restrict__ rep
 // ------------------------------------------------------------- host side
 struct ac4_md {
     int R = 0, prec = 0, ntot = 0, nblk = 0, ncell_tot = 0, nact_tot = 0, cap = 192, stride = 0, max_ncell = 0;
-    int max_fnblk = 0;  // force blocks of the largest slot
     std::vector<RepC> reps_h;
     RepC *reps = nullptr;
     ChainS *chain = nullptr;
@@ -1908,6 +1984,8 @@ struct ac4_md {
     int *xmid = nullptr;                       // per cell: first slot of its upper x-half
     int *lblk_rep = nullptr, *lblk_first = nullptr;  // list-build block table (LPB particles per block)
     double *partial = nullptr;
+    double *gpart = nullptr;                             // EndArgs
+    unsigned *gdone = nullptr, *rdone = nullptr, *bdone = nullptr;  // finished blocks and groups (EndArgs), blocks of k_bin
     double *mid = nullptr;  // per replica: the chain's eta, p_eta after the start-of-step half
     PartArrays P{}, A{};  // primary and permutation scratch
     void **ftab = nullptr;  // their pointers on the device (PART_FIELDS of P, then of A)
@@ -2160,7 +2238,6 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         blk_off += R.nblk;
         fblk_off += R.fnblk;
         md->max_ncell = std::max(md->max_ncell, cap_cells);
-        md->max_fnblk = std::max(md->max_fnblk, R.fnblk);
         md->reps_h.push_back(R);  // idle: n = 0
     }
     md->t_brep = brep; md->t_bfirst = bfirst; md->t_bidx = bidx;
@@ -2208,6 +2285,8 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     ALLOC(reps, nslots) ALLOC(chain, nslots) ALLOC(blk_rep, md->nblk) ALLOC(blk_first, md->nblk) ALLOC(blk_idx, md->nblk)
     ALLOC(blkd, md->nblk) ALLOC(fblk, md->fnblk) ALLOC(lblk_rep, md->lnblk) ALLOC(lblk_first, md->lnblk)
     ALLOC(wl_item, (size_t)md->nblk + md->lnblk + md->ncb) ALLOC(wl_n, 4) ALLOC(ranges, (size_t)off_cell * NRANGE) ALLOC(xmid, off_cell) ALLOC(cblk_rep, off_cell) ALLOC(cblk_cell, off_cell) ALLOC(partial, 4 * (size_t)md->fnblk) ALLOC(mid, 6 * (size_t)nslots)
+    ALLOC(gpart, 4 * (size_t)md->fnblk) ALLOC(gdone, md->fnblk) ALLOC(rdone, (size_t)nslots * DONE_PAD)
+    ALLOC(bdone, (size_t)nslots * DONE_PAD)
     if (md->en_apart) { ALLOC(eblk, md->enblk) ALLOC(epart, 2 * (size_t)md->enblk) }
     ALLOC(fx, off) ALLOC(fy, off) ALLOC(fz, off) ALLOC(xo, off) ALLOC(yo, off) ALLOC(zo, off) ALLOC(pos4, off) ALLOC(posq, off)
     ALLOC(cell_mem, (size_t)off_cell * CELL_CAP) ALLOC(nn, off) ALLOC(nn_ref, off) ALLOC(nl, (size_t)md->cap * off) ALLOC(cnt, off_cell) ALLOC(start, off_cell)
@@ -2363,7 +2442,7 @@ extern "C" int ac4_md_destroy(ac4_md *md) {
                     md->lblk_rep, md->lblk_first, md->wl_item, md->wl_n, md->ranges, md->xmid,
                     md->cblk_rep, md->cblk_cell, md->ox, md->oy, md->oz, md->ov_q, md->ov_q2,
                     md->ov_step, md->ov_cnt, md->ov_n, md->ov_list, md->ov_out,
-                    md->partial, md->mid, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo, md->pos4, md->posq, md->cell_mem, md->shuf_ent, md->shuf_ent_n, md->nn,
+                    md->partial, md->mid, md->gpart, md->gdone, md->rdone, md->bdone, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo, md->pos4, md->posq, md->cell_mem, md->shuf_ent, md->shuf_ent_n, md->nn,
                     md->nn_ref, md->nl,
                     md->cnt, md->start, md->members, md->kx, md->ky, md->kz, md->ex, md->ey, md->ez, md->et};
     for (void *q : ptrs)
@@ -2937,9 +3016,10 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
     if (with_zero)
         hipLaunchKernelGGL(k_cell_zero, dim3(md->R, cy), dim3(BLK), 0, s, md->reps, md->chain, md->cnt, md->wl_n);
     hipLaunchKernelGGL(k_bin, dim3(md->nblk), dim3(BLK), 0, s, md->reps, md->chain, md->blk_rep, md->blk_first,
-                       md->P.x, md->P.y, md->P.z, md->P.id, md->cnt, md->P.cell_of, md->cell_mem, md->P.cell_ref);
-    hipLaunchKernelGGL(k_bin_end, dim3(md->R), dim3(md->max_ncell > BIN_END_T ? BIN_END_T : BLK), 0, s, md->reps, md->chain,
-                       md->cnt, md->start, wl);
+                       md->P.x, md->P.y, md->P.z, md->P.id, md->cnt, md->P.cell_of, md->cell_mem, md->P.cell_ref,
+                       md->max_ncell <= BIN_FUSE_CELLS ? 1 : 0, md->bdone, md->start, wl);
+    if (md->max_ncell > BIN_FUSE_CELLS)
+        hipLaunchKernelGGL(k_bin_end, dim3(md->R), dim3(BIN_END_T), 0, s, md->reps, md->chain, md->cnt, md->start, wl);
     hipLaunchKernelGGL(k_cell_sort, dim3(gc), dim3(BLK), 0, s, md->reps, wl, md->cnt, md->start,
                        md->cell_mem, md->members, md->ranges, md->xmid, md->P, md->A,
                        PosCopies{md->pos4, md->posq, md->xo, md->yo, md->zo});
@@ -2989,7 +3069,8 @@ static int launch_force_kernel(ac4_md *md) {
                                : k_force<false, KICK, EN, -2>;
     hipLaunchKernelGGL(kern, dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, md->stream, md->reps, md->fblk, md->pos4,
                        md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->P.act, md->kx, md->ky, md->kz, md->fx,
-                       md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk);
+                       md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk,
+                       EndArgs{md->chain, md->mid, md->gpart, md->gdone, md->rdone, md->en_apart ? 1 : 0});
     AC4_HIP(hipGetLastError());
     return AC4_OK;
 }
@@ -3008,23 +3089,10 @@ template <bool KICK, bool EN>
 static int launch_force_pass(ac4_md *md) {
     return md->prec == AC4_FP32 ? launch_force_kernel<true, KICK, EN>(md) : launch_force_kernel<false, KICK, EN>(md);
 }
-template <bool KICK, bool EN>
-static int launch_force_end(ac4_md *md) {
-    auto kern = k_force_end<KICK, EN>;
-    hipLaunchKernelGGL(kern, dim3(md->R), dim3(md->max_fnblk > 64 ? 256 : 64), 0, md->stream, md->reps, md->chain,
-                       md->partial, md->en_apart ? 1 : 0, md->mid);
-    AC4_HIP(hipGetLastError());
-    return AC4_OK;
-}
 // energy: form the pair energy and virial in this pass
 template <bool KICK>
 static int launch_force(ac4_md *md, bool energy) {
-    if (energy && !md->en_apart) {
-        TRY((launch_force_pass<KICK, true>(md)));
-        return launch_force_end<KICK, true>(md);
-    }
-    TRY((launch_force_pass<KICK, false>(md)));
-    return launch_force_end<KICK, false>(md);
+    return energy && !md->en_apart ? launch_force_pass<KICK, true>(md) : launch_force_pass<KICK, false>(md);
 }
 
 static void launch_shuffle(ac4_md *md, int force, hipStream_t s) {
@@ -3204,8 +3272,9 @@ extern "C" int ac4_md_relax(ac4_md *md, int nsteps, double f_start, double f_end
 
 // Eager steps with HIP events (on the handle's stream) around each launch
 // group; ms = average ms per step of {first_half, rebuild group, force,
-// shuffle, force end}: the force entry is k_force alone, the last k_force_end;
-// where the shuffle runs inside k_first_half its time is in the first entry
+// shuffle, force end}: the per-replica sums and the chain update run in
+// k_force's last workgroups, and the last entry is the empty interval between
+// two events; where the shuffle runs inside k_first_half its time is in the first entry
 // and the fourth is the empty interval between two events.
 extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
     AC4_REQUIRE(md && nsteps > 0 && ms, AC4_EARG, "kernel_times: bad arguments");
@@ -3222,10 +3291,8 @@ extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
         AC4_HIP(hipEventRecord(ev[2], s));
         TRY(launch_rebuild(md));
         AC4_HIP(hipEventRecord(ev[3], s));
-        const bool en = k == nsteps - 1 && !md->en_apart;
-        TRY((en ? launch_force_pass<true, true>(md) : launch_force_pass<true, false>(md)));
+        TRY(launch_force<true>(md, k == nsteps - 1));
         AC4_HIP(hipEventRecord(ev[4], s));
-        TRY((en ? launch_force_end<true, true>(md) : launch_force_end<true, false>(md)));
         AC4_HIP(hipEventRecord(ev[5], s));
         AC4_HIP(hipEventSynchronize(ev[5]));
         float t[5];

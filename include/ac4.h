@@ -143,9 +143,10 @@ int ac4_md_rebuilds(ac4_md *md, int r);
 /* Measurement hook (no reference counterpart): nsteps eager steps timed with
  * HIP events on the handle's stream around each launch group; ms (5 doubles)
  * = average milliseconds per step of {first half, rebuild group, force pass,
- * shuffle, force end (per-replica sums and chain update)}.  Where the handle
- * runs the shuffle inside the first-half kernel (small active sets), the
- * shuffle's time is part of the first entry. */
+ * shuffle, force end}.  The per-replica sums and the chain update are part of
+ * the force pass and the last entry is empty; where the handle runs the
+ * shuffle inside the first-half kernel (small active sets), the shuffle's time
+ * is part of the first entry. */
 int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms);
 /* Waits for all device work of the handle; reports deferred device errors
  * (list/cell overflow). */

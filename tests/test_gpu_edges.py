@@ -93,6 +93,37 @@ def test_force_team_widths(gpu, prec, n):
     assert np.allclose(pa, pb, rtol=1e-11 if prec == 0 else 1e-6)
 
 
+# What the last workgroups of the force pass and of the binning do for a whole
+# replica: part of a group of 64 blocks of 16 or 64 particles, a whole one and one
+# more, more than 4 groups, cells below and above the limit of the scan in the
+# binning pass; several replicas of different sizes in one handle.
+@pytest.mark.parametrize("sizes", [(256,), (1024,), (1025,), (16385,), (131073,), (700, 256, 2048, 500)])
+def test_sums_and_cells_of_the_last_workgroup(gpu, sizes):
+    md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 10, 3 + r) for r, n in enumerate(sizes)])
+    for r, n in enumerate(sizes):
+        s = gpu.init_lattice(n, 0.5, n)
+        xs = [s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")]
+        md.set_state(r, *xs, s["type"], s["act_tag"], s["kx"], s["ky"], s["kz"])
+    md.relax(20)
+    for r in range(len(sizes)):
+        md.init_chain(r)
+    for k in (1, 40):
+        md.step(k)
+        seen = [(md.stats(r), md.get_state(r), np.stack(md.forces(r))) for r in range(len(sizes))]
+        pv = md.calculate_forces()  # new cells and lists of the same positions
+        for r, n in enumerate(sizes):
+            st, g, f = seen[r]
+            p2 = sum((g[k] ** 2).sum() for k in ("px", "py", "pz"))
+            assert np.isclose(st["ke"], 0.5 * p2, rtol=1e-12, atol=0)  # sums of n terms of one sign
+            assert abs(st["drift"] - g["px"].sum()) <= 1e-13 * np.abs(g["px"]).sum()
+            assert np.allclose((st["pe"], st["virial"]), pv[r], rtol=1e-10, atol=1e-12)
+            # about 100 terms of up to a few hundred times the rms force cancel: 100 * 300 * 2^-53
+            f2 = np.stack(md.forces(r))
+            assert np.abs(f - f2).max() <= 4e-12 * max(1.0, np.sqrt((f2 ** 2).mean()))
+    assert all(md.rebuilds(r) > 2 for r in range(len(sizes)))
+    md.close()
+
+
 # Particle counts around the tiles of the frame kernel (256) and of the Fs
 # kernel (32, loads of 256), and one large enough for several of each per
 # workgroup; with and without the B particles.
