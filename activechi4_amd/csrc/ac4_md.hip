@@ -1768,12 +1768,15 @@ struct EndArgs {
 // combined by a fixed butterfly.  Each block hands over its partial sums of
 // p^2 and p_x, and with EN of PE and virial; the last block of each FORCE_GRP
 // adds theirs up (lane k block k, a fixed butterfly), the replica's last group
-// adds the groups' in a fixed order and updates the chain (force_end).  Two levels: atomics on one line are done one after the other.
-// As a kernel of their own after this
-// one, sums and update took 3.5 us of N=1000's step, 5.1 of N=50000's and
-// 11.4 of N=1e6's.  A block's loads form a short chain (block table, then position,
-// list length, active index and momentum together, then list, then
-// neighbour positions): on small boxes, a few waves per CU, the launch is as
+// adds the groups' in a fixed order and updates the chain (force_end).  Two
+// levels: atomics on one line are done one after the other.  As a kernel of
+// their own after this one, sums and update took 3.5 us of N=1000's step, 5.1
+// of N=50000's and 11.4 of N=1e6's; with them, and the scan of the cell
+// counts, inside: 19.7 -> 17.3 us per graph step at N=1000 FP64, 22.9 -> 20.8
+// at 10000 FP32, 65.8 -> 62.0 on the 64-replica ensemble, 359 -> 349 at 1e6.
+// A block's loads form a short chain (block table, then position, list
+// length, active index and momentum together, then list, then neighbour
+// positions): on small boxes, a few waves per CU, the launch is as
 // long as that chain.  Each loaded where it was used, with the constants
 // divided out per lane and the sums shuffled through LDS: 7.2 us at N=1000
 // FP64 and 11.0 at N=10000 FP32 (four lanes); this 5.9 and 7.0 (sixteen).
