@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
+#include <chrono>
 #include <vector>
 #include <map>
 #include "ac4_internal.h"
@@ -61,9 +62,9 @@ __device__ __forceinline__ double wrapn(double v, int times) {
     return v;
 }
 
-template <int NV>
+template <int NV, int T = ABLK>
 __device__ __forceinline__ void block_sum_store(double (&v)[NV], double *out) {
-    __shared__ double s_red[NV][ABLK / 64];
+    __shared__ double s_red[NV][T / 64];
     for (int k = 0; k < NV; k++) {
         double w = ac4_wave_sum(v[k]);
         if ((threadIdx.x & 63) == 0) s_red[k][threadIdx.x >> 6] = w;
@@ -71,46 +72,83 @@ __device__ __forceinline__ void block_sum_store(double (&v)[NV], double *out) {
     __syncthreads();
     if (threadIdx.x < NV) {
         double s = 0.0;
-        for (int w = 0; w < ABLK / 64; w++) s += s_red[threadIdx.x][w];
+        for (int w = 0; w < T / 64; w++) s += s_red[threadIdx.x][w];
         out[threadIdx.x] = s;
     }
 }
 
-// One pushed frame against the origins of its jobs: grid (blocks, jobs, plus
-// one row copying the frame to place `keep` when keep >= 0).  Block b takes
-// particles [b*ppb, (b+1)*ppb), ppb a multiple of ABLK.  Per job:
-//  MSD sums (msd_pos.c:64-76) to msdp[(p0*gridDim.x + b)*3 + v];
-//  overlap count (overlap.c:61-84) to ovp[p1*gridDim.x + b];
-//  S4's overlap mask (S4Qt.c:125-133): bit i of mask[p1*nwords + i/32], count
-//  to s4p[p1*gridDim.x + b]; its coordinates take the reference's per-lag
-//  single-if wraps (wrapn) exactly as it applies them.
-// k_msd_pairs and k_counts add the blocks up, for all pairs at once.  A
-// frame has about one job, so each launch is a latency of a few
-// microseconds whatever it does: three kernels, each with a reduction kernel
-// of its own, the jobs copied from the host and a synchronisation per walk
-// took 83 us per frame of 50000 particles (MSD, overlap, S4 masks); one
-// launch and one synchronisation take 18.
-__global__ void __launch_bounds__(ABLK) k_frame(const Job *__restrict__ jobs, int nj, int n, int ppb, double L,
-                                                double param, const double *__restrict__ x,
-                                                const double *__restrict__ y, const double *__restrict__ z,
-                                                const int *__restrict__ ty, int flag, int obs, Origins org, int keep,
-                                                double *msdp, int *ovp, int *s4p, int nwords,
-                                                unsigned *mask) {
-    const int b = blockIdx.x, i0 = b * ppb, i1 = min(n, i0 + ppb), lane = threadIdx.x & 63;
-    if ((int)blockIdx.y >= nj) {  // the frame is an origin: keep it
-        double *ox = org.at(keep, 0), *oy = org.at(keep, 1), *oz = org.at(keep, 2);
-        for (int i = i0 + threadIdx.x; i < i1; i += ABLK) {
+// The pushed frame: its arrays (device), n particles, the types the caller may
+// leave out (flag), and what tells the host that it has been read.
+struct Frame {
+    const double *x, *y, *z;
+    const int *ty;
+    int n, flag;
+    double L, param;
+    int obs;
+    Origins org;
+    int keep;             // place the frame is copied to, or -1
+    // read(): every workgroup says when it has read its part of the frame; the
+    // last one stores seq to the host's word, so the caller may have its
+    // arrays back (null: nobody waits).  Groups of READ_GRP workgroups, then
+    // the groups: atomics on one line are done one after the other (about 8
+    // ns each), so the counts lie a line apart.
+    unsigned *count, *word, seq;
+};
+#define READ_GRP 64
+#define READ_PAD 32
+__device__ __forceinline__ void frame_read(const Frame &F, int b, int nb) {  // one thread of workgroup b of nb
+    if (!F.word) return;
+    const auto last = [](unsigned *c, int of) {
+        if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != (unsigned)of) return false;
+        __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next frame
+        return true;
+    };
+    const int g = b / READ_GRP, ng = (nb + READ_GRP - 1) / READ_GRP;
+    if (!last(F.count + (1 + g) * READ_PAD, min(READ_GRP, nb - g * READ_GRP))) return;
+    if (ng > 1 && !last(F.count, ng)) return;
+    __hip_atomic_store(F.word, F.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// What k_frame and k_frame_fs leave per pair and block of particles:
+// MSD sums (msd_pos.c:64-76) in msdp[(p0*nb + b)*3 + v];
+// overlap count (overlap.c:61-84) in ovp[p1*nb + b];
+// S4's overlap mask (S4Qt.c:125-133), bit i of mask[p1*nwords + i/32], count
+// in s4p[p1*nb + b].
+struct FrameOut {
+    int ppb, nb;  // particles per block (a multiple of the block's threads), blocks
+    double *msdp;
+    int *ovp, *s4p, nwords;
+    unsigned *mask;
+};
+
+// One pushed frame against the origins of its jobs: block b of row `row` on T
+// threads (a row per job, then one that copies the frame to its place as an
+// origin); workgroup wg of nwg.  S4's coordinates take the reference's
+// per-lag single-if wraps (wrapn) exactly as it applies them.
+template <int T>
+__device__ __forceinline__ void frame_block(const Job *__restrict__ jobs, int nj, int row, int b, const Frame &F,
+                                            const FrameOut &O, int wg, int nwg) {
+    const double *__restrict__ x = F.x, *__restrict__ y = F.y, *__restrict__ z = F.z;
+    const int *__restrict__ ty = F.ty;
+    const int obs = F.obs, n = F.n, flag = F.flag;
+    const double L = F.L, param = F.param;
+    const int i0 = b * O.ppb, i1 = min(n, i0 + O.ppb), lane = threadIdx.x & 63;
+    if (row >= nj) {  // the frame is an origin: keep it
+        double *ox = F.org.at(F.keep, 0), *oy = F.org.at(F.keep, 1), *oz = F.org.at(F.keep, 2);
+        for (int i = i0 + threadIdx.x; i < i1; i += T) {
             ox[i] = x[i];
             oy[i] = y[i];
             oz[i] = z[i];
         }
+        __syncthreads();
+        if (threadIdx.x == 0) frame_read(F, wg, nwg);
         return;
     }
-    const Job J = jobs[blockIdx.y];
-    const double *ox = org.at(J.org, 0), *oy = org.at(J.org, 1), *oz = org.at(J.org, 2);
+    const Job J = jobs[row];
+    const double *ox = F.org.at(J.org, 0), *oy = F.org.at(J.org, 1), *oz = F.org.at(J.org, 2);
     double v[3] = {0.0, 0.0, 0.0};
     int nov = 0, ns4 = 0;
-    for (int t = i0; t < i1; t += ABLK) {
+    for (int t = i0; t < i1; t += T) {
         const int i = t + threadIdx.x;
         bool ov = false, s4 = false;
         if (i < i1) {
@@ -144,21 +182,35 @@ __global__ void __launch_bounds__(ABLK) k_frame(const Job *__restrict__ jobs, in
         if (J.p1 >= 0 && (obs & AC4_OBS_S4)) {
             const unsigned long long m = __ballot(s4);
             const int w = (t + (threadIdx.x & ~63)) >> 5;  // first of the wave's two words
-            unsigned *row = mask + (size_t)J.p1 * nwords;
-            if (lane == 0 && w < nwords) row[w] = (unsigned)m;
-            if (lane == 1 && w + 1 < nwords) row[w + 1] = (unsigned)(m >> 32);
+            unsigned *row = O.mask + (size_t)J.p1 * O.nwords;
+            if (lane == 0 && w < O.nwords) row[w] = (unsigned)m;
+            if (lane == 1 && w + 1 < O.nwords) row[w + 1] = (unsigned)(m >> 32);
             ns4 += __popcll(m);
         }
     }
-    __shared__ int s_c[2][ABLK / 64];
+    __shared__ int s_c[2][T / 64];
     if (lane == 0) { s_c[0][threadIdx.x >> 6] = nov; s_c[1][threadIdx.x >> 6] = ns4; }
-    if (J.p0 >= 0) block_sum_store<3>(v, msdp + ((size_t)J.p0 * gridDim.x + b) * 3);
     __syncthreads();
+    if (threadIdx.x == 0) frame_read(F, wg, nwg);
+    if (J.p0 >= 0) block_sum_store<3, T>(v, O.msdp + ((size_t)J.p0 * O.nb + b) * 3);
     if (J.p1 >= 0 && threadIdx.x < 2 && (obs & (threadIdx.x == 0 ? AC4_OBS_OVERLAP : AC4_OBS_S4))) {
         int c = 0;
-        for (int w = 0; w < ABLK / 64; w++) c += s_c[threadIdx.x][w];
-        (threadIdx.x == 0 ? ovp : s4p)[(size_t)J.p1 * gridDim.x + b] = c;
+        for (int w = 0; w < T / 64; w++) c += s_c[threadIdx.x][w];
+        (threadIdx.x == 0 ? O.ovp : O.s4p)[(size_t)J.p1 * O.nb + b] = c;
     }
+}
+
+// The frame without Fs: grid (blocks, rows).  k_msd_pairs and k_counts add the
+// blocks up, for all pairs at once.  A frame has about one job, so a push is
+// latencies whatever it does: three kernels, each with a reduction kernel of
+// its own, the jobs copied from the host and a synchronisation per walk took
+// 83 us per frame of 50000 particles (MSD, overlap, S4); one launch and one synchronisation 21.4,
+// one launch whose workgroups say that they have read the frame 15.9 (the
+// host's word arrives 4 us before the stream's end is seen: 7.7 against 11.8
+// us for an empty kernel).
+__global__ void __launch_bounds__(ABLK) k_frame(const Job *__restrict__ jobs, int nj, Frame F, FrameOut O) {
+    frame_block<ABLK>(jobs, nj, blockIdx.y, blockIdx.x, F, O, blockIdx.y * gridDim.x + blockIdx.x,
+                      gridDim.x * gridDim.y);
 }
 
 // out[p*3 + v] = the MSD sums of pair p over its nb blocks, in a fixed order;
@@ -229,6 +281,7 @@ __constant__ int c_pcol[AC4_NQ];     // first column of each GetQ vector
 #define FS_TILES 14    // accumulated 16 x 16 tiles: 3 x {cos, sin}, then the (0, k, i) group's 8
 #define FS_LOAD 256    // particles whose displacements are loaded together
 #define FS_NBLK 256    // workgroups per pair, at most
+#define FS_WAIT 32     // jobs whose partials one reduction takes, at least (at most 21 MB)
 #define FS_SETS 4      // sets of four waves per workgroup
 #define FS_T (256 * FS_SETS)
 
@@ -261,20 +314,18 @@ __device__ __forceinline__ void fs_entry(const double *s_t, int o0, int o1, int 
     s = t0[(r + 6) * 16] + t1[r * 16];
 }
 
-// grid (blocks of ppb particles, jobs), ppb a multiple of FS_P;
-// partial[((job*gridDim.x+blk)*AC4_NQ*2) + n] = cos sum, + AC4_NQ + n = sin
-// sum, averaged over the vector's permutations.
-__global__ void __launch_bounds__(FS_T) k_fs(const Job *__restrict__ jobs, int n, int ppb,
-                                            const double *__restrict__ x, const double *__restrict__ y,
-                                            const double *__restrict__ z, const int *__restrict__ ty, int flag,
-                                            Origins org, double *partial) {
+// Block blk (ppb particles, a multiple of FS_P) of job J; out[n] = cos sum,
+// out[AC4_NQ + n] = sin sum, averaged over the vector's permutations.
+__device__ __forceinline__ void fs_block(const Job &J, int blk, int ppb, const Frame &F, double *__restrict__ out, int wg,
+                                         int nwg) {
+    const double *__restrict__ x = F.x, *__restrict__ y = F.y, *__restrict__ z = F.z;
+    const int *__restrict__ ty = F.ty;
+    const int n = F.n, flag = F.flag;
     __shared__ double s_t[FS_LDS];
     __shared__ double s_p[3][FS_LOAD];
     __shared__ double s_use[FS_LOAD];
-    const Job J = jobs[blockIdx.y];
-    if (J.p1 < 0) return;
     const int t = threadIdx.x, lane = t & 63, set = t >> 8, wv = (t >> 6) & 3, i16 = lane & 15, k4 = lane >> 4;
-    const double *ox = org.at(J.org, 0), *oy = org.at(J.org, 1), *oz = org.at(J.org, 2);
+    const double *ox = F.org.at(J.org, 0), *oy = F.org.at(J.org, 1), *oz = F.org.at(J.org, 2);
     // for the end: this thread's permuted vector, and of its output value the columns
     const int pc = min(t, S4_NCOL - 1), o0 = c_pv[3 * pc], o1 = c_pv[3 * pc + 1], o2 = c_pv[3 * pc + 2];
     const int oq = t < 2 * AC4_NQ ? t % AC4_NQ : 0, od = c_dg[oq], oc = c_pcol[oq];
@@ -291,7 +342,7 @@ __global__ void __launch_bounds__(FS_T) k_fs(const Job *__restrict__ jobs, int n
         const int cq = 16 * q + i16;
         kb[q] = cq < 3 * FS_M ? fs_ax(cq / FS_M, cq % FS_M + 1, 0) : fs_ax(0, 0, 0);
     }
-    const int i0 = blockIdx.x * ppb, i1 = min(n, i0 + ppb);
+    const int i0 = blk * ppb, i1 = min(n, i0 + ppb);
     for (int tb = i0; tb < i1; tb += FS_P) {
         const int lb = (tb - i0) & (FS_LOAD - 1);  // the tile among the loaded particles
         if (lb == 0 && t < FS_LOAD) {
@@ -311,7 +362,10 @@ __global__ void __launch_bounds__(FS_T) k_fs(const Job *__restrict__ jobs, int n
             s_p[0][t] = p0; s_p[1][t] = p1; s_p[2][t] = p2;
             s_use[t] = use;
         }
-        if (lb == 0) __syncthreads();
+        if (lb == 0) {
+            __syncthreads();
+            if (t == FS_T - 1 && tb + FS_LOAD >= i1) frame_read(F, wg, nwg);
+        }
         if (t < FS_P) {
             s_t[fs_ax(0, 0, 0) + t] = s_use[lb + t];  // the column of ones
             s_t[fs_ax(0, 0, 1) + t] = 0.0;
@@ -392,8 +446,31 @@ __global__ void __launch_bounds__(FS_T) k_fs(const Job *__restrict__ jobs, int n
         const double *src = s_t + (t < AC4_NQ ? 0 : S4_NCOL) + oc;
         double v = 0.0;
         for (int k = 0; k < od; k++) v += src[k];
-        partial[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * (AC4_NQ * 2) + t] = od == 1 ? v : v / (double)od;
+        out[t] = od == 1 ? v : v / (double)od;
     }
+}
+
+// The frame with Fs in one launch: workgroups [0, nj*fs_nb) Fs, a job's block
+// each (partial[(job*fs_nb + blk)*2*AC4_NQ + value]), the rest `rows` rows of
+// O.nb frame blocks.  As two launches, a reduction and the stream's end waited
+// for: 25.6 us per frame of 1000 particles, all four observables, and 31.7 of
+// 20011, Fs alone; this, the partials of FS_WAIT jobs reduced together, 11.1
+// and 16.8.
+__global__ void __launch_bounds__(FS_T) k_frame_fs(const Job *__restrict__ jobs, int nj, int nf, int fs_nb, int fs_ppb,
+                                                   Frame F, FrameOut O, double *partial) {
+    const int wg = blockIdx.x, nwg = gridDim.x;
+    if (wg >= nj * fs_nb) {
+        const int k = wg - nj * fs_nb;
+        frame_block<FS_T>(jobs, nf, k / O.nb, k % O.nb, F, O, wg, nwg);
+        return;
+    }
+    const int j = wg / fs_nb;
+    const Job J = jobs[j];
+    if (J.p1 < 0) {
+        if (threadIdx.x == 0) frame_read(F, wg, nwg);
+        return;
+    }
+    fs_block(J, wg - j * fs_nb, fs_ppb, F, partial + (size_t)wg * (AC4_NQ * 2), wg, nwg);
 }
 
 // ---------------------------------------------------------------- S4
@@ -402,7 +479,7 @@ __global__ void __launch_bounds__(FS_T) k_fs(const Job *__restrict__ jobs, int n
 // position at the lag (|r(t) - r0| < a), averaged over q's permutations.
 // The phase depends on the origin frame alone, so it is evaluated once per
 // origin and shared by all of that origin's lags:
-//   k_frame     at each lag frame: the overlap mask of the pair, one bit per
+//   k_frame(_fs) at each lag frame: the overlap mask of the pair, one bit per
 //               particle (and the overlap count of the pair);
 //   k_s4_origin when the origin's last lag has been masked: the phase matrix
 //               P[particle][573 permuted vectors] times the mask matrix
@@ -595,6 +672,7 @@ struct ac4_ana {
     double *d_part = nullptr, *d_msdp = nullptr;
     int *d_ovp = nullptr, *d_s4p = nullptr;  // per block: overlap counts of the overlap and the S4 rule
     Job *d_jobs = nullptr;
+    unsigned *d_read = nullptr, *h_read = nullptr, seq = 0;  // Frame::count, ::word (pinned), ::seq
     bool stale = false;         // frames came in since d_msd, d_ov and d_s4m were formed from the blocks' values
     // S4 by origin: pair ids per origin (CSR, walk order), origins whose
     // last lag is frame pos, the pairs' overlap masks and the chunk partials
@@ -605,6 +683,7 @@ struct ac4_ana {
     unsigned *d_s4mask = nullptr;
     double *d_s4part = nullptr;
     int nwords = 0, s4_wpw = 1, s4_nchunk = 1;
+    int fs_j0 = 0, fs_j1 = 0, fs_wait = 0;  // jobs whose Fs partials are in d_part, how many it holds
     int max_jobs = 0, ppb = ABLK, nb = 0, fs_ppb = FS_P, fs_nb = 0;
     std::vector<int> vx, vy, vz, qsq;
     std::vector<double> qval;
@@ -809,8 +888,9 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vz), an->vz.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_dg), dg.data(), sizeof(int) * AC4_NQ));
     if ((rc = set_columns(an, dg)) != AC4_OK) return fail(rc);
-    // blocks of k_frame: one tile of ABLK particles each up to 256 of them, then more tiles per block
-    an->ppb = ABLK * ((n + 256 * ABLK - 1) / (256 * ABLK));
+    // blocks of a frame row: one tile of the block's threads each up to 256 of them, then more tiles per block
+    const int fb = obs & AC4_OBS_FS ? FS_T : ABLK;
+    an->ppb = fb * ((n + 256 * fb - 1) / (256 * fb));
     an->nb = (n + an->ppb - 1) / an->ppb;
     an->fs_ppb = FS_P * ((n + FS_NBLK * FS_P - 1) / (FS_NBLK * FS_P));
     an->fs_nb = (n + an->fs_ppb - 1) / an->fs_ppb;
@@ -825,6 +905,10 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     if (!an->jobs.empty() && hipMemcpy(an->d_jobs, an->jobs.data(), sizeof(Job) * an->jobs.size(),
                                        hipMemcpyHostToDevice) != hipSuccess) return fail(AC4_EHIP);
     if (!get(&an->org.f, (size_t)3 * n * std::max(places, 1), false)) return fail(AC4_EHIP);
+    const int wgs = an->max_jobs * (an->fs_nb + an->nb) + an->nb;  // workgroups of a frame, at most
+    if (!get(&an->d_read, (size_t)(2 + wgs / READ_GRP) * READ_PAD, true)) return fail(AC4_EHIP);
+    if (hipHostMalloc((void **)&an->h_read, 64, hipHostMallocDefault) != hipSuccess) return fail(AC4_EHIP);
+    *an->h_read = 0;
     if (!get(&an->cur, (size_t)3 * n, false) || !get(&an->cur_t, n, false)) return fail(AC4_EHIP);
     if (obs & AC4_OBS_MSD)
         if (!get(&an->d_msd, 3 * np0, true) || !get(&an->d_msdp, 3 * np0 * an->nb, true)) return fail(AC4_EHIP);
@@ -832,7 +916,8 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
         if (!get(&an->d_ov, np1, true) || !get(&an->d_ovp, np1 * an->nb, true)) return fail(AC4_EHIP);
     if (obs & AC4_OBS_FS)
         if (!get(&an->d_fs, 2 * AC4_NQ * np1, true) ||
-            !get(&an->d_part, (size_t)an->max_jobs * an->fs_nb * AC4_NQ * 2, false)) return fail(AC4_EHIP);
+            !get(&an->d_part, (size_t)(an->fs_wait = std::max(an->max_jobs, FS_WAIT)) * an->fs_nb * AC4_NQ * 2, false))
+            return fail(AC4_EHIP);
     if (obs & AC4_OBS_S4) {
         if (hipMalloc(&an->d_s4, sizeof(double) * 2 * AC4_NQ * (size_t)np1) != hipSuccess) return fail(AC4_EHIP);
         if (!get(&an->d_s4m, np1, true) || !get(&an->d_s4p, np1 * an->nb, true)) return fail(AC4_EHIP);
@@ -846,10 +931,11 @@ extern "C" int ac4_ana_destroy(ac4_ana *an) {
     if (!an) return AC4_OK;
     if (an->stream) (void)hipStreamSynchronize(an->stream);
     void *ptrs[] = {an->org.f, an->cur, an->cur_t, an->d_msd, an->d_msdp, an->d_ov, an->d_ovp, an->d_s4, an->d_s4m, an->d_s4p,
-                    an->d_fs, an->d_part, an->d_jobs,
+                    an->d_fs, an->d_part, an->d_jobs, an->d_read,
                     an->d_s4_opairs, an->d_s4mask, an->d_s4part};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (an->h_read) (void)hipHostFree(an->h_read);
     for (auto &W : an->W) ac4_walk_free(&W.w);
     if (an->stream) (void)hipStreamDestroy(an->stream);
     delete an;
@@ -858,31 +944,59 @@ extern "C" int ac4_ana_destroy(ac4_ana *an) {
 
 extern "C" int ac4_ana_gap(const ac4_ana *an) { return an ? an->gap : AC4_EARG; }
 
+static void reduce_fs(ac4_ana *an) {
+    if (an->fs_j1 > an->fs_j0)
+        hipLaunchKernelGGL(k_reduce_jobs, dim3(an->fs_j1 - an->fs_j0, (2 * AC4_NQ + 63) / 64), dim3(256), 0, an->stream,
+                           an->d_jobs + an->fs_j0, an->fs_nb, 2 * AC4_NQ, an->d_part, an->d_fs);
+    an->fs_j0 = an->fs_j1;
+}
+
+// Returns when the frame of the last launch has been read, i.e. its last
+// workgroup has stored h_read; should the word not come (a failed launch), or
+// take long, the stream's end, with its error, is waited for instead.
+static int wait_read(ac4_ana *an) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (unsigned k = 1; __atomic_load_n(an->h_read, __ATOMIC_ACQUIRE) != an->seq; k++)
+        if ((k & 255) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+            AC4_HIP(hipStreamSynchronize(an->stream));
+            break;
+        }
+    return AC4_OK;
+}
+
 // Runs every job of the frame whose arrays (device) are x, y, z, t; keep: the
-// origin place the frame is copied to, or -1.
+// origin place the frame is copied to, or -1; wait: return when the arrays have
+// been read.
 static int process_frame(ac4_ana *an, int pos, const double *x, const double *y, const double *z, const int *t,
-                         int keep) {
+                         int keep, bool wait) {
     hipStream_t s = an->stream;
     const int j0 = an->jptr[pos], nj = an->jptr[pos + 1] - j0;
-    const int nf = an->obs & (AC4_OBS_MSD | AC4_OBS_OVERLAP | AC4_OBS_S4) ? nj : 0;  // Fs has its own kernel
-    if (nf > 0 || keep >= 0) {
-        hipLaunchKernelGGL(k_frame, dim3(an->nb, nf + (keep >= 0 ? 1 : 0)), dim3(ABLK), 0, s, an->d_jobs + j0, nf, an->n,
-                           an->ppb, an->L, an->param, x, y, z, t, an->flag, an->obs, an->org, keep, an->d_msdp,
-                           an->d_ovp, an->d_s4p, an->nwords, an->d_s4mask);
-        an->stale = true;
-    }
-    if (nj > 0 && (an->obs & AC4_OBS_FS)) {
-        hipLaunchKernelGGL(k_fs, dim3(an->fs_nb, nj), dim3(FS_T), 0, s, an->d_jobs + j0, an->n, an->fs_ppb, x, y, z, t,
-                           an->flag, an->org, an->d_part);
-        hipLaunchKernelGGL(k_reduce_jobs, dim3(nj, (2 * AC4_NQ + 63) / 64), dim3(256), 0, s, an->d_jobs + j0, an->fs_nb,
-                           2 * AC4_NQ, an->d_part, an->d_fs);
+    const int nf = an->obs & (AC4_OBS_MSD | AC4_OBS_OVERLAP | AC4_OBS_S4) ? nj : 0;  // rows of pairs
+    const int rows = nf + (keep >= 0 ? 1 : 0), nfs = an->obs & AC4_OBS_FS ? nj : 0;
+    if (rows + nfs == 0) return AC4_OK;  // no pair ends here (so no origin's last lag either), nothing to keep
+    const Frame F{x, y, z, t, an->n, an->flag, an->L, an->param, an->obs, an->org, keep, an->d_read,
+                  wait ? an->h_read : nullptr, wait ? ++an->seq : 0u};
+    const FrameOut O{an->ppb, an->nb, an->d_msdp, an->d_ovp, an->d_s4p, an->nwords, an->d_s4mask};
+    if (rows > 0) an->stale = true;
+    if (nfs > 0) {
+        // the partials of the jobs [fs_j0, fs_j1) wait for their reduction
+        if (j0 != an->fs_j1 || j0 + nj - an->fs_j0 > an->fs_wait) {
+            reduce_fs(an);
+            an->fs_j0 = j0;
+        }
+        an->fs_j1 = j0 + nj;
+        hipLaunchKernelGGL(k_frame_fs, dim3(nfs * an->fs_nb + rows * an->nb), dim3(FS_T), 0, s, an->d_jobs + j0, nfs, nf,
+                           an->fs_nb, an->fs_ppb, F, O,
+                           an->d_part + (size_t)(j0 - an->fs_j0) * an->fs_nb * (AC4_NQ * 2));
+    } else {
+        hipLaunchKernelGGL(k_frame, dim3(an->nb, rows), dim3(ABLK), 0, s, an->d_jobs + j0, nf, F, O);
     }
     AC4_HIP(hipGetLastError());
     // origins whose last lag this frame was: their S4 sums, before another
     // origin takes their place
     if (an->obs & AC4_OBS_S4)
         for (int o : an->s4_end[pos]) TRY(s4_origin(an, o));
-    return AC4_OK;
+    return wait ? wait_read(an) : AC4_OK;
 }
 
 static int push_common(ac4_ana *an, int pos, const double *x, const double *y, const double *z, const int *t,
@@ -908,8 +1022,8 @@ static int push_common(ac4_ana *an, int pos, const double *x, const double *y, c
         keep = -1;
     }
     an->resident[pos] = an->place[pos] >= 0;
-    TRY(process_frame(an, pos, x, y, z, t, keep));
-    AC4_HIP(hipStreamSynchronize(s));  // the caller may reuse its arrays
+    TRY(process_frame(an, pos, x, y, z, t, keep, !host));  // the caller may reuse its arrays
+    if (host) AC4_HIP(hipStreamSynchronize(s));
     // origins no pair needs any more (their places may be taken from now on)
     for (int f = an->last_pos + 1; f <= pos; f++)
         for (int o : an->ends[f]) an->resident[o] = 0;
@@ -976,6 +1090,8 @@ static void split_phase(const std::vector<double> &in, int ns, std::vector<doubl
 
 // Every pair's MSD sums and overlap counts from its blocks' values
 static int sum_blocks(ac4_ana *an) {
+    reduce_fs(an);
+    AC4_HIP(hipGetLastError());
     if (!an->stale) return AC4_OK;
     const int np0 = an->W[0].w.np, np1 = an->W[1].w.np;
     if ((an->obs & AC4_OBS_MSD) && np0 > 0)

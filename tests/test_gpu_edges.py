@@ -1,6 +1,8 @@
 """Kernels at the sizes where their tilings can go wrong: edges of tiles,
 remainders, the smallest and largest of their ranges, against the oracle or a
 64-bit restatement."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -187,3 +189,40 @@ def _walk(frames, gap):
             off = off + 1 if int(off * 1.4) == off else int(off * 1.4)
         k += 1
     return out
+
+
+# Frames pushed from one set of device arrays that are overwritten as soon as
+# the push returns, against host pushes: one workgroup, one and more groups of
+# 64, Fs with and without the other observables, more pairs than one reduction
+# of Fs takes and a frame left out between them.
+@pytest.mark.parametrize("n,obs", [(1, 15), (700, 7), (700, 8), (2049, 15), (70001, 15), (70001, 3)])
+def test_device_arrays_reused_after_the_push(gpu, n, obs):
+    frames = list(range(60))
+    X, Y, Z, T = trajgen.make_frames(n, frames, 5 + n, 0.08, 1.0)
+    L = max(4.0, (n / 1.2) ** (1.0 / 3.0))
+    hip = ctypes.CDLL("libamdhip64.so")  # the runtime the library has loaded
+    dev = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(dev), ctypes.c_size_t(28 * n)) == 0
+    at = [dev.value + 8 * n * k for k in range(4)]  # x, y, z, types
+    out = []
+    for device in (False, True):
+        an = gpu.Analysis(n, L, frames, gap=10, obs=obs)
+        for f in range(len(frames)):
+            if f == 21:
+                continue
+            if not device:
+                an.push(f, X[f], Y[f], Z[f], T[f])
+                continue
+            src = [np.ascontiguousarray(v) for v in (X[f], Y[f], Z[f], np.asarray(T[f], dtype=np.int32))]
+            for d, v in zip(at, src):
+                assert hip.hipMemcpy(ctypes.c_void_p(d), v.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(v.nbytes), 1) == 0
+            assert gpu.lib.ac4_ana_push_frame_device(an.h, f, *at) == 0
+            assert hip.hipMemset(dev, 255, ctypes.c_size_t(28 * n)) == 0
+        an.finalize()
+        got = [an.pairs(o) for o in (gpu.OBS_MSD, gpu.OBS_OVERLAP, gpu.OBS_S4, gpu.OBS_FS) if obs & o]
+        out.append([v for g in got for v in (g if isinstance(g, tuple) else (g,))])
+        an.close()
+    hip.hipFree(dev)
+    assert not obs & 8 or len(out[0][-1]) > 32
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
