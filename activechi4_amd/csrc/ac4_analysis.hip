@@ -481,19 +481,219 @@ __global__ void __launch_bounds__(FS_T) k_frame_fs(const Job *__restrict__ jobs,
 // origin and shared by all of that origin's lags:
 //   k_frame(_fs) at each lag frame: the overlap mask of the pair, one bit per
 //               particle (and the overlap count of the pair);
-//   k_s4_origin when the origin's last lag has been masked: the phase matrix
-//               P[particle][573 permuted vectors] times the mask matrix
-//               M[particle][lags] on FP64 matrix cores, P formed in registers
+//   k_s4_origin when the origin's last lag has been masked: the mask matrix
+//               M[lags][particle] times the phase matrix P[particle][573
+//               permuted vectors] on FP64 matrix cores, P formed in registers
 //               and never stored;
-//   k_s4_reduce sums the chunk partials in a fixed order and averages each
-//               vector's permutations.
-// This evaluates 573 sincos per particle per origin instead of per pair.
+//   k_s4_reduce sums the chunk partials in a fixed order and divides by the
+//               number of each vector's permutations.
+//
+// As in Fs a phase is a product of one factor each of two tables (the axis
+// factors exp(2 pi i m x), m = 0 ... 21, and the products (j, j) of two axes),
+// built per tile of particles in LDS: 63 sincos and 45 products per particle
+// for 573 phases of four multiplications, where a sincos per phase (34
+// instructions) took 2/5 of the time.  One workgroup takes its particles
+// through all 36 column tiles (12 waves, three tiles each), so the tables are
+// built once.  The lags are 16 rows per v_mfma_f64_16x16x4f64 and, for what is
+// left of them, 4 per v_mfma_f64_4x4x4f64 (four blocks of 4 x 4, the four
+// columns each of the same B operand; the same rate, 64 against 68 TFLOP/s
+// measured): 22 lags cost 24 rows, not 32.  The bound is the issue of the FP64 matrix
+// and vector instructions, which share their rate: of 78.7 us at 50000
+// particles and 22 lags 52 are the products, 10 the tables; a workgroup per
+// chunk and column tile with a sincos per phase took 110, its reduction of
+// 576 columns per lag 13.5 (k_s4_reduce's 324 values 4.8).
 #define S4_NCT (S4_NCOL / 16) // column tiles
-#define S4_RT_MAX 4           // lag rows of one pass: up to 64 lags
-#define S4_CHUNKS 64          // particle chunks a pass is split into (at most)
+#define S4_WAVES 12
+#define S4_CPW (S4_NCT / S4_WAVES)  // column tiles of a wave
+#define S4_T (64 * S4_WAVES)
+#define S4_LAGS 32     // lags of one pass, at most
+#define S4_CHUNKS 256  // workgroups of a pass, at most
+#define S4_SMALL 3072  // particles up to which k_s4_small is the faster one
+#define S4_SMALL_CHUNKS 64
 
-// One origin, one pass of up to RT*16 of its lags: grid (chunks, S4_NCT),
-// 256 threads.  Wave w of block (c, ct) takes the mask words
+// The table rows (cos; sin at + FS_RL) whose product is the permuted vector (o0, o1, o2)
+__device__ __forceinline__ void s4_rows(int o0, int o1, int o2, int &u, int &v) {
+    const int o[3] = {o0, o1, o2};
+    if (o0 != 0 && o1 != 0 && o2 != 0) {  // (i, j, j): the odd component with the product of the equal ones
+        const int a = o1 == o2 ? 0 : (o0 == o2 ? 1 : 2), j = a == 0 ? o1 : o0;
+        u = fs_ax(a, o[a], 0);
+        v = fs_pr(a, j, 0);
+        return;
+    }
+    // up to two components; axis 0's m = 0 is the row of ones
+    const int a = o0 != 0 ? 0 : (o1 != 0 ? 1 : 2), b = o2 != 0 ? 2 : 1;
+    u = o[a] != 0 ? fs_ax(a, o[a], 0) : fs_ax(0, 0, 0);
+    v = b != a && o[b] != 0 ? fs_ax(b, o[b], 0) : fs_ax(0, 0, 0);
+}
+
+// One origin, one pass of nl <= 16*NT16 + 4*NT4 of its lags: grid (chunks of
+// ppb particles), tiles of tp <= FS_P particles (both multiples of 4).
+// v_mfma_f64_16x16x4f64: lane l = i + 16k holds A[i][k] (mask bit of lag i,
+// particle k) and B[k][j] with j = i (phase of vector j for particle k); the
+// accumulator's element e of lane l is row l/16 + 4*e, column l%16.
+// v_mfma_f64_4x4x4f64: the same B; lane l holds A[l%4][l/16], and the
+// accumulator of lane l is row l/16, column l%16.
+// part[((chunk*nl + lag)*2 + {cos,sin})*AC4_NQ + vector]: sums over the
+// vector's permutations.
+template <int NT16, int NT4>
+__global__ void __launch_bounds__(S4_T) k_s4_origin(const double *__restrict__ x0, const double *__restrict__ y0,
+                                                    const double *__restrict__ z0, int n, int nwords,
+                                                    const unsigned *__restrict__ mask, const int *__restrict__ lags,
+                                                    int nl, int ppb, int tp, double *__restrict__ part) {
+    constexpr int NR = NT16 + NT4, ROWS = 16 * NT16 + 4 * NT4;
+    constexpr int LDS = FS_LDS > ROWS * S4_NCOL ? FS_LDS : ROWS * S4_NCOL;
+    __shared__ double s_t[LDS];  // the tables, then the sums of one of cos and sin
+    __shared__ double s_p[3][FS_P];
+    __shared__ int s_dc[AC4_NQ];  // permutations and first column of each vector, for the end
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, i16 = lane & 15, k4 = lane >> 4, pp = t & (FS_P - 1);
+    int u[S4_CPW], v[S4_CPW];
+#pragma unroll
+    for (int c = 0; c < S4_CPW; c++) {
+        const int col = (wv * S4_CPW + c) * 16 + i16;
+        s4_rows(c_pv[3 * col], c_pv[3 * col + 1], c_pv[3 * col + 2], u[c], v[c]);
+    }
+    const unsigned *mrow[NR];  // this lane's lag of each row tile
+    bool live[NR];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int l = r < NT16 ? 16 * r + i16 : 16 * NT16 + 4 * (r - NT16) + (lane & 3);
+        live[r] = l < nl;
+        mrow[r] = mask + (size_t)lags[live[r] ? l : 0] * nwords;
+    }
+    ac4_d4 ac[S4_CPW][NT16 > 0 ? NT16 : 1], as[S4_CPW][NT16 > 0 ? NT16 : 1];
+    double bc[S4_CPW][NT4 > 0 ? NT4 : 1], bs[S4_CPW][NT4 > 0 ? NT4 : 1];
+#pragma unroll
+    for (int c = 0; c < S4_CPW; c++) {
+        for (int r = 0; r < NT16; r++) ac[c][r] = as[c][r] = ac4_d4{0.0, 0.0, 0.0, 0.0};
+        for (int r = 0; r < NT4; r++) bc[c][r] = bs[c][r] = 0.0;
+    }
+    const int i0 = blockIdx.x * ppb, i1 = min(n, i0 + ppb);
+    // exp(i q.r0) is periodic in r0 with the box, so the stored origin
+    // coordinate is used as it is, whatever single-if wraps the reference
+    // applies to it at a given lag.  A particle past n has no mask bit: its
+    // (clamped) phase is multiplied by zero; so has one of the next chunk.
+    const double *src = t < FS_P ? x0 : (t < 2 * FS_P ? y0 : z0);
+    double p = t < 3 * FS_P ? src[min(i0 + pp, n - 1)] : 0.0;
+    if (t < AC4_NQ) s_dc[t] = c_pcol[t] << 3 | c_dg[t];
+    if (t < FS_P) {
+        s_t[fs_ax(0, 0, 0) + t] = 1.0;
+        s_t[fs_ax(0, 0, 1) + t] = 0.0;
+    }
+    for (int tb = i0; tb < i1; tb += tp) {
+        if (t < 3 * FS_P) s_p[t / FS_P][pp] = p;
+        // the mask words of this tile, loaded while its tables are built
+        const int w = tb >> 5, sh = tb & 31, cnt = min(tp, i1 - tb);
+        unsigned mw[NR], mx[NR];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            mw[r] = mrow[r][w];
+            mx[r] = mrow[r][sh + cnt > 32 ? w + 1 : w];
+        }
+        __syncthreads();
+        if (t < 3 * FS_P) p = src[min(tb + tp + pp, n - 1)];  // the next tile's
+        for (int e = t / FS_P; e < 3 * FS_M; e += S4_T / FS_P) {
+            const int a = e / FS_M, m = e - a * FS_M + 1;
+            const double q = s_p[a][pp], f = fma((double)m, q, -rint((double)m * q));
+            double sn, cs;
+            ac4_sincos_turns(f, &sn, &cs);
+            s_t[fs_ax(a, m, 0) + pp] = cs;
+            s_t[fs_ax(a, m, 1) + pp] = sn;
+        }
+        __syncthreads();
+        for (int e = t / FS_P; e < 3 * FS_J; e += S4_T / FS_P) {
+            const int a = e / FS_J, j = e - a * FS_J + 1, b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+            const double cb = s_t[fs_ax(b, j, 0) + pp], sb = s_t[fs_ax(b, j, 1) + pp], cc = s_t[fs_ax(c, j, 0) + pp],
+                         sc = s_t[fs_ax(c, j, 1) + pp];
+            s_t[fs_pr(a, j, 0) + pp] = fma(cb, cc, -(sb * sc));
+            s_t[fs_pr(a, j, 1) + pp] = fma(sb, cc, cb * sc);
+        }
+        __syncthreads();
+        // the bits of the tile's particles, its first one lowest
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const unsigned long long m = (unsigned long long)mx[r] << 32 | mw[r];
+            mw[r] = live[r] ? (unsigned)(m >> sh) & (cnt < 32 ? (1u << cnt) - 1u : ~0u) : 0u;
+        }
+        for (int st = 0; st < tp; st += 4) {
+            const int q = st + k4;
+            double a[NR];
+#pragma unroll
+            for (int r = 0; r < NR; r++) a[r] = (mw[r] >> q) & 1u ? 1.0 : 0.0;
+#pragma unroll
+            for (int c = 0; c < S4_CPW; c++) {
+                const double uc = s_t[u[c] + q], us = s_t[u[c] + FS_RL + q], vc = s_t[v[c] + q], vs = s_t[v[c] + FS_RL + q];
+                const double pc = fma(uc, vc, -(us * vs)), ps = fma(us, vc, uc * vs);
+#pragma unroll
+                for (int r = 0; r < NT16; r++) {
+                    ac[c][r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], pc, ac[c][r], 0, 0, 0);
+                    as[c][r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], ps, as[c][r], 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < NT4; r++) {
+                    bc[c][r] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[NT16 + r], pc, bc[c][r], 0, 0, 0);
+                    bs[c][r] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[NT16 + r], ps, bs[c][r], 0, 0, 0);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const int oq = t % AC4_NQ, od = s_dc[oq] & 7, oc = s_dc[oq] >> 3;  // this thread's vector, its columns
+#pragma unroll
+    for (int sn = 0; sn < 2; sn++) {
+#pragma unroll
+        for (int c = 0; c < S4_CPW; c++) {
+            double *d = &s_t[(wv * S4_CPW + c) * 16 + i16 + k4 * S4_NCOL];
+#pragma unroll
+            for (int r = 0; r < NT16; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) d[(16 * r + 4 * e) * S4_NCOL] = sn ? as[c][r][e] : ac[c][r][e];
+#pragma unroll
+            for (int r = 0; r < NT4; r++) d[(16 * NT16 + 4 * r) * S4_NCOL] = sn ? bs[c][r] : bc[c][r];
+        }
+        __syncthreads();
+        // thread t: vector t % AC4_NQ of lags t / AC4_NQ, + S4_T / AC4_NQ, ...
+        for (int l = t / AC4_NQ; l < nl && t < S4_T / AC4_NQ * AC4_NQ; l += S4_T / AC4_NQ) {
+            const double *w = s_t + l * S4_NCOL + oc;
+            double sum = w[0];
+            if (od > 1) sum = (sum + w[1]) + w[2];
+            if (od > 3) sum = ((sum + w[3]) + w[4]) + w[5];
+            part[(((size_t)blockIdx.x * nl + l) * 2 + sn) * AC4_NQ + oq] = sum;
+        }
+        __syncthreads();
+    }
+}
+
+// Per lag l of the pass and value v (v < AC4_NQ: cos sum of vector v, else
+// sin sum of vector v - AC4_NQ): grid (nl, ceil(2*AC4_NQ/64)), 1024 threads.
+// Wave w sums chunks w, w+16, ..., the 16 wave sums are added in order and
+// divided by the number of permutations.  s4[pair*2*AC4_NQ + v].
+#define S4_RW 16
+__global__ void __launch_bounds__(64 * S4_RW) k_s4_reduce(const double *__restrict__ part, int nchunk, int nl,
+                                                          const int *__restrict__ lags, double *__restrict__ s4) {
+    const int l = blockIdx.x;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int v = blockIdx.y * 64 + lane;
+    const bool ok = v < 2 * AC4_NQ;
+    const double *src = part + (size_t)l * 2 * AC4_NQ + (ok ? v : 0);
+    double acc = 0.0;
+#pragma unroll 4
+    for (int c = wv; c < nchunk; c += S4_RW) acc += src[(size_t)c * nl * 2 * AC4_NQ];
+    __shared__ double s_w[S4_RW][64];
+    s_w[wv][lane] = acc;
+    __syncthreads();
+    if (wv == 0 && ok) {
+        double tot = s_w[0][lane];
+        for (int w = 1; w < S4_RW; w++) tot += s_w[w][lane];
+        s4[(size_t)lags[l] * 2 * AC4_NQ + v] = tot / (double)c_dg[v < AC4_NQ ? v : v - AC4_NQ];
+    }
+}
+
+// The same for small systems (n <= S4_SMALL), where the launch is as long as
+// one workgroup: a workgroup per chunk and column tile, each phase by a sincos
+// of its own, the waves' particles split further.  us per origin with its
+// reduction, 22 lags: 1000 particles 12.0 against k_s4_origin's 18.2, 4000 the
+// same, 50000 124 against 83.5.
+// One pass of up to RT*16 lags: grid (chunks, S4_NCT), 256 threads.  Wave w of block (c, ct) takes the mask words
 // [(4c+w)*wpw, (4c+w+1)*wpw) -- 32 particles each, 4 per MFMA step -- and
 // the 16 permuted vectors of column tile ct.  v_mfma_f64_16x16x4f64 operand
 // layout: lane l = i + 16k holds A[i][k] (mask bit of lag i, particle k) and
@@ -502,7 +702,7 @@ __global__ void __launch_bounds__(FS_T) k_frame_fs(const Job *__restrict__ jobs,
 // sums are added in wave order through LDS, and the block writes
 // part[((c*rows + row)*2 + {cos,sin})*S4_NCOL + column].
 template <int RT>
-__global__ void __launch_bounds__(256) k_s4_origin(const double *__restrict__ x0, const double *__restrict__ y0,
+__global__ void __launch_bounds__(256) k_s4_small(const double *__restrict__ x0, const double *__restrict__ y0,
                                                    const double *__restrict__ z0, int n, int nwords,
                                                    const unsigned *__restrict__ mask, const int *__restrict__ lags,
                                                    int nl, int wpw, double *__restrict__ part) {
@@ -569,7 +769,7 @@ __global__ void __launch_bounds__(256) k_s4_origin(const double *__restrict__ x0
 // Wave w sums chunks w, w+4, ... (each over the vector's permutations in
 // order); the four wave sums are added in wave order and divided by the
 // number of permutations.  s4[pair*2*AC4_NQ + v].
-__global__ void __launch_bounds__(256) k_s4_reduce(const double *__restrict__ part, int nchunk, int rows,
+__global__ void __launch_bounds__(256) k_s4_small_reduce(const double *__restrict__ part, int nchunk, int rows,
                                                    const int *__restrict__ lags, double *__restrict__ s4) {
     const int l = blockIdx.x;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -682,7 +882,7 @@ struct ac4_ana {
     int *d_s4_opairs = nullptr;
     unsigned *d_s4mask = nullptr;
     double *d_s4part = nullptr;
-    int nwords = 0, s4_wpw = 1, s4_nchunk = 1;
+    int nwords = 0, s4_ppb = 16, s4_tp = 16, s4_nchunk = 1, s4_wpw = 1;
     int fs_j0 = 0, fs_j1 = 0, fs_wait = 0;  // jobs whose Fs partials are in d_part, how many it holds
     int max_jobs = 0, ppb = ABLK, nb = 0, fs_ppb = FS_P, fs_nb = 0;
     std::vector<int> vx, vy, vz, qsq;
@@ -801,41 +1001,56 @@ static int s4_setup(ac4_ana *an) {
         if (an->W[1].last_use[o] >= 0) an->s4_end[an->W[1].last_use[o]].push_back(o);
     an->s4_done.assign(an->nframes, 0);
     an->nwords = (an->n + 31) / 32;
-    an->s4_wpw = std::max(1, (an->nwords + 4 * S4_CHUNKS - 1) / (4 * S4_CHUNKS));
-    an->s4_nchunk = (an->nwords + 4 * an->s4_wpw - 1) / (4 * an->s4_wpw);
+    an->s4_wpw = std::max(1, (an->nwords + 4 * S4_SMALL_CHUNKS - 1) / (4 * S4_SMALL_CHUNKS));
+    // chunks: at least 16 particles each, at most S4_CHUNKS of them; the tiles of a chunk as even as they go
+    an->s4_ppb = std::max(16, 4 * ((an->n + 4 * S4_CHUNKS - 1) / (4 * S4_CHUNKS)));
+    an->s4_nchunk = (an->n + an->s4_ppb - 1) / an->s4_ppb;
+    const int nt = (an->s4_ppb + FS_P - 1) / FS_P;
+    an->s4_tp = 4 * ((an->s4_ppb / 4 + nt - 1) / nt);
+    size_t part = (size_t)an->s4_nchunk * S4_LAGS * 2 * AC4_NQ;
+    if (an->n <= S4_SMALL) {
+        an->s4_nchunk = (an->nwords + 4 * an->s4_wpw - 1) / (4 * an->s4_wpw);
+        part = (size_t)an->s4_nchunk * S4_LAGS * 2 * S4_NCOL;
+    }
     const size_t np1 = std::max(w.np, 1);
     AC4_HIP(hipMalloc(&an->d_s4_opairs, sizeof(int) * np1));
     AC4_HIP(hipMemcpy(an->d_s4_opairs, an->s4_opairs.data(), sizeof(int) * np1, hipMemcpyHostToDevice));
     AC4_HIP(hipMalloc(&an->d_s4mask, sizeof(unsigned) * np1 * an->nwords));
-    AC4_HIP(hipMalloc(&an->d_s4part, sizeof(double) * (size_t)an->s4_nchunk * 16 * S4_RT_MAX * 2 * S4_NCOL));
+    AC4_HIP(hipMalloc(&an->d_s4part, sizeof(double) * part));
     AC4_HIP(hipMemset(an->d_s4mask, 0, sizeof(unsigned) * np1 * an->nwords));
     AC4_HIP(hipMemset(an->d_s4, 0, sizeof(double) * 2 * AC4_NQ * np1));
     return AC4_OK;
 }
 
 // The S4 sums of every pair of origin o, from its resident frame and the
-// masks its lags left; passes of up to 16*S4_RT_MAX lags.
+// masks its lags left; passes of up to S4_LAGS lags.
 static int s4_origin(ac4_ana *an, int o) {
     AC4_REQUIRE(an->resident[o], AC4_ESTATE, "S4: origin frame %d is not resident", o);
     const double *ox = an->org.at(an->place[o], 0), *oy = an->org.at(an->place[o], 1), *oz = an->org.at(an->place[o], 2);
     hipStream_t s = an->stream;
     const int b = an->s4_optr[o], e = an->s4_optr[o + 1];
-    for (int p0 = b; p0 < e; p0 += 16 * S4_RT_MAX) {
-        const int nl = std::min(16 * S4_RT_MAX, e - p0), rt = (nl + 15) / 16;
-        const int *lags = an->d_s4_opairs + p0;
-        const dim3 g(an->s4_nchunk, S4_NCT);
-        switch (rt) {
-            case 1: hipLaunchKernelGGL(k_s4_origin<1>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
-                                       an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
-            case 2: hipLaunchKernelGGL(k_s4_origin<2>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
-                                       an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
-            case 3: hipLaunchKernelGGL(k_s4_origin<3>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
-                                       an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
-            default: hipLaunchKernelGGL(k_s4_origin<4>, g, dim3(256), 0, s, ox, oy, oz, an->n, an->nwords,
-                                        an->d_s4mask, lags, nl, an->s4_wpw, an->d_s4part); break;
+    for (int p0 = b; p0 < e; p0 += S4_LAGS) {
+        const int nl = std::min(S4_LAGS, e - p0);
+        if (an->n <= S4_SMALL) {
+            const int rt = (nl + 15) / 16;
+            hipLaunchKernelGGL(rt == 1 ? k_s4_small<1> : k_s4_small<2>, dim3(an->s4_nchunk, S4_NCT), dim3(256), 0, s, ox, oy, oz,
+                               an->n, an->nwords, an->d_s4mask, an->d_s4_opairs + p0, nl, an->s4_wpw, an->d_s4part);
+            hipLaunchKernelGGL(k_s4_small_reduce, dim3(nl, (2 * AC4_NQ + 63) / 64), dim3(256), 0, s, an->d_s4part,
+                               an->s4_nchunk, rt * 16, an->d_s4_opairs + p0, an->d_s4);
+            AC4_HIP(hipGetLastError());
+            continue;
         }
-        hipLaunchKernelGGL(k_s4_reduce, dim3(nl, (2 * AC4_NQ + 63) / 64), dim3(256), 0, s, an->d_s4part,
-                           an->s4_nchunk, rt * 16, lags, an->d_s4);
+        // row tiles of 16 lags, the rest in tiles of 4; more than 12 are a tile of 16 as well
+        const int nt16 = (nl + 3) / 16, nt4 = std::max(0, nl - 16 * nt16 + 3) / 4;
+        const int *lags = an->d_s4_opairs + p0;
+        auto *k = nt16 == 2 ? k_s4_origin<2, 0>
+                  : nt16 == 1 ? (nt4 == 0 ? k_s4_origin<1, 0> : nt4 == 1 ? k_s4_origin<1, 1>
+                                 : nt4 == 2 ? k_s4_origin<1, 2> : k_s4_origin<1, 3>)
+                              : (nt4 == 1 ? k_s4_origin<0, 1> : nt4 == 2 ? k_s4_origin<0, 2> : k_s4_origin<0, 3>);
+        hipLaunchKernelGGL(k, dim3(an->s4_nchunk), dim3(S4_T), 0, s, ox, oy, oz, an->n, an->nwords, an->d_s4mask, lags, nl,
+                           an->s4_ppb, an->s4_tp, an->d_s4part);
+        hipLaunchKernelGGL(k_s4_reduce, dim3(nl, (2 * AC4_NQ + 63) / 64), dim3(64 * S4_RW), 0, s, an->d_s4part,
+                           an->s4_nchunk, nl, lags, an->d_s4);
         AC4_HIP(hipGetLastError());
     }
     an->s4_done[o] = 1;

@@ -226,3 +226,24 @@ def test_device_arrays_reused_after_the_push(gpu, n, obs):
     assert not obs & 8 or len(out[0][-1]) > 32
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# S4 by origin with every split of the lags into row tiles of 16 and 4 (and
+# two passes), sizes at the line between its two kernels, chunks that end in
+# the middle of a mask word, and tiles of less than 32 particles.
+@pytest.mark.parametrize("n,nf,nl", [(3073, 5, 2), (3100, 11, 5), (3100, 26, 12), (3073, 30, 14), (3079, 36, 17),
+                                     (3072, 46, 22), (3100, 46, 22), (3100, 54, 26), (3100, 64, 31), (3100, 90, 44),
+                                     (40001, 11, 5)])
+def test_s4_lag_tiles(gpu, n, nf, nl):
+    frames = list(range(nf))
+    X, Y, Z, T = trajgen.make_frames(n, frames, 11 + n + nf, 0.03, 1.0)
+    L = (n / 1.2) ** (1.0 / 3.0)
+    an = gpu.Analysis(n, L, frames, gap=nf + 1, factor=1.01, obs=4)
+    for f in range(nf):
+        an.push(f, X[f], Y[f], Z[f], T[f])
+    an.finalize()
+    v, m = an.pairs(gpu.OBS_S4)
+    an.close()
+    o = OL.phase("s4", n, L, X, Y, Z, T, frames, nf + 1, factor=1.01)
+    assert len(m) == nl and np.array_equal(m, o["mask"]) and m.max() > 0
+    assert np.abs(v - o["pairs"]).max() < 1e-12 * n  # a term is off by at most a few 1e-14
