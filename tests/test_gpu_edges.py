@@ -247,3 +247,32 @@ def test_s4_lag_tiles(gpu, n, nf, nl):
     o = OL.phase("s4", n, L, X, Y, Z, T, frames, nf + 1, factor=1.01)
     assert len(m) == nl and np.array_equal(m, o["mask"]) and m.max() > 0
     assert np.abs(v - o["pairs"]).max() < 1e-12 * n  # a term is off by at most a few 1e-14
+
+
+# Columns of the written form (one to three digits and a point and five digits
+# between tabs) next to others of nearly that form, in any column; workgroups
+# of 256 lines whose text fits the staged 96 bytes a line and whose does not;
+# segment and 16-byte edges by the varying lengths.  Bit for bit the host
+# reader's values.
+@pytest.mark.parametrize("n,blanks", [(1, 0), (255, 0), (257, 0), (3000, 0), (600, 90)])
+def test_text_columns_of_every_width(gpu, n, blanks):
+    rng = np.random.default_rng(n)
+    forms = ["%.5f", "%.5f", "%.5f", "%.5f", "%.4f", "%.6f", "%.0f", "%.5f ", " %.5f", "%+.5f", "%010.5f", "%.9f"]
+    lines = []
+    for i in range(2 * n):
+        v = rng.normal(0.0, 1.0, 3) * 10.0 ** rng.integers(-6, 5, 3)
+        f = [forms[k] for k in (rng.integers(0, 4, 3) if i % 3 else rng.integers(0, len(forms), 3))]
+        sep = "\t" if i % 5 else "\t " if i % 2 else " "
+        t = str(rng.integers(0, 3)) if i % 4 else str(rng.integers(-12, 120))
+        lines.append(sep.join([f[k] % v[k] for k in range(3)] + [t]) + " " * (blanks if i % 7 else 0))
+    text = ("\n".join(lines) + "\n").encode()
+    tf = gpu.TextFrames(n, len(text) + 64)
+    k, used = tf.parse(text)
+    assert k == 2 and used == len(text)
+    pos = 0
+    for f in range(2):
+        x, y, z, t, u = gpu.parse_frame(text[pos:], n)
+        pos += u
+        for a, b in zip(tf.frame(f), (x, y, z, t)):
+            assert np.array_equal(a, b) and np.array_equal(np.signbit(a), np.signbit(b))
+    tf.close()
