@@ -2011,10 +2011,14 @@ struct ac4_md {
     // frame text on the device (ac4_md_format_frame): 80-byte line slots in
     // reference order, line lengths, the joined text, per-block byte offsets
     // (the total after the last block) and a flag
+    // frame text: a slot of 80 bytes per line and its length, the bytes of each
+    // block of lines, and in pinned memory two pieces of the joined text (one
+    // for a frame of one piece) and the words k_fmt_* leave for the host
     char *fmt_dev = nullptr, *fmt_txt = nullptr;
     unsigned char *fmt_len_dev = nullptr;
-    long long *fmt_boff = nullptr;
-    int *fmt_bad = nullptr;
+    int *fmt_bsum = nullptr;
+    long long *fmt_meta = nullptr;  // [0, 1]: bytes of a piece, [2]: a value for the host's formatter
+    hipEvent_t fmt_ev[2] = {nullptr, nullptr};
     size_t fmt_cap = 0;
     unsigned int *ov_cnt = nullptr;
     int *ov_n = nullptr;
@@ -2437,6 +2441,22 @@ extern "C" int ac4_md_create(int n_rep, const ac4_replica_params *p, int precisi
     return AC4_OK;
 }
 
+static void free_fmt(ac4_md *md) {
+    for (void *q : {(void *)md->fmt_dev, (void *)md->fmt_len_dev, (void *)md->fmt_bsum})
+        if (q) (void)hipFree(q);
+    for (void *q : {(void *)md->fmt_txt, (void *)md->fmt_meta})
+        if (q) (void)hipHostFree(q);
+    for (hipEvent_t &ev : md->fmt_ev) {
+        if (ev) (void)hipEventDestroy(ev);
+        ev = nullptr;
+    }
+    md->fmt_dev = md->fmt_txt = nullptr;
+    md->fmt_len_dev = nullptr;
+    md->fmt_bsum = nullptr;
+    md->fmt_meta = nullptr;
+    md->fmt_cap = 0;
+}
+
 extern "C" int ac4_md_destroy(ac4_md *md) {
     if (!md) return AC4_OK;
     if (md->stream) (void)hipStreamSynchronize(md->stream);
@@ -2450,9 +2470,7 @@ extern "C" int ac4_md_destroy(ac4_md *md) {
                     md->cnt, md->start, md->members, md->kx, md->ky, md->kz, md->ex, md->ey, md->ez, md->et};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
-    for (void *q : {(void *)md->fmt_dev, (void *)md->fmt_txt, (void *)md->fmt_len_dev, (void *)md->fmt_boff,
-                    (void *)md->fmt_bad})
-        if (q) (void)hipFree(q);
+    free_fmt(md);
     free_parts(md->P);
     free_parts(md->A);
     if (md->ftab) (void)hipFree(md->ftab);
@@ -2746,6 +2764,10 @@ extern "C" int ac4_md_set_chain(ac4_md *md, int r, const double *c9) {
 // q/10^5 "." q%10^5 with the sign of v.  Values with |v| >= 1e12 or not
 // finite set *bad (the host formats those frames).
 __device__ __forceinline__ char *fmt_put_u64(char *o, unsigned long long v) {
+    if (v < 10) {
+        *o++ = (char)('0' + (int)v);
+        return o;
+    }
     char t[24];
     int k = 0;
     do {
@@ -2755,7 +2777,7 @@ __device__ __forceinline__ char *fmt_put_u64(char *o, unsigned long long v) {
     while (k) *o++ = t[--k];
     return o;
 }
-__device__ char *fmt5_dev(char *o, double v, int *bad) {
+__device__ __forceinline__ char *fmt5_dev(char *o, double v, int *bad) {
     const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
     const int neg = (int)(bits >> 63), ex = (int)((bits >> 52) & 0x7ff);
     const unsigned long long frac = bits & ((1ull << 52) - 1);
@@ -2784,27 +2806,41 @@ __device__ char *fmt5_dev(char *o, double v, int *bad) {
         return o;
     }
     if (neg) *o++ = '-';
-    o = fmt_put_u64(o, q / 100000ull);
+    unsigned fp;
+    if (q < 1000ull * 100000ull) {  // up to three digits before the point: 32-bit arithmetic
+        const unsigned q32 = (unsigned)q, ip = q32 / 100000u;
+        fp = q32 - ip * 100000u;
+        if (ip >= 100u) *o++ = (char)('0' + ip / 100u);
+        if (ip >= 10u) *o++ = (char)('0' + ip / 10u % 10u);
+        *o++ = (char)('0' + ip % 10u);
+    } else {
+        o = fmt_put_u64(o, q / 100000ull);
+        fp = (unsigned)(q % 100000ull);
+    }
     *o++ = '.';
-    unsigned long long fp = q % 100000ull;
+#pragma unroll
     for (int d = 4; d >= 0; d--) {
-        o[d] = (char)('0' + fp % 10ull);
-        fp /= 10ull;
+        o[d] = (char)('0' + fp % 10u);
+        fp /= 10u;
     }
     return o + 5;
 }
 
 // line of the particle in slot s of replica R, written to slot id[s] (its
-// reference index) of out (80 bytes each)
+// reference index) of out (FMT_LINE bytes each), formed in LDS and stored 16
+// bytes at a time (50000 lines: 6.2 us; formed in scratch memory and stored
+// byte by byte 11.7)
+#define FMT_LINE 80
 __global__ void __launch_bounds__(BLK) k_fmt_frame(const RepC *__restrict__ reps, int r, const double *__restrict__ xu,
                                                    const double *__restrict__ yu, const double *__restrict__ zu,
                                                    const int *__restrict__ type, const int *__restrict__ id,
-                                                   char *out, unsigned char *len, int *bad) {
+                                                   char *out, unsigned char *len, long long *meta) {
+    __shared__ uint4 s_line[BLK][FMT_LINE / 16];
     const RepC R = reps[r];
     const int s = blockIdx.x * BLK + threadIdx.x;
     if (s >= R.n) return;
     const int g = R.off + s, i = id[g];
-    char line[80];
+    char *const line = (char *)s_line[threadIdx.x];
     int b = 0;
     char *o = fmt5_dev(line, xu[g], &b);
     *o++ = '\t';
@@ -2821,69 +2857,72 @@ __global__ void __launch_bounds__(BLK) k_fmt_frame(const RepC *__restrict__ reps
     }
     *o++ = '\n';
     const int k = (int)(o - line);
-    char *dst = out + (size_t)i * 80;
-    for (int c = 0; c < k; c++) dst[c] = line[c];
+    uint4 *dst = (uint4 *)(out + (size_t)i * FMT_LINE);
+#pragma unroll
+    for (int c = 0; c < FMT_LINE / 16; c++)
+        if (16 * c < k) dst[c] = s_line[threadIdx.x][c];
     len[i] = (unsigned char)k;
-    if (b) atomicOr(bad, 1);
+    if (b) meta[2] = 1;  // pinned; every writer stores the same
 }
 
 // bytes of each block of BLK lines (reference order)
-__global__ void __launch_bounds__(BLK) k_fmt_bsum(int n, const unsigned char *__restrict__ len,
-                                                  long long *__restrict__ boff) {
-    __shared__ int sum;
-    if (threadIdx.x == 0) sum = 0;
-    __syncthreads();
+__global__ void __launch_bounds__(BLK) k_fmt_bsum(int n, const unsigned char *__restrict__ len, int *__restrict__ bsum) {
+    __shared__ int s_w[BLK / 64];
     const int i = blockIdx.x * BLK + threadIdx.x;
-    if (i < n) atomicAdd(&sum, (int)len[i]);
+    const int w = ac4_wave_sum_i(i < n ? (int)len[i] : 0);
+    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = w;
     __syncthreads();
-    if (threadIdx.x == 0) boff[blockIdx.x] = sum;
+    if (threadIdx.x == 0) bsum[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
 }
 
-// exclusive prefix of the nb block sums in place, the total to boff[nb]; one
-// workgroup of FMT_SCAN threads, each scanning a contiguous chunk
-#define FMT_SCAN 1024
-__global__ void __launch_bounds__(FMT_SCAN) k_fmt_scan(int nb, long long *__restrict__ boff) {
-    __shared__ long long part[FMT_SCAN];
-    const int t = threadIdx.x, chunk = (nb + FMT_SCAN - 1) / FMT_SCAN;
-    const int lo = min(nb, t * chunk), hi = min(nb, lo + chunk);
-    long long acc = 0;
-    for (int b = lo; b < hi; b++) acc += boff[b];
-    part[t] = acc;
-    __syncthreads();
-    for (int d = 1; d < FMT_SCAN; d <<= 1) {  // inclusive Hillis-Steele scan
-        const long long v = t >= d ? part[t - d] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    long long run = part[t] - acc;
-    for (int b = lo; b < hi; b++) {
-        const long long v = boff[b];
-        boff[b] = run;
-        run += v;
-    }
-    if (t == FMT_SCAN - 1) boff[nb] = part[t];
-}
-
-// line i from its slot to its place in the joined text
-__global__ void __launch_bounds__(BLK) k_fmt_pack(int n, const char *__restrict__ slots,
-                                                  const unsigned char *__restrict__ len,
-                                                  const long long *__restrict__ boff, char *__restrict__ txt) {
-    __shared__ int sc[BLK];
-    const int t = threadIdx.x, i = blockIdx.x * BLK + t;
+// One piece of the text: lines of the blocks [b0, b0 + gridDim.x) from their
+// slots to txt (pinned host memory), and the piece's bytes to *bytes.  A block
+// adds up the blocks of the piece before it, joins its lines in LDS and stores
+// the joined text 16 bytes at a time, so that the bus carries whole words.
+#define FMT_PIECE 128  // blocks of a piece, at most
+__global__ void __launch_bounds__(BLK) k_fmt_pack(int n, int b0, const char *__restrict__ slots,
+                                                  const unsigned char *__restrict__ len, const int *__restrict__ bsum,
+                                                  char *__restrict__ txt, long long *bytes) {
+    __shared__ uint4 s_buf[BLK * FMT_LINE / 16 + 1];
+    __shared__ int s_w[2][BLK / 64];
+    char *const s_txt = (char *)s_buf;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, b = b0 + blockIdx.x, i = b * BLK + t;
+    static_assert(FMT_PIECE <= BLK, "one block sum per thread");
     const int k = i < n ? (int)len[i] : 0;
-    sc[t] = k;
-    __syncthreads();
-    for (int d = 1; d < BLK; d <<= 1) {
-        const int v = t >= d ? sc[t - d] : 0;
-        __syncthreads();
-        sc[t] += v;
-        __syncthreads();
+    uint4 v[FMT_LINE / 16];
+    const uint4 *src = (const uint4 *)(slots + (size_t)(i < n ? i : 0) * FMT_LINE);
+#pragma unroll
+    for (int c = 0; c < FMT_LINE / 16; c++)
+        if (16 * c < k) v[c] = src[c];
+    const int before = ac4_wave_sum_i(t < (int)blockIdx.x ? bsum[b0 + t] : 0);
+    int at = k;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(at, o, 64);
+        if (lane >= o) at += u;
     }
-    if (i >= n) return;
-    char *dst = txt + boff[blockIdx.x] + (sc[t] - k);
-    const char *src = slots + (size_t)i * 80;
-    for (int c = 0; c < k; c++) dst[c] = src[c];
+    if (lane == 63) s_w[0][w] = at;
+    if (lane == 0) s_w[1][w] = before;  // the wave's sum is in its first lane
+    __syncthreads();
+    const int off = s_w[1][0] + s_w[1][1] + s_w[1][2] + s_w[1][3], h = off & 15;
+    at += h - k;
+    for (int q = 0; q < w; q++) at += s_w[0][q];
+    const int end = h + s_w[0][0] + s_w[0][1] + s_w[0][2] + s_w[0][3];  // the block's text: s_txt[h, end)
+#pragma unroll
+    for (int c = 0; c < FMT_LINE / 16; c++) {
+        const unsigned u[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
+#pragma unroll
+        for (int q = 0; q < 16; q++)
+            if (16 * c + q < k) s_txt[at + 16 * c + q] = (char)(u[q / 4] >> (8 * (q % 4)));
+    }
+    __syncthreads();
+    char *const dst = txt + (off - h);
+    for (int q = 16 * t; q < end; q += 16 * BLK) {
+        if (q >= h && q + 16 <= end)
+            *(uint4 *)(dst + q) = s_buf[q / 16];
+        else  // words shared with the neighbouring blocks
+            for (int c = max(q, h); c < min(q + 16, end); c++) dst[c] = s_txt[c];
+    }
+    if (t == 0 && blockIdx.x == gridDim.x - 1) *bytes = off - h + end;
 }
 
 // data_coor.out text of replica r's current frame (x_u, y_u, z_u, type in
@@ -2895,42 +2934,57 @@ extern "C" long long ac4_md_format_frame(ac4_md *md, int r, char *out, long long
     const RepC &R = md->reps_h[r];
     const int n = R.n;
     AC4_REQUIRE(out && cap >= 80LL * n, AC4_EARG, "format_frame: buffer needs 80 bytes a line");
-    const int nb = (n + BLK - 1) / BLK;
+    const int nb = (n + BLK - 1) / BLK, np = (nb + FMT_PIECE - 1) / FMT_PIECE;
+    const auto piece_bytes = [](int blocks) { return (size_t)std::min(blocks, FMT_PIECE) * BLK * FMT_LINE; };
     if ((size_t)n > md->fmt_cap) {
-        for (void *q : {(void *)md->fmt_dev, (void *)md->fmt_txt, (void *)md->fmt_len_dev, (void *)md->fmt_boff,
-                        (void *)md->fmt_bad})
-            if (q) (void)hipFree(q);
-        md->fmt_dev = md->fmt_txt = nullptr;
-        md->fmt_len_dev = nullptr;
-        md->fmt_boff = nullptr;
-        md->fmt_bad = nullptr;
-        md->fmt_cap = 0;
+        free_fmt(md);
         const size_t cn = (size_t)n;
-        AC4_HIP(hipMalloc(&md->fmt_dev, 80 * cn));
-        AC4_HIP(hipMalloc(&md->fmt_txt, 80 * cn));
+        AC4_HIP(hipMalloc(&md->fmt_dev, FMT_LINE * cn));
         AC4_HIP(hipMalloc(&md->fmt_len_dev, cn));
-        AC4_HIP(hipMalloc(&md->fmt_boff, sizeof(long long) * (nb + 1)));
-        AC4_HIP(hipMalloc(&md->fmt_bad, sizeof(int)));
+        AC4_HIP(hipMalloc(&md->fmt_bsum, sizeof(int) * nb));
+        AC4_HIP(hipHostMalloc((void **)&md->fmt_txt, piece_bytes(nb) * (np > 1 ? 2 : 1), hipHostMallocDefault));
+        AC4_HIP(hipHostMalloc((void **)&md->fmt_meta, 3 * sizeof(long long), hipHostMallocDefault));
+        for (hipEvent_t &ev : md->fmt_ev) AC4_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         md->fmt_cap = cn;
     }
     if (n == 0) return 0;
     hipStream_t s = md->stream;
-    AC4_HIP(hipMemsetAsync(md->fmt_bad, 0, sizeof(int), s));
+    volatile long long *meta = md->fmt_meta;
+    meta[2] = 0;
     hipLaunchKernelGGL(k_fmt_frame, dim3(nb), dim3(BLK), 0, s, md->reps, r, md->P.xu, md->P.yu, md->P.zu, md->P.type,
-                       md->P.id, md->fmt_dev, md->fmt_len_dev, md->fmt_bad);
+                       md->P.id, md->fmt_dev, md->fmt_len_dev, md->fmt_meta);
+    hipLaunchKernelGGL(k_fmt_bsum, dim3(nb), dim3(BLK), 0, s, n, md->fmt_len_dev, md->fmt_bsum);
     AC4_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_fmt_bsum, dim3(nb), dim3(BLK), 0, s, n, md->fmt_len_dev, md->fmt_boff);
-    AC4_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_fmt_scan, dim3(1), dim3(FMT_SCAN), 0, s, nb, md->fmt_boff);
-    AC4_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_fmt_pack, dim3(nb), dim3(BLK), 0, s, n, (const char *)md->fmt_dev,
-                       (const unsigned char *)md->fmt_len_dev, (const long long *)md->fmt_boff, md->fmt_txt);
-    AC4_HIP(hipGetLastError());
-    int bad = 0;
+    // the pieces over the bus straight from their kernel, two under way; the
+    // host copies one to the caller's buffer while the next is written.  A
+    // copy from the device to the caller's pageable memory takes 90 us for the
+    // 1.55 MB of 50000 lines, this way 27 over the bus and 18 by memcpy; the
+    // whole call 142 -> 82 us (the two small results alone, copied to pageable
+    // memory, took 20 of it)
+    const auto pack = [&](int p) {
+        const int b0 = p * FMT_PIECE;
+        hipLaunchKernelGGL(k_fmt_pack, dim3(std::min(FMT_PIECE, nb - b0)), dim3(BLK), 0, s, n, b0, md->fmt_dev,
+                           md->fmt_len_dev, md->fmt_bsum, md->fmt_txt + (p & 1) * piece_bytes(nb), md->fmt_meta + (p & 1));
+        if (p + 1 < np) AC4_HIP(hipEventRecord(md->fmt_ev[p & 1], s));
+        AC4_HIP(hipGetLastError());
+        return AC4_OK;
+    };
+    for (int p = 0; p < std::min(np, 2); p++) TRY(pack(p));
+    bool bad = false;
     long long total = 0;
-    AC4_HIP(hipMemcpyAsync(&bad, md->fmt_bad, sizeof(int), hipMemcpyDeviceToHost, s));
-    AC4_HIP(hipMemcpyAsync(&total, md->fmt_boff + nb, sizeof(long long), hipMemcpyDeviceToHost, s));
-    AC4_HIP(hipStreamSynchronize(s));
+    for (int p = 0; p < np && !bad; p++) {
+        if (p + 1 < np)
+            AC4_HIP(hipEventSynchronize(md->fmt_ev[p & 1]));
+        else
+            AC4_HIP(hipStreamSynchronize(s));
+        bad = meta[2] != 0;  // known with the first piece
+        const long long k = meta[p & 1];
+        AC4_REQUIRE(k > 0 && k <= (long long)piece_bytes(nb) && total + k <= (long long)FMT_LINE * n, AC4_ESTATE,
+                    "format_frame: piece of %lld bytes", k);
+        if (!bad) memcpy(out + total, md->fmt_txt + (p & 1) * piece_bytes(nb), (size_t)k);
+        total += k;
+        if (!bad && p + 2 < np) TRY(pack(p + 2));
+    }
     if (bad) {  // a value the device formatter does not cover: the host formats the frame
         std::vector<double> x(n), y(n), z(n);
         std::vector<int> id, ty(n);
@@ -2941,9 +2995,6 @@ extern "C" long long ac4_md_format_frame(ac4_md *md, int r, char *out, long long
         TRY(fetch_unpermuted(md, r, (const int *)md->P.type, ty.data(), id));
         return ac4_format_frame(n, x.data(), y.data(), z.data(), ty.data(), out, cap);
     }
-    AC4_REQUIRE(total > 0 && total <= 80LL * n, AC4_ESTATE, "format_frame: joined text of %lld bytes", total);
-    AC4_HIP(hipMemcpyAsync(out, md->fmt_txt, (size_t)total, hipMemcpyDeviceToHost, s));
-    AC4_HIP(hipStreamSynchronize(s));
     return total;
 }
 

@@ -276,3 +276,22 @@ def test_text_columns_of_every_width(gpu, n, blanks):
         for a, b in zip(tf.frame(f), (x, y, z, t)):
             assert np.array_equal(a, b) and np.array_equal(np.signbit(a), np.signbit(b))
     tf.close()
+
+
+# Frame text in one, exactly one, two and three pieces of 128 blocks of 256
+# lines, a small replica through the buffers of a large one, columns of one to
+# twelve digits before the point, and a value the host has to format.
+@pytest.mark.parametrize("sizes", [(256, 257), (32768,), (32769, 300), (65793, 256)])
+def test_frame_text_pieces(gpu, sizes):
+    md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 200, 7) for n in sizes])
+    rng = np.random.default_rng(sum(sizes))
+    for r, n in enumerate(sizes):
+        for big in (0.0, 1e12):
+            xu = rng.normal(0.0, 1.0, (3, n)) * 10.0 ** rng.integers(-7, 11, (3, n))
+            xu[:, ::3] = np.round(xu[:, ::3], 6) + 5e-6  # halves of the last digit
+            xu[0, -1] = big
+            x = rng.random((3, n))
+            ty = rng.integers(-9, 120, n).astype(np.int32) if big else (rng.random(n) < 0.2).astype(np.int32)
+            md.set_state(r, *x, *xu, *x, (ty & 1))
+            assert md.format_frame(r) == gpu.format_frame(*xu, ty & 1)
+    md.close()
