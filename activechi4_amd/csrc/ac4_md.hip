@@ -55,8 +55,11 @@ struct RepC {
     double qscale;  // L / 2^32: real length of one unit of a fixed-point coordinate
     double skin;    // Verlet skin: list radii 2.5 sigma_ab + skin, rebuild criterion
     float qs2;      // qscale^2 in FP32
-    int xcull;      // list teams skip the far x-half of the cells beside along x (configure_rep)
+    int xcull;      // a cell's slots are ordered by x-half, which list teams may skip (configure_rep)
     int enblk, eblk_off;   // blocks of the energy pass (k_energy), 0 without it
+    float lcut[3];         // qscreen_cut of species pair ab
+    float lr2[2];          // what a particle of species a reaches in any list, squared, with a margin of 2e-3
+    float rnc, cell, fix2cell;  // 1/nc, L/nc, nc/2^32
     float rcq[3], c2i[3];  // species pair ab: cutoff^2 in fixed-point units^2, C2 / sigma^2 (FP32 path)
 };
 
@@ -876,7 +879,7 @@ __global__ void __launch_bounds__(BLK) k_commit(const RepC *__restrict__ reps, c
 // pair); pairs are stored when ((dx*dx+dy*dy)+dz*dz)*L*L < (2.5 sigma_ab +
 // skin)^2.  The reference list (< 2.85^2 for every pair,
 // cell_list+forces.c:129-130) is counted beside it.
-__device__ __forceinline__ double list_cut2(int ab, double skin) {
+__host__ __device__ __forceinline__ double list_cut2(int ab, double skin) {
     const double rc = (ab == 0 ? (2.5 * 1.00) : (ab == 1 ? (2.5 * 0.80) : (2.5 * 0.88))) + skin;
     return rc * rc;
 }
@@ -890,6 +893,16 @@ __device__ __forceinline__ size_t nl_at(const RepC &R, int cap, int k, int i) {
     return (size_t)R.off * cap + (((size_t)(k >> R.lc) * R.n + i) << R.lc) + (k & ((1 << R.lc) - 1));
 }
 
+// The particle's position at slot j; a 32-bit byte offset for the 12-byte
+// records (a handle of 2^32 / 12 slots does not fit the memory).
+__device__ __forceinline__ QPos ld_pos(const QPos *p, int j) {
+    const unsigned u = (unsigned)j;
+    unsigned u3;  // 3u by a shift and an add; the compiler's product by 12 is a multiplication at a quarter of the rate
+    asm("v_lshl_add_u32 %0, %1, 1, %1" : "=v"(u3) : "v"(u));
+    return *(const QPos *)((const char *)p + (size_t)(u3 << 2));
+}
+__device__ __forceinline__ double4 ld_pos(const double4 *p, int j) { return p[j]; }
+
 // Dynamics-list screen shared by every builder (so all of them keep exactly
 // the same pairs): minimum image from the fixed-point positions, r^2 in FP32
 // in fixed-point units (fused multiply-adds) against the list radius plus a
@@ -902,8 +915,11 @@ __device__ __forceinline__ bool qscreen(const QPos &pi, const QPos &q, float ua,
     return __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < ((q.x & 1u) ? ub : ua);
 }
 // list radius^2 of species pair ab plus the screen's margin, in fixed-point units^2
+__host__ __device__ __forceinline__ float qscreen_cut_of(int ab, double skin, float qs2) {
+    return (float)((list_cut2(ab, skin) + 1e-3) / (double)qs2);
+}
 __device__ __forceinline__ float qscreen_cut(int ab, const RepC &R) {
-    return (float)((list_cut2(ab, R.skin) + 1e-3) / (double)R.qs2);
+    return ab == 0 ? R.lcut[0] : (ab == 1 ? R.lcut[1] : R.lcut[2]);
 }
 
 #define NL_UNROLL 8
@@ -996,27 +1012,40 @@ __global__ void __launch_bounds__(BLK) k_nlist(const RepC *__restrict__ reps, Ch
 // every lane of a team is active at each ballot.  FP32 screen with the margin
 // described at k_nlist.
 //
-// The stencil's slot ranges are cut into chunks of NLT candidates, listed by
-// the team in its LDS row (ct, CH_CAP entries), and the team takes CH_PER
-// chunks per round, with CH_PER loads in flight per lane across range
-// boundaries: about half the dependent rounds of a range-by-range walk, the
-// same candidates in the same order.  A stencil of more than CH_CAP chunks
-// (crowded cells, narrow teams) is walked range by range.
+// The stencil's slot ranges, trimmed to what the particle can reach, are cut
+// into groups of CH_GRP candidates, listed by the team in its LDS row (ct,
+// CH_CAP entries): a step of the walk takes the next NLT / CH_GRP groups, one
+// round CH_PER steps, with CH_PER loads in flight per lane across range
+// boundaries; the same candidates in the same order as a range-by-range walk,
+// which a stencil of more than CH_CAP groups (crowded cells) takes.  (Chunks
+// of one range per step left 1 lane in 4 of a step idle.)
 //
-// Where the replica allows it (RepC::xcull), the range holding the cell
-// beside the home cell along x on the far side loses that cell's far x-half:
-// its start moves to the cell's xmid for a particle in the upper x-half of
-// its own cell (the cell below), its end for one in the lower half (the cell
-// above).  Those candidates are at least one cell width away, beyond every
-// list radius, so the lists are the same pairs in the same order; each of the
-// 9 rows loses half a cell, 1/6 of the candidates.
-#define CH_CAP 64
+// Trimming: a row of cells beside the particle's own along y or z is at least
+// d away, d^2 the sum of the squared distances to the faces between; along x
+// the row is needed up to sqrt(rl^2 - d^2) from the particle, rl the largest
+// list radius of its species.  The cell below or above along x goes where its
+// face is farther, or its far half where that is farther and the cells' slots
+// are ordered by x-half (RepC::xcull, xmid), or the whole row.  What goes is
+// beyond every list radius, so the lists are the same pairs in the same order.
+// Of 27 cells' candidates 18 are left without the halves, 16 with (species A;
+// 13.6 of B), where the halves alone left 22.5.
+//
+// The walk is bound by vector instructions, about 30 per step (screen, place,
+// store).  With the trimming, which costs some 200 per particle pair of a wave:
+// 62.4 -> 59.8 us per step on the 64-replica ensemble, 50.3 -> 48.9 at N=50000
+// FP64.  TRIM = false leaves it out, for handles without a replica ordered by
+// x-half: one box of 1e6 (cells of 2.852, skin 0.35) builds its lists in 840 us
+// without and 926 with it (895 before the step lost its multiplication by 12
+// and the ballots their detour over a register).
+#define CH_CAP 128
+#define CH_GRP 16
 #define CH_PER 4
-template <int NLT, bool CULL>
+template <int NLT, bool TRIM>
 __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, ChainS *chain,
                                                const QPos *__restrict__ posq, const int *__restrict__ cell_of,
-                                               const int2 *__restrict__ ranges,
+                                               const int2 *__restrict__ ranges, const int *__restrict__ start,
                                                const int *__restrict__ xmid, int *nn, int *nl, int cap, int2 *ct) {
+    constexpr int GPS = NLT / CH_GRP;  // groups of a step
     const int lane = threadIdx.x & 63, t = lane & (NLT - 1);
     const unsigned long long tmask = (NLT == 64 ? ~0ull : ((1ull << (NLT & 63)) - 1ull)) << (lane & ~(NLT - 1));
     const unsigned long long below = (1ull << lane) - 1ull;
@@ -1027,36 +1056,38 @@ __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, Chai
     const int2 *rgs = ranges + (size_t)(R.off_cell + cg) * NRANGE;
     const float ua = qscreen_cut(ti, R), ub = qscreen_cut(ti + 1, R);
     int count = 0;
-    auto inlist = [&](const QPos &q) -> bool { return qscreen(pi, q, ua, ub); };
+    // the lanes whose candidate k at q is in the list (qscreen, as a wave mask:
+    // the two compares' masks and-ed, the radius picked by the species bit)
+    auto inlist = [&](const QPos &q, int k) -> unsigned long long {
+        const float dx = (float)(int)(pi.x - q.x), dy = (float)(int)(pi.y - q.y), dz = (float)(int)(pi.z - q.z);
+        const int m = __builtin_amdgcn_sbfe((int)q.x, 0, 1);
+        const float cut = __int_as_float((m & __float_as_int(ub)) | (~m & __float_as_int(ua)));
+        return __builtin_amdgcn_fcmpf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)), cut, 4) &  // ordered <
+               __builtin_amdgcn_uicmp((unsigned)k, (unsigned)g, 33);                                      // !=
+    };
     // entry p of this particle's list at nlb[(p >> lc) * nC + (p & cm)] (nl_at
     // relative to entry 0; 24-bit products, n < 2^21 is checked at creation)
     int *const nlb = nl + nl_at(R, cap, 0, i);
     const unsigned nC = (unsigned)R.n << R.lc, cm = (1u << R.lc) - 1u;
     const int lc = R.lc;
-    // a hit's place: the team's hits of lower lanes (the wave's lower hits,
-    // mbcnt, less those of the teams below) after the team's count so far
-    auto emit = [&](bool hit, int k) {
-        const unsigned long long b = __ballot(hit);
+    // a hit's place: the team's count so far and its hits of lower lanes
+    // (mbcnt of the ballot word that holds the team)
+    const unsigned mlo = NLT == 32 && lane >= 32 ? 0u : ~0u;
+    auto emit = [&](unsigned long long b, int k) {
         const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
-        const int wr = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-        int rank, tot;
+        unsigned pos, tot;
         if (NLT == 64) {
-            rank = wr;
+            pos = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, (unsigned)count));
             tot = __popcll(b);
         } else if (NLT == 32) {
-            const bool up = lane >= 32;
-            const int pl = __popc(lo), ph = __popc(hi);
-            rank = wr - (up ? pl : 0);
-            tot = up ? ph : pl;
+            pos = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo & mlo, (unsigned)count));
+            tot = __popc((lo & mlo) | (hi & ~mlo));
         } else {
             const unsigned long long m = b & tmask;
-            rank = __popcll(m & below);
+            pos = count + __popcll(m & below);
             tot = __popcll(m);
         }
-        if (hit) {
-            const unsigned pos = (unsigned)(count + rank);
-            if (pos < (unsigned)cap) nlb[__umul24(pos >> lc, nC) + (pos & cm)] = k;
-        }
+        if (__builtin_amdgcn_inverse_ballot_w64(b) && pos < (unsigned)cap) nlb[__umul24(pos >> lc, nC) + (pos & cm)] = k;
         count += tot;
     };
     // the home cell's stencil as slot ranges (k_cell_sort), in stencil order:
@@ -1065,49 +1096,85 @@ __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, Chai
     int2 ra = make_int2(0, 0), rb = make_int2(0, 0);
     if (t < NRANGE) ra = rgs[t];
     if (NLT < NRANGE && t + NLT < NRANGE) rb = rgs[t + NLT];
-    if (CULL && R.xcull) {
-        const int nc = R.nc, cx = cg % nc, cy = (cg / nc) % nc, cz = cg / (nc * nc);
-        const bool up = g >= xmid[R.off_cell + cg];
-        // the cell whose far half goes, and the part of its row's runs
-        // holding it (xruns: part 1 where the home cell is at either end)
-        const int xc = up ? (cx == 0 ? nc - 1 : cx - 1) : (cx == nc - 1 ? 0 : cx + 1);
-        const int qp = (!up && (cx == 0 || cx == nc - 1)) ? 1 : 0;
-        auto cull = [&](int q, int2 &rg) {
-            if (q >= NRANGE || (q & 1) != qp) return;
-            const int row = q >> 1, iz = row / 3, iy = row - 3 * iz;
-            const int yy = (cy + iy + nc - 1) % nc, zz = (cz + iz + nc - 1) % nc;
-            const int m = xmid[R.off_cell + xc + yy * nc + zz * nc * nc];
-            if (up) rg.x = m;
-            else rg.y = m;
+    if (TRIM && R.nc >= 3) {
+        const int nc = R.nc;
+        const auto div = [&](int a, int &m) {  // a / nc and the remainder
+            int q = (int)((float)a * R.rnc);
+            m = a - q * nc;
+            if (m < 0) { q--; m += nc; }
+            if (m >= nc) { q++; m -= nc; }
+            return q;
         };
-        cull(t, ra);
-        if (NLT < NRANGE) cull(t + NLT, rb);
+        int cx, cy;
+        const int cz = div(div(cg, cx), cy);
+        // distances to the faces of the particle's cell (FP32 errors of 1e-5 are within lr2's margin)
+        const float cell = R.cell, xl = ((float)pi.x * R.fix2cell - (float)cx) * cell,
+                    yl = ((float)pi.y * R.fix2cell - (float)cy) * cell, zl = ((float)pi.z * R.fix2cell - (float)cz) * cell;
+        const float xr = cell - xl, rl2 = ti ? R.lr2[1] : R.lr2[0];
+        const float xlh = R.xcull ? xl + 0.5f * cell : 0.0f, xrh = R.xcull ? xr + 0.5f * cell : 0.0f;
+        const bool first = cx == 0, last = cx == nc - 1;
+        const auto trim = [&](int q, int2 &rg) {
+            const int row = q >> 1, part = q & 1, iz = row / 3, iy = row - 3 * iz;
+            const float dy = iy == 1 ? 0.0f : (iy == 0 ? yl : cell - yl), dz = iz == 1 ? 0.0f : (iz == 0 ? zl : cell - zl);
+            const float reach2 = rl2 - dy * dy - dz * dz;
+            if (reach2 <= 0.0f) rg.y = rg.x;
+            if (rg.x >= rg.y) return;
+            int yy = cy + iy - 1, zz = cz + iz - 1;
+            yy = yy < 0 ? nc - 1 : (yy == nc ? 0 : yy);
+            zz = zz < 0 ? nc - 1 : (zz == nc ? 0 : zz);
+            const int rb = R.off_cell + __mul24(__mul24(zz, nc) + yy, nc);
+            // the row's part 0 holds the cell below along x, part 1 at either end of the row the cell above (xruns)
+            const bool out = xl * xl >= reach2, outr = xr * xr >= reach2;
+            if (part == 0 && (out || xlh * xlh >= reach2)) {
+                const int *const p = out ? start + cx : xmid + (first ? nc - 1 : cx - 1);
+                const int v = p[rb] + (out ? R.off : 0);
+                rg.x = out && first ? rg.y : v;
+            }
+            if (part == (first || last ? 1 : 0) && (outr || xrh * xrh >= reach2)) {
+                const int *const p = (outr ? start : xmid) + (last ? 0 : cx + 1);
+                const int v = p[rb] + (outr ? R.off : 0);
+                rg.y = outr && last ? rg.x : v;
+            }
+        };
+        trim(t, ra);
+        if (NLT < NRANGE) trim(t + NLT, rb);
     }
-    const int na = (ra.y - ra.x + NLT - 1) / NLT, nb = (rb.y - rb.x + NLT - 1) / NLT;
-    int pa = na, pb = nb;  // inclusive scans over the team
-    for (int o = 1; o < NLT; o <<= 1) {
-        const int ua = __shfl_up(pa, o, NLT), ub = __shfl_up(pb, o, NLT);
-        if (t >= o) { pa += ua; pb += ub; }
-    }
-    const int tot_a = __shfl(pa, NLT - 1, NLT), nch = tot_a + __shfl(pb, NLT - 1, NLT);
-    if (nch <= CH_CAP) {
-        for (int j = 0; j < na; j++) ct[pa - na + j] = make_int2(ra.x + j * NLT, min(NLT, ra.y - ra.x - j * NLT));
-        for (int j = 0; j < nb; j++)
-            ct[tot_a + pb - nb + j] = make_int2(rb.x + j * NLT, min(NLT, rb.y - rb.x - j * NLT));
-        if (t < CH_PER) ct[nch + t] = make_int2(0, 0);  // empty chunks up to the next whole round
+    const int na = (ra.y - ra.x + CH_GRP - 1) / CH_GRP, nb = (rb.y - rb.x + CH_GRP - 1) / CH_GRP;
+    // inclusive scans over the team: within rows of 16 lanes, then the rows
+    const auto scan = [&](int v) {
+        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr 1, 2, 4, 8
+        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+        if (NLT >= 32) v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 to rows 1 and 3
+        if (NLT == 64) v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 to rows 2 and 3
+        return v;
+    };
+    const int pa = scan(na), pb = NLT < NRANGE ? scan(nb) : 0;
+    const int tot_a = __shfl(pa, NLT - 1, NLT), ngr = tot_a + (NLT < NRANGE ? __shfl(pb, NLT - 1, NLT) : 0);
+    if (ngr <= CH_CAP) {
+#pragma nounroll
+        for (int j = 0; j < na; j++) ct[pa - na + j] = make_int2(ra.x + j * CH_GRP, min(CH_GRP, ra.y - ra.x - j * CH_GRP));
+        if (NLT < NRANGE)
+            for (int j = 0; j < nb; j++)
+                ct[tot_a + pb - nb + j] = make_int2(rb.x + j * CH_GRP, min(CH_GRP, rb.y - rb.x - j * CH_GRP));
+        for (int j = t; j < CH_PER * GPS; j += NLT) ct[ngr + j] = make_int2(0, 0);  // empty ones up to the next whole round
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the row is read by the other lanes
-        for (int c0 = 0; c0 < nch; c0 += CH_PER) {
+        const int2 *const cl = ct + t / CH_GRP;
+        const int tg = t & (CH_GRP - 1);
+        for (int c0 = 0; c0 < ngr; c0 += CH_PER * GPS) {
             int2 ch[CH_PER];
+            int k[CH_PER];
             QPos qv[CH_PER];
 #pragma unroll
-            for (int u = 0; u < CH_PER; u++) ch[u] = ct[c0 + u];
-#pragma unroll
-            for (int u = 0; u < CH_PER; u++) qv[u] = posq[t < ch[u].y ? ch[u].x + t : g];
+            for (int u = 0; u < CH_PER; u++) ch[u] = cl[c0 + u * GPS];
 #pragma unroll
             for (int u = 0; u < CH_PER; u++) {
-                const int k = ch[u].x + t;
-                emit((t < ch[u].y) & (k != g) & inlist(qv[u]), k);
+                k[u] = tg < ch[u].y ? ch[u].x + tg : g;  // g itself: no candidate
+                qv[u] = ld_pos(posq, k[u]);
             }
+#pragma unroll
+            for (int u = 0; u < CH_PER; u++) emit(inlist(qv[u], k[u]), k[u]);
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // reads done before the row is rewritten
     } else {
@@ -1115,13 +1182,12 @@ __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, Chai
             const int2 rg = rgs[q];
             const int s2 = rg.x, e2 = rg.y;
             // two candidates per lane, both loaded before either is used
-            // (indices clamped into [s2, e2), validity applied after)
+            // (an index past the range is replaced by g, which is no candidate)
             for (int k0 = s2; k0 < e2; k0 += 2 * NLT) {
-                const int ka = k0 + t, kb = k0 + NLT + t;
-                const QPos qa = posq[min(ka, e2 - 1)], qb = posq[min(kb, e2 - 1)];
-                const bool ha = inlist(qa) && ka < e2 && ka != g, hb = inlist(qb) && kb < e2 && kb != g;
-                emit(ha, ka);
-                emit(hb, kb);
+                const int ka = k0 + t < e2 ? k0 + t : g, kb = k0 + NLT + t < e2 ? k0 + NLT + t : g;
+                const QPos qa = ld_pos(posq, ka), qb = ld_pos(posq, kb);
+                emit(inlist(qa, ka), ka);
+                emit(inlist(qb, kb), kb);
             }
         }
     }
@@ -1134,23 +1200,20 @@ __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, Chai
 // Fixed grid over the step's list blocks (LPB particles each, one team per
 // particle); plain block order spreads the few rebuilding replicas over all
 // XCDs.
-// CULL: the x-half culling compiled in (handles with a replica that allows
-// it); without it the kernel keeps the registers of the plain walk (N=10^6:
-// 2.45e9 against 2.55e9 particle-steps/s with the culling code present but
-// unused).
-template <int NLT, bool MOVE, bool CULL>
+template <int NLT, bool MOVE, bool TRIM>
 __global__ void __launch_bounds__(NLT * LPB) k_nlist_team(const RepC *__restrict__ reps, ChainS *chain,
                                                           const int *__restrict__ lblk_rep,
                                                           const int *__restrict__ lblk_first, WorkList wl,
                                                           const QPos *__restrict__ posq,
                                                           const int *__restrict__ cell_of,
                                                           const int2 *__restrict__ ranges,
+                                                          const int *__restrict__ start,
                                                           const int *__restrict__ xmid, int *nn, int *nl, int cap,
                                                           void *const *__restrict__ ftab) {
-    __shared__ int2 s_ct[LPB][CH_CAP + CH_PER];  // each team's chunk list, then empty chunks
+    __shared__ int2 s_ct[LPB][CH_CAP + CH_PER * NLT / CH_GRP];  // each team's groups, then empty ones
     const int nit = wl.n[1];
     for (int it = blockIdx.x; it < nit; it += gridDim.x) {
-        const int b = wl.item[wl.off_l + it], r = lblk_rep[b];
+        const int b = __builtin_amdgcn_readfirstlane(wl.item[wl.off_l + it]), r = __builtin_amdgcn_readfirstlane(lblk_rep[b]);
         const RepC R = reps[r];
         // MOVE: the block's LPB particles go back from the permuted copy
         // (second half of ftab) to the primary arrays (first half) here
@@ -1167,7 +1230,7 @@ __global__ void __launch_bounds__(NLT * LPB) k_nlist_team(const RepC *__restrict
             cv = cf < 9 ? ((const long long *)ftab[PART_FIELDS + cf])[cg] : ((const int *)ftab[PART_FIELDS + cf])[cg];
         const int i = lblk_first[b] + (int)threadIdx.x / NLT;
         if (i < R.n)  // whole team
-            nlist_team_one<NLT, CULL>(R, r, i, chain, posq, cell_of, ranges, xmid, nn, nl, cap, s_ct[threadIdx.x / NLT]);
+            nlist_team_one<NLT, TRIM>(R, r, i, chain, posq, cell_of, ranges, start, xmid, nn, nl, cap, s_ct[threadIdx.x / NLT]);
         if (cpy) {
             if (cf < 9) ((long long *)ftab[cf])[cg] = cv;
             else ((int *)ftab[cf])[cg] = (int)cv;
@@ -1554,14 +1617,6 @@ struct PairAcc<true> {
         oz = fz * R.qscale;
     }
 };
-
-// The particle's position at slot j; a 32-bit byte offset for the 12-byte
-// records (a handle of 2^32 / 12 slots does not fit the memory).
-__device__ __forceinline__ QPos ld_pos(const QPos *p, int j) {
-    const unsigned u = (unsigned)j;
-    return *(const QPos *)((const char *)p + (size_t)(u * 12u));
-}
-__device__ __forceinline__ double4 ld_pos(const double4 *p, int j) { return p[j]; }
 
 // Sum over each aligned group of 2^lw lanes (2^lw <= 16), in every lane of it:
 // lane exchanges within a row of 16 (quad permutes, then mirrors of the half
@@ -2135,8 +2190,14 @@ static const char *configure_rep(RepC &R, const ac4_replica_params &q) {
     if (R.ncell > R.cap_cells) return "density below the slot's cell capacity (0.5)";
     R.qscale = R.L / 4294967296.0;
     R.qs2 = (float)(R.qscale * R.qscale);
+    R.rnc = 1.0f / (float)R.nc;
+    R.cell = (float)(R.L / R.nc);
+    R.fix2cell = (float)(R.nc / 4294967296.0);
+    R.lr2[0] = (float)(list_cut2(0, R.skin) + 2e-3);
+    R.lr2[1] = (float)(list_cut2(2, R.skin) + 2e-3);
     for (int ab = 0; ab < 3; ab++) {  // cutoff (r/sigma)^2 < 6.25 (cell_list+forces.c:189)
         const double sig = ab == 0 ? 1.00 : (ab == 1 ? 0.80 : 0.88);
+        R.lcut[ab] = qscreen_cut_of(ab, R.skin, R.qs2);
         R.rcq[ab] = (float)(K_LCUTSQR * sig * sig / (double)R.qs2);
         R.c2i[ab] = (float)(K_C2 / (sig * sig));
     }
@@ -3090,16 +3151,16 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
                            md->nl, md->stride, md->cap);
     else if (md->nlist_mode >= 2) {
         const int w = md->nlist_mode == 2 ? 16 : (md->nlist_mode == 3 ? 32 : 64);
-        bool cull = false;  // any replica whose list teams may cull (the kernel checks each replica)
-        for (int r = 0; r < md->R; r++) cull |= md->reps_h[r].n > 0 && md->reps_h[r].xcull;
-        auto kern = cull ? (w == 16 ? (team_moves ? k_nlist_team<16, true, true> : k_nlist_team<16, false, true>)
+        bool trim = false;  // any replica whose cells are ordered by x-half
+        for (int r = 0; r < md->R; r++) trim |= md->reps_h[r].n > 0 && md->reps_h[r].xcull;
+        auto kern = trim ? (w == 16 ? (team_moves ? k_nlist_team<16, true, true> : k_nlist_team<16, false, true>)
                                     : (w == 32 ? (team_moves ? k_nlist_team<32, true, true> : k_nlist_team<32, false, true>)
                                                : k_nlist_team<64, false, true>))
                          : (w == 16 ? (team_moves ? k_nlist_team<16, true, false> : k_nlist_team<16, false, false>)
                                     : (w == 32 ? (team_moves ? k_nlist_team<32, true, false> : k_nlist_team<32, false, false>)
                                                : k_nlist_team<64, false, false>));
         hipLaunchKernelGGL(kern, dim3(gl), dim3(w * LPB), 0, s, md->reps, md->chain, md->lblk_rep, md->lblk_first, wl,
-                           md->posq, md->A.cell_of, md->ranges, md->xmid, md->nn, md->nl, md->cap, md->ftab);
+                           md->posq, md->A.cell_of, md->ranges, md->start, md->xmid, md->nn, md->nl, md->cap, md->ftab);
     }
     else if (md->nlist_mode == 0)
         hipLaunchKernelGGL(k_nlist_cell, dim3(md->ncell_tot), dim3(64), 0, s, md->reps, md->chain, md->cblk_rep,

@@ -295,3 +295,32 @@ def test_frame_text_pieces(gpu, sizes):
             md.set_state(r, *x, *xu, *x, (ty & 1))
             assert md.format_frame(r) == gpu.format_frame(*xu, ty & 1)
     md.close()
+
+
+# The list teams' trimmed stencils against the thread-per-particle builder,
+# which takes every candidate: two, three and more cells per axis, cells at
+# least and less than 0.01 wider than the largest list radius (ordered by x-half
+# or not), small and large skins, a dilute box.
+@pytest.mark.parametrize("n,rho,skin", [(400, 1.2, 0.35), (753, 1.2, 0.35), (1000, 1.2, 0.35), (1790, 1.2, 0.35),
+                                        (4100, 1.2, 0.35), (1500, 0.5, 0.35), (2600, 1.2, 0.2), (2600, 1.2, 0.6)])
+def test_trimmed_list_teams(gpu, n, rho, skin):
+    out = []
+    for mode in (1, 2, 3, 4):
+        gpu.set_tuning(0, mode)
+        gpu.set_skin(skin)
+        try:
+            md = gpu.MD([gpu.ReplicaParams(n, rho, 1.0, 1.0, -1, 20, 3)], precision=gpu.FP32)
+        finally:
+            gpu.set_tuning()
+            gpu.set_skin()
+        s = gpu.init_lattice(n, 1.0, n)
+        md.set_state(0, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], s["act_tag"],
+                     s["kx"], s["ky"], s["kz"])
+        md.relax(60)
+        md.init_chain(0)
+        md.step(80)
+        assert md.rebuilds(0) > 3
+        out.append(md.export_xu()[0])
+        md.close()
+    for o in out[1:]:
+        assert np.array_equal(o, out[0])
