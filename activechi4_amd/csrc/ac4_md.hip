@@ -2081,6 +2081,7 @@ struct ac4_md {
     hipStream_t stream = nullptr;
     // captured steps: [0] one step, [1] GRAPH_CHUNK steps in one graph
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    int eager = 0;  // steps ac4_md_step launched one by one since the graphs were last dropped
     hipGraph_t graph[2] = {nullptr, nullptr};
     bool have_forces = false;
     int nlist_mode = 0;
@@ -2410,6 +2411,7 @@ static int h2d(T *dst, const T *src, size_t n, hipStream_t s);
 static void drop_graphs(ac4_md *md) {
     for (int k = 0; k < 2; k++) {
         if (md->gexec[k]) { (void)hipGraphExecDestroy(md->gexec[k]); md->gexec[k] = nullptr; }
+        md->eager = 0;
         if (md->graph[k]) { (void)hipGraphDestroy(md->graph[k]); md->graph[k] = nullptr; }
     }
 }
@@ -3301,13 +3303,6 @@ extern "C" int ac4_md_calculate_forces(ac4_md *md, double *out2) {
     return check_err(md);
 }
 
-extern "C" int ac4_md_step(ac4_md *md, int nsteps) {
-    AC4_REQUIRE(md && nsteps >= 0, AC4_EARG, "bad arguments");
-    if (!md->have_forces) TRY(ac4_md_calculate_forces(md, nullptr));
-    for (int k = 0; k < nsteps; k++) TRY(launch_step(md, k == nsteps - 1));
-    return nsteps > 0 ? launch_energy(md, true) : AC4_OK;
-}
-
 // Steps are replayed from captured graphs: GRAPH_CHUNK steps per launch (one
 // launch per ten steps instead of one per step: 1.53e9 -> 1.60e9
 // particle-steps/s on the 64-replica ensemble in three launch groups; 25 steps
@@ -3343,6 +3338,34 @@ static int ready_graphs(ac4_md *md) {
     for (int k = 0; k < 2; k++)
         if (!md->gexec[k]) TRY(capture_steps(md, k));
     return AC4_OK;
+}
+
+// Steps launched one by one.  On a small handle the five launches of a step
+// cost the host more than the step takes on the device (us per step launched
+// and replayed: N=1000 FP64 23.1 and 17.3, 8000 26.3 and 20.8, N=16000 FP32
+// 28.1 and 23.0), and capturing GRAPH_CHUNK steps about 1.1 ms: once a
+// handle of at most STEP_GRAPH_N particles has launched STEP_GRAPH_PAY steps
+// that way, its further calls replay whole chunks from the graph, as
+// ac4_md_step_graph does (the same kernels and arguments: the results are the
+// same bit for bit), and launch the rest.  Larger handles are bound by the
+// device (N=50000 FP64: 50.2 and 48.9); short runs never pay for a capture.
+#define STEP_GRAPH_N 32768
+#define STEP_GRAPH_PAY 300
+extern "C" int ac4_md_step(ac4_md *md, int nsteps) {
+    AC4_REQUIRE(md && nsteps >= 0, AC4_EARG, "bad arguments");
+    if (!md->have_forces) TRY(ac4_md_calculate_forces(md, nullptr));
+    int k = 0;
+    if (md->ntot <= STEP_GRAPH_N && nsteps >= GRAPH_CHUNK && (md->gexec[1] || md->eager >= STEP_GRAPH_PAY)) {
+        if (!md->gexec[1] && capture_steps(md, 1) != AC4_OK) {
+            (void)hipGetLastError();
+            md->eager = 0;  // launched as before, another try later
+        }
+        for (; md->gexec[1] && nsteps - k >= GRAPH_CHUNK; k += GRAPH_CHUNK)
+            AC4_HIP(hipGraphLaunch(md->gexec[1], md->stream));
+    }
+    md->eager = std::min(md->eager + nsteps - k, STEP_GRAPH_PAY);
+    for (; k < nsteps; k++) TRY(launch_step(md, k == nsteps - 1));
+    return nsteps > 0 ? launch_energy(md, true) : AC4_OK;
 }
 
 extern "C" int ac4_md_step_graph(ac4_md *md, int nsteps) {

@@ -324,3 +324,35 @@ def test_trimmed_list_teams(gpu, n, rho, skin):
         md.close()
     for o in out[1:]:
         assert np.array_equal(o, out[0])
+
+
+# A small handle's steps past the few hundred after which they are replayed
+# from a graph, in calls of whole chunks of 25 and remainders, against steps
+# launched one by one; the tables change in between (another job in the slot).
+@pytest.mark.parametrize("prec,n", [(0, 700), (1, 3000)])
+def test_steps_replayed_after_a_while(gpu, prec, n):
+    def start(md, seed):
+        s = gpu.init_lattice(n, 0.5, seed)
+        md.set_state(0, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], s["act_tag"],
+                     s["kx"], s["ky"], s["kz"])
+        md.relax(40)
+        md.init_chain(0)
+    out = []
+    for calls in ([260, 60, 25, 110, 1, 26], [1] * 24 * 20 + [2]):
+        md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 30, 3)], precision=prec)
+        start(md, 5)
+        for k in calls:
+            md.step(k)
+        got = [md.get_state(0), md.stats(0), md.get_chain(0)]
+        md.set_rebuild_criterion(1)
+        for k in calls:
+            md.step(k)
+        out.append(got + [md.get_state(0), md.stats(0), md.get_chain(0), md.rebuilds(0)])
+        md.close()
+    assert sum([260, 60, 25, 110, 1, 26]) == 24 * 20 + 2
+    for a, b in zip(*out):
+        if isinstance(a, dict):
+            for k in a:
+                assert np.array_equal(a[k], b[k]), k
+        else:
+            assert np.array_equal(a, b)
