@@ -36,6 +36,9 @@
 #define PR_THREADS 256
 #define CG_CAP 64            // neighbours per particle within 1.3 sigma (about 13 at rho = 1.2)
 #define GU_TILE 256
+#define GU_REC 8             // doubles of a particle: wrapped origin position, displacement, its components, padding
+#define GU_SPLIT 4           // threads that share a row of a tile
+#define GU_T (GU_SPLIT * GU_TILE)
 #define GU_LDS_BINS 6144     // bins per pass: 6144 * 20 B = 120 KB of LDS
 #define GU_BATCH (64u << 20) // bytes of displacements of one launch's origins
 #define PR_TIME_STEP 0.005   // Analysis/global.h:19
@@ -244,7 +247,7 @@ __global__ void __launch_bounds__(PR_THREADS) k_cg_count(const double *__restric
 // active particles m (ascending index act[m]) of each origin of a batch
 // (grid: particle blocks x origins, frame offsets fo[o] = {origin, lag}):
 // displacement to the lag frame (guu.c:151-180) and wrapped origin position
-// (LoadOrigin) to g[o][7][na]; the block's sums of L*L*r2 and r (the terms of
+// (LoadOrigin) to the record g[o][m]; the block's sums of L*L*r2 and r (the terms of
 // MSDtPP and MDtPP, guu.c:172-173) to acc[(o*gridDim.x + block)*2], added up
 // by the host in origin and block order.  (One thread adding them in
 // particle order took 301 us per origin at 5000 active particles, more than
@@ -255,22 +258,22 @@ __global__ void __launch_bounds__(PR_THREADS) k_gu_disp(const double *__restrict
                                                         int na, double L, double *gall, double *acc) {
     const int m = blockIdx.x * PR_THREADS + threadIdx.x;
     const size_t f0 = (size_t)fo[blockIdx.y].x * n, ft = (size_t)fo[blockIdx.y].y * n;
-    double *g = gall + (size_t)blockIdx.y * 7 * na;
+    double *g = gall + ((size_t)blockIdx.y * na + m) * GU_REC;
     double msd = 0.0, md = 0.0;
     if (m < na) {
         const int i = act[m];
         const double dx = pr_mi(X[ft + i] - X[f0 + i]), dy = pr_mi(Y[ft + i] - Y[f0 + i]),
                      dz = pr_mi(Z[ft + i] - Z[f0 + i]);
         const double r2 = (dx * dx + dy * dy + dz * dz);
-        g[0 * (size_t)na + m] = pr_wrap(X[f0 + i]);
-        g[1 * (size_t)na + m] = pr_wrap(Y[f0 + i]);
-        g[2 * (size_t)na + m] = pr_wrap(Z[f0 + i]);
         md = L * sqrt(r2);  // drt
         msd = L * L * r2;
-        g[3 * (size_t)na + m] = md;
-        g[4 * (size_t)na + m] = L * dx;
-        g[5 * (size_t)na + m] = L * dy;
-        g[6 * (size_t)na + m] = L * dz;
+        g[0] = pr_wrap(X[f0 + i]);
+        g[1] = pr_wrap(Y[f0 + i]);
+        g[2] = pr_wrap(Z[f0 + i]);
+        g[3] = md;
+        g[4] = L * dx;
+        g[5] = L * dy;
+        g[6] = L * dz;
     }
     __shared__ double s_w[2][PR_THREADS / 64];
     msd = ac4_wave_sum(msd);
@@ -288,14 +291,18 @@ __global__ void __launch_bounds__(PR_THREADS) k_gu_disp(const double *__restrict
 }
 
 // (int)(sqrt(r2) / bin), the bin of guu.c:205-206 with its correctly rounded
-// sqrt and division.  A 32-bit estimate decides wherever it is further from
-// a whole number than its error: r2 rounded to FP32, v_sqrt_f32 (1 ulp) and
-// one product with the rounded 1/bin are together within 3e-7 relative, taken
-// as 1e-6; about one pair in a hundred at 3500 bins takes the exact form.
-__device__ __forceinline__ int gu_bin(double r2, double bin, float rbin) {
-    const float e = __builtin_amdgcn_sqrtf((float)r2) * rbin;
-    const float f = floorf(e), m = 1e-6f * e + 1e-6f;
-    if (e - f > m && f + 1.0f - e > m) return (int)f;
+// sqrt and division.  An estimate decides wherever it is further from a whole
+// number than its error: r2 times v_rsq_f64 (5.3e-8 relative measured over
+// 2.7e8 values) is the square root to 5e-15 after one Newton step, and the
+// products after it round to 2e-16; 1e-11 is taken, relative.  r2 = 0 gives
+// NaN and the exact form.  (A 32-bit estimate, taken as 1e-6, left every fifth
+// wave of 64 pairs to the exact form: 622 against 500 us for 20 origins of
+// 5000 active particles.)
+__device__ __forceinline__ int gu_bin(double r2, double bin, double rbin) {
+    const double y = __builtin_amdgcn_rsq(r2), t = r2 * y;
+    const double e = fma(t * 0.5, fma(-t, y, 1.0), t) * rbin;
+    const double f = floor(e), m = 1e-11 * e;
+    if (e - f > m && f + 1.0 - e > m) return (int)f;
     return (int)(sqrt(r2) / bin);
 }
 
@@ -303,84 +310,86 @@ __device__ __forceinline__ int gu_bin(double r2, double bin, float rbin) {
 // origin of the batch, bins [b0, b0+nbins), item i = origin i / ntri, tile
 // i % ntri; workgroup w takes items w, w + gridDim.x, ... and keeps one
 // histogram in LDS over all of them, written to its own rows of pc/p1/p2 at
-// the end (k_gu_reduce adds the workgroups in order).  Bound by the FP64
-// pair arithmetic and the LDS atomics.  One launch per origin, a workgroup per
-// tile, each flushed by global atomics: 135 us per origin on 210 workgroups at
-// 5000 active particles; a persistent grid over 20 origins takes 60 us each.
-// Two threads share a row (half of the tile's columns each).
-__global__ void __launch_bounds__(2 * GU_TILE) k_gu_hist(const double *__restrict__ gall, int na, double L, double bin,
-                                                         float rbin, int maxbin, int b0, int nbins, int ntile,
+// the end (k_gu_reduce adds the workgroups in order).  Bound by the issue of
+// the FP64 pair arithmetic (46 instructions) beside three LDS atomics per
+// pair.  GU_SPLIT threads share a row (a part of the tile's columns each), so
+// that two workgroups of 16 waves fit a CU; a column is the same for a whole
+// wave and its record comes by scalar loads, which leaves the LDS to the
+// histogram.  One launch per origin, a workgroup per tile, each flushed by
+// global atomics: 135 us per origin on 210 workgroups at 5000 active particles;
+// a persistent grid over 20 origins with the columns in LDS 60, with 16 waves
+// per workgroup 42, with scalar loads 31, with the 64-bit bin estimate 25.
+__global__ void __launch_bounds__(GU_T) k_gu_hist(const double *__restrict__ gall, int na, double L, double bin,
+                                                         double rbin, int b0, int nbins, int ntile,
                                                          int ntri, int nitem, unsigned int *__restrict__ pc,
                                                          double *__restrict__ p1, double *__restrict__ p2) {
     extern __shared__ unsigned char s_raw[];
     unsigned int *s_c = (unsigned int *)s_raw;
     double *s_1 = (double *)(s_raw + ((sizeof(unsigned int) * nbins + 15) & ~(size_t)15));
     double *s_2 = s_1 + nbins;
-    __shared__ double s_col[7][GU_TILE];
-    const int t = threadIdx.x, row = t & (GU_TILE - 1), half = t / GU_TILE;
-    for (int b = t; b < nbins; b += 2 * GU_TILE) {
+    const int t = threadIdx.x, row = t & (GU_TILE - 1), part = __builtin_amdgcn_readfirstlane(t / GU_TILE);
+    for (int b = t; b < nbins; b += GU_T) {
         s_c[b] = 0;
         s_1[b] = 0.0;
         s_2[b] = 0.0;
     }
+    __syncthreads();
     for (int it = blockIdx.x; it < nitem; it += gridDim.x) {
         const int o = it / ntri;
-        const double *g = gall + (size_t)o * 7 * na;
+        const double *g = gall + (size_t)o * GU_REC * na;
         // tile (tr, tc), tr <= tc, of the triangle
         int q = it - o * ntri, tr = 0;
         while (q >= ntile - tr) {
             q -= ntile - tr;
             tr++;
         }
-        const int tc = tr + q;
-        __syncthreads();  // the previous item's columns are read (and the bins cleared)
-        for (int k = t; k < 7 * GU_TILE; k += 2 * GU_TILE) {
-            const int a = k / GU_TILE, c = tc * GU_TILE + k % GU_TILE;
-            if (c < na) s_col[a][k % GU_TILE] = g[(size_t)a * na + c];
-        }
-        __syncthreads();
-        const int mi = tr * GU_TILE + row;
+        const int mi = tr * GU_TILE + row, j0 = (tr + q) * GU_TILE + part * (GU_TILE / GU_SPLIT);
+        const int j1 = min(j0 + GU_TILE / GU_SPLIT, na);
         if (mi >= na) continue;
-        const double xi = g[mi], yi = g[(size_t)na + mi], zi = g[2 * (size_t)na + mi];
-        const double ri = g[3 * (size_t)na + mi], ui = g[4 * (size_t)na + mi], vi = g[5 * (size_t)na + mi],
-                     wi = g[6 * (size_t)na + mi];
-        const int j1 = min((half + 1) * (GU_TILE / 2), na - tc * GU_TILE);
-        for (int jj = half * (GU_TILE / 2); jj < j1; jj++) {
-            if (tc * GU_TILE + jj <= mi) continue;
-            // guu.c:198-213: x0_j - x0_i, one correction
-            const double dx = pr_mi(s_col[0][jj] - xi), dy = pr_mi(s_col[1][jj] - yi), dz = pr_mi(s_col[2][jj] - zi);
+        const double *gi = g + (size_t)mi * GU_REC;
+        const double xi = gi[0], yi = gi[1], zi = gi[2], ri = gi[3], ui = gi[4], vi = gi[5], wi = gi[6];
+        for (int j = j0; j < j1; j++) {
+            if (j <= mi) continue;
+            const double *c = g + (size_t)j * GU_REC;  // the same for the whole wave: scalar loads
+            // guu.c:198-213: x0_j - x0_i, one correction (pr_mi; rint differs
+            // from it in the sign of a difference of exactly a half alone)
+            double dx = c[0] - xi, dy = c[1] - yi, dz = c[2] - zi;
+            dx -= rint(dx);
+            dy -= rint(dy);
+            dz -= rint(dz);
             const double r2 = L * L * (dx * dx + dy * dy + dz * dz);
-            const int index = gu_bin(r2, bin, rbin);
-            if (index < maxbin && index >= b0 && index < b0 + nbins) {
-                const int b = index - b0;
+            const int b = gu_bin(r2, bin, rbin) - b0;
+            if ((unsigned)b < (unsigned)nbins) {  // b0 + nbins <= the number of bins
                 atomicAdd(&s_c[b], 1u);
-                atomicAdd(&s_1[b], 2.0 * (ri * s_col[3][jj]));
-                atomicAdd(&s_2[b], 2.0 * (ui * s_col[4][jj] + vi * s_col[5][jj] + wi * s_col[6][jj]));
+                atomicAdd(&s_1[b], 2.0 * (ri * c[3]));
+                atomicAdd(&s_2[b], 2.0 * (ui * c[4] + vi * c[5] + wi * c[6]));
             }
         }
     }
     __syncthreads();
     const size_t w0 = (size_t)blockIdx.x * nbins;
-    for (int b = t; b < nbins; b += 2 * GU_TILE) {
+    for (int b = t; b < nbins; b += GU_T) {
         pc[w0 + b] = s_c[b];
         p1[w0 + b] = s_1[b];
         p2[w0 + b] = s_2[b];
     }
 }
 
-// the workgroups' histograms added to the totals in workgroup order: 64 bins
-// per workgroup of 256 threads, each quarter of the threads every fourth
-// histogram
-__global__ void __launch_bounds__(256) k_gu_reduce(const unsigned int *__restrict__ pc, const double *__restrict__ p1,
-                                                   const double *__restrict__ p2, int nw, int nbins, int b0,
-                                                   unsigned long long *hc, double *h1, double *h2) {
-    __shared__ unsigned long long s_c[4][64];
-    __shared__ double s_1[4][64], s_2[4][64];
+// the workgroups' histograms added to the totals in a fixed order: 64 bins per
+// workgroup, its wave q every GU_RW-th histogram, then the waves in order
+#define GU_RW 16
+__global__ void __launch_bounds__(64 * GU_RW) k_gu_reduce(const unsigned int *__restrict__ pc,
+                                                          const double *__restrict__ p1, const double *__restrict__ p2,
+                                                          int nw, int nbins, int b0, unsigned long long *hc, double *h1,
+                                                          double *h2) {
+    __shared__ unsigned long long s_c[GU_RW][64];
+    __shared__ double s_1[GU_RW][64], s_2[GU_RW][64];
     const int l = threadIdx.x & 63, q = threadIdx.x >> 6, b = blockIdx.x * 64 + l;
     unsigned long long c = 0;
     double a1 = 0.0, a2 = 0.0;
     if (b < nbins)
-        for (int w = q; w < nw; w += 4) {
+#pragma unroll 4
+        for (int w = q; w < nw; w += GU_RW) {
             const size_t k = (size_t)w * nbins + b;
             c += pc[k];
             a1 += p1[k];
@@ -391,9 +400,14 @@ __global__ void __launch_bounds__(256) k_gu_reduce(const unsigned int *__restric
     s_2[q][l] = a2;
     __syncthreads();
     if (q == 0 && b < nbins) {
-        hc[b0 + b] += s_c[0][l] + s_c[1][l] + s_c[2][l] + s_c[3][l];
-        h1[b0 + b] += ((s_1[0][l] + s_1[1][l]) + s_1[2][l]) + s_1[3][l];
-        h2[b0 + b] += ((s_2[0][l] + s_2[1][l]) + s_2[2][l]) + s_2[3][l];
+        for (int w = 1; w < GU_RW; w++) {
+            c += s_c[w][l];
+            a1 += s_1[w][l];
+            a2 += s_2[w][l];
+        }
+        hc[b0 + b] += c;
+        h1[b0 + b] += a1;
+        h2[b0 + b] += a2;
     }
 }
 
@@ -564,38 +578,37 @@ extern "C" int ac4_frames_guu(ac4_frames *f, const int *act_tag, int gap, double
     const int pass_bins = std::min(maxbin, GU_LDS_BINS);
     const size_t lds = ((sizeof(unsigned int) * pass_bins + 15) & ~(size_t)15) + sizeof(double) * 2 * pass_bins;
     // origins of one launch: as many as GU_BATCH bytes of displacements hold
-    const size_t per = sizeof(double) * 7 * (size_t)std::max(na, 1);
+    const size_t per = sizeof(double) * GU_REC * (size_t)std::max(na, 1);
     const int batch = (int)std::max<size_t>(1, std::min<size_t>(std::max(on, 1), std::min<size_t>(GU_BATCH / per, 65535)));
     // the persistent grid: the workgroups that are resident together
-    // (160 KB of LDS per CU, at most four of eight waves)
+    // (160 KB of LDS per CU, at most two of sixteen waves)
     int dev = 0, ncu = 256;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) ncu = 256;
-    const size_t lds_all = lds + sizeof(double) * 7 * GU_TILE;
-    const int grid = ncu * (int)std::max<size_t>(1, std::min<size_t>(4, 163840 / lds_all));
+    const int grid = ncu * (int)std::max<size_t>(1, std::min<size_t>(2, 163840 / lds));
     const int dblk = (na + PR_THREADS - 1) / PR_THREADS;
+    // one allocation: act and fo (one copy in), the totals and k_gu_disp's
+    // sums (one copy out), then the batch's records and the partial histograms
+    const size_t mb = std::max(maxbin, 1), pb = (size_t)grid * std::max(pass_bins, 1);
+    const size_t in_b = sizeof(int2) * std::max(on, 1) + ((sizeof(int) * std::max(na, 1) + 7) & ~(size_t)7);
+    const size_t out_n = 3 * mb + (size_t)2 * std::max(on, 1) * std::max(dblk, 1);  // 64-bit words
     AcDevBuf B;
-    int *d_act;
-    int2 *d_fo;
-    double *d_g, *d_acc, *d_h1, *d_h2, *d_p1, *d_p2;
-    unsigned int *d_pc;
-    unsigned long long *d_hc;
-    PTRY(B.get(&d_act, std::max(na, 1)));
-    PTRY(B.get(&d_fo, std::max(on, 1)));
-    PTRY(B.get(&d_g, (size_t)batch * 7 * std::max(na, 1)));
-    PTRY(B.get(&d_acc, (size_t)2 * std::max(on, 1) * std::max(dblk, 1)));
-    PTRY(B.get(&d_hc, std::max(maxbin, 1)));
-    PTRY(B.get(&d_h1, std::max(maxbin, 1)));
-    PTRY(B.get(&d_h2, std::max(maxbin, 1)));
-    PTRY(B.get(&d_pc, (size_t)grid * std::max(pass_bins, 1)));
-    PTRY(B.get(&d_p1, (size_t)grid * std::max(pass_bins, 1)));
-    PTRY(B.get(&d_p2, (size_t)grid * std::max(pass_bins, 1)));
+    char *d_all;
+    PTRY(B.get(&d_all, in_b + 8 * out_n + sizeof(double) * ((size_t)batch * GU_REC * std::max(na, 1) + 2 * pb) +
+                           sizeof(unsigned int) * pb));
+    int2 *const d_fo = (int2 *)d_all;
+    int *const d_act = (int *)(d_fo + std::max(on, 1));
+    unsigned long long *const d_hc = (unsigned long long *)(d_all + in_b);
+    double *const d_h1 = (double *)(d_hc + mb), *const d_h2 = d_h1 + mb, *const d_acc = d_h2 + mb,
+           *const d_g = (double *)d_hc + out_n, *const d_p1 = d_g + (size_t)batch * GU_REC * std::max(na, 1),
+           *const d_p2 = d_p1 + pb;
+    unsigned int *const d_pc = (unsigned int *)(d_p2 + pb);
     hipStream_t s = v.s;
-    if (na) AC4_HIP(hipMemcpyAsync(d_act, act.data(), sizeof(int) * na, hipMemcpyHostToDevice, s));
-    if (on) AC4_HIP(hipMemcpyAsync(d_fo, fo.data(), sizeof(int2) * on, hipMemcpyHostToDevice, s));
-    AC4_HIP(hipMemsetAsync(d_hc, 0, sizeof(unsigned long long) * std::max(maxbin, 1), s));
-    AC4_HIP(hipMemsetAsync(d_h1, 0, sizeof(double) * std::max(maxbin, 1), s));
-    AC4_HIP(hipMemsetAsync(d_h2, 0, sizeof(double) * std::max(maxbin, 1), s));
+    std::vector<char> in(in_b, 0);
+    if (on) memcpy(in.data(), fo.data(), sizeof(int2) * on);
+    if (na) memcpy(in.data() + sizeof(int2) * std::max(on, 1), act.data(), sizeof(int) * na);
+    AC4_HIP(hipMemcpyAsync(d_all, in.data(), in_b, hipMemcpyHostToDevice, s));
+    AC4_HIP(hipMemsetAsync(d_hc, 0, 8 * 3 * mb, s));
     AC4_HIP(hipFuncSetAttribute((const void *)k_gu_hist, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     for (int o0 = 0; na && o0 < on; o0 += batch) {
         const int no = std::min(batch, on - o0);
@@ -606,23 +619,20 @@ extern "C" int ac4_frames_guu(ac4_frames *f, const int *act_tag, int gap, double
         const int nitem = (int)all, gw = std::min(grid, nitem);
         for (int b0 = 0; b0 < maxbin; b0 += pass_bins) {
             const int nbins = std::min(pass_bins, maxbin - b0);
-            hipLaunchKernelGGL(k_gu_hist, dim3(gw), dim3(2 * GU_TILE), lds, s, d_g, na, L, bin, (float)(1.0 / bin),
-                               maxbin, b0, nbins, ntile, ntri, nitem, d_pc, d_p1, d_p2);
-            hipLaunchKernelGGL(k_gu_reduce, dim3((nbins + 63) / 64), dim3(256), 0, s, d_pc, d_p1, d_p2, gw, nbins, b0,
+            hipLaunchKernelGGL(k_gu_hist, dim3(gw), dim3(GU_T), lds, s, d_g, na, L, bin, 1.0 / bin,
+                               b0, nbins, ntile, ntri, nitem, d_pc, d_p1, d_p2);
+            hipLaunchKernelGGL(k_gu_reduce, dim3((nbins + 63) / 64), dim3(64 * GU_RW), 0, s, d_pc, d_p1, d_p2, gw, nbins, b0,
                                d_hc, d_h1, d_h2);
         }
         AC4_HIP(hipGetLastError());
     }
-    std::vector<unsigned long long> hc(std::max(maxbin, 1));
-    std::vector<double> h1(std::max(maxbin, 1)), h2(std::max(maxbin, 1)), part((size_t)2 * on * dblk);
-    AC4_HIP(hipMemcpyAsync(hc.data(), d_hc, sizeof(unsigned long long) * maxbin, hipMemcpyDeviceToHost, s));
-    AC4_HIP(hipMemcpyAsync(h1.data(), d_h1, sizeof(double) * maxbin, hipMemcpyDeviceToHost, s));
-    AC4_HIP(hipMemcpyAsync(h2.data(), d_h2, sizeof(double) * maxbin, hipMemcpyDeviceToHost, s));
-    if (!part.empty())
-        AC4_HIP(hipMemcpyAsync(part.data(), d_acc, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
+    std::vector<unsigned long long> res(out_n, 0);
+    AC4_HIP(hipMemcpyAsync(res.data(), d_hc, 8 * out_n, hipMemcpyDeviceToHost, s));
     AC4_HIP(hipStreamSynchronize(s));
+    const unsigned long long *const hc = res.data();
+    const double *const h1 = (const double *)(hc + mb), *const h2 = h1 + mb, *const part = h2 + mb;
     double acc[2] = {0.0, 0.0};
-    for (size_t k = 0; k < part.size(); k++) acc[k & 1] += part[k];
+    for (size_t k = 0; k < (size_t)2 * on * dblk; k++) acc[k & 1] += part[k];
     // guu.c:250-276
     const double MSDt = acc[0] / ((double)n * (double)on);
     const double MDt = acc[1] / ((double)n * (double)on);
