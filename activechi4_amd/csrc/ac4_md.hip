@@ -617,7 +617,7 @@ __device__ __forceinline__ void bin_end(const RepC &R, int r, const int *cnt, in
 }
 
 // The same as a kernel of its own, one workgroup per replica, for handles
-// with a slot of more than BIN_FUSE_CELLS cells, whose scan would be long for
+// with a job of more than BIN_FUSE_CELLS cells, whose scan would be long for
 // a k_bin workgroup (BIN_END_T threads there).
 #define BIN_FUSE_CELLS 4096
 __global__ void __launch_bounds__(BIN_END_T) k_bin_end(const RepC *__restrict__ reps,
@@ -2031,12 +2031,16 @@ struct ac4_md {
     int lw = 0, lc = 3, vec = 1;  // force teams: log2 lanes, log2 list chunk, list reading (k_force's VEC)
     int *cblk_rep = nullptr, *cblk_cell = nullptr;
     int fnblk = 0, lnblk = 0, ncb = 0;
-    int shuf_kcap = 0;     // largest Nact whose directions k_shuffle keeps in LDS
+    int shuf_kmax = 0;     // room for directions in LDS (bytes), at most
+    int shuf_kcap = 0;     // largest Nact whose directions the shuffle keeps in LDS
     int shuf_bmax = 0;     // swap blocks of the largest slot, 0 without the parallel shuffle path
     int2 *shuf_ent = nullptr;  // its per-block source maps
     int *shuf_ent_n = nullptr;
     size_t shuf_lds = 0;   // dynamic LDS of k_shuffle
-    bool shuf_fused = false;  // the shuffle runs in k_first_half's first workgroups
+    // by the jobs in the slots (job_rules): the shuffle runs in k_first_half's
+    // first workgroups; else k_shuffle, the parallel path or both are launched;
+    // the scan of the cell counts is k_bin's
+    bool shuf_fused = false, shuf_serial = true, shuf_par = false, bin_fuse = false;
     int *wl_item = nullptr, *wl_n = nullptr;  // rebuild work list (WorkList)
     int2 *ranges = nullptr;                    // per cell: stencil slot ranges (NRANGE)
     int *xmid = nullptr;                       // per cell: first slot of its upper x-half
@@ -2160,6 +2164,31 @@ extern "C" int ac4_set_tuning(int tpp, int nlist_mode) {
     g_tpp = tpp;
     g_nlist_mode = nlist_mode;
     return AC4_OK;
+}
+
+// Launch rules that follow the jobs in the slots (the capacities while no slot
+// holds one): the shuffle is k_first_half's when no job needs the parallel
+// path and its LDS leaves that kernel at least 5 workgroups per CU; a launch
+// that no job needs is left out (each costs 1.6 to 4.5 us a step even where it
+// returns at once: N=50000, whose slot could hold 50000 active particles and
+// holds 5000, took three for the shuffle and one for the scan; 1e6 one).
+static void job_rules(ac4_md *md) {
+    bool any = false, small = false, large = false;
+    int k = 0, ncell = 0;
+    for (const RepC &R : md->reps_h) any |= R.n > 0;
+    for (const RepC &R : md->reps_h) {
+        if (any && R.n == 0) continue;
+        const int na = any ? R.nact : R.cap_n;
+        k = std::max(k, na);
+        ncell = std::max(ncell, any ? R.ncell : R.cap_cells);
+        (md->shuf_bmax > 0 && na > SHUF_PAR_MIN ? large : small) = true;
+    }
+    md->shuf_kcap = std::min(md->shuf_kmax, (k + 15) & ~15);
+    md->shuf_lds = SHUF_CH * sizeof(unsigned int) + (size_t)md->shuf_kcap;
+    md->shuf_serial = small || !any;
+    md->shuf_par = md->shuf_bmax > 0 && (large || !any);
+    md->shuf_fused = !md->shuf_par && md->shuf_lds <= 32768;
+    md->bin_fuse = ncell <= BIN_FUSE_CELLS;
 }
 
 // Job-dependent fields of a slot (the capacity-dependent ones are fixed at
@@ -2330,21 +2359,19 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) lds = 65536;
         for (int r = 0; r < nslots; r++) cap_max = std::max(cap_max, cap_n[r]);
         const int room = lds - (int)(SHUF_CH * sizeof(unsigned int));
-        md->shuf_kcap = std::max(0, std::min(room, (cap_max + 15) & ~15));
-        md->shuf_lds = SHUF_CH * sizeof(unsigned int) + (size_t)md->shuf_kcap;
+        md->shuf_kmax = std::max(0, std::min(room, (cap_max + 15) & ~15));
+        md->shuf_lds = SHUF_CH * sizeof(unsigned int) + (size_t)md->shuf_kmax;
         if (md->shuf_lds > 65536 &&
             (hipFuncSetAttribute((const void *)k_shuffle, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)md->shuf_lds) != hipSuccess ||
              hipFuncSetAttribute((const void *)k_shuf_apply, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)md->shuf_lds) != hipSuccess)) {
             (void)hipGetLastError();
-            md->shuf_kcap = 65536 - (int)(SHUF_CH * sizeof(unsigned int));
-            md->shuf_lds = 65536;
+            md->shuf_kmax = 65536 - (int)(SHUF_CH * sizeof(unsigned int));
         }
         md->shuf_bmax = cap_max > SHUF_PAR_MIN ? (cap_max + SHUF_M - 1) / SHUF_M : 0;
-        // in k_first_half when its LDS leaves that kernel at least 5 workgroups per CU
-        md->shuf_fused = md->shuf_bmax == 0 && md->shuf_lds <= 32768;
     }
+    job_rules(md);
     int rc = AC4_OK;
 #define ALLOC(ptr, n) if ((rc = dalloc(&md->ptr, (size_t)(n))) != AC4_OK) { ac4_md_destroy(md); return rc; }
     if (md->shuf_bmax > 0) {
@@ -2445,6 +2472,7 @@ static int refresh_tables(ac4_md *md) {
     hipStream_t s = md->stream;
     AC4_HIP(hipStreamSynchronize(s));
     drop_graphs(md);
+    job_rules(md);
     TRY(h2d(md->blk_rep, br.data(), br.size(), s)); TRY(h2d(md->blk_first, bf.data(), bf.size(), s));
     TRY(h2d(md->blk_idx, bi.data(), bi.size(), s));
     TRY(h2d(md->blkd, bd.data(), bd.size(), s)); TRY(h2d(md->fblk, fd.data(), fd.size(), s));
@@ -3134,8 +3162,8 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
         hipLaunchKernelGGL(k_cell_zero, dim3(md->R, cy), dim3(BLK), 0, s, md->reps, md->chain, md->cnt, md->wl_n);
     hipLaunchKernelGGL(k_bin, dim3(md->nblk), dim3(BLK), 0, s, md->reps, md->chain, md->blk_rep, md->blk_first,
                        md->P.x, md->P.y, md->P.z, md->P.id, md->cnt, md->P.cell_of, md->cell_mem, md->P.cell_ref,
-                       md->max_ncell <= BIN_FUSE_CELLS ? 1 : 0, md->bdone, md->start, wl);
-    if (md->max_ncell > BIN_FUSE_CELLS)
+                       md->bin_fuse ? 1 : 0, md->bdone, md->start, wl);
+    if (!md->bin_fuse)
         hipLaunchKernelGGL(k_bin_end, dim3(md->R), dim3(BIN_END_T), 0, s, md->reps, md->chain, md->cnt, md->start, wl);
     hipLaunchKernelGGL(k_cell_sort, dim3(gc), dim3(BLK), 0, s, md->reps, wl, md->cnt, md->start,
                        md->cell_mem, md->members, md->ranges, md->xmid, md->P, md->A,
@@ -3213,9 +3241,10 @@ static int launch_force(ac4_md *md, bool energy) {
 }
 
 static void launch_shuffle(ac4_md *md, int force, hipStream_t s) {
-    hipLaunchKernelGGL(k_shuffle, dim3(md->R, 3), dim3(256), md->shuf_lds, s, md->reps, md->chain, md->kx, md->ky,
-                       md->kz, force, md->shuf_kcap, md->shuf_bmax > 0 ? 1 : 0);
-    if (md->shuf_bmax > 0) {  // slots that can hold more than SHUF_PAR_MIN active particles
+    if (md->shuf_serial)
+        hipLaunchKernelGGL(k_shuffle, dim3(md->R, 3), dim3(256), md->shuf_lds, s, md->reps, md->chain, md->kx, md->ky,
+                           md->kz, force, md->shuf_kcap, md->shuf_bmax > 0 ? 1 : 0);
+    if (md->shuf_par) {  // more than SHUF_PAR_MIN active particles
         hipLaunchKernelGGL(k_shuf_part, dim3(md->shuf_bmax, 3, md->R), dim3(64), 0, s, md->reps, md->chain, force,
                            md->shuf_bmax, md->shuf_ent, md->shuf_ent_n);
         hipLaunchKernelGGL(k_shuf_apply, dim3(md->R, 3), dim3(2 * SHUF_M), md->shuf_lds, s, md->reps, md->chain,

@@ -356,3 +356,34 @@ def test_steps_replayed_after_a_while(gpu, prec, n):
                 assert np.array_equal(a[k], b[k]), k
         else:
             assert np.array_equal(a, b)
+
+
+# The shuffle inside the half-kick kernel, as its own launch, on the parallel
+# path, and both of the last two for a handle whose replicas need them; cells
+# scanned by the binning pass and by a kernel of their own.  Each replica alone
+# gives what it gives beside the others, direction for direction.
+@pytest.mark.parametrize("acts", [(300, 9000), (300, 17000), (16384, 16385), (300, 9000, 17000)])
+def test_shuffle_launches_by_the_jobs(gpu, acts):
+    def start(r_list):
+        gpu.set_tuning(4)
+        try:
+            md = gpu.MD([gpu.ReplicaParams(120000 if a == 17000 else 20000, 1.2, 0.5, 1.0, a, 5, 3 + a) for a in r_list])
+        finally:
+            gpu.set_tuning()
+        for r, a in enumerate(r_list):
+            n = md.n(r)
+            s = gpu.init_lattice(n, 0.5, n)
+            rng = np.random.default_rng(a)
+            tag = np.full(n, -1, np.int32)
+            tag[rng.permutation(n)[:a]] = np.arange(a)
+            ks = [rng.integers(0, 2, a).astype(np.int32) * 2 - 1 for _ in range(3)]
+            md.set_state(r, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], tag, *ks)
+        md.step(12)
+        out = [md.get_state(r) for r in range(len(r_list))]
+        md.close()
+        return out
+    both = start(acts)
+    for r, a in enumerate(acts):
+        alone = start([a])[0]
+        for k in ("kx", "ky", "kz", "xu", "px"):
+            assert np.array_equal(alone[k], both[r][k]), (a, k)
