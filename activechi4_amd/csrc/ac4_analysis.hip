@@ -270,15 +270,19 @@ __constant__ int c_pcol[AC4_NQ];     // first column of each GetQ vector
 // then in each set of four waves wave w < 3 takes the product of axis w with
 // the other two (real and imaginary parts, four MFMAs) and one of the eight
 // tiles of the (0, k, i) group, wave 3 the other five.  The FS_SETS sets
-// take every FS_SETS-th MFMA step and are added in order at the end: a frame
-// has about one pair, so the launch is as long as one workgroup's tiles, and
-// four waves per SIMD make them shorter.  1000 and 20011 particles, per pair:
-// one sincos per vector and particle 33.6 and 59.5 us, this 9.5 and 17.6 (one
-// set of waves, the displacements loaded per tile: 13.3 and 27.5).
-#define FS_P 32        // particles of a tile
+// take every FS_SETS-th MFMA step and are added at the end in a fixed order: a
+// frame has about one pair, so the launch is as long as one workgroup's tiles,
+// and four waves per SIMD make them shorter.  Tiles of 16 particles: the 63
+// factors of each are one round of the workgroup's threads, a set has one
+// MFMA step, and a small frame's workgroups hold half as many particles.  1000
+// and 20011 particles, per pair: one sincos per vector and particle 33.6 and
+// 59.5 us, this 8.2 and 15.8 (tiles of 32 and the sets added one after the
+// other 9.5 and 17.4; one set of waves, the displacements loaded per tile 13.3
+// and 27.5).
+#define FS_P 16        // particles of a tile
 #define FS_M 21        // largest component of a GetQ vector
 #define FS_J 15        // largest j of the (i, j, j) vectors
-#define FS_RL (FS_P + 1)  // row of a table: FS_P values, padded against bank conflicts
+#define FS_RL 33       // row of a table: up to 32 values, padded against bank conflicts
 #define FS_TILES 14    // accumulated 16 x 16 tiles: 3 x {cos, sin}, then the (0, k, i) group's 8
 #define FS_LOAD 256    // particles whose displacements are loaded together
 #define FS_NBLK 256    // workgroups per pair, at most
@@ -420,13 +424,15 @@ __device__ __forceinline__ void fs_block(const Job &J, int blk, int ppb, const F
         }
         __syncthreads();
     }
-    // the accumulated tiles to LDS (element e of lane l: row l/16 + 4*e, column l%16)
-    for (int w = 0; w < FS_SETS; w++) {
-        if (set == w)
+    // the accumulated tiles to LDS (element e of lane l: row l/16 + 4*e, column
+    // l%16): sets 0 and 1 to two areas, sets 2 and 3 added to them
+    static_assert(FS_SETS == 4 && 2 * FS_TILES * 256 <= FS_LDS, "two areas of tiles in the tables' place");
+    for (int w = 0; w < 2; w++) {
+        if (set >> 1 == w)
 #pragma unroll
             for (int q = 0; q < 5; q++) {
                 if (wv < 3 && q >= 3) continue;
-                const int tile = wv < 3 ? (q < 2 ? 2 * wv + q : 6 + wv) : 9 + q;
+                const int tile = (set & 1) * FS_TILES + (wv < 3 ? (q < 2 ? 2 * wv + q : 6 + wv) : 9 + q);
                 for (int e = 0; e < 4; e++) {
                     double *d = &s_t[tile * 256 + (k4 + 4 * e) * 16 + i16];
                     *d = w == 0 ? acc[q][e] : *d + acc[q][e];
@@ -436,7 +442,13 @@ __device__ __forceinline__ void fs_block(const Job &J, int blk, int ppb, const F
     }
     // the permuted vectors' sums, then each vector's average over its permutations
     double c = 0.0, sn = 0.0;
-    if (t < S4_NCOL - 3) fs_entry(s_t, o0, o1, o2, c, sn);
+    if (t < S4_NCOL - 3) {
+        double c1, s1;
+        fs_entry(s_t, o0, o1, o2, c, sn);
+        fs_entry(s_t + FS_TILES * 256, o0, o1, o2, c1, s1);
+        c += c1;
+        sn += s1;
+    }
     __syncthreads();
     if (t < S4_NCOL) {
         s_t[t] = c;
@@ -456,7 +468,7 @@ __device__ __forceinline__ void fs_block(const Job &J, int blk, int ppb, const F
 // O.nb frame blocks.  As two launches, a reduction and the stream's end waited
 // for: 25.6 us per frame of 1000 particles, all four observables, and 31.7 of
 // 20011, Fs alone; this, the partials of FS_WAIT jobs reduced together, 11.1
-// and 16.8.
+// and 16.8 (with Fs tiles of 32).
 __global__ void __launch_bounds__(FS_T) k_frame_fs(const Job *__restrict__ jobs, int nj, int nf, int fs_nb, int fs_ppb,
                                                    Frame F, FrameOut O, double *partial) {
     const int wg = blockIdx.x, nwg = gridDim.x;
@@ -504,6 +516,7 @@ __global__ void __launch_bounds__(FS_T) k_frame_fs(const Job *__restrict__ jobs,
 // chunk and column tile with a sincos per phase took 110, its reduction of
 // 576 columns per lag 13.5 (k_s4_reduce's 324 values 4.8).
 #define S4_NCT (S4_NCOL / 16) // column tiles
+#define S4_P 32        // particles of a tile, at most
 #define S4_WAVES 12
 #define S4_CPW (S4_NCT / S4_WAVES)  // column tiles of a wave
 #define S4_T (64 * S4_WAVES)
@@ -528,7 +541,7 @@ __device__ __forceinline__ void s4_rows(int o0, int o1, int o2, int &u, int &v) 
 }
 
 // One origin, one pass of nl <= 16*NT16 + 4*NT4 of its lags: grid (chunks of
-// ppb particles), tiles of tp <= FS_P particles (both multiples of 4).
+// ppb particles), tiles of tp <= S4_P particles (both multiples of 4).
 // v_mfma_f64_16x16x4f64: lane l = i + 16k holds A[i][k] (mask bit of lag i,
 // particle k) and B[k][j] with j = i (phase of vector j for particle k); the
 // accumulator's element e of lane l is row l/16 + 4*e, column l%16.
@@ -544,9 +557,9 @@ __global__ void __launch_bounds__(S4_T) k_s4_origin(const double *__restrict__ x
     constexpr int NR = NT16 + NT4, ROWS = 16 * NT16 + 4 * NT4;
     constexpr int LDS = FS_LDS > ROWS * S4_NCOL ? FS_LDS : ROWS * S4_NCOL;
     __shared__ double s_t[LDS];  // the tables, then the sums of one of cos and sin
-    __shared__ double s_p[3][FS_P];
+    __shared__ double s_p[3][S4_P];
     __shared__ int s_dc[AC4_NQ];  // permutations and first column of each vector, for the end
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, i16 = lane & 15, k4 = lane >> 4, pp = t & (FS_P - 1);
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, i16 = lane & 15, k4 = lane >> 4, pp = t & (S4_P - 1);
     int u[S4_CPW], v[S4_CPW];
 #pragma unroll
     for (int c = 0; c < S4_CPW; c++) {
@@ -573,15 +586,15 @@ __global__ void __launch_bounds__(S4_T) k_s4_origin(const double *__restrict__ x
     // coordinate is used as it is, whatever single-if wraps the reference
     // applies to it at a given lag.  A particle past n has no mask bit: its
     // (clamped) phase is multiplied by zero; so has one of the next chunk.
-    const double *src = t < FS_P ? x0 : (t < 2 * FS_P ? y0 : z0);
-    double p = t < 3 * FS_P ? src[min(i0 + pp, n - 1)] : 0.0;
+    const double *src = t < S4_P ? x0 : (t < 2 * S4_P ? y0 : z0);
+    double p = t < 3 * S4_P ? src[min(i0 + pp, n - 1)] : 0.0;
     if (t < AC4_NQ) s_dc[t] = c_pcol[t] << 3 | c_dg[t];
-    if (t < FS_P) {
+    if (t < S4_P) {
         s_t[fs_ax(0, 0, 0) + t] = 1.0;
         s_t[fs_ax(0, 0, 1) + t] = 0.0;
     }
     for (int tb = i0; tb < i1; tb += tp) {
-        if (t < 3 * FS_P) s_p[t / FS_P][pp] = p;
+        if (t < 3 * S4_P) s_p[t / S4_P][pp] = p;
         // the mask words of this tile, loaded while its tables are built
         const int w = tb >> 5, sh = tb & 31, cnt = min(tp, i1 - tb);
         unsigned mw[NR], mx[NR];
@@ -591,8 +604,8 @@ __global__ void __launch_bounds__(S4_T) k_s4_origin(const double *__restrict__ x
             mx[r] = mrow[r][sh + cnt > 32 ? w + 1 : w];
         }
         __syncthreads();
-        if (t < 3 * FS_P) p = src[min(tb + tp + pp, n - 1)];  // the next tile's
-        for (int e = t / FS_P; e < 3 * FS_M; e += S4_T / FS_P) {
+        if (t < 3 * S4_P) p = src[min(tb + tp + pp, n - 1)];  // the next tile's
+        for (int e = t / S4_P; e < 3 * FS_M; e += S4_T / S4_P) {
             const int a = e / FS_M, m = e - a * FS_M + 1;
             const double q = s_p[a][pp], f = fma((double)m, q, -rint((double)m * q));
             double sn, cs;
@@ -601,7 +614,7 @@ __global__ void __launch_bounds__(S4_T) k_s4_origin(const double *__restrict__ x
             s_t[fs_ax(a, m, 1) + pp] = sn;
         }
         __syncthreads();
-        for (int e = t / FS_P; e < 3 * FS_J; e += S4_T / FS_P) {
+        for (int e = t / S4_P; e < 3 * FS_J; e += S4_T / S4_P) {
             const int a = e / FS_J, j = e - a * FS_J + 1, b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
             const double cb = s_t[fs_ax(b, j, 0) + pp], sb = s_t[fs_ax(b, j, 1) + pp], cc = s_t[fs_ax(c, j, 0) + pp],
                          sc = s_t[fs_ax(c, j, 1) + pp];
@@ -1008,7 +1021,7 @@ static int s4_setup(ac4_ana *an) {
     // chunks: at least 16 particles each, at most S4_CHUNKS of them; the tiles of a chunk as even as they go
     an->s4_ppb = std::max(16, 4 * ((an->n + 4 * S4_CHUNKS - 1) / (4 * S4_CHUNKS)));
     an->s4_nchunk = (an->n + an->s4_ppb - 1) / an->s4_ppb;
-    const int nt = (an->s4_ppb + FS_P - 1) / FS_P;
+    const int nt = (an->s4_ppb + S4_P - 1) / S4_P;
     an->s4_tp = 4 * ((an->s4_ppb / 4 + nt - 1) / nt);
     size_t part = (size_t)an->s4_nchunk * S4_LAGS * 2 * AC4_NQ;
     if (an->n <= S4_SMALL) {

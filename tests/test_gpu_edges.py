@@ -127,9 +127,10 @@ def test_sums_and_cells_of_the_last_workgroup(gpu, sizes):
 
 
 # Particle counts around the tiles of the frame kernel (256) and of the Fs
-# kernel (32, loads of 256), and one large enough for several of each per
+# kernel (16, loads of 256), and one large enough for several of each per
 # workgroup; with and without the B particles.
-@pytest.mark.parametrize("n,flag", [(1, 0), (31, 0), (32, 1), (33, 0), (255, 1), (257, 0), (513, 0), (70001, 1)])
+@pytest.mark.parametrize("n,flag", [(1, 0), (15, 0), (17, 1), (31, 0), (32, 1), (33, 0), (255, 1), (257, 0), (513, 0),
+                                    (70001, 1)])
 def test_frame_and_fs_tile_edges(gpu, n, flag):
     frames = [0, 1, 2, 3, 10, 11]
     X, Y, Z, T = trajgen.make_frames(n, frames, 7 + n, 0.08, 1.0)
