@@ -1646,16 +1646,13 @@ __device__ __forceinline__ double wave_sum_rows(double v) {
     return (r[0] + r[1]) + (r[2] + r[3]);
 }
 
-// VEC consecutive list entries in one load.  (A nontemporal load of the list
+// VEC consecutive list entries, 1 or 8.  (A nontemporal load of the list
 // measured 79 against 56 us per k_force launch on the 64-replica ensemble:
 // the list stream is better served by the caches.)
 template <int VEC>
 __device__ __forceinline__ void ld_list(const int *p, int *j) {
     if (VEC == 1) {
         j[0] = p[0];
-    } else if (VEC == 2) {
-        const int2 a = *(const int2 *)p;
-        j[0] = a.x; j[1] = a.y;
     } else {
 #pragma unroll
         for (int q = 0; q < VEC; q += 4) {
@@ -1671,10 +1668,9 @@ __device__ __forceinline__ void ld_list(const int *p, int *j) {
 // too (an entry past m is replaced by g before it is used as an index).
 // VEC = 1: lane t of W takes entries t, t + W, ... (row c of the walk is
 // entries c*W ... c*W + W - 1, cs list words apart); the others read chunks
-// of 8 entries, cs words apart, with W = 8 / |VEC| lanes: VEC > 1 takes VEC
-// consecutive entries of a chunk in one load, VEC < -1 entries t, t + W, ...
-// of it, |VEC| rows per chunk, and six entries per group (FP64 only: 128
-// vector registers in k_force instead of 148, four waves per SIMD instead of
+// of 8 entries, cs words apart, with W = 8 / |VEC| lanes: VEC = 8 the whole
+// chunk, VEC = -2 entries t, t + 4 of it, two rows per chunk, and in FP64 six
+// entries per group (128 vector registers in k_force instead of 148, four waves per SIMD instead of
 // three; us per step at N=50000 50.7 -> 50.1, 80000 63.5 -> 61.4, 200000
 // 104 -> 99.5.  Teams of 8 and 16 lanes, whose lists are one or two groups,
 // keep eight: 22.0 against 22.8 at N=10000).
@@ -1683,7 +1679,7 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
                                           const PosT *__restrict__ pos, const PosT &pi, Acc &acc) {
     constexpr int V = VEC > 1 ? VEC : 1;    // entries of a load
     constexpr int RC = VEC < 0 ? -VEC : 1;  // rows per step of cs
-    constexpr int G = VEC < 0 ? 6 : 8;      // entries of a group
+    constexpr int G = VEC < 0 && sizeof(PosT) == 32 ? 6 : 8;  // entries of a group
     constexpr int NR = G / V;               // rows of a group
     const int rl = W * V, full = m / rl;    // entries of a row, whole rows
     int c = 0, jn[G];
@@ -2139,12 +2135,13 @@ static void free_parts(PartArrays &a) {
 //   FP64  10000: 39.9 30.5 25.5 24.5 23.7    20000: 47.8 38.1 35.7 33.7 35.1
 //         50000: 56.6 52.1 51.2 51.9 56.6   100000: 79.7 75.9 72.0 78.3 87.2
 //        200000:  121  113  106  121  143   500000:  288  252  252  292  361
-// On large FP32 handles two lanes reading four entries of a chunk at a time
-// (k_force, VEC = 4) take 194 at 500000; one lane was the rule before.
-static int force_width(double cap_tot, int prec) {
+// Four FP32 lanes reading a chunk's entries strided (k_force, VEC = -2) take
+// 177.6 at 500000, 118.7 at 300000 and 44.6 at 70000; reading two consecutive
+// ones 181.6, 122.5 and 45.4; eight lanes 194.9, 127.2 and 45.4.
+static int force_width(double cap_tot) {
     if (cap_tot <= 14000.0) return 16;
     if (cap_tot <= 32768.0) return 8;
-    return prec == AC4_FP32 && cap_tot > 160000.0 ? 2 : 4;
+    return 4;
 }
 static int g_tpp = 0, g_nlist_mode = 3;
 static double g_skin = K_SKIN;
@@ -2285,18 +2282,17 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     while ((1 << ltpp) < tpp) ltpp++;
     // lanes per particle in the force kernel: the pinned width, else by the
     // handle's total capacity (FORCE_W)
-    const int W = g_tpp ? tpp : std::max(tpp > 1 ? tpp : 1, force_width(cap_tot, precision));
+    const int W = g_tpp ? tpp : std::max(tpp > 1 ? tpp : 1, force_width(cap_tot));
     while ((1 << md->lw) < W) md->lw++;
     md->en_apart = precision == AC4_FP32 && W != tpp;
     md->elw = ltpp;
     md->lc = tpp == 1 ? 3 : ltpp;
-    // a chunk of 8 entries read by fewer lanes: FP32 teams take consecutive
-    // entries in one load each; FP64 teams (and more than one lane) take
-    // every W-th, so that the lanes of a gather are on neighbouring entries:
-    // the 32-byte records of four are one or two lines (N=100000, four lanes:
-    // 72 against 79 us per step), the 12-byte ones mostly one either way
-    md->vec = W < (1 << md->lc) ? (1 << md->lc) / W : 1;
-    if (precision == AC4_FP64 && W > 1 && md->vec > 1) md->vec = -md->vec;
+    // a chunk of 8 entries read by four lanes: every fourth entry each, so
+    // that the lanes of a gather are on neighbouring entries, which are mostly
+    // neighbouring slots: two consecutive entries each make the gathers of a
+    // wave reach more lines (us per step, FP64 N=100000 72 against 79, FP32
+    // N=1e6 343 against 352); one lane takes all 8
+    md->vec = W < (1 << md->lc) ? (W > 1 ? -((1 << md->lc) / W) : 8) : 1;
     for (int r = 0; r < nslots; r++) {
         RepC R;
         memset(&R, 0, sizeof R);
@@ -3205,13 +3201,10 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
 
 template <bool FP32, bool KICK, bool EN>
 static int launch_force_kernel(ac4_md *md) {
-    // FP32 teams read consecutive entries of a chunk, FP64 ones (four lanes)
-    // strided ones; en_apart: no energy in this kernel
+    // a team of four on chunks of 8 has its energy apart in FP32 (en_apart)
     auto kern = md->vec == 8 ? k_force<FP32, KICK, EN, 8>
                 : md->vec == 1 ? k_force<FP32, KICK, EN, 1>
-                : md->vec == 4 ? k_force<true, KICK, false, 4>
-                : md->vec == 2 ? k_force<true, KICK, false, 2>
-                               : k_force<false, KICK, EN, -2>;
+                               : k_force<FP32, KICK, EN && !FP32, -2>;
     hipLaunchKernelGGL(kern, dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, md->stream, md->reps, md->fblk, md->pos4,
                        md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->P.act, md->kx, md->ky, md->kz, md->fx,
                        md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk,
