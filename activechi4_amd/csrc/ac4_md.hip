@@ -1662,24 +1662,25 @@ __device__ __forceinline__ void ld_list(const int *p, int *j) {
     }
 }
 
-// A team's walk of particle g's list of m entries, eight entries per lane and
+// A team's walk of particle g's list of m entries, G entries per lane and
 // group: the positions of a group are gathered together while the indices of
 // the next are loaded; the last, partial group has its loads issued together
 // too (an entry past m is replaced by g before it is used as an index).
 // VEC = 1: lane t of W takes entries t, t + W, ... (row c of the walk is
 // entries c*W ... c*W + W - 1, cs list words apart); the others read chunks
 // of 8 entries, cs words apart, with W = 8 / |VEC| lanes: VEC = 8 the whole
-// chunk, VEC = -2 entries t, t + 4 of it, two rows per chunk, and in FP64 six
-// entries per group (128 vector registers in k_force instead of 148, four waves per SIMD instead of
-// three; us per step at N=50000 50.7 -> 50.1, 80000 63.5 -> 61.4, 200000
-// 104 -> 99.5.  Teams of 8 and 16 lanes, whose lists are one or two groups,
-// keep eight: 22.0 against 22.8 at N=10000).
+// chunk, VEC = -2 entries t, t + 4 of it, two rows per chunk.  In FP64 a group
+// is six entries with VEC = -2 and four with VEC = 1: 128 and 108 vector
+// registers in k_force instead of 148, four waves per SIMD instead of three (us
+// per step, N=50000 50.7 -> 50.1, 80000 63.5 -> 61.4, 200000 104 -> 99.5;
+// teams of 8, N=20000 29.2 -> 28.7, 30000 34.6 -> 33.6; of 16 the same).
 template <int VEC, bool EN, class PosT, class Acc>
 __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t, int m, int g,
                                           const PosT *__restrict__ pos, const PosT &pi, Acc &acc) {
     constexpr int V = VEC > 1 ? VEC : 1;    // entries of a load
     constexpr int RC = VEC < 0 ? -VEC : 1;  // rows per step of cs
-    constexpr int G = VEC < 0 && sizeof(PosT) == 32 ? 6 : 8;  // entries of a group
+    constexpr bool WIDE = sizeof(PosT) == 32;                       // FP64
+    constexpr int G = WIDE && VEC < 0 ? 6 : WIDE && VEC == 1 ? 4 : 8;  // entries of a group
     constexpr int NR = G / V;               // rows of a group
     const int rl = W * V, full = m / rl;    // entries of a row, whole rows
     int c = 0, jn[G];
