@@ -430,7 +430,7 @@ class MD:
 
     def kernel_times(self, nsteps):
         """Average ms per step of {first_half, rebuild, force, shuffle,
-        force_end} (HIP events; force is k_force alone)."""
+        force_end} (HIP events; force includes the sums and the chain update, force_end is empty)."""
         o = np.empty(5)
         _check(lib.ac4_md_kernel_times(self.h, nsteps, _dp(o)))
         return dict(zip(["first_half", "rebuild", "force", "shuffle", "force_end"], o))

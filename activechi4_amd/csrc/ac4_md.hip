@@ -2116,9 +2116,9 @@ static void free_parts(PartArrays &a) {
 }
 
 // Kernel shape of handles created afterwards.  tpp: lanes per particle in
-// the force kernel, 1..16, or 0 = automatic (the widest team with at most
-// TPP_LANES lanes over the handle's total capacity, so small handles still
-// fill the device and large ones keep one thread per particle).  The team
+// the force kernel and of the list's layout, 1..16, or 0 = automatic (the
+// layout the widest with at most TPP_LANES lanes over the handle's total
+// capacity, the force team at least force_width of it).  The team
 // width fixes the order of each particle's force sum, so results are bitwise
 // reproducible for a given handle shape.  nlist_mode: dynamics list builder,
 // 0 = one wave per cell, 1 = one thread per particle, 2/3/4 = teams of

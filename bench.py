@@ -857,8 +857,8 @@ def main():
                      "kernel": "k_force<fp32,kick>", "bytes_per_particle": FORCE_BYTES_PER_PARTICLE,
                      "particles_per_launch": ntot,
                      "note": "one k_force launch over the whole ensemble at the timed run's kernel shape "
-                             "(HIP events, eager; the per-replica sums and chain update, k_force_end, are "
-                             "timed apart); the timed run splits the same particles into %d concurrent "
+                             "(HIP events, eager; with the per-replica sums and chain update); "
+                             "the timed run splits the same particles into %d concurrent "
                              "launch groups" % groups,
                      "whole_step": {"bytes_per_particle_step": STEP_BYTES_PER_PARTICLE,
                                     "achieved": value * STEP_BYTES_PER_PARTICLE / 1e9,
