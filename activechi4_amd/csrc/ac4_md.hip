@@ -2080,10 +2080,13 @@ struct ac4_md {
     int *ov_n = nullptr;
     int *et = nullptr;
     hipStream_t stream = nullptr;
-    // captured steps: [0] one step, [1] GRAPH_CHUNK steps in one graph
+    // recorded steps: [0] one step, [1] GRAPH_CHUNK steps in one graph
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int eager = 0;  // steps ac4_md_step launched one by one since the graphs were last dropped
     hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraph_t rec = nullptr;  // the graph that put() adds its launches to, or null
+    hipGraphNode_t rec_end = nullptr;
+    hipError_t rec_err = hipSuccess;
     bool have_forces = false;
     int nlist_mode = 0;
 };
@@ -2444,7 +2447,7 @@ static void drop_graphs(ac4_md *md) {
 // occupied), in slot order: the step's launch grids skip idle slots, whose
 // blocks would only exit.  A replica's blocks, and so its arithmetic (every
 // per-replica sum runs over its own blocks in their order), do not change.
-// The captured step graphs are dropped: their grids change.
+// The recorded step graphs are dropped: their grids change.
 static int refresh_tables(ac4_md *md) {
     bool any = false;
     for (const RepC &R : md->reps_h) any |= R.n > 0;
@@ -3145,37 +3148,61 @@ extern "C" int ac4_md_set_rebuild_criterion(ac4_md *md, int criterion) {
     return put_chains(md, c);
 }
 
+// A launch of the step's chain: on the handle's stream, or, while steps are
+// recorded, as the next node of the graph.  Stream capture would fail other
+// threads: while any stream is being captured, their calls on the null stream
+// (a plain hipMemcpy, the creation of another handle) return an error, in every
+// capture mode, and can end the capture.
+template <class... P>
+static void put(ac4_md *md, void (*kern)(P...), dim3 grid, dim3 block, size_t lds,
+                typename std::common_type<P>::type... a) {
+    void *args[] = {(void *)&a...};
+    if (!md->rec) {
+        (void)hipLaunchKernel((const void *)kern, grid, block, args, lds, md->stream);  // the callers ask hipGetLastError
+        return;
+    }
+    hipKernelNodeParams q{};
+    q.func = (void *)kern;
+    q.gridDim = grid;
+    q.blockDim = block;
+    q.sharedMemBytes = (unsigned)lds;
+    q.kernelParams = args;
+    hipGraphNode_t node = nullptr;
+    const hipError_t e = hipGraphAddKernelNode(&node, md->rec, &md->rec_end, md->rec_end ? 1 : 0, &q);
+    if (e == hipSuccess) md->rec_end = node;
+    else if (md->rec_err == hipSuccess) md->rec_err = e;
+}
+
 // Cell counts are cleared by k_first_half inside a step; outside a step
 // (update_cell_list) with_zero clears them first.
 // fixed grid of the work-list kernels: enough workgroups to fill the device
 #define WL_GRID 1024
 #define TEAM_MOVE_N 400000
 static int launch_rebuild(ac4_md *md, bool with_zero = false) {
-    hipStream_t s = md->stream;
     const int cy = (md->max_ncell + BLK - 1) / BLK;
     const WorkList wl{md->wl_item, md->wl_n, md->nblk, md->nblk + md->lnblk};
     const int gb = std::min(md->nblk, WL_GRID), gl = std::min(md->lnblk, WL_GRID), gc = std::min(md->ncb, WL_GRID);
     if (with_zero)
-        hipLaunchKernelGGL(k_cell_zero, dim3(md->R, cy), dim3(BLK), 0, s, md->reps, md->chain, md->cnt, md->wl_n);
-    hipLaunchKernelGGL(k_bin, dim3(md->nblk), dim3(BLK), 0, s, md->reps, md->chain, md->blk_rep, md->blk_first,
-                       md->P.x, md->P.y, md->P.z, md->P.id, md->cnt, md->P.cell_of, md->cell_mem, md->P.cell_ref,
-                       md->bin_fuse ? 1 : 0, md->bdone, md->start, wl);
+        put(md, k_cell_zero, dim3(md->R, cy), dim3(BLK), 0, md->reps, md->chain, md->cnt, md->wl_n);
+    put(md, k_bin, dim3(md->nblk), dim3(BLK), 0, md->reps, md->chain, md->blk_rep, md->blk_first,
+        md->P.x, md->P.y, md->P.z, md->P.id, md->cnt, md->P.cell_of, md->cell_mem, md->P.cell_ref,
+        md->bin_fuse ? 1 : 0, md->bdone, md->start, wl);
     if (!md->bin_fuse)
-        hipLaunchKernelGGL(k_bin_end, dim3(md->R), dim3(BIN_END_T), 0, s, md->reps, md->chain, md->cnt, md->start, wl);
-    hipLaunchKernelGGL(k_cell_sort, dim3(gc), dim3(BLK), 0, s, md->reps, wl, md->cnt, md->start,
-                       md->cell_mem, md->members, md->ranges, md->xmid, md->P, md->A,
-                       PosCopies{md->pos4, md->posq, md->xo, md->yo, md->zo});
+        put(md, k_bin_end, dim3(md->R), dim3(BIN_END_T), 0, md->reps, md->chain, md->cnt, md->start, wl);
+    put(md, k_cell_sort, dim3(gc), dim3(BLK), 0, md->reps, wl, md->cnt, md->start,
+        md->cell_mem, md->members, md->ranges, md->xmid, md->P, md->A,
+        PosCopies{md->pos4, md->posq, md->xo, md->yo, md->zo});
     // 16- and 32-lane list teams of handles up to TEAM_MOVE_N particles move
     // the permuted arrays back themselves (measured: 64 replicas, 1.5e5
     // particles, 134.5 -> 130.0 us per step; one box of 1e6, 686 -> 701 us)
     const bool team_moves = !with_zero && (md->nlist_mode == 2 || md->nlist_mode == 3) && md->ntot <= TEAM_MOVE_N;
     if (!team_moves)
-        hipLaunchKernelGGL(k_commit, dim3(gb), dim3(BLK), 0, s, md->reps, md->blk_rep, md->blk_first, wl, md->P,
-                           md->A);
+        put(md, k_commit, dim3(gb), dim3(BLK), 0, md->reps, md->blk_rep, md->blk_first, wl, md->P,
+            md->A);
     if (with_zero)  // update_cell_list: the reference's FP64 test and its 2.85 count
-        hipLaunchKernelGGL(k_nlist<true>, dim3(md->nblk), dim3(BLK), 0, s, md->reps, md->chain, md->blk_rep,
-                           md->blk_first, md->pos4, md->posq, md->P.cell_of, md->cnt, md->start, md->nn, md->nn_ref,
-                           md->nl, md->stride, md->cap);
+        put(md, k_nlist<true>, dim3(md->nblk), dim3(BLK), 0, md->reps, md->chain, md->blk_rep,
+            md->blk_first, md->pos4, md->posq, md->P.cell_of, md->cnt, md->start, md->nn, md->nn_ref,
+            md->nl, md->stride, md->cap);
     else if (md->nlist_mode >= 2) {
         const int w = md->nlist_mode == 2 ? 16 : (md->nlist_mode == 3 ? 32 : 64);
         bool trim = false;  // any replica whose cells are ordered by x-half
@@ -3186,16 +3213,16 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
                          : (w == 16 ? (team_moves ? k_nlist_team<16, true, false> : k_nlist_team<16, false, false>)
                                     : (w == 32 ? (team_moves ? k_nlist_team<32, true, false> : k_nlist_team<32, false, false>)
                                                : k_nlist_team<64, false, false>));
-        hipLaunchKernelGGL(kern, dim3(gl), dim3(w * LPB), 0, s, md->reps, md->chain, md->lblk_rep, md->lblk_first, wl,
-                           md->posq, md->A.cell_of, md->ranges, md->start, md->xmid, md->nn, md->nl, md->cap, md->ftab);
+        put(md, kern, dim3(gl), dim3(w * LPB), 0, md->reps, md->chain, md->lblk_rep, md->lblk_first, wl,
+            md->posq, md->A.cell_of, md->ranges, md->start, md->xmid, md->nn, md->nl, md->cap, md->ftab);
     }
     else if (md->nlist_mode == 0)
-        hipLaunchKernelGGL(k_nlist_cell, dim3(md->ncell_tot), dim3(64), 0, s, md->reps, md->chain, md->cblk_rep,
-                           md->cblk_cell, md->posq, md->cnt, md->start, md->nn, md->nl, md->cap);
+        put(md, k_nlist_cell, dim3(md->ncell_tot), dim3(64), 0, md->reps, md->chain, md->cblk_rep,
+            md->cblk_cell, md->posq, md->cnt, md->start, md->nn, md->nl, md->cap);
     else
-        hipLaunchKernelGGL(k_nlist<false>, dim3(md->nblk), dim3(BLK), 0, s, md->reps, md->chain, md->blk_rep,
-                           md->blk_first, md->pos4, md->posq, md->P.cell_of, md->cnt, md->start, md->nn, md->nn_ref,
-                           md->nl, md->stride, md->cap);
+        put(md, k_nlist<false>, dim3(md->nblk), dim3(BLK), 0, md->reps, md->chain, md->blk_rep,
+            md->blk_first, md->pos4, md->posq, md->P.cell_of, md->cnt, md->start, md->nn, md->nn_ref,
+            md->nl, md->stride, md->cap);
     AC4_HIP(hipGetLastError());
     return AC4_OK;
 }
@@ -3206,10 +3233,10 @@ static int launch_force_kernel(ac4_md *md) {
     auto kern = md->vec == 8 ? k_force<FP32, KICK, EN, 8>
                 : md->vec == 1 ? k_force<FP32, KICK, EN, 1>
                                : k_force<FP32, KICK, EN && !FP32, -2>;
-    hipLaunchKernelGGL(kern, dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, md->stream, md->reps, md->fblk, md->pos4,
-                       md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->P.act, md->kx, md->ky, md->kz, md->fx,
-                       md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk,
-                       EndArgs{md->chain, md->mid, md->gpart, md->gdone, md->rdone, md->en_apart ? 1 : 0});
+    put(md, kern, dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, md->reps, md->fblk, md->pos4,
+        md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->P.act, md->kx, md->ky, md->kz, md->fx,
+        md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk,
+        EndArgs{md->chain, md->mid, md->gpart, md->gdone, md->rdone, md->en_apart ? 1 : 0});
     AC4_HIP(hipGetLastError());
     return AC4_OK;
 }
@@ -3217,10 +3244,10 @@ static int launch_force_kernel(ac4_md *md) {
 // or after calculate_forces' pass.
 static int launch_energy(ac4_md *md, bool step) {
     if (!md->en_apart) return AC4_OK;
-    hipLaunchKernelGGL((md->elw ? k_energy<1> : k_energy<8>), dim3(xcd_grid(md->enblk)), dim3(BLK), 0, md->stream,
-                       md->reps, md->eblk, md->posq, md->nn, md->nl, md->cap, md->elw, md->epart, md->enblk);
-    hipLaunchKernelGGL(k_energy_end, dim3(md->R), dim3(256), 0, md->stream, md->reps, md->chain, md->epart,
-                       step ? 1 : 0);
+    put(md, (md->elw ? k_energy<1> : k_energy<8>), dim3(xcd_grid(md->enblk)), dim3(BLK), 0,
+        md->reps, md->eblk, md->posq, md->nn, md->nl, md->cap, md->elw, md->epart, md->enblk);
+    put(md, k_energy_end, dim3(md->R), dim3(256), 0, md->reps, md->chain, md->epart,
+        step ? 1 : 0);
     AC4_HIP(hipGetLastError());
     return AC4_OK;
 }
@@ -3234,31 +3261,31 @@ static int launch_force(ac4_md *md, bool energy) {
     return energy && !md->en_apart ? launch_force_pass<KICK, true>(md) : launch_force_pass<KICK, false>(md);
 }
 
-static void launch_shuffle(ac4_md *md, int force, hipStream_t s) {
+static void launch_shuffle(ac4_md *md, int force) {
     if (md->shuf_serial)
-        hipLaunchKernelGGL(k_shuffle, dim3(md->R, 3), dim3(256), md->shuf_lds, s, md->reps, md->chain, md->kx, md->ky,
-                           md->kz, force, md->shuf_kcap, md->shuf_bmax > 0 ? 1 : 0);
+        put(md, k_shuffle, dim3(md->R, 3), dim3(256), md->shuf_lds, md->reps, md->chain, md->kx, md->ky,
+            md->kz, force, md->shuf_kcap, md->shuf_bmax > 0 ? 1 : 0);
     if (md->shuf_par) {  // more than SHUF_PAR_MIN active particles
-        hipLaunchKernelGGL(k_shuf_part, dim3(md->shuf_bmax, 3, md->R), dim3(64), 0, s, md->reps, md->chain, force,
-                           md->shuf_bmax, md->shuf_ent, md->shuf_ent_n);
-        hipLaunchKernelGGL(k_shuf_apply, dim3(md->R, 3), dim3(2 * SHUF_M), md->shuf_lds, s, md->reps, md->chain,
-                           md->kx, md->ky, md->kz, force, md->shuf_kcap, md->shuf_bmax, md->shuf_ent,
-                           md->shuf_ent_n);
+        put(md, k_shuf_part, dim3(md->shuf_bmax, 3, md->R), dim3(64), 0, md->reps, md->chain, force,
+            md->shuf_bmax, md->shuf_ent, md->shuf_ent_n);
+        put(md, k_shuf_apply, dim3(md->R, 3), dim3(2 * SHUF_M), md->shuf_lds, md->reps, md->chain,
+            md->kx, md->ky, md->kz, force, md->shuf_kcap, md->shuf_bmax, md->shuf_ent,
+            md->shuf_ent_n);
     }
 }
 // with_shuffle: the step's shuffle runs in k_first_half's first 3*R
 // workgroups (handles whose shuffle LDS is small, see shuf_fused)
 static void launch_first_half(ac4_md *md, bool with_shuffle) {
     const ShufArgs sa{md->kx, md->ky, md->kz, md->shuf_kcap, with_shuffle ? 3 * md->R : 0};
-    hipLaunchKernelGGL(k_first_half, dim3(md->nblk + sa.nblk), dim3(BLK), with_shuffle ? md->shuf_lds : 0, md->stream,
-                       md->reps, md->chain, md->blkd, md->P.x, md->P.y, md->P.z, md->P.xu, md->P.yu,
-                       md->P.zu, md->P.px, md->P.py, md->P.pz, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo,
-                       md->P.type, md->pos4, md->posq, md->prec == AC4_FP32 ? 1 : 0, md->chain, md->blk_idx, md->cnt,
-                       md->wl_n, md->mid, sa);
+    put(md, k_first_half, dim3(md->nblk + sa.nblk), dim3(BLK), with_shuffle ? md->shuf_lds : 0,
+        md->reps, md->chain, md->blkd, md->P.x, md->P.y, md->P.z, md->P.xu, md->P.yu,
+        md->P.zu, md->P.px, md->P.py, md->P.pz, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo,
+        md->P.type, md->pos4, md->posq, md->prec == AC4_FP32 ? 1 : 0, md->chain, md->blk_idx, md->cnt,
+        md->wl_n, md->mid, sa);
 }
 
 // One MD step, one chain of launches on the handle's stream (also when
-// captured in a graph).  The shuffle, which only the force kernel needs, once
+// recorded in a graph).  The shuffle, which only the force kernel needs, once
 // ran on a second graph branch beside the half kick and the rebuild: the
 // fork and join cost more than the overlap gave (about 9 us per step).  It
 // now runs inside k_first_half where its LDS allows, else as k_shuffle first.
@@ -3269,7 +3296,7 @@ static int launch_step(ac4_md *md, bool last) {
     if (md->shuf_fused) {
         launch_first_half(md, true);
     } else {
-        launch_shuffle(md, 0, md->stream);
+        launch_shuffle(md, 0);
         launch_first_half(md, false);
     }
     AC4_HIP(hipGetLastError());
@@ -3326,29 +3353,29 @@ extern "C" int ac4_md_calculate_forces(ac4_md *md, double *out2) {
     return check_err(md);
 }
 
-// Steps are replayed from captured graphs: GRAPH_CHUNK steps per launch (one
+// Steps are replayed from recorded graphs: GRAPH_CHUNK steps per launch (one
 // launch per ten steps instead of one per step: 1.53e9 -> 1.60e9
 // particle-steps/s on the 64-replica ensemble in three launch groups; 25 steps
 // instead of ten: 2.093e9 -> 2.101e9), and a one-step graph for the remainder.  Every step's kernels and arguments are the same (the step
 // state lives on the device), so a chunk replays exactly the steps launched
 // one by one.
 #define GRAPH_CHUNK 25
-static int capture_steps(ac4_md *md, int k) {
+static int record_steps(ac4_md *md, int k) {
     const int m = k ? GRAPH_CHUNK : 1;
-    AC4_HIP(hipStreamBeginCapture(md->stream, hipStreamCaptureModeThreadLocal));
+    hipGraph_t g = nullptr;
+    AC4_HIP(hipGraphCreate(&g, 0));
+    md->rec = g;
+    md->rec_end = nullptr;
+    md->rec_err = hipSuccess;
     int rc = AC4_OK;
     for (int q = 0; q < m && rc == AC4_OK; q++) rc = launch_step(md, q == m - 1);
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamEndCapture(md->stream, &g);
-    if (rc != AC4_OK || e != hipSuccess) {  // nothing of a failed capture is kept
-        if (g) (void)hipGraphDestroy(g);
-        if (rc != AC4_OK) return rc;
-        AC4_HIP(e);
-    }
+    md->rec = nullptr;
     hipGraphExec_t x = nullptr;
-    e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
+    hipError_t e = md->rec_err;
+    if (rc == AC4_OK && e == hipSuccess) e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+    if (rc != AC4_OK || e != hipSuccess) {  // nothing of a failed recording is kept
         (void)hipGraphDestroy(g);
+        if (rc != AC4_OK) return rc;
         AC4_HIP(e);
     }
     md->graph[k] = g;
@@ -3359,19 +3386,19 @@ static int capture_steps(ac4_md *md, int k) {
 static int ready_graphs(ac4_md *md) {
     if (!md->have_forces) TRY(ac4_md_calculate_forces(md, nullptr));
     for (int k = 0; k < 2; k++)
-        if (!md->gexec[k]) TRY(capture_steps(md, k));
+        if (!md->gexec[k]) TRY(record_steps(md, k));
     return AC4_OK;
 }
 
 // Steps launched one by one.  On a small handle the five launches of a step
 // cost the host more than the step takes on the device (us per step launched
 // and replayed: N=1000 FP64 23.1 and 17.3, 8000 26.3 and 20.8, N=16000 FP32
-// 28.1 and 23.0), and capturing GRAPH_CHUNK steps about 1.1 ms: once a
+// 28.1 and 23.0), and recording GRAPH_CHUNK steps about 1.1 ms: once a
 // handle of at most STEP_GRAPH_N particles has launched STEP_GRAPH_PAY steps
 // that way, its further calls replay whole chunks from the graph, as
 // ac4_md_step_graph does (the same kernels and arguments: the results are the
 // same bit for bit), and launch the rest.  Larger handles are bound by the
-// device (N=50000 FP64: 50.2 and 48.9); short runs never pay for a capture.
+// device (N=50000 FP64: 50.2 and 48.9); short runs never pay for a recording.
 #define STEP_GRAPH_N 32768
 #define STEP_GRAPH_PAY 300
 extern "C" int ac4_md_step(ac4_md *md, int nsteps) {
@@ -3379,7 +3406,7 @@ extern "C" int ac4_md_step(ac4_md *md, int nsteps) {
     if (!md->have_forces) TRY(ac4_md_calculate_forces(md, nullptr));
     int k = 0;
     if (md->ntot <= STEP_GRAPH_N && nsteps >= GRAPH_CHUNK && (md->gexec[1] || md->eager >= STEP_GRAPH_PAY)) {
-        if (!md->gexec[1] && capture_steps(md, 1) != AC4_OK) {
+        if (!md->gexec[1] && record_steps(md, 1) != AC4_OK) {
             (void)hipGetLastError();
             md->eager = 0;  // launched as before, another try later
         }
@@ -3409,7 +3436,7 @@ extern "C" int ac4_md_step_graph_multi(ac4_md *const *mds, int nh, int nsteps) {
         AC4_REQUIRE(mds[h], AC4_EARG, "step_graph_multi: handle %d is NULL", h);
         for (int q = 0; q < h; q++)
             AC4_REQUIRE(mds[q] != mds[h], AC4_EARG, "step_graph_multi: handle %d appears twice", h);
-        TRY(ready_graphs(mds[h]));  // forces and the captured steps of every handle first
+        TRY(ready_graphs(mds[h]));  // forces and the recorded steps of every handle first
     }
     for (int k = 0; k < nsteps / GRAPH_CHUNK; k++)
         for (int h = 0; h < nh; h++) AC4_HIP(hipGraphLaunch(mds[h]->gexec[1], mds[h]->stream));
@@ -3446,7 +3473,7 @@ extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
     double acc[5] = {0, 0, 0, 0, 0};
     for (int k = 0; k < nsteps; k++) {
         AC4_HIP(hipEventRecord(ev[0], s));
-        if (!md->shuf_fused) launch_shuffle(md, 0, s);
+        if (!md->shuf_fused) launch_shuffle(md, 0);
         AC4_HIP(hipEventRecord(ev[1], s));
         launch_first_half(md, md->shuf_fused);
         AC4_HIP(hipEventRecord(ev[2], s));
@@ -3468,7 +3495,7 @@ extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
 
 extern "C" int ac4_md_shuffle(ac4_md *md) {
     AC4_REQUIRE(md, AC4_EARG, "NULL handle");
-    launch_shuffle(md, 1, md->stream);
+    launch_shuffle(md, 1);
     AC4_HIP(hipGetLastError());
     std::vector<ChainS> c;
     TRY(get_chains(md, c));  // synchronises

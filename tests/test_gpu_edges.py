@@ -2,6 +2,7 @@
 remainders, the smallest and largest of their ranges, against the oracle or a
 64-bit restatement."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -388,3 +389,41 @@ def test_shuffle_launches_by_the_jobs(gpu, acts):
         alone = start([a])[0]
         for k in ("kx", "ky", "kz", "xu", "px"):
             assert np.array_equal(alone[k], both[r][k]), (a, k)
+
+
+# Another thread's calls on the null stream (copies, the creation of handles)
+# while a handle's steps are recorded: they succeed, and the steps are those
+# of a handle alone.
+def test_steps_recorded_beside_the_null_stream(gpu):
+    hip = ctypes.CDLL("libamdhip64.so")
+    n, codes, stop = 600, [], threading.Event()
+    s = gpu.init_lattice(n, 0.5, 5)
+
+    def steps():
+        md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 30, 3)])
+        md.set_state(0, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], s["act_tag"],
+                     s["kx"], s["ky"], s["kz"])
+        md.step(300)
+        md.step(50)
+        out = md.get_state(0)
+        md.close()
+        return out
+
+    def copies():
+        d, h = ctypes.c_void_p(), np.zeros(16)
+        codes.append(hip.hipMalloc(ctypes.byref(d), ctypes.c_size_t(128)))
+        while not stop.is_set():
+            codes.append(hip.hipMemcpy(h.ctypes.data_as(ctypes.c_void_p), d, ctypes.c_size_t(128), 2))
+        hip.hipFree(d)
+
+    alone = steps()
+    t = threading.Thread(target=copies)
+    t.start()
+    try:
+        for _ in range(5):
+            got = steps()
+            assert all(np.array_equal(got[k], alone[k]) for k in ("x", "px", "kx"))
+    finally:
+        stop.set()
+        t.join()
+    assert len(codes) > 100 and not any(codes)
