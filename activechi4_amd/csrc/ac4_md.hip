@@ -2141,9 +2141,13 @@ static void free_parts(PartArrays &a) {
 //        200000:  121  113  106  121  143   500000:  288  252  252  292  361
 // Four FP32 lanes reading a chunk's entries strided (k_force, VEC = -2) take
 // 177.6 at 500000, 118.7 at 300000 and 44.6 at 70000; reading two consecutive
-// ones 181.6, 122.5 and 45.4; eight lanes 194.9, 127.2 and 45.4.
+// ones 181.6, 122.5 and 45.4; eight lanes 194.9, 127.2 and 45.4.  The lines lie
+// where the automatic list layout changes (TPP_LANES), so that handles between
+// which a checkpoint can move, those of one layout, have one force width and
+// the restored replica goes on bit for bit (14500 and 16000 particles at 8 and
+// 16 lanes: FP32 22.4 and 22.1, 22.5 and 22.9; FP64 23.5 and 24.0, 24.1 and 24.4).
 static int force_width(double cap_tot) {
-    if (cap_tot <= 14000.0) return 16;
+    if (cap_tot <= 16384.0) return 16;
     if (cap_tot <= 32768.0) return 8;
     return 4;
 }

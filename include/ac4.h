@@ -279,8 +279,10 @@ int ac4_md_fix_drift(ac4_md *md, int r, double *mean3);
  * counters), so a run resumed from it is bitwise the uninterrupted run (the
  * reference's restart is not exact: it redraws the chain momenta).  Restore
  * into a slot configured with the same replica parameters in a handle of the
- * same shape (precision, team width, skin); other replicas of the handle are
- * not touched.  Sizes in bytes. */
+ * same shape (precision, skin, and team width: pinned alike, or automatic in
+ * both; between a pinned and an automatic handle of one list layout it goes on
+ * with the other's summation order); other replicas of the handle are not
+ * touched.  Sizes in bytes. */
 long long ac4_md_checkpoint_size(ac4_md *md, int r);
 int ac4_md_checkpoint(ac4_md *md, int r, void *buf, long long cap);
 int ac4_md_restore(ac4_md *md, int r, const void *buf, long long len);

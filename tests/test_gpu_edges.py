@@ -427,3 +427,29 @@ def test_steps_recorded_beside_the_null_stream(gpu):
         stop.set()
         t.join()
     assert len(codes) > 100 and not any(codes)
+
+
+# A checkpoint goes on bit for bit in every handle of its layout: capacities at
+# both ends of the layout of four lanes, alone and beside another replica.
+@pytest.mark.parametrize("prec", [0, 1])
+def test_checkpoint_between_capacities_of_a_layout(gpu, prec):
+    def relaxed(sizes):
+        md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 30, 3) for n in sizes], precision=prec)
+        for r, n in enumerate(sizes):
+            s = gpu.init_lattice(n, 0.5, 5)
+            md.set_state(r, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"],
+                         s["act_tag"], s["kx"], s["ky"], s["kz"])
+        md.relax(40)  # every replica has its forces before the restore
+        for r in range(len(sizes)):
+            md.init_chain(r)
+        return md
+    a, b = relaxed([8300]), relaxed([8300, 16384 - 8300])
+    a.step(20)
+    b.restore(0, a.checkpoint(0))
+    for md in (a, b):
+        md.step(60)
+    x, y = a.get_state(0), b.get_state(0)
+    assert all(np.array_equal(x[k], y[k]) for k in x)
+    assert np.array_equal(a.get_chain(0), b.get_chain(0))
+    a.close()
+    b.close()
