@@ -662,7 +662,7 @@ __global__ void __launch_bounds__(BLK) k_bin(const RepC *__restrict__ reps, Chai
         // list teams cull (RepC::xcull) the x bit is highest, so each x-half
         // of a cell is one slot range (k_cell_sort); elsewhere the z bit (one
         // N=10^6 box: 2.48e9 against 2.45e9 particle-steps/s with x highest).
-        // n < 2^21, so the id fits below bit 21.
+        // n <= 2^21, so the id fits below bit 21.
         const int ox = clampc((int)floor(sx * (2 * R.nc)), 2 * R.nc) & 1,
                   oy = clampc((int)floor(sy * (2 * R.nc)), 2 * R.nc) & 1,
                   oz = clampc((int)floor(sz * (2 * R.nc)), 2 * R.nc) & 1;
@@ -1065,11 +1065,12 @@ __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, Chai
         return __builtin_amdgcn_fcmpf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)), cut, 4) &  // ordered <
                __builtin_amdgcn_uicmp((unsigned)k, (unsigned)g, 33);                                      // !=
     };
-    // entry p of this particle's list at nlb[(p >> lc) * nC + (p & cm)] (nl_at
-    // relative to entry 0; 24-bit products, n < 2^21 is checked at creation)
+    // entry p of this particle's list at nlb[(p & ~cm) * n + (p & cm)] (nl_at
+    // relative to entry 0: p >> lc chunks of n << lc entries).  Both factors
+    // fit 24 bits in every layout (n <= 2^21 is checked at creation), which n
+    // times the chunk length does not.
     int *const nlb = nl + nl_at(R, cap, 0, i);
-    const unsigned nC = (unsigned)R.n << R.lc, cm = (1u << R.lc) - 1u;
-    const int lc = R.lc;
+    const unsigned cm = (1u << R.lc) - 1u;
     // a hit's place: the team's count so far and its hits of lower lanes
     // (mbcnt of the ballot word that holds the team)
     const unsigned mlo = NLT == 32 && lane >= 32 ? 0u : ~0u;
@@ -1087,7 +1088,7 @@ __device__ __forceinline__ void nlist_team_one(const RepC &R, int r, int i, Chai
             pos = count + __popcll(m & below);
             tot = __popcll(m);
         }
-        if (__builtin_amdgcn_inverse_ballot_w64(b) && pos < (unsigned)cap) nlb[__umul24(pos >> lc, nC) + (pos & cm)] = k;
+        if (__builtin_amdgcn_inverse_ballot_w64(b) && pos < (unsigned)cap) nlb[__umul24(pos & ~cm, (unsigned)R.n) + (pos & cm)] = k;
         count += tot;
     };
     // the home cell's stencil as slot ranges (k_cell_sort), in stencil order:
@@ -2306,7 +2307,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         memset(&R, 0, sizeof R);
         const int cn = cap_n[r];
         if (cn < 2) { delete md; ac4_set_error("slot %d: capacity %d < 2", r, cn); return AC4_EARG; }
-        // list addressing in the team builders uses 24-bit products of n*8
+        // the cell sort's keys hold ids below 2^21, list addressing uses 24-bit products with n
         if (cn > (1 << 21)) { delete md; ac4_set_error("slot %d: capacity %d > 2^21", r, cn); return AC4_EARG; }
         R.cap_n = cn;
         R.skin = g_skin;

@@ -453,3 +453,25 @@ def test_checkpoint_between_capacities_of_a_layout(gpu, prec):
     assert np.array_equal(a.get_chain(0), b.get_chain(0))
     a.close()
     b.close()
+
+
+# A list layout whose chunks of 16 entries times the particles pass 2^24: the
+# team builders store the lists the thread-per-particle builder stores.
+@pytest.mark.parametrize("n", [1048576, 1048600])
+def test_list_addresses_of_large_boxes(gpu, n):
+    s = gpu.init_lattice(n, 0.5, 11)
+    out = []
+    for mode in (1, 2, 3, 4):
+        gpu.set_tuning(16, mode)
+        try:
+            md = gpu.MD([gpu.ReplicaParams(n, 1.2, 1.0, 1.0, -1, 20, 3)], precision=gpu.FP32)
+        finally:
+            gpu.set_tuning()
+        md.set_state(0, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], s["act_tag"],
+                     s["kx"], s["ky"], s["kz"])
+        md.relax(40)
+        assert md.rebuilds(0) > 1
+        out.append((md.export_xu()[0], np.stack(md.forces(0))))
+        md.close()
+    for xu, f in out[1:]:
+        assert np.array_equal(xu, out[0][0]) and np.array_equal(f, out[0][1])
