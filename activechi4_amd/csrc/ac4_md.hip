@@ -1931,15 +1931,16 @@ __global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, co
         last = 0;
         if (lane == 0) last = last_done(E.rdone + D.rep * DONE_PAD, ngr);
         if (!__builtin_amdgcn_readfirstlane(last)) return;
-        const bool few = ngr <= 4;  // one after the other, else lane k groups k, k + 64, ...
+        // lane k groups k, k + 64, ..., then the butterfly: groups past the
+        // particles add zeros, so the slot's capacity does not show in the sums
         for (int q = 0; q < 4; q++) a4[q] = 0.0;
-        for (int k = few ? 0 : lane; k < ngr; k += few ? 1 : 64)
+        for (int k = lane; k < ngr; k += 64)
 #pragma unroll
             for (int q = 0; q < 4; q++)
                 if (EN || q == 0 || q == 3) a4[q] += ld_agent(gp + 4 * k + q);
 #pragma unroll
         for (int q = 0; q < 4; q++)
-            if (!few && (EN || q == 0 || q == 3)) a4[q] = wave_sum_rows(a4[q]);
+            if (EN || q == 0 || q == 3) a4[q] = wave_sum_rows(a4[q]);
     }
     if (lane == 0) {
         ChainS c0;

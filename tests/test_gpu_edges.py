@@ -475,3 +475,31 @@ def test_list_addresses_of_large_boxes(gpu, n):
         md.close()
     for xu, f in out[1:]:
         assert np.array_equal(xu, out[0][0]) and np.array_equal(f, out[0][1])
+
+
+# A checkpoint goes on bit for bit in a larger slot of its handle: replicas
+# whose force blocks are four groups of 64, in slots of four and of five, at
+# force teams of 16, 8 and 4 lanes.
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n,caps", [(4000, (4000, 5000)), (8000, (8000, 9000)), (16000, (16000, 17000))])
+def test_checkpoint_between_slot_capacities(gpu, n, caps, prec):
+    h = ctypes.c_void_p()
+    assert gpu.lib.ac4_md_create_slots(2, (ctypes.c_int * 2)(*caps), prec, ctypes.byref(h)) == 0
+    md = gpu.MD.__new__(gpu.MD)
+    md.h, md.params = h, [gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 30, 3)] * 2
+    for r in range(2):
+        assert gpu.lib.ac4_md_assign(h, r, ctypes.byref(md.params[r])) == 0
+        s = gpu.init_lattice(n, 0.5, 5)
+        md.set_state(r, *[s[k] for k in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], s["act_tag"],
+                     s["kx"], s["ky"], s["kz"])
+    md.relax(40)
+    md.init_chain(0)
+    md.step(20)
+    md.restore(1, md.checkpoint(0))
+    for _ in range(60):  # the sum of p^2 of every step: its last bit seldom survives in the thermostat
+        md.step(1)
+        assert md.stats(0) == md.stats(1)
+    x, y = md.get_state(0), md.get_state(1)
+    assert all(np.array_equal(x[k], y[k]) for k in x)
+    assert np.array_equal(md.get_chain(0), md.get_chain(1))
+    md.close()
