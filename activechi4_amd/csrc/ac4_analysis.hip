@@ -1240,6 +1240,12 @@ static int push_common(ac4_ana *an, int pos, const double *x, const double *y, c
         AC4_REQUIRE(an->resident[an->jorg[j]], AC4_ESTATE, "origin frame %d of pair %d was not pushed", an->jorg[j],
                     an->jobs[j].p0 >= 0 ? an->jobs[j].p0 : an->jobs[j].p1);
     hipStream_t s = an->stream;
+    // origins whose last lag was left out: the S4 sums of the lags that came,
+    // before this frame takes a place
+    if (an->obs & AC4_OBS_S4)
+        for (int f = an->last_pos + 1; f < pos; f++)
+            for (int o : an->s4_end[f])
+                if (an->resident[o] && !an->s4_done[o]) TRY(s4_origin(an, o));
     const size_t n = an->n, b = sizeof(double) * n;
     int keep = an->place[pos];
     if (host) {  // an origin frame straight to its place
@@ -1346,7 +1352,7 @@ static int sum_blocks(ac4_ana *an) {
 extern "C" int ac4_ana_finalize(ac4_ana *an) {
     AC4_REQUIRE(an, AC4_EARG, "NULL handle");
     if (an->finalized) return AC4_OK;
-    if (an->obs & AC4_OBS_S4)  // origins whose last lag frame was never pushed
+    if (an->obs & AC4_OBS_S4)  // origins whose last lag frame is past the last one pushed
         for (int o = 0; o < an->nframes; o++)
             if (!an->s4_done[o] && an->resident[o] && an->s4_optr[o + 1] > an->s4_optr[o]) TRY(s4_origin(an, o));
     TRY(sum_blocks(an));

@@ -503,3 +503,34 @@ def test_checkpoint_between_slot_capacities(gpu, n, caps, prec):
     assert all(np.array_equal(x[k], y[k]) for k in x)
     assert np.array_equal(md.get_chain(0), md.get_chain(1))
     md.close()
+
+
+# S4 and Fs of an origin whose last lag frame is left out: the lags that came
+# are those of the full walk.  The next frame that comes is a lag frame, or an
+# origin that takes a place of the resident frames itself, or there is none;
+# both S4 kernels.
+@pytest.mark.parametrize("n,obs", [(300, 15), (300, 4), (3100, 12)])
+def test_origins_without_their_last_lag(gpu, n, obs):
+    frames = trajgen.case_frames(3, 30)
+    left_out = [frames.index(t) for t in (42, 46, 52, 72, 102)]
+    X, Y, Z, T = trajgen.make_frames(n, frames, 5, 0.08, 1.0)
+    L = (n / 1.2) ** (1.0 / 3.0)
+    an = gpu.Analysis(n, L, frames, gap=30, obs=obs)
+    for f in range(len(frames)):
+        if f not in left_out:
+            an.push(f, X[f], Y[f], Z[f], T[f])
+    an.finalize()
+    walk = _walk(frames, 30)
+    here = ~np.isin([frames.index(o + l) for o, l in walk], left_out)
+    last = {o: o + l for o, l in walk}
+    assert set(last.values()) <= {frames[k] for k in left_out} and here.sum() > 20
+    os4 = OL.phase("s4", n, L, X, Y, Z, T, frames, 30)
+    v, m = an.pairs(gpu.OBS_S4)
+    assert np.array_equal(m[here], os4["mask"][here]) and m[here].min() > 0 and not m[~here].any()
+    # a term is off by at most a few 1e-14
+    assert np.abs(v[here] - os4["pairs"][here]).max() < 1e-12 * n and not v[~here].any()
+    if obs & 8:
+        ofs = OL.phase("fs", n, L, X, Y, Z, T, frames, 30)
+        w = an.pairs(gpu.OBS_FS)
+        assert np.abs(w[here] - ofs["pairs"][here]).max() < 1e-12 * n and not w[~here].any()
+    an.close()
