@@ -534,3 +534,20 @@ def test_origins_without_their_last_lag(gpu, n, obs):
         w = an.pairs(gpu.OBS_FS)
         assert np.abs(w[here] - ofs["pairs"][here]).max() < 1e-12 * n and not w[~here].any()
     an.close()
+
+
+# Boxes of no bin, one bin and two: an empty histogram, and the pairs' counts.
+@pytest.mark.parametrize("L,nbin", [(0.004, 0), (0.0101, 1), (0.0201, 2)])
+def test_guu_boxes_of_few_bins(gpu, L, nbin):
+    n, frames = 300, trajgen.case_frames(5, 40)
+    X, Y, Z, _ = trajgen.make_frames(n, frames, 31, 0.3, 1.0)
+    act = np.ones(n, dtype=np.int32)
+    fr = gpu.Frames(n, L, len(frames))
+    for k, t in enumerate(frames):
+        fr.push(X[k], Y[k], Z[k], t)
+    h, fn, no = fr.guu(act, 40, 0.06)
+    fr.close()
+    assert h.shape == (3, nbin) and no > 0
+    if nbin:
+        ho, fno, noo = OL.guu(n, L, X, Y, Z, act, frames, 40, 0.06)
+        assert (fn, no) == (fno, noo) and np.array_equal(h[0], ho[0])
