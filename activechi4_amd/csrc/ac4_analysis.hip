@@ -902,6 +902,7 @@ struct ac4_ana {
     std::vector<int> vx, vy, vz, qsq;
     std::vector<double> qval;
     hipStream_t stream = nullptr;
+    int dev = 0;                // the device the handle was made on
     bool finalized = false;
     // slot results
     std::vector<double> m0, m1, m2, c, x4, s4c, s4s, s4c2, s4s2, fsc, fss, fsc2, fss2;
@@ -1113,7 +1114,7 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     }
     int rc = AC4_OK;
     auto fail = [&](int e) { ac4_ana_destroy(an); return e; };
-    if (hipStreamCreate(&an->stream) != hipSuccess) return fail(AC4_EHIP);
+    if (hipGetDevice(&an->dev) != hipSuccess || hipStreamCreate(&an->stream) != hipSuccess) return fail(AC4_EHIP);
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vx), an->vx.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vy), an->vy.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vz), an->vz.data(), sizeof(int) * AC4_NQ));
@@ -1230,8 +1231,21 @@ static int process_frame(ac4_ana *an, int pos, const double *x, const double *y,
     return wait ? wait_read(an) : AC4_OK;
 }
 
+// p is memory of the device dev, which its kernels read where it is (another
+// device's may not be mapped there, nor the host's): 0.06 us, so a push of
+// device arrays takes 0.25 of its 12 us for asking
+static bool on_device(const void *p, int dev) {
+    hipPointerAttribute_t a = {};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeDevice && a.device == dev;
+    (void)hipGetLastError();
+    return false;
+}
+
+// kind: hipMemcpyHostToDevice for host arrays, which are copied;
+// hipMemcpyDefault for arrays the kernels read where they are, or of another
+// device or the host, copied too
 static int push_common(ac4_ana *an, int pos, const double *x, const double *y, const double *z, const int *t,
-                       bool host) {
+                       hipMemcpyKind kind) {
     AC4_REQUIRE(an && pos >= 0 && pos < an->nframes && x && y && z && t, AC4_EARG, "push_frame: bad arguments");
     AC4_REQUIRE(pos > an->last_pos, AC4_ESTATE, "push_frame: frame %d after %d (frames must increase)", pos,
                 an->last_pos);
@@ -1248,19 +1262,21 @@ static int push_common(ac4_ana *an, int pos, const double *x, const double *y, c
                 if (an->resident[o] && !an->s4_done[o]) TRY(s4_origin(an, o));
     const size_t n = an->n, b = sizeof(double) * n;
     int keep = an->place[pos];
-    if (host) {  // an origin frame straight to its place
+    const bool copy = kind != hipMemcpyDefault || !on_device(x, an->dev) || !on_device(y, an->dev) ||
+                      !on_device(z, an->dev) || !on_device(t, an->dev);
+    if (copy) {  // an origin frame straight to its place
         double *dx = an->cur, *dy = dx + n, *dz = dy + n;
         if (keep >= 0) { dx = an->org.at(keep, 0); dy = an->org.at(keep, 1); dz = an->org.at(keep, 2); }
-        AC4_HIP(hipMemcpyAsync(dx, x, b, hipMemcpyHostToDevice, s));
-        AC4_HIP(hipMemcpyAsync(dy, y, b, hipMemcpyHostToDevice, s));
-        AC4_HIP(hipMemcpyAsync(dz, z, b, hipMemcpyHostToDevice, s));
-        AC4_HIP(hipMemcpyAsync(an->cur_t, t, sizeof(int) * n, hipMemcpyHostToDevice, s));
+        AC4_HIP(hipMemcpyAsync(dx, x, b, kind, s));
+        AC4_HIP(hipMemcpyAsync(dy, y, b, kind, s));
+        AC4_HIP(hipMemcpyAsync(dz, z, b, kind, s));
+        AC4_HIP(hipMemcpyAsync(an->cur_t, t, sizeof(int) * n, kind, s));
         x = dx; y = dy; z = dz; t = an->cur_t;
         keep = -1;
     }
     an->resident[pos] = an->place[pos] >= 0;
-    TRY(process_frame(an, pos, x, y, z, t, keep, !host));  // the caller may reuse its arrays
-    if (host) AC4_HIP(hipStreamSynchronize(s));
+    TRY(process_frame(an, pos, x, y, z, t, keep, !copy));  // the caller may reuse its arrays
+    if (copy) AC4_HIP(hipStreamSynchronize(s));
     // origins no pair needs any more (their places may be taken from now on)
     for (int f = an->last_pos + 1; f <= pos; f++)
         for (int o : an->ends[f]) an->resident[o] = 0;
@@ -1270,12 +1286,12 @@ static int push_common(ac4_ana *an, int pos, const double *x, const double *y, c
 
 extern "C" int ac4_ana_push_frame(ac4_ana *an, int pos, const double *x, const double *y, const double *z,
                                   const int *type) {
-    return push_common(an, pos, x, y, z, type, true);
+    return push_common(an, pos, x, y, z, type, hipMemcpyHostToDevice);
 }
 
 extern "C" int ac4_ana_push_frame_device(ac4_ana *an, int pos, const double *x, const double *y, const double *z,
                                          const int *type) {
-    return push_common(an, pos, x, y, z, type, false);
+    return push_common(an, pos, x, y, z, type, hipMemcpyDefault);
 }
 
 extern "C" int ac4_md_device_xu(ac4_md *md, int r, const double **xu, const double **yu, const double **zu,
@@ -1287,7 +1303,7 @@ extern "C" int ac4_ana_push_md(ac4_ana *an, int pos, ac4_md *md, int r) {
     TRY(ac4_md_device_xu(md, r, &x, &y, &z, &t, &n));
     AC4_REQUIRE(an && n == an->n, AC4_EARG, "push_md: replica has %d particles, analysis expects %d", n,
                 an ? an->n : -1);
-    return push_common(an, pos, x, y, z, t, false);
+    return push_common(an, pos, x, y, z, t, hipMemcpyDefault);
 }
 
 // The slots' sums of a walk's pair values, for the slots that have pairs

@@ -449,7 +449,9 @@ int ac4_ana_push_frame(ac4_ana *an, int pos, const double *x, const double *y,
                        const double *z, const int *type);
 /* Same from device arrays (in-situ analysis of a running MD handle).  Returns
  * when the arrays have been read and may be overwritten or freed; the results
- * are waited for where they are asked for (get, finalize, write). */
+ * are waited for where they are asked for (get, finalize, write).  Arrays of
+ * the device the handle was made on are read where they are; arrays of another
+ * device or of the host are copied first. */
 int ac4_ana_push_frame_device(ac4_ana *an, int pos, const double *dx,
                               const double *dy, const double *dz,
                               const int *dtype);

@@ -551,3 +551,45 @@ def test_guu_boxes_of_few_bins(gpu, L, nbin):
     if nbin:
         ho, fno, noo = OL.guu(n, L, X, Y, Z, act, frames, 40, 0.06)
         assert (fn, no) == (fno, noo) and np.array_equal(h[0], ho[0])
+
+
+# The device push copies arrays that the handle's device may not read where
+# they are: pageable and pinned host memory, all of the arrays or one of them,
+# overwritten as soon as the push returns.
+@pytest.mark.parametrize("n,obs", [(700, 15), (2049, 3)])
+@pytest.mark.parametrize("where", ["pageable", "pinned", "types"])
+def test_device_push_of_other_memory(gpu, n, obs, where):
+    frames = trajgen.case_frames(3, 30)
+    X, Y, Z, T = trajgen.make_frames(n, frames, 5 + n, 0.08, 1.0)
+    L = (n / 1.2) ** (1.0 / 3.0)
+    hip = ctypes.CDLL("libamdhip64.so")  # the runtime the library has loaded
+    dev, pin = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(dev), ctypes.c_size_t(28 * n)) == 0
+    assert hip.hipHostMalloc(ctypes.byref(pin), ctypes.c_size_t(28 * n), 0) == 0
+    own = np.zeros(28 * n, dtype=np.uint8)
+    base = {"pageable": own.ctypes.data, "pinned": pin.value, "types": dev.value}[where]
+    at = [base + 8 * n * k for k in range(4)]  # x, y, z, types
+    if where == "types":
+        at[3] = own.ctypes.data
+    out = []
+    for device in (False, True):
+        an = gpu.Analysis(n, L, frames, gap=30, obs=obs)
+        for f in range(len(frames)):
+            if not device:
+                an.push(f, X[f], Y[f], Z[f], T[f])
+                continue
+            src = [np.ascontiguousarray(v) for v in (X[f], Y[f], Z[f], np.asarray(T[f], dtype=np.int32))]
+            for d, v in zip(at, src):
+                assert hip.hipMemcpy(ctypes.c_void_p(d), v.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(v.nbytes), 4) == 0
+            assert gpu.lib.ac4_ana_push_frame_device(an.h, f, *at) == 0
+            for d, v in zip(at, src):
+                w = np.full(v.nbytes, 255, dtype=np.uint8)
+                assert hip.hipMemcpy(ctypes.c_void_p(d), w.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(w.nbytes), 4) == 0
+        an.finalize()
+        got = [an.pairs(o) for o in (gpu.OBS_MSD, gpu.OBS_OVERLAP, gpu.OBS_S4, gpu.OBS_FS) if obs & o]
+        out.append([v for g in got for v in (g if isinstance(g, tuple) else (g,))])
+        an.close()
+    hip.hipFree(dev)
+    hip.hipHostFree(pin)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
