@@ -5,6 +5,7 @@ force error on 100 configurations of a run, and the overlap Q(t) of an
 ensemble in FP32 against the same ensemble in FP64."""
 import numpy as np
 import pytest
+from scipy.spatial import cKDTree
 
 import oracle_lib as OL
 from test_gpu_md import _chain0, make_md
@@ -158,3 +159,40 @@ def test_forces_at_one_million_particles(gpu):
     assert err64 < 1e-12
     assert err32 <= 1e-5
     assert net < 1e-10
+
+
+@pytest.mark.parametrize("n", [1000, 50000])
+def test_fp64_energy_and_virial_against_extended_precision(gpu, n):
+    """FP64 pair energy and virial against the same sums in 80-bit arithmetic,
+    on a displaced lattice with many close pairs, whose terms magnify an error
+    of r^2 that all pairs share."""
+    LD = np.longdouble
+    rng = np.random.default_rng(5)
+    s = gpu.init_lattice(n, 0.5, n)
+    x = np.stack([(s[k] + rng.normal(0, 0.03 / n ** (1 / 3), n)) % 1.0 for k in ("x", "y", "z")])
+    L = float(np.power(n / 1.2, 0.33333333))
+    md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 0.0, -1, 200, 3)], precision=gpu.FP64)
+    md.set_state(0, *x, *x, s["px"], s["py"], s["pz"], s["type"], s["act_tag"], s["kx"], s["ky"], s["kz"])
+    got = md.calculate_forces()[0]
+    md.close()
+    i, j = cKDTree(x.T, boxsize=1.0).query_pairs(2.51 / L, output_type="ndarray").T
+    d = x[:, i].astype(LD) - x[:, j].astype(LD)
+    d -= np.rint(d)
+    r2 = (d * d).sum(0) * LD(L) * LD(L)
+    ab = s["type"][i] + s["type"][j]
+    sg2 = np.array([1.0, 0.80 * 0.80, 0.88 * 0.88])[ab].astype(LD)
+    ep = np.array([1.0, 1.5, 0.5])[ab]
+    ros = r2 / sg2
+    ok = ros < 6.25
+    r2, sg2, ep, ros = r2[ok], sg2[ok], ep[ok], ros[ok]
+    c0, c2, s6 = LD(0.0162665594880), LD(-0.001949973872640), (1 / ros) ** 3
+    pe = 4 * ep * (s6 * (s6 - 1) + c0 + c2 * ros)
+    w = 8 * ep * (6 * s6 * (s6 - LD(0.5)) - c2 * ros)  # r^2 times the gradient
+    # A pair's r^2 carries about 1.5 roundings, 1/r^2 and s^2 one each, and a
+    # term in s^12 six times their sum, sqrt(1.5^2 + 1 + 1) * 6 / sqrt(3) = 7 in
+    # the mean square; four standard deviations of the sum of independent
+    # pairs.  The sums add four roundings of the total.
+    dev = 4 * 7 * np.sqrt(((ep * (s6 * s6 + s6)) ** 2).sum())
+    tol = 2.0 ** -53 * (dev * np.array([4, 16]) + 4 * np.array([abs(pe.sum()), abs(w.sum()) / 3]))
+    assert abs(got[0] - pe.sum()) <= tol[0] and abs(got[1] - w.sum() / 3) <= tol[1], \
+        (got - np.array([pe.sum(), w.sum() / 3])) / tol
