@@ -2108,16 +2108,58 @@ static int dalloc(T **p, size_t n) {
     return AC4_OK;
 }
 
-static int alloc_parts(PartArrays &a, size_t n) {
-    int rc;
-    double **d[] = {&a.x, &a.y, &a.z, &a.xu, &a.yu, &a.zu, &a.px, &a.py, &a.pz};
-    for (double **q : d)
-        if ((rc = dalloc(q, n)) != AC4_OK) return rc;
-    int **i[] = {&a.type, &a.act, &a.id, &a.cell_ref, &a.cell_of};
-    for (int **q : i)
-        if ((rc = dalloc(q, n)) != AC4_OK) return rc;
+template <class F>
+static int each_part(PartArrays &a, size_t n, F get) {
+    for (double **q : {&a.x, &a.y, &a.z, &a.xu, &a.yu, &a.zu, &a.px, &a.py, &a.pz}) TRY(get(q, n));
+    for (int **q : {&a.type, &a.act, &a.id, &a.cell_ref, &a.cell_of}) TRY(get(q, n));
     return AC4_OK;
 }
+
+// What slots add up to, and the device arrays a handle of that many has: the
+// list creation allocates and ac4_md_slot_bytes adds up, get(&array, count).
+struct SlotCounts {
+    size_t slots, n, cells, nblk, fnblk, lnblk, ncb;  // particles, cells, blocks of each kind
+    size_t enblk;                                     // blocks of the energy pass, 0 without it
+    size_t shuf;                                      // swap blocks of the parallel shuffle, 0 without it
+};
+template <class F>
+static int each_array(ac4_md *md, const SlotCounts &k, F get) {
+    if (k.shuf) { TRY(get(&md->shuf_ent, k.shuf * 2 * SHUF_M)); TRY(get(&md->shuf_ent_n, k.shuf)); }
+    TRY(get(&md->reps, k.slots)); TRY(get(&md->chain, k.slots)); TRY(get(&md->mid, 6 * k.slots));
+    TRY(get(&md->blk_rep, k.nblk)); TRY(get(&md->blk_first, k.nblk)); TRY(get(&md->blk_idx, k.nblk));
+    TRY(get(&md->blkd, k.nblk)); TRY(get(&md->fblk, k.fnblk));
+    TRY(get(&md->lblk_rep, k.lnblk)); TRY(get(&md->lblk_first, k.lnblk));
+    TRY(get(&md->wl_item, k.nblk + k.lnblk + k.ncb)); TRY(get(&md->wl_n, (size_t)4));
+    TRY(get(&md->ranges, k.cells * NRANGE)); TRY(get(&md->xmid, k.cells));
+    TRY(get(&md->cblk_rep, k.cells)); TRY(get(&md->cblk_cell, k.cells));
+    TRY(get(&md->cell_mem, k.cells * CELL_CAP)); TRY(get(&md->cnt, k.cells)); TRY(get(&md->start, k.cells));
+    TRY(get(&md->partial, 4 * k.fnblk)); TRY(get(&md->gpart, 4 * k.fnblk)); TRY(get(&md->gdone, k.fnblk));
+    TRY(get(&md->rdone, k.slots * DONE_PAD)); TRY(get(&md->bdone, k.slots * DONE_PAD));
+    if (k.enblk) { TRY(get(&md->eblk, k.enblk)); TRY(get(&md->epart, 2 * k.enblk)); }
+    for (double **q : {&md->fx, &md->fy, &md->fz, &md->xo, &md->yo, &md->zo}) TRY(get(q, k.n));
+    TRY(get(&md->pos4, k.n)); TRY(get(&md->posq, k.n));
+    TRY(get(&md->nn, k.n)); TRY(get(&md->nn_ref, k.n)); TRY(get(&md->nl, md->cap * k.n)); TRY(get(&md->members, k.n));
+    TRY(get(&md->kx, k.n)); TRY(get(&md->ky, k.n)); TRY(get(&md->kz, k.n));  // n_act is n at most
+    TRY(each_part(md->P, k.n, get)); TRY(each_part(md->A, k.n, get));
+    return get(&md->ftab, (size_t)2 * PART_FIELDS);
+}
+// those of the reference-order export and of the overlap accumulators
+template <class F>
+static int each_export_array(ac4_md *md, size_t n, F get) {
+    TRY(get(&md->ex, n)); TRY(get(&md->ey, n)); TRY(get(&md->ez, n));
+    return get(&md->et, n);
+}
+template <class F>
+static int each_overlap_array(ac4_md *md, size_t slots, size_t n, size_t n_origin, size_t n_lags, F get) {
+    for (double **q : {&md->ox, &md->oy, &md->oz}) TRY(get(q, n * n_origin));
+    TRY(get(&md->ov_q, slots * (n_lags + 1))); TRY(get(&md->ov_q2, slots * (n_lags + 1)));
+    TRY(get(&md->ov_n, slots * (n_lags + 1)));
+    TRY(get(&md->ov_cnt, slots * n_origin)); TRY(get(&md->ov_step, slots * n_origin));
+    TRY(get(&md->ov_list, slots));
+    return get(&md->ov_out, 3 * (n_lags + 1));
+}
+static const auto alloc_array = [](auto **p, size_t n) { return dalloc(p, n); };
+
 static void free_parts(PartArrays &a) {
     void *q[] = {a.x, a.y, a.z, a.xu, a.yu, a.zu, a.px, a.py, a.pz, a.type, a.act, a.id, a.cell_ref, a.cell_of};
     for (void *v : q)
@@ -2262,6 +2304,9 @@ static void fresh_chain(ChainS &c, const RepC &R) {
     c.force_rebuild = R.n > 0 ? 1 : 0;
 }
 
+// cells a slot of capacity cn can hold: those of the least dense box (rho 0.5)
+static int slot_cells(int cn) { return (int)pow((int)(pow((double)cn / 0.5, 1.0 / 3.0) / K_CELL_CUT) + 1, 3); }
+
 // cap_rule > 0: the automatic force team width is taken for that total
 // capacity instead of the handle's own (a server's launch groups share one
 // kernel shape, so a job's arithmetic does not depend on its group)
@@ -2320,8 +2365,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         R.off = off;
         R.off_act = off_act;
         R.off_cell = off_cell;
-        // the densest box a slot can hold sets its cell capacity (rho >= 0.5)
-        const int cap_cells = (int)pow((int)(pow((double)cn / 0.5, 1.0 / 3.0) / K_CELL_CUT) + 1, 3);
+        const int cap_cells = slot_cells(cn);
         R.cap_cells = cap_cells;
         R.tpp = tpp;
         R.ltpp = ltpp;
@@ -2384,22 +2428,9 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     }
     job_rules(md);
     int rc = AC4_OK;
-#define ALLOC(ptr, n) if ((rc = dalloc(&md->ptr, (size_t)(n))) != AC4_OK) { ac4_md_destroy(md); return rc; }
-    if (md->shuf_bmax > 0) {
-        ALLOC(shuf_ent, (size_t)nslots * 3 * md->shuf_bmax * 2 * SHUF_M)
-        ALLOC(shuf_ent_n, (size_t)nslots * 3 * md->shuf_bmax)
-    }
-    ALLOC(reps, nslots) ALLOC(chain, nslots) ALLOC(blk_rep, md->nblk) ALLOC(blk_first, md->nblk) ALLOC(blk_idx, md->nblk)
-    ALLOC(blkd, md->nblk) ALLOC(fblk, md->fnblk) ALLOC(lblk_rep, md->lnblk) ALLOC(lblk_first, md->lnblk)
-    ALLOC(wl_item, (size_t)md->nblk + md->lnblk + md->ncb) ALLOC(wl_n, 4) ALLOC(ranges, (size_t)off_cell * NRANGE) ALLOC(xmid, off_cell) ALLOC(cblk_rep, off_cell) ALLOC(cblk_cell, off_cell) ALLOC(partial, 4 * (size_t)md->fnblk) ALLOC(mid, 6 * (size_t)nslots)
-    ALLOC(gpart, 4 * (size_t)md->fnblk) ALLOC(gdone, md->fnblk) ALLOC(rdone, (size_t)nslots * DONE_PAD)
-    ALLOC(bdone, (size_t)nslots * DONE_PAD)
-    if (md->en_apart) { ALLOC(eblk, md->enblk) ALLOC(epart, 2 * (size_t)md->enblk) }
-    ALLOC(fx, off) ALLOC(fy, off) ALLOC(fz, off) ALLOC(xo, off) ALLOC(yo, off) ALLOC(zo, off) ALLOC(pos4, off) ALLOC(posq, off)
-    ALLOC(cell_mem, (size_t)off_cell * CELL_CAP) ALLOC(nn, off) ALLOC(nn_ref, off) ALLOC(nl, (size_t)md->cap * off) ALLOC(cnt, off_cell) ALLOC(start, off_cell)
-    ALLOC(members, off) ALLOC(kx, off_act) ALLOC(ky, off_act) ALLOC(kz, off_act)
-#undef ALLOC
-    if ((rc = alloc_parts(md->P, off)) != AC4_OK || (rc = alloc_parts(md->A, off)) != AC4_OK) { ac4_md_destroy(md); return rc; }
+    const SlotCounts counts{(size_t)nslots, (size_t)off, (size_t)off_cell, (size_t)md->nblk, (size_t)md->fnblk,
+                            (size_t)md->lnblk, (size_t)md->ncb, (size_t)md->enblk, (size_t)nslots * 3 * md->shuf_bmax};
+    if ((rc = each_array(md, counts, alloc_array)) != AC4_OK) { ac4_md_destroy(md); return rc; }
     {
         void *tab[2 * PART_FIELDS];
         for (int k = 0; k < 2; k++) {
@@ -2408,7 +2439,6 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
                                     a.type, a.act, a.id, a.cell_ref, a.cell_of};
             for (int q = 0; q < PART_FIELDS; q++) tab[k * PART_FIELDS + q] = f[q];
         }
-        if ((rc = dalloc(&md->ftab, 2 * PART_FIELDS)) != AC4_OK) { ac4_md_destroy(md); return rc; }
         if (hipMemcpy(md->ftab, tab, sizeof tab, hipMemcpyHostToDevice) != hipSuccess) {
             ac4_md_destroy(md);
             ac4_set_error("ac4_md_create: field table upload failed");
@@ -2583,27 +2613,26 @@ extern "C" int ac4_md_destroy(ac4_md *md) {
 
 extern "C" int ac4_md_total_particles(const ac4_md *md) { return md ? md->ntot : 0; }
 
-// Device bytes a slot of capacity cap_n adds to a handle, from the sizes
-// ac4_md_create_slots and ac4_md_overlap_enable allocate (the reference-order
-// export buffers included; the parallel-shuffle tables counted at their
-// largest, as if this slot were the largest of its handle).
+// Device bytes a slot of capacity cap_n adds to a handle: the arrays
+// ac4_md_create_slots and ac4_md_overlap_enable allocate and the
+// reference-order export's, the force blocks counted at the widest team (16
+// lanes a particle), the energy pass as if the handle had one and the
+// parallel-shuffle tables at their largest, as if this slot were the largest
+// of its handle.
 extern "C" long long ac4_md_slot_bytes(int cap_n, int n_origin, int n_lags) {
     if (cap_n < 2 || n_origin < 0 || n_lags < 0) return AC4_EARG;
-    const long long n = cap_n;
-    const long long cells = (long long)pow((int)(pow((double)cap_n / 0.5, 1.0 / 3.0) / K_CELL_CUT) + 1, 3);
-    const long long nblk = (n + BLK - 1) / BLK, lnblk = (n + LPB - 1) / LPB;
-    const long long fnb = (n * 16 + BLK - 1) / BLK;  // force blocks at the widest team (16 lanes a particle)
-    const long long ncb = (cells + BLK / 64 - 1) / (BLK / 64);
+    const size_t n = cap_n, cells = slot_cells(cap_n), fnb = (n * 16 + BLK - 1) / BLK;
+    const SlotCounts k{1, n, cells, (n + BLK - 1) / BLK, fnb, (n + LPB - 1) / LPB, (cells + BLK / 64 - 1) / (BLK / 64), fnb,
+                       cap_n > SHUF_PAR_MIN ? 3 * ((n + SHUF_M - 1) / SHUF_M) : 0};
+    ac4_md md;  // for the arrays' types
     long long b = 0;
-    b += n * (6 * 8 + 32 + 12 + 2 * 4 + 192LL * 4 + 4 + 3);         // forces, xold, pos copies, counts, list, members, k
-    b += 2 * n * (9 * 8 + 5 * 4);                                    // particle arrays and their scratch copy
-    b += n * (3 * 8 + 4);                                            // reference-order export
-    b += cells * ((long long)NRANGE * 8 + 3 * 4 + (long long)CELL_CAP * 8 + 2 * 4);
-    b += nblk * (3 * 4 + 16) + fnb * (2 * 16 + 16) + lnblk * 2 * 4;  // block tables, energy partials
-    b += (nblk + lnblk + ncb) * 4 + fnb * 4 * 8;                     // work list, force partials
-    b += (long long)sizeof(RepC) + (long long)sizeof(ChainS) + 6 * 8;
-    if (cap_n > SHUF_PAR_MIN) b += 3LL * 2 * ((n + SHUF_M - 1) / SHUF_M) * SHUF_M * 4 + 3LL * ((n + SHUF_M - 1) / SHUF_M) * 4;
-    if (n_origin > 0) b += n * 24LL * n_origin + (long long)n_origin * 12 + (long long)(n_lags + 1) * 20;
+    const auto add = [&](auto **p, size_t count) {
+        b += (long long)(sizeof(**p) * count);
+        return AC4_OK;
+    };
+    (void)each_array(&md, k, add);
+    (void)each_export_array(&md, n, add);
+    if (n_origin > 0) (void)each_overlap_array(&md, 1, n, n_origin, n_lags, add);
     return b;
 }
 
@@ -3566,8 +3595,7 @@ extern "C" int ac4_philox4x32(const uint32_t *ctr4, const uint32_t *key2, uint32
 extern "C" int ac4_md_export_all(ac4_md *md, double *xu, double *yu, double *zu) {
     AC4_REQUIRE(md && xu && yu && zu, AC4_EARG, "export_all: bad arguments");
     if (!md->ex) {
-        TRY(dalloc(&md->ex, md->ntot)); TRY(dalloc(&md->ey, md->ntot)); TRY(dalloc(&md->ez, md->ntot));
-        TRY(dalloc(&md->et, md->ntot));
+        TRY(each_export_array(md, md->ntot, alloc_array));
     }
     hipLaunchKernelGGL(k_export, dim3(md->nblk), dim3(BLK), 0, md->stream, md->reps, md->blk_rep, md->blk_first,
                        md->P.id, md->P.xu, md->P.yu, md->P.zu, md->P.type, md->ex, md->ey, md->ez, md->et, -1);
@@ -3586,13 +3614,7 @@ extern "C" int ac4_md_overlap_enable(ac4_md *md, int sample_every, int origin_ev
                 AC4_EARG, "overlap_enable: bad arguments (origin_every must be a multiple of sample_every)");
     AC4_REQUIRE(!md->ox, AC4_ESTATE, "overlap accumulators already enabled");
     md->ov = OvCfg{sample_every, origin_every, n_origin, n_lags, a * a};
-    const size_t snap = (size_t)md->ntot * n_origin, acc = (size_t)md->R * (n_lags + 1);
-    TRY(dalloc(&md->ox, snap)); TRY(dalloc(&md->oy, snap)); TRY(dalloc(&md->oz, snap));
-    TRY(dalloc(&md->ov_q, acc)); TRY(dalloc(&md->ov_q2, acc)); TRY(dalloc(&md->ov_n, acc));
-    TRY(dalloc(&md->ov_cnt, (size_t)md->R * n_origin));
-    TRY(dalloc(&md->ov_step, (size_t)md->R * n_origin));
-    TRY(dalloc(&md->ov_list, (size_t)md->R));
-    TRY(dalloc(&md->ov_out, 3 * (size_t)(n_lags + 1)));
+    TRY(each_overlap_array(md, md->R, md->ntot, n_origin, n_lags, alloc_array));
     std::vector<long long> none((size_t)md->R * n_origin, -1);
     AC4_HIP(hipMemcpy(md->ov_step, none.data(), sizeof(long long) * none.size(), hipMemcpyHostToDevice));
     return AC4_OK;
@@ -3666,8 +3688,7 @@ extern "C" int ac4_md_device_xu(ac4_md *md, int r, const double **xu, const doub
                                 const int **type, int *n) {
     TRY(check_rep(md, r));
     if (!md->ex) {
-        TRY(dalloc(&md->ex, md->ntot)); TRY(dalloc(&md->ey, md->ntot)); TRY(dalloc(&md->ez, md->ntot));
-        TRY(dalloc(&md->et, md->ntot));
+        TRY(each_export_array(md, md->ntot, alloc_array));
     }
     hipLaunchKernelGGL(k_export, dim3(md->nblk), dim3(BLK), 0, md->stream, md->reps, md->blk_rep, md->blk_first,
                        md->P.id, md->P.xu, md->P.yu, md->P.zu, md->P.type, md->ex, md->ey, md->ez, md->et, r);

@@ -593,3 +593,30 @@ def test_device_push_of_other_memory(gpu, n, obs, where):
     hip.hipHostFree(pin)
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# What a handle takes of the device's memory is what ac4_md_slot_bytes says of
+# its slots, which the server plans with: the largest slots at the widest team,
+# where every block table has its full size.
+def test_slot_bytes_cover_the_handle(gpu):
+    hip = ctypes.CDLL("libamdhip64.so")  # the runtime the library has loaded
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    caps = [1 << 21] * 4
+    gpu.set_tuning(16)
+    try:
+        for c in ([1000], caps):  # the first loads the code and what else the runtime keeps
+            h, f0 = ctypes.c_void_p(), free()
+            assert gpu.lib.ac4_md_create_slots(len(c), (ctypes.c_int * len(c))(*c), 0, ctypes.byref(h)) == 0
+            used = f0 - free()
+            assert gpu.lib.ac4_md_destroy(h) == 0
+    finally:
+        gpu.set_tuning()
+    # the export's arrays are allocated when first used; each of about 70
+    # arrays is rounded up to 2 MiB at most
+    want = sum(gpu.slot_bytes(c) for c in caps) - 28 * sum(caps)
+    assert used <= want + 70 * (2 << 20), (used, want)
