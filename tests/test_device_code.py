@@ -6,8 +6,9 @@ agent-scope release/acquire ordering) compiles on gfx950 to a write-back and
 an invalidation of the XCD's L2 (``buffer_wbl2`` / ``buffer_inv``).  Issued by
 every workgroup of the force kernel it cost the neighbour gathers of all the
 other workgroups their L2 lines (k_force 42.7 against 55.8 us on the
-64-replica ensemble without it), so the per-replica reductions run as kernels
-of their own; this test keeps such instructions out of every kernel."""
+64-replica ensemble without it), so what workgroups hand over inside a kernel
+goes through relaxed agent-scope stores and loads; this test keeps such
+instructions out of every kernel."""
 import os
 import shutil
 import subprocess

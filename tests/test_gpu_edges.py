@@ -69,8 +69,8 @@ def test_shell_runs_against_direct_sums(gpu, n, npairs, nshell, ndir):
     assert np.allclose(s4d, want, rtol=1e-9, atol=1e-9 * (ph ** 2).max() / n)
 
 
-# One size in each range of the automatic force team (16, 8, 4 and 2 lanes,
-# with the list layouts of 16, 8, 4, 2 and one nominal lanes) against one
+# Sizes of the automatic force team of 16 and of 4 lanes (those of 8 lanes
+# below), with the list layouts of 16, 8, 4 and one nominal lanes, against one
 # pinned lane: the same pair terms, summed in FP64 in another order.
 @pytest.mark.parametrize("prec,n", [(0, 700), (0, 6000), (0, 9001), (0, 14001), (0, 33001), (1, 700), (1, 6000),
                                     (1, 9001), (1, 14001), (1, 33001), (1, 160001)])
@@ -94,6 +94,14 @@ def test_force_team_widths(gpu, prec, n):
     assert np.abs(fa - fb).max() <= 4e-12 * np.sqrt((fb ** 2).mean())
     # energy and virial: FP32 partial sums of eight pairs in FP32 mode
     assert np.allclose(pa, pb, rtol=1e-11 if prec == 0 else 1e-6)
+
+
+# The team of 8 lanes, on the list layout of two: the range's edges and a size
+# between them.
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [16385, 20000, 32768])
+def test_force_team_of_eight_lanes(gpu, prec, n):
+    test_force_team_widths(gpu, prec, n)
 
 
 # What the last workgroups of the force pass and of the binning do for a whole
