@@ -26,7 +26,7 @@
 #define ABLK 256
 #define A_PI 3.14159265358979 // Analysis/global.h:14
 
-__constant__ int c_vx[AC4_NQ], c_vy[AC4_NQ], c_vz[AC4_NQ], c_dg[AC4_NQ];
+__constant__ int c_dg[AC4_NQ];  // permutations of each GetQ vector
 
 struct Job {       // one (origin, lag) pair evaluated against the pushed frame
     int org;       // the origin's place among the resident frames
@@ -1115,9 +1115,6 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     int rc = AC4_OK;
     auto fail = [&](int e) { ac4_ana_destroy(an); return e; };
     if (hipGetDevice(&an->dev) != hipSuccess || hipStreamCreate(&an->stream) != hipSuccess) return fail(AC4_EHIP);
-    AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vx), an->vx.data(), sizeof(int) * AC4_NQ));
-    AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vy), an->vy.data(), sizeof(int) * AC4_NQ));
-    AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_vz), an->vz.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_dg), dg.data(), sizeof(int) * AC4_NQ));
     if ((rc = set_columns(an, dg)) != AC4_OK) return fail(rc);
     // blocks of a frame row: one tile of the block's threads each up to 256 of them, then more tiles per block

@@ -223,7 +223,7 @@ __device__ __forceinline__ bool last_done(unsigned *count, int of) {
 }
 
 // Rebuild work of one step: the blocks of the replicas due for a rebuild,
-// appended by k_bin_end for each such replica, so the kernels after
+// appended by bin_end for each such replica, so the kernels after
 // k_bin run a fixed grid over this list instead of one workgroup per block of
 // every replica (most of which would have nothing to do).  n[0]: particle
 // blocks of BLK (global block ids); n[1]: list blocks of LPB particles
@@ -2071,12 +2071,10 @@ struct ac4_md {
     std::vector<int> t_brep, t_bfirst, t_bidx, t_ffirst, t_lrep, t_lfirst, t_b0, t_f0, t_l0;
     int *ov_list = nullptr;     // replica list of ac4_md_overlap_chi4
     double *ov_out = nullptr;   // its per-lag results
-    // frame text on the device (ac4_md_format_frame): 80-byte line slots in
-    // reference order, line lengths, the joined text, per-block byte offsets
-    // (the total after the last block) and a flag
-    // frame text: a slot of 80 bytes per line and its length, the bytes of each
-    // block of lines, and in pinned memory two pieces of the joined text (one
-    // for a frame of one piece) and the words k_fmt_* leave for the host
+    // frame text (ac4_md_format_frame): a slot of 80 bytes per line in
+    // reference order and its length, the bytes of each block of lines, and in
+    // pinned memory two pieces of the joined text (one for a frame of one
+    // piece) and the words k_fmt_* leave for the host
     char *fmt_dev = nullptr, *fmt_txt = nullptr;
     unsigned char *fmt_len_dev = nullptr;
     int *fmt_bsum = nullptr;
@@ -2341,7 +2339,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     }
     while ((1 << ltpp) < tpp) ltpp++;
     // lanes per particle in the force kernel: the pinned width, else by the
-    // handle's total capacity (FORCE_W)
+    // handle's total capacity
     const int W = g_tpp ? tpp : std::max(tpp > 1 ? tpp : 1, force_width(cap_tot));
     while ((1 << md->lw) < W) md->lw++;
     md->en_apart = precision == AC4_FP32 && W != tpp;
@@ -3091,7 +3089,11 @@ extern "C" long long ac4_md_format_frame(ac4_md *md, int r, char *out, long long
     // copy from the device to the caller's pageable memory takes 90 us for the
     // 1.55 MB of 50000 lines, this way 27 over the bus and 18 by memcpy; the
     // whole call 142 -> 82 us (the two small results alone, copied to pageable
-    // memory, took 20 of it)
+    // memory, took 20 of it).  Pages of the pinned pieces cost the host 1.6 us
+    // each when it first reads them, in a handle's first frame: 100000 lines
+    // 0.34 -> 0.93 ms, then 218 -> 142 us a frame (200000: 0.54 -> 1.11 ms, 376
+    // -> 226 us).  Pieces of a half and a quarter of the size: 0.62 and 0.51 ms,
+    // but 154 and 204 us (271 and 365).
     const auto pack = [&](int p) {
         const int b0 = p * FMT_PIECE;
         hipLaunchKernelGGL(k_fmt_pack, dim3(std::min(FMT_PIECE, nb - b0)), dim3(BLK), 0, s, n, b0, md->fmt_dev,
