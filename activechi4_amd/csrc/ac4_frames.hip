@@ -49,6 +49,7 @@ extern "C" int ac4_md_device_xu(ac4_md *md, int r, const double **xu, const doub
 #define SHELL_RUN 27   // shells of a run: the middle one and SHELL_H on either side
 #define SHELL_H 13
 #define PH_THREADS 512 // threads of k_fr_phase and particles of its tile
+#define FOLD_SEQ 8     // teams folded one after the other
 #define FR_BLOCKS 256  // its workgroups of one launch: one per CU
 #define FR_PAIRS 32    // pairs of one launch, at most
 
@@ -208,16 +209,23 @@ __global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restric
             }
         }
     }
-    // the shells' sums from the products, folded over the teams in team order
+    // the shells' sums from the products, folded over the teams: in team order
+    // up to FOLD_SEQ teams, else in two rounds, the first F teams every F-th
+    // one's, then team 0 theirs (one shell and direction, 512 teams: in team
+    // order the fold alone took 300 us)
     double *o = part + (size_t)blockIdx.x * ndir * nshell * 2;
     int te = t;
     asm volatile("" : "+v"(te));  // the role again, not kept in registers over the loop
-    const int role = te % T, d = role / nrole, g0 = (role - d * nrole) * NG;
+    const int role = te % T, d = role / nrole, g0 = (role - d * nrole) * NG, tm = te / T;
+    int F = 1;
+    if (S > FOLD_SEQ)
+        while (F * F < S) F++;
 #pragma unroll
     for (int u = 0; u < NG; u++) {
         const int kc = (g0 + u) * SHELL_RUN + SHELL_H;
 #pragma unroll
         for (int h = 0; h <= SHELL_H; h++) {
+            if (u * SHELL_RUN + SHELL_H - h >= nshell) continue;  // no role has either shell
             // shells kc + h and kc - h: {C+, S+, C-, S-} (h = 0: the first two)
             double v[4];
             if (h == 0) {
@@ -233,12 +241,22 @@ __global__ void __launch_bounds__(PH_THREADS) k_fr_phase(const double *__restric
 #pragma unroll
                 for (int q = 0; q < 4; q++) s_f[q * PH_THREADS + t] = v[q];
                 __syncthreads();
-                if (team == 0)
-                    for (int w = 1; w < S; w++)
+                if (F > 1) {
+                    if (tm < F)
+                        for (int w = tm + F; w < S; w += F)
+#pragma unroll
+                            for (int q = 0; q < 4; q++) v[q] += s_f[q * PH_THREADS + w * T + role];
+                    __syncthreads();
+#pragma unroll
+                    for (int q = 0; q < 4; q++) s_f[q * PH_THREADS + t] = v[q];
+                    __syncthreads();
+                }
+                if (tm == 0)
+                    for (int w = 1; w < (F > 1 ? F : S); w++)
 #pragma unroll
                         for (int q = 0; q < 4; q++) v[q] += s_f[q * PH_THREADS + w * T + role];
             }
-            if (team == 0) {
+            if (tm == 0) {
                 const int kp = kc + h, km = kc - h;
                 if (kp < nshell) {
                     o[2 * ((size_t)d * nshell + kp)] = v[0];

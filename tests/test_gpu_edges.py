@@ -69,6 +69,13 @@ def test_shell_runs_against_direct_sums(gpu, n, npairs, nshell, ndir):
     assert np.allclose(s4d, want, rtol=1e-9, atol=1e-9 * (ph ** 2).max() / n)
 
 
+# The fold over the teams, eight and nine of them and more, and part of one run
+# of shells: only the lower half of it, the middle one, one above.
+@pytest.mark.parametrize("nshell,ndir", [(1, 1), (1, 56), (13, 64), (13, 57), (14, 32), (15, 56), (27, 2), (40, 56)])
+def test_shell_teams_and_part_runs(gpu, nshell, ndir):
+    test_shell_runs_against_direct_sums(gpu, 700, 2, nshell, ndir)
+
+
 # Sizes of the automatic force team of 16 and of 4 lanes (those of 8 lanes
 # below), with the list layouts of 16, 8, 4 and one nominal lanes, against one
 # pinned lane: the same pair terms, summed in FP64 in another order.
