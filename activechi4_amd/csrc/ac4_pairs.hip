@@ -581,12 +581,15 @@ extern "C" int ac4_frames_guu(ac4_frames *f, const int *act_tag, int gap, double
     const size_t per = sizeof(double) * GU_REC * (size_t)std::max(na, 1);
     const int batch = (int)std::max<size_t>(1, std::min<size_t>(std::max(on, 1), std::min<size_t>(GU_BATCH / per, 65535)));
     // the persistent grid: the workgroups that are resident together
-    // (160 KB of LDS per CU, at most two of sixteen waves); a box of less than
+    // (160 KB of LDS per CU, at most two of sixteen waves), no more than a
+    // batch has tiles; a box of less than
     // two bins' length has no bins and no LDS
     int dev = 0, ncu = 256;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) ncu = 256;
-    const int grid = ncu * (int)std::max<size_t>(1, std::min<size_t>(2, 163840 / std::max<size_t>(lds, 1)));
+    const long long items = std::max<long long>(1, std::min<long long>((long long)ntri * batch, 2147483647LL));
+    const int grid = (int)std::min<long long>(
+        items, ncu * (long long)std::max<size_t>(1, std::min<size_t>(2, 163840 / std::max<size_t>(lds, 1))));
     const int dblk = (na + PR_THREADS - 1) / PR_THREADS;
     // one allocation: act and fo (one copy in), the totals and k_gu_disp's
     // sums (one copy out), then the batch's records and the partial histograms
