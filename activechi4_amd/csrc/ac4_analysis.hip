@@ -886,7 +886,7 @@ struct ac4_ana {
     double *d_part = nullptr, *d_msdp = nullptr;
     int *d_ovp = nullptr, *d_s4p = nullptr;  // per block: overlap counts of the overlap and the S4 rule
     Job *d_jobs = nullptr;
-    unsigned *d_read = nullptr, *h_read = nullptr, seq = 0;  // Frame::count, ::word (pinned), ::seq
+    unsigned *d_read = nullptr, *h_read = nullptr, seq = 0;  // Frame::count, ::word (pinned, with the first device push), ::seq
     bool stale = false;         // frames came in since d_msd, d_ov and d_s4m were formed from the blocks' values
     // S4 by origin: pair ids per origin (CSR, walk order), origins whose
     // last lag is frame pos, the pairs' overlap masks and the chunk partials
@@ -901,6 +901,7 @@ struct ac4_ana {
     int max_jobs = 0, ppb = ABLK, nb = 0, fs_ppb = FS_P, fs_nb = 0;
     std::vector<int> vx, vy, vz, qsq;
     std::vector<double> qval;
+    char *mem = nullptr;        // all of them
     hipStream_t stream = nullptr;
     int dev = 0;                // the device the handle was made on
     bool finalized = false;
@@ -1003,9 +1004,9 @@ static int set_columns(ac4_ana *an, const std::vector<int> &dg) {
     return AC4_OK;
 }
 
-// S4 by origin: the per-origin pair lists and the device buffers.  Masks and sums start at zero, so a pair whose lag
-// frame never arrives contributes nothing.
-static int s4_setup(ac4_ana *an) {
+// S4 by origin: the per-origin pair lists and the sizes.  Returns the number of
+// chunk partials of a pass.
+static size_t s4_setup(ac4_ana *an) {
     const ac4_walk_t &w = an->W[1].w;
     an->s4_optr.assign(an->nframes + 1, 0);
     for (int p = 0; p < w.np; p++) an->s4_optr[w.cur[p] + 1]++;
@@ -1029,14 +1030,7 @@ static int s4_setup(ac4_ana *an) {
         an->s4_nchunk = (an->nwords + 4 * an->s4_wpw - 1) / (4 * an->s4_wpw);
         part = (size_t)an->s4_nchunk * S4_LAGS * 2 * S4_NCOL;
     }
-    const size_t np1 = std::max(w.np, 1);
-    AC4_HIP(hipMalloc(&an->d_s4_opairs, sizeof(int) * np1));
-    AC4_HIP(hipMemcpy(an->d_s4_opairs, an->s4_opairs.data(), sizeof(int) * np1, hipMemcpyHostToDevice));
-    AC4_HIP(hipMalloc(&an->d_s4mask, sizeof(unsigned) * np1 * an->nwords));
-    AC4_HIP(hipMalloc(&an->d_s4part, sizeof(double) * part));
-    AC4_HIP(hipMemset(an->d_s4mask, 0, sizeof(unsigned) * np1 * an->nwords));
-    AC4_HIP(hipMemset(an->d_s4, 0, sizeof(double) * 2 * AC4_NQ * np1));
-    return AC4_OK;
+    return part;
 }
 
 // The S4 sums of every pair of origin o, from its resident frame and the
@@ -1125,33 +1119,59 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     an->fs_nb = (n + an->fs_ppb - 1) / an->fs_ppb;
     an->max_jobs = std::max(an->max_jobs, 1);
     const size_t np0 = std::max(an->W[0].w.np, 1), np1 = std::max(an->W[1].w.np, 1);
+    // one allocation, the zeroed arrays first: masks and sums start at zero, so
+    // that a pair whose lag frame never arrives contributes nothing (1000
+    // particles, all four observables, an allocation and a fill for each array:
+    // 353 us to create and destroy, this 200)
+    struct Array {
+        void **p;
+        size_t bytes;
+    };
+    std::vector<Array> arrays[2];  // zeroed, not zeroed
     auto get = [&](auto **p, size_t count, bool zero) {
-        if (hipMalloc((void **)p, sizeof(**p) * count) != hipSuccess) return false;
-        return !zero || hipMemset(*p, 0, sizeof(**p) * count) == hipSuccess;
+        arrays[zero ? 0 : 1].push_back({(void **)p, (sizeof(**p) * count + 255) & ~(size_t)255});
     };
     an->org.n = (size_t)n;
-    if (!get(&an->d_jobs, std::max<size_t>(an->jobs.size(), 1), false)) return fail(AC4_EHIP);
+    get(&an->d_jobs, std::max<size_t>(an->jobs.size(), 1), false);
+    get(&an->org.f, (size_t)3 * n * std::max(places, 1), false);
+    const int wgs = an->max_jobs * (an->fs_nb + an->nb) + an->nb;  // workgroups of a frame, at most
+    get(&an->d_read, (size_t)(2 + wgs / READ_GRP) * READ_PAD, true);
+    get(&an->cur, (size_t)3 * n, false);
+    get(&an->cur_t, n, false);
+    if (obs & AC4_OBS_MSD) { get(&an->d_msd, 3 * np0, true); get(&an->d_msdp, 3 * np0 * an->nb, true); }
+    if (obs & AC4_OBS_OVERLAP) { get(&an->d_ov, np1, true); get(&an->d_ovp, np1 * an->nb, true); }
+    if (obs & AC4_OBS_FS) {
+        an->fs_wait = std::max(an->max_jobs, FS_WAIT);
+        get(&an->d_fs, 2 * AC4_NQ * np1, true);
+        get(&an->d_part, (size_t)an->fs_wait * an->fs_nb * AC4_NQ * 2, false);
+    }
+    if (obs & AC4_OBS_S4) {
+        const size_t part = s4_setup(an);
+        get(&an->d_s4, 2 * AC4_NQ * np1, true);
+        get(&an->d_s4m, np1, true);
+        get(&an->d_s4p, np1 * an->nb, true);
+        get(&an->d_s4mask, np1 * an->nwords, true);
+        get(&an->d_s4_opairs, np1, false);
+        get(&an->d_s4part, part, false);
+    }
+    size_t bytes[2] = {0, 0};
+    for (int k = 0; k < 2; k++)
+        for (const Array &v : arrays[k]) bytes[k] += v.bytes;
+    if (hipMalloc((void **)&an->mem, bytes[0] + bytes[1]) != hipSuccess) {
+        ac4_set_error("ac4_ana_create: cannot allocate %zu bytes", bytes[0] + bytes[1]);
+        return fail(AC4_EHIP);
+    }
+    char *at = an->mem;
+    for (int k = 0; k < 2; k++)
+        for (const Array &v : arrays[k]) {
+            *v.p = at;
+            at += v.bytes;
+        }
+    if (hipMemset(an->mem, 0, bytes[0]) != hipSuccess) return fail(AC4_EHIP);
     if (!an->jobs.empty() && hipMemcpy(an->d_jobs, an->jobs.data(), sizeof(Job) * an->jobs.size(),
                                        hipMemcpyHostToDevice) != hipSuccess) return fail(AC4_EHIP);
-    if (!get(&an->org.f, (size_t)3 * n * std::max(places, 1), false)) return fail(AC4_EHIP);
-    const int wgs = an->max_jobs * (an->fs_nb + an->nb) + an->nb;  // workgroups of a frame, at most
-    if (!get(&an->d_read, (size_t)(2 + wgs / READ_GRP) * READ_PAD, true)) return fail(AC4_EHIP);
-    if (hipHostMalloc((void **)&an->h_read, 64, hipHostMallocDefault) != hipSuccess) return fail(AC4_EHIP);
-    *an->h_read = 0;
-    if (!get(&an->cur, (size_t)3 * n, false) || !get(&an->cur_t, n, false)) return fail(AC4_EHIP);
-    if (obs & AC4_OBS_MSD)
-        if (!get(&an->d_msd, 3 * np0, true) || !get(&an->d_msdp, 3 * np0 * an->nb, true)) return fail(AC4_EHIP);
-    if (obs & AC4_OBS_OVERLAP)
-        if (!get(&an->d_ov, np1, true) || !get(&an->d_ovp, np1 * an->nb, true)) return fail(AC4_EHIP);
-    if (obs & AC4_OBS_FS)
-        if (!get(&an->d_fs, 2 * AC4_NQ * np1, true) ||
-            !get(&an->d_part, (size_t)(an->fs_wait = std::max(an->max_jobs, FS_WAIT)) * an->fs_nb * AC4_NQ * 2, false))
-            return fail(AC4_EHIP);
-    if (obs & AC4_OBS_S4) {
-        if (hipMalloc(&an->d_s4, sizeof(double) * 2 * AC4_NQ * (size_t)np1) != hipSuccess) return fail(AC4_EHIP);
-        if (!get(&an->d_s4m, np1, true) || !get(&an->d_s4p, np1 * an->nb, true)) return fail(AC4_EHIP);
-        if ((rc = s4_setup(an)) != AC4_OK) return fail(rc);
-    }
+    if ((obs & AC4_OBS_S4) && hipMemcpy(an->d_s4_opairs, an->s4_opairs.data(), sizeof(int) * np1,
+                                        hipMemcpyHostToDevice) != hipSuccess) return fail(AC4_EHIP);
     *out = an;
     return AC4_OK;
 }
@@ -1159,11 +1179,7 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
 extern "C" int ac4_ana_destroy(ac4_ana *an) {
     if (!an) return AC4_OK;
     if (an->stream) (void)hipStreamSynchronize(an->stream);
-    void *ptrs[] = {an->org.f, an->cur, an->cur_t, an->d_msd, an->d_msdp, an->d_ov, an->d_ovp, an->d_s4, an->d_s4m, an->d_s4p,
-                    an->d_fs, an->d_part, an->d_jobs, an->d_read,
-                    an->d_s4_opairs, an->d_s4mask, an->d_s4part};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    if (an->mem) (void)hipFree(an->mem);
     if (an->h_read) (void)hipHostFree(an->h_read);
     for (auto &W : an->W) ac4_walk_free(&W.w);
     if (an->stream) (void)hipStreamDestroy(an->stream);
@@ -1270,6 +1286,10 @@ static int push_common(ac4_ana *an, int pos, const double *x, const double *y, c
         AC4_HIP(hipMemcpyAsync(an->cur_t, t, sizeof(int) * n, kind, s));
         x = dx; y = dy; z = dz; t = an->cur_t;
         keep = -1;
+    }
+    if (!copy && !an->h_read) {  // 30 us; host pushes do without it
+        AC4_HIP(hipHostMalloc((void **)&an->h_read, 64, hipHostMallocDefault));
+        *an->h_read = 0;
     }
     an->resident[pos] = an->place[pos] >= 0;
     TRY(process_frame(an, pos, x, y, z, t, keep, !copy));  // the caller may reuse its arrays
