@@ -35,7 +35,7 @@ struct ac4_textframes {
     int *d_bcnt = nullptr, *d_boff = nullptr, *d_lend = nullptr, *d_meta = nullptr;  // meta: lines, first bad, frames, last end
     double *d_x = nullptr, *d_y = nullptr, *d_z = nullptr;
     int *d_t = nullptr;
-    int *h_meta = nullptr;              // pinned copy of meta
+    int *h_meta = nullptr;              // copy of meta, after the chunk's bytes in the pinned buffer
     int max_frames = 0;                 // frames the parsed arrays hold
     hipStream_t s = nullptr;
 };
@@ -275,7 +275,6 @@ extern "C" int ac4_textframes_destroy(ac4_textframes *t) {
     if (!t) return AC4_OK;
     if (t->s) (void)hipStreamSynchronize(t->s);
     if (t->h_text) (void)hipHostFree(t->h_text);
-    if (t->h_meta) (void)hipHostFree(t->h_meta);
     void *d[] = {t->d_text, t->d_bcnt, t->d_boff, t->d_lend, t->d_meta, t->d_x, t->d_y, t->d_z, t->d_t};
     for (void *q : d)
         if (q) (void)hipFree(q);
@@ -302,8 +301,9 @@ extern "C" int ac4_textframes_create(int n, long long chunk_bytes, ac4_textframe
     const long long nb = cap / TX_SEG, ml = (long long)t->max_frames * n;
     auto fail = [&](int e) { ac4_textframes_destroy(t); return e; };
     if (hipStreamCreate(&t->s) != hipSuccess) return fail(AC4_EHIP);
-    if (hipHostMalloc((void **)&t->h_text, (size_t)cap, hipHostMallocDefault) != hipSuccess) return fail(AC4_EHIP);
-    if (hipHostMalloc((void **)&t->h_meta, sizeof(int) * 4, hipHostMallocDefault) != hipSuccess) return fail(AC4_EHIP);
+    if (hipHostMalloc((void **)&t->h_text, (size_t)cap + sizeof(int) * 4, hipHostMallocDefault) != hipSuccess)
+        return fail(AC4_EHIP);
+    t->h_meta = (int *)(t->h_text + cap);  // cap is whole segments
     if (hipMalloc(&t->d_text, (size_t)cap) != hipSuccess || hipMalloc(&t->d_bcnt, sizeof(int) * nb) != hipSuccess ||
         hipMalloc(&t->d_boff, sizeof(int) * nb) != hipSuccess ||
         hipMalloc(&t->d_lend, sizeof(int) * (size_t)t->lines_cap) != hipSuccess ||
