@@ -1481,6 +1481,11 @@ __global__ void __launch_bounds__(BLK) k_export(const RepC *__restrict__ reps, c
 template <bool FP32>
 struct PairAcc;
 
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ double uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)), __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
 // 1/a for a normal positive a: the hardware's estimate (v_rcp_f64) and two
 // Newton steps, within an ulp; a fifth of the instructions of a division.
 __device__ __forceinline__ double rcp_newton(double a) {
@@ -1504,13 +1509,14 @@ struct PairAcc<false> {
     // error is the same for all pairs and adds up where theirs cancel.  Relative
     // error of the pair energy of displaced lattices of 1000 and 50000: with L*L
     // rounded 1.8e-15 and 1.0e-15, so 3e-17 and 1.8e-16, for one instruction of
-    // a pair (50000 particles 1.4 % of the step).
+    // a pair (50000 particles 0.3 % of the step).
     double fx = 0, fy = 0, fz = 0, pe = 0, vir = 0;
     double L2, L2r;
     double rc[2], s2c[2], e4[2], e8[2], c2i[2];  // value of species 0, difference of species 1
     __device__ __forceinline__ PairAcc(int ti, const RepC &R) {
-        L2 = R.L * R.L;
-        L2r = fma(R.L, R.L, -L2);
+        const double l2 = R.L * R.L;  // of the workgroup's replica: in scalar registers
+        L2 = uniform(l2);
+        L2r = uniform(fma(R.L, R.L, -l2));
         // (ti, tj) -> ab = ti + tj: sigma {1, 0.8, 0.88}, epsilon {1, 1.5, 0.5} (cell_list+forces.c:19-20)
         const auto pick = [ti](double v0, double v1, double v2, double (&out)[2]) {
             const double a = ti ? v1 : v0;
@@ -1676,7 +1682,7 @@ __device__ __forceinline__ void ld_list(const int *p, int *j) {
 // entries c*W ... c*W + W - 1, cs list words apart); the others read chunks
 // of 8 entries, cs words apart, with W = 8 / |VEC| lanes: VEC = 8 the whole
 // chunk, VEC = -2 entries t, t + 4 of it, two rows per chunk.  In FP64 a group
-// is six entries with VEC = -2 and four with VEC = 1: 128 and 108 vector
+// is six entries with VEC = -2 and four with VEC = 1: 126 and 106 vector
 // registers in k_force instead of 148, four waves per SIMD instead of three (us
 // per step, N=50000 50.7 -> 50.1, 80000 63.5 -> 61.4, 200000 104 -> 99.5;
 // teams of 8, N=20000 29.2 -> 28.7, 30000 34.6 -> 33.6; of 16 the same).
