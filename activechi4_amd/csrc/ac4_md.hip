@@ -56,7 +56,6 @@ struct RepC {
     double skin;    // Verlet skin: list radii 2.5 sigma_ab + skin, rebuild criterion
     float qs2;      // qscale^2 in FP32
     int xcull;      // a cell's slots are ordered by x-half, which list teams may skip (configure_rep)
-    int enblk, eblk_off;   // blocks of the energy pass (k_energy), 0 without it
     float lcut[3];         // qscreen_cut of species pair ab
     float lr2[2];          // what a particle of species a reaches in any list, squared, with a margin of 2e-3
     float rnc, cell, fix2cell;  // 1/nc, L/nc, nc/2^32
@@ -1529,9 +1528,9 @@ struct PairAcc<false> {
         pick(8.0 * 1.0, 8.0 * 1.5, 8.0 * 0.5, e8);
         pick(K_C2 / (1.00 * 1.00), K_C2 / (0.80 * 0.80), K_C2 / (0.88 * 0.88), c2i);
     }
-    template <bool EN>
+    template <int EN>
     __device__ __forceinline__ void flush() {}
-    template <bool EN>
+    template <int EN>
     __device__ __forceinline__ void add(const double4 &pi, const double4 &pj) {
         double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         dx -= rint(dx);
@@ -1591,8 +1590,9 @@ struct PairAcc<true> {
         pick(R.rcq[0], R.rcq[1], R.rcq[2], rcq);
         pick(R.c2i[0], R.c2i[1], R.c2i[2], c2i);
     }
-    template <bool EN>
-    __device__ __forceinline__ void add(const QPos &pi, const QPos &pj) {
+    // the pair's force added up; energy(species of the partner, gradient, r^2, s^6, C2/sigma^2) within the cutoff
+    template <class F>
+    __device__ __forceinline__ void pair(const QPos &pi, const QPos &pj, F energy) {
         const float dx = (float)(int)(pi.x - pj.x);
         const float dy = (float)(int)(pi.y - pj.y);
         const float dz = (float)(int)(pi.z - pj.z);
@@ -1610,13 +1610,57 @@ struct PairAcc<true> {
             fx += (double)(grad * dx);
             fy += (double)(grad * dy);
             fz += (double)(grad * dz);
-            if (EN) {
-                gpe += (b ? e4[1] : e4[0]) * __builtin_fmaf(s6, s6 - 1.0f, __builtin_fmaf(c2, r2, (float)K_C0));
-                gvir = __builtin_fmaf(grad, r2, gvir);
-            }
+            energy(b, grad, r2, s6, c2);
         }
     }
-    template <bool EN>
+    __device__ __forceinline__ float pot(bool b, float r2, float s6, float c2) const {
+        return (b ? e4[1] : e4[0]) * __builtin_fmaf(s6, s6 - 1.0f, __builtin_fmaf(c2, r2, (float)K_C0));
+    }
+    template <int EN>
+    __device__ __forceinline__ void add(const QPos &pi, const QPos &pj) {
+        pair(pi, pj, [&](bool b, float grad, float r2, float s6, float c2) {
+            if (EN) {
+                gpe += pot(b, r2, s6, c2);
+                gvir = __builtin_fmaf(grad, r2, gvir);
+            }
+        });
+    }
+    // the pair's terms of the energy and the virial (a factor each of two), zero beyond the cutoff, for chain()
+    __device__ __forceinline__ void add_terms(const QPos &pi, const QPos &pj, float &p, float &gr, float &rr) {
+        pair(pi, pj, [&](bool b, float grad, float r2, float s6, float c2) {
+            p = pot(b, r2, s6, c2);
+            gr = grad;
+            rr = r2;
+        });
+    }
+    // The terms of eight entries per lane of the team, summed as the list
+    // layout's team, RAT times narrower, sums them: its lane's entries of eight
+    // rows in order, then widened; src[k]: the lane (times 4) that has the
+    // entries of rows k, k + RAT, ...  Every lane of the team sums what its
+    // layout lane does.
+    template <int RAT, bool QUAD>
+    __device__ __forceinline__ void chain(const float (&p)[8], const float (&gr)[8], const float (&rr)[8],
+                                          const int (&src)[RAT]) {
+        const auto from = [&](float v, int k) {
+            const int i = __float_as_int(v);
+            if (!QUAD) return __int_as_float(__builtin_amdgcn_ds_bpermute(src[k], i));
+            return __int_as_float(k == 0   ? __builtin_amdgcn_update_dpp(0, i, 0x00, 0xf, 0xf, true)  // quad_perm k k k k
+                                  : k == 1 ? __builtin_amdgcn_update_dpp(0, i, 0x55, 0xf, 0xf, true)
+                                  : k == 2 ? __builtin_amdgcn_update_dpp(0, i, 0xaa, 0xf, 0xf, true)
+                                           : __builtin_amdgcn_update_dpp(0, i, 0xff, 0xf, 0xf, true));
+        };
+#pragma unroll
+        for (int j = 0; j < RAT; j++) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int u = (8 * j + i) / RAT, k = (8 * j + i) % RAT;
+                gpe += from(p[u], k);
+                gvir = __builtin_fmaf(from(gr[u], k), from(rr[u], k), gvir);
+            }
+            flush<1>();
+        }
+    }
+    template <int EN>
     __device__ __forceinline__ void flush() {
         if (EN) {
             pe += (double)gpe; vir += (double)gvir;
@@ -1686,8 +1730,10 @@ __device__ __forceinline__ void ld_list(const int *p, int *j) {
 // registers in k_force instead of 148, four waves per SIMD instead of three (us
 // per step, N=50000 50.7 -> 50.1, 80000 63.5 -> 61.4, 200000 104 -> 99.5;
 // teams of 8, N=20000 29.2 -> 28.7, 30000 34.6 -> 33.6; of 16 the same).
-template <int VEC, bool EN, class PosT, class Acc>
-__device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t, int m, int g,
+// EN = 1: the energy's FP32 terms are summed for eight entries of the lane;
+// EN = 2, 4: as the list layout's team, EN times narrower, would (2^lt lanes).
+template <int VEC, int EN, class PosT, class Acc>
+__device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int lt, int t, int m, int g,
                                           const PosT *__restrict__ pos, const PosT &pi, Acc &acc) {
     constexpr int V = VEC > 1 ? VEC : 1;    // entries of a load
     constexpr int RC = VEC < 0 ? -VEC : 1;  // rows per step of cs
@@ -1695,6 +1741,13 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
     constexpr int G = WIDE && VEC < 0 ? 6 : WIDE && VEC == 1 ? 4 : 8;  // entries of a group
     constexpr int NR = G / V;               // rows of a group
     const int rl = W * V, full = m / rl;    // entries of a row, whole rows
+    [[maybe_unused]] int src[EN > 1 ? EN : 1];
+    if constexpr (EN > 1) {
+        static_assert(G == 8 && V == 1, "chain() takes eight entries of a lane");
+#pragma unroll
+        for (int k = 0; k < EN; k++)
+            src[k] = (((int)threadIdx.x & 63 & ~(W - 1)) + (t & ((1 << lt) - 1)) + (k << lt)) * 4;
+    }
     int c = 0, jn[G];
     if (NR <= full) {
 #pragma unroll
@@ -1710,12 +1763,19 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
 #pragma unroll
             for (int r = 0; r < NR; r++) ld_list<V>(lp + (r / RC) * cs + (r % RC) * W, jn + V * r);
         }
+        if constexpr (EN > 1) {
+            float p[G] = {}, gr[G] = {}, rr[G] = {};
 #pragma unroll
-        for (int u = 0; u < G; u++) acc.template add<EN>(pi, q[u]);
-        acc.template flush<EN>();
+            for (int u = 0; u < G; u++) acc.add_terms(pi, q[u], p[u], gr[u], rr[u]);
+            acc.template chain<EN, (VEC < 0)>(p, gr, rr, src);
+        } else {
+#pragma unroll
+            for (int u = 0; u < G; u++) acc.template add<EN>(pi, q[u]);
+            acc.template flush<EN>();
+        }
     }
     const int k0 = c * rl + t * V;  // this lane's first entry of the last group
-    if (k0 < m) {
+    if (EN > 1 ? c * rl < m : k0 < m) {  // chain() takes the whole team
         int jt[G];
         PosT q[G];
 #pragma unroll
@@ -1730,10 +1790,18 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
         }
 #pragma unroll
         for (int u = 0; u < G; u++) q[u] = ld_pos(pos, k0 + (u / V) * rl + u % V < m ? jt[u] : g);
+        if constexpr (EN > 1) {
+            float p[G] = {}, gr[G] = {}, rr[G] = {};
 #pragma unroll
-        for (int u = 0; u < G; u++)
-            if (k0 + (u / V) * rl + u % V < m) acc.template add<EN>(pi, q[u]);
-        acc.template flush<EN>();
+            for (int u = 0; u < G; u++)
+                if (k0 + u * rl < m) acc.add_terms(pi, q[u], p[u], gr[u], rr[u]);
+            acc.template chain<EN, (VEC < 0)>(p, gr, rr, src);
+        } else {
+#pragma unroll
+            for (int u = 0; u < G; u++)
+                if (k0 + (u / V) * rl + u % V < m) acc.template add<EN>(pi, q[u]);
+            acc.template flush<EN>();
+        }
     }
 }
 
@@ -1741,11 +1809,12 @@ __device__ __forceinline__ void walk_list(const int *lp, size_t cs, int W, int t
 // virial, p_x} (PE and virial with EN only) to the end-of-step chain update.
 // c0: the chain as it is; eta, peta: after the start-of-step half
 // (k_first_half).  EN: the pass summed the pair energy and virial (the last
-// step of a call; they are only reported).  apart: k_energy forms them after
-// the call's last step, and Heff is stored without the pair energy for it.
+// step of a call; they are only reported).  late: Heff's pair energy is added
+// last, by this step or, without EN, by a pass after the call's last step
+// (step, not KICK; launch_energy): the same sum either way.
 template <bool KICK, bool EN>
 __device__ __forceinline__ void force_end(const RepC &R, ChainS &c, const ChainS &c0, double *eta, double *peta,
-                                          const double *a4, int apart) {
+                                          const double *a4, int late, int step) {
     double S = a4[0], pe = a4[1], vir = a4[2], spx = a4[3];  // pe, vir: zero without EN
     pe = 0.5 * pe;                  // every pair seen from both sides
     vir = (0.5 * vir) / (3.0e0);   // cell_list+forces.c:220
@@ -1753,7 +1822,11 @@ __device__ __forceinline__ void force_end(const RepC &R, ChainS &c, const ChainS
         c.pe = pe;
         c.vir = vir;
     }
-    if (!KICK) return;
+    if (!KICK) {
+        if (EN && step) c.heff = c.heff + pe;
+        return;
+    }
+    const double pe0 = late ? 0.0 : pe, pe1 = late ? pe : 0.0;
     const bool rebuilt = need_rebuild(R, c0);
     if (c0.mode == 2) {
         // NVE: plain velocity Verlet (AdvanceTimeNVE, MDcode/time_evolve.c:39-171,
@@ -1764,7 +1837,7 @@ __device__ __forceinline__ void force_end(const RepC &R, ChainS &c, const ChainS
         c.ke = ke;
         c.inst_T = 2.0 * ke / R.dof;
         c.drift = spx;
-        if (EN || apart) c.heff = ke + pe;
+        if (EN || late) c.heff = ke + pe0 + pe1;
         if (rebuilt) c.rebuilds = c0.rebuilds + 1;
         c.maxbits = 0ull;
         c.force_rebuild = 0;
@@ -1784,7 +1857,7 @@ __device__ __forceinline__ void force_end(const RepC &R, ChainS &c, const ChainS
         c.ke = ke;
         c.inst_T = 2.0 * ke / R.dof;
         c.drift = spx * s2;
-        if (EN || apart) c.heff = ke + pe;
+        if (EN || late) c.heff = ke + pe0 + pe1;
         c.ramp_k = c0.ramp_k + 1;
         if (c0.ramp_k + 1 >= c0.ramp_n) c.mode = 0;
         if (rebuilt) c.rebuilds = c0.rebuilds + 1;
@@ -1801,11 +1874,11 @@ __device__ __forceinline__ void force_end(const RepC &R, ChainS &c, const ChainS
     c.ke = ke;
     c.inst_T = 2.0 * ke / R.dof;     // :524
     c.drift = spx * s2;
-    if (EN || apart) {
-        double heff = ke + pe + eta[0] * R.T * R.dof;  // print.c:85-87
+    if (EN || late) {
+        double heff = ke + pe0 + eta[0] * R.T * R.dof;  // print.c:85-87
         for (int k = 0; k < 3; k++) heff = heff + peta[k] * peta[k] / (2.0 * c0.q[k]);
         for (int k = 1; k < 3; k++) heff = heff + R.T * eta[k];
-        c.heff = heff;
+        c.heff = heff + pe1;
     }
     if (rebuilt) c.rebuilds = c0.rebuilds + 1;
     c.maxbits = 0ull;
@@ -1823,7 +1896,7 @@ struct EndArgs {
     const double *mid;
     double *gpart;
     unsigned *gdone, *rdone;
-    int apart;
+    int late, step;  // force_end
 };
 
 // Pair forces: a team of W = 2^lw lanes per particle (fixed per handle at
@@ -1844,15 +1917,20 @@ struct EndArgs {
 // long as that chain.  Each loaded where it was used, with the constants
 // divided out per lane and the sums shuffled through LDS: 7.2 us at N=1000
 // FP64 and 11.0 at N=10000 FP32 (four lanes); this 5.9 and 7.0 (sixteen).
-// EN = false leaves out the pair energy and virial, which every step
-// overwrites and only the call's last one reports: 9 of 55 instructions of
-// an FP32 pair.  (FP32 handles whose team is not the list layout's form them in
-// k_energy.)
-template <bool FP32, bool KICK, bool EN, int VEC>
+// EN = 0 leaves out the pair energy and virial, which every step overwrites
+// and only the call's last one reports: 9 of 55 instructions of an FP32 pair.
+// FP32 handles whose team is 2 or 4 times the list layout's take EN = 2 or 4,
+// which sums the FP32 terms of eight entries as the layout's team does, so that
+// the partial sums, whose rounding shows in the seventh to ninth digit of the
+// energy, do not depend on the force team's width (walk_list): a third more of
+// the pass.  us of a call of one step, 8000, 160001 and 500000 particles: with
+// the energy in two kernels of its own after it 32.6, 156 and 292, this 27.6,
+// 140 and 254.
+template <bool FP32, bool KICK, int EN, int VEC>
 __global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, const BlkD *__restrict__ fblk,
                                                const double4 *__restrict__ pos4, const QPos *__restrict__ posq,
                                                const int *__restrict__ nn,
-                                               const int *__restrict__ nl, int cap, int lw, int lc,
+                                               const int *__restrict__ nl, int cap, int lw, int lc, int lt,
                                                const int *__restrict__ act,
                                                const int8_t *__restrict__ kx, const int8_t *__restrict__ ky,
                                                const int8_t *__restrict__ kz, double *fx, double *fy, double *fz,
@@ -1886,10 +1964,12 @@ __global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, co
     // entries are W * n words apart; else the chunks of 8 entries, 8 * n
     const size_t e0 = (size_t)(VEC > 1 ? t * VEC : t);
     const int *lp = nl + (size_t)D.off * cap + ((((e0 >> lc) * D.n + (g - D.off)) << lc) + (e0 & ((1u << lc) - 1u)));
-    walk_list<VEC, EN>(lp, (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, pos, pi, acc);
+    walk_list<VEC, EN>(lp, (size_t)D.n * (VEC == 1 ? W : 8), W, lt, t, m, g, pos, pi, acc);
     acc.result(Fx, Fy, Fz, R);
-    v_pe = acc.pe;
-    v_vir = acc.vir;
+    if (EN <= 1 || t >> lt == 0) {  // EN > 1: the layout's lanes
+        v_pe = acc.pe;
+        v_vir = acc.vir;
+    }
     Fx = team_sum(Fx, lw);
     Fy = team_sum(Fy, lw);
     Fz = team_sum(Fz, lw);
@@ -1960,70 +2040,8 @@ __global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, co
             c0 = E.chain[D.rep];
             for (int k = 0; k < 3; k++) { eta[k] = E.mid[6 * D.rep + k]; peta[k] = E.mid[6 * D.rep + 3 + k]; }
         }
-        force_end<KICK, EN>(R, E.chain[D.rep], c0, eta, peta, a4, E.apart);
+        force_end<KICK, EN != 0>(R, E.chain[D.rep], c0, eta, peta, a4, E.late, E.step);
     }
-}
-
-// Pair energy and virial of FP32 handles whose force team is not the list
-// layout's team of 2^lw lanes: that team walks the list (entries t, t + W, ...;
-// one lane: chunks of 8) and sums the FP32 terms of eight entries before it
-// widens them, so the partial sums, whose rounding shows in the seventh to
-// ninth digit of the energy, do not depend on the force kernel's width.  Runs
-// once per call, after its last step (k_energy_end then completes the step's
-// reported values).
-template <int VEC>
-__global__ void __launch_bounds__(BLK) k_energy(const RepC *__restrict__ reps, const BlkD *__restrict__ eblk,
-                                                const QPos *__restrict__ posq, const int *__restrict__ nn,
-                                                const int *__restrict__ nl, int cap, int lw, double *epart, int nb) {
-    __shared__ double s_red[2][BLK / 64];
-    const int b = xcd_block(nb);
-    if (b < 0) return;
-    const BlkD D = eblk[b];
-    const int W = 1 << lw, t = threadIdx.x & (W - 1), i = D.first + (threadIdx.x >> lw);
-    const bool valid = i < D.n;
-    const int il = valid ? i : 0, g = D.off + il;
-    const QPos pi = ld_pos(posq, g);
-    const int m = valid ? nn[g] : 0;
-    PairAcc<true> acc(ptype(pi), reps[D.rep]);
-    walk_list<VEC, true>(nl + (size_t)D.off * cap + (size_t)il * (VEC == 1 ? W : 8) + t,
-                         (size_t)D.n * (VEC == 1 ? W : 8), W, t, m, g, posq, pi, acc);
-    const double v[2] = {wave_sum_rows(acc.pe), wave_sum_rows(acc.vir)};
-    if ((threadIdx.x & 63) == 0)
-        for (int q = 0; q < 2; q++) s_red[q][threadIdx.x >> 6] = v[q];
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        double s = 0.0;
-        for (int w = 0; w < BLK / 64; w++) s += s_red[threadIdx.x][w];
-        epart[2 * (size_t)b + threadIdx.x] = s;
-    }
-}
-
-// After k_energy, one workgroup per replica: its energy and virial, and with
-// step the pair energy in Heff (force_end stored it without).
-__global__ void __launch_bounds__(256) k_energy_end(const RepC *__restrict__ reps, ChainS *chain,
-                                                    const double *__restrict__ epart, int step) {
-    __shared__ double s_w[2][4];
-    const int r = blockIdx.x, w = threadIdx.x >> 6;
-    const RepC &R = reps[r];
-    if (R.n == 0) return;  // idle slot
-    double pe = 0.0, vir = 0.0;
-    for (int k = threadIdx.x; k < R.enblk; k += 256) {
-        const double *pp = epart + 2 * (size_t)(R.eblk_off + k);
-        pe += pp[0];
-        vir += pp[1];
-    }
-    pe = wave_sum_rows(pe);
-    vir = wave_sum_rows(vir);
-    if ((threadIdx.x & 63) == 0) { s_w[0][w] = pe; s_w[1][w] = vir; }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int k = 1; k < 4; k++) { pe += s_w[0][k]; vir += s_w[1][k]; }
-    pe = 0.5 * pe;                 // every pair seen from both sides
-    vir = (0.5 * vir) / (3.0e0);  // cell_list+forces.c:220
-    ChainS &c = chain[r];
-    c.pe = pe;
-    c.vir = vir;
-    if (step) c.heff = c.heff + pe;
 }
 
 // ------------------------------------------------------------- host side
@@ -2034,10 +2052,7 @@ struct ac4_md {
     ChainS *chain = nullptr;
     int *blk_rep = nullptr, *blk_first = nullptr, *blk_idx = nullptr;
     BlkD *blkd = nullptr, *fblk = nullptr;  // particle blocks (k_first_half) and force blocks
-    bool en_apart = false;  // the energy in a pass of its own (k_energy), with the list layout's team:
-    BlkD *eblk = nullptr;   // its block table,
-    double *epart = nullptr;  // its partial sums {pe, virial} per block,
-    int enblk = 0, elw = 0;   // its blocks, log2 of its lanes per particle
+    int en = 1, lt = 0;  // the energy's order (k_force's EN), log2 of the list layout's lanes per particle
     int lw = 0, lc = 3, vec = 1;  // force teams: log2 lanes, log2 list chunk, list reading (k_force's VEC)
     int *cblk_rep = nullptr, *cblk_cell = nullptr;
     int fnblk = 0, lnblk = 0, ncb = 0;
@@ -2123,7 +2138,6 @@ static int each_part(PartArrays &a, size_t n, F get) {
 // list creation allocates and ac4_md_slot_bytes adds up, get(&array, count).
 struct SlotCounts {
     size_t slots, n, cells, nblk, fnblk, lnblk, ncb;  // particles, cells, blocks of each kind
-    size_t enblk;                                     // blocks of the energy pass, 0 without it
     size_t shuf;                                      // swap blocks of the parallel shuffle, 0 without it
 };
 template <class F>
@@ -2139,7 +2153,6 @@ static int each_array(ac4_md *md, const SlotCounts &k, F get) {
     TRY(get(&md->cell_mem, k.cells * CELL_CAP)); TRY(get(&md->cnt, k.cells)); TRY(get(&md->start, k.cells));
     TRY(get(&md->partial, 4 * k.fnblk)); TRY(get(&md->gpart, 4 * k.fnblk)); TRY(get(&md->gdone, k.fnblk));
     TRY(get(&md->rdone, k.slots * DONE_PAD)); TRY(get(&md->bdone, k.slots * DONE_PAD));
-    if (k.enblk) { TRY(get(&md->eblk, k.enblk)); TRY(get(&md->epart, 2 * k.enblk)); }
     for (double **q : {&md->fx, &md->fy, &md->fz, &md->xo, &md->yo, &md->zo}) TRY(get(q, k.n));
     TRY(get(&md->pos4, k.n)); TRY(get(&md->posq, k.n));
     TRY(get(&md->nn, k.n)); TRY(get(&md->nn_ref, k.n)); TRY(get(&md->nl, md->cap * k.n)); TRY(get(&md->members, k.n));
@@ -2348,8 +2361,8 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     // handle's total capacity
     const int W = g_tpp ? tpp : std::max(tpp > 1 ? tpp : 1, force_width(cap_tot));
     while ((1 << md->lw) < W) md->lw++;
-    md->en_apart = precision == AC4_FP32 && W != tpp;
-    md->elw = ltpp;
+    md->lt = ltpp;
+    md->en = precision == AC4_FP32 ? W / tpp : 1;  // force_width and the layout's rule: 1, 2 or 4
     md->lc = tpp == 1 ? 3 : ltpp;
     // a chunk of 8 entries read by four lanes: every fourth entry each, so
     // that the lanes of a gather are on neighbouring entries, which are mostly
@@ -2381,8 +2394,6 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         R.fnblk = (cn + ppb - 1) / ppb;
         R.fblk_off = fblk_off;
         for (int k = 0; k < R.fnblk; k++) { ffirst.push_back(k * ppb); fd.push_back(BlkD{r, k * ppb, off, 0}); }
-        R.enblk = md->en_apart ? (cn * tpp + BLK - 1) / BLK : 0;
-        md->enblk += R.enblk;
         R.lblk_off = (int)lrep.size();
         R.lnblk = (cn + LPB - 1) / LPB;
         for (int k = 0; k < R.lnblk; k++) { lrep.push_back(r); lfirst.push_back(k * LPB); }
@@ -2433,7 +2444,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     job_rules(md);
     int rc = AC4_OK;
     const SlotCounts counts{(size_t)nslots, (size_t)off, (size_t)off_cell, (size_t)md->nblk, (size_t)md->fnblk,
-                            (size_t)md->lnblk, (size_t)md->ncb, (size_t)md->enblk, (size_t)nslots * 3 * md->shuf_bmax};
+                            (size_t)md->lnblk, (size_t)md->ncb, (size_t)nslots * 3 * md->shuf_bmax};
     if ((rc = each_array(md, counts, alloc_array)) != AC4_OK) { ac4_md_destroy(md); return rc; }
     {
         void *tab[2 * PART_FIELDS];
@@ -2497,7 +2508,7 @@ static int refresh_tables(ac4_md *md) {
     bool any = false;
     for (const RepC &R : md->reps_h) any |= R.n > 0;
     std::vector<int> br, bf, bi, lr, lf;
-    std::vector<BlkD> bd, fd, ed;
+    std::vector<BlkD> bd, fd;
     for (int r = 0; r < md->R; r++) {
         RepC &R = md->reps_h[r];
         if (any && R.n == 0) continue;
@@ -2508,8 +2519,6 @@ static int refresh_tables(ac4_md *md) {
         for (int k = 0; k < R.nblk; k++) bd.push_back(BlkD{r, md->t_bfirst[md->t_b0[r] + k], R.off, R.n});
         R.fblk_off = (int)fd.size();
         for (int k = 0; k < R.fnblk; k++) fd.push_back(BlkD{r, md->t_ffirst[md->t_f0[r] + k], R.off, R.n});
-        R.eblk_off = (int)ed.size();
-        for (int k = 0; k < R.enblk; k++) ed.push_back(BlkD{r, k * (BLK >> md->elw), R.off, R.n});
         R.lblk_off = (int)lr.size();
         lr.insert(lr.end(), md->t_lrep.begin() + md->t_l0[r], md->t_lrep.begin() + md->t_l0[r] + R.lnblk);
         lf.insert(lf.end(), md->t_lfirst.begin() + md->t_l0[r], md->t_lfirst.begin() + md->t_l0[r] + R.lnblk);
@@ -2521,13 +2530,11 @@ static int refresh_tables(ac4_md *md) {
     TRY(h2d(md->blk_rep, br.data(), br.size(), s)); TRY(h2d(md->blk_first, bf.data(), bf.size(), s));
     TRY(h2d(md->blk_idx, bi.data(), bi.size(), s));
     TRY(h2d(md->blkd, bd.data(), bd.size(), s)); TRY(h2d(md->fblk, fd.data(), fd.size(), s));
-    if (!ed.empty()) TRY(h2d(md->eblk, ed.data(), ed.size(), s));
     TRY(h2d(md->lblk_rep, lr.data(), lr.size(), s)); TRY(h2d(md->lblk_first, lf.data(), lf.size(), s));
     TRY(h2d(md->reps, md->reps_h.data(), md->reps_h.size(), s));
     AC4_HIP(hipStreamSynchronize(s));
     md->nblk = (int)br.size();
     md->fnblk = (int)fd.size();
-    md->enblk = (int)ed.size();
     md->lnblk = (int)lr.size();
     return AC4_OK;
 }
@@ -2597,7 +2604,7 @@ extern "C" int ac4_md_destroy(ac4_md *md) {
     if (!md) return AC4_OK;
     if (md->stream) (void)hipStreamSynchronize(md->stream);
     drop_graphs(md);
-    void *ptrs[] = {md->reps, md->chain, md->blk_rep, md->blk_first, md->blk_idx, md->blkd, md->fblk, md->eblk, md->epart,
+    void *ptrs[] = {md->reps, md->chain, md->blk_rep, md->blk_first, md->blk_idx, md->blkd, md->fblk,
                     md->lblk_rep, md->lblk_first, md->wl_item, md->wl_n, md->ranges, md->xmid,
                     md->cblk_rep, md->cblk_cell, md->ox, md->oy, md->oz, md->ov_q, md->ov_q2,
                     md->ov_step, md->ov_cnt, md->ov_n, md->ov_list, md->ov_out,
@@ -2620,13 +2627,12 @@ extern "C" int ac4_md_total_particles(const ac4_md *md) { return md ? md->ntot :
 // Device bytes a slot of capacity cap_n adds to a handle: the arrays
 // ac4_md_create_slots and ac4_md_overlap_enable allocate and the
 // reference-order export's, the force blocks counted at the widest team (16
-// lanes a particle), the energy pass as if the handle had one and the
-// parallel-shuffle tables at their largest, as if this slot were the largest
-// of its handle.
+// lanes a particle) and the parallel-shuffle tables at their largest, as if
+// this slot were the largest of its handle.
 extern "C" long long ac4_md_slot_bytes(int cap_n, int n_origin, int n_lags) {
     if (cap_n < 2 || n_origin < 0 || n_lags < 0) return AC4_EARG;
     const size_t n = cap_n, cells = slot_cells(cap_n), fnb = (n * 16 + BLK - 1) / BLK;
-    const SlotCounts k{1, n, cells, (n + BLK - 1) / BLK, fnb, (n + LPB - 1) / LPB, (cells + BLK / 64 - 1) / (BLK / 64), fnb,
+    const SlotCounts k{1, n, cells, (n + BLK - 1) / BLK, fnb, (n + LPB - 1) / LPB, (cells + BLK / 64 - 1) / (BLK / 64),
                        cap_n > SHUF_PAR_MIN ? 3 * ((n + SHUF_M - 1) / SHUF_M) : 0};
     ac4_md md;  // for the arrays' types
     long long b = 0;
@@ -3275,39 +3281,39 @@ static int launch_rebuild(ac4_md *md, bool with_zero = false) {
     return AC4_OK;
 }
 
-template <bool FP32, bool KICK, bool EN>
-static int launch_force_kernel(ac4_md *md) {
-    // a team of four on chunks of 8 has its energy apart in FP32 (en_apart)
-    auto kern = md->vec == 8 ? k_force<FP32, KICK, EN, 8>
-                : md->vec == 1 ? k_force<FP32, KICK, EN, 1>
-                               : k_force<FP32, KICK, EN && !FP32, -2>;
+template <bool FP32, bool KICK, int EN>
+static int launch_force_kernel(ac4_md *md, bool step) {
+    auto kern = k_force<FP32, KICK, EN, 1>;
+    if constexpr (EN <= 1) {
+        if (md->vec == 8) kern = k_force<FP32, KICK, EN, 8>;
+    }
+    if constexpr (FP32 ? EN == 0 || EN == 4 : true) {
+        if (md->vec < 0) kern = k_force<FP32, KICK, EN, -2>;
+    }
     put(md, kern, dim3(xcd_grid(md->fnblk)), dim3(BLK), 0, md->reps, md->fblk, md->pos4,
-        md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->P.act, md->kx, md->ky, md->kz, md->fx,
+        md->posq, md->nn, md->nl, md->cap, md->lw, md->lc, md->lt, md->P.act, md->kx, md->ky, md->kz, md->fx,
         md->fy, md->fz, md->P.px, md->P.py, md->P.pz, md->partial, md->fnblk,
-        EndArgs{md->chain, md->mid, md->gpart, md->gdone, md->rdone, md->en_apart ? 1 : 0});
+        EndArgs{md->chain, md->mid, md->gpart, md->gdone, md->rdone, md->en > 1 ? 1 : 0, step ? 1 : 0});
     AC4_HIP(hipGetLastError());
     return AC4_OK;
 }
-// The energy of en_apart handles, after the last of the call's steps (step)
-// or after calculate_forces' pass.
-static int launch_energy(ac4_md *md, bool step) {
-    if (!md->en_apart) return AC4_OK;
-    put(md, (md->elw ? k_energy<1> : k_energy<8>), dim3(xcd_grid(md->enblk)), dim3(BLK), 0,
-        md->reps, md->eblk, md->posq, md->nn, md->nl, md->cap, md->elw, md->epart, md->enblk);
-    put(md, k_energy_end, dim3(md->R), dim3(256), 0, md->reps, md->chain, md->epart,
-        step ? 1 : 0);
-    AC4_HIP(hipGetLastError());
-    return AC4_OK;
-}
-template <bool KICK, bool EN>
-static int launch_force_pass(ac4_md *md) {
-    return md->prec == AC4_FP32 ? launch_force_kernel<true, KICK, EN>(md) : launch_force_kernel<false, KICK, EN>(md);
-}
-// energy: form the pair energy and virial in this pass
+// energy: form the pair energy and virial in this pass (without KICK always);
+// step: also complete Heff (after a step without them)
 template <bool KICK>
-static int launch_force(ac4_md *md, bool energy) {
-    return energy && !md->en_apart ? launch_force_pass<KICK, true>(md) : launch_force_pass<KICK, false>(md);
+static int launch_force(ac4_md *md, bool energy, bool step = false) {
+    if constexpr (KICK) {
+        if (!energy)
+            return md->prec == AC4_FP32 ? launch_force_kernel<true, true, 0>(md, step) : launch_force_kernel<false, true, 0>(md, step);
+    }
+    if (md->prec != AC4_FP32) return launch_force_kernel<false, KICK, 1>(md, step);
+    return md->en == 1   ? launch_force_kernel<true, KICK, 1>(md, step)
+           : md->en == 2 ? launch_force_kernel<true, KICK, 2>(md, step)
+                         : launch_force_kernel<true, KICK, 4>(md, step);
 }
+// The energy after a call whose last step is the end of a recorded chunk, on
+// handles that form it in the layout's order (EN > 1: a third more of the
+// pass, so chunks leave it out): the forces once more, with it.
+static int launch_energy(ac4_md *md) { return md->en > 1 ? launch_force<false>(md, true, true) : AC4_OK; }
 
 static void launch_shuffle(ac4_md *md, int force) {
     if (md->shuf_serial)
@@ -3338,8 +3344,7 @@ static void launch_first_half(ac4_md *md, bool with_shuffle) {
 // fork and join cost more than the overlap gave (about 9 us per step).  It
 // now runs inside k_first_half where its LDS allows, else as k_shuffle first.
 // last: the call's last step, whose pair energy and virial a caller can read
-// (each step overwrites them, so the steps before it do not form them; the
-// callers follow it with launch_energy).
+// (each step overwrites them, so the steps before it do not form them).
 static int launch_step(ac4_md *md, bool last) {
     if (md->shuf_fused) {
         launch_first_half(md, true);
@@ -3393,7 +3398,6 @@ extern "C" int ac4_md_calculate_forces(ac4_md *md, double *out2) {
     for (auto &e : c) stale |= e.force_rebuild != 0;
     if (stale) TRY(force_rebuild_all(md));
     TRY(launch_force<false>(md, true));
-    TRY(launch_energy(md, false));
     TRY(get_chains(md, c));
     if (out2)
         for (int r = 0; r < md->R; r++) { out2[2 * r] = c[r].pe; out2[2 * r + 1] = c[r].vir; }
@@ -3416,7 +3420,7 @@ static int record_steps(ac4_md *md, int k) {
     md->rec_end = nullptr;
     md->rec_err = hipSuccess;
     int rc = AC4_OK;
-    for (int q = 0; q < m && rc == AC4_OK; q++) rc = launch_step(md, q == m - 1);
+    for (int q = 0; q < m && rc == AC4_OK; q++) rc = launch_step(md, q == m - 1 && md->en == 1);
     md->rec = nullptr;
     hipGraphExec_t x = nullptr;
     hipError_t e = md->rec_err;
@@ -3462,16 +3466,26 @@ extern "C" int ac4_md_step(ac4_md *md, int nsteps) {
             AC4_HIP(hipGraphLaunch(md->gexec[1], md->stream));
     }
     md->eager = std::min(md->eager + nsteps - k, STEP_GRAPH_PAY);
+    if (k > 0 && k == nsteps) return launch_energy(md);
     for (; k < nsteps; k++) TRY(launch_step(md, k == nsteps - 1));
-    return nsteps > 0 ? launch_energy(md, true) : AC4_OK;
+    return AC4_OK;
+}
+
+// A step after the chunks: from the one-step graph, or, the call's last one
+// where that graph leaves the energy out, launched.
+static int launch_rest(ac4_md *md, bool last) {
+    if (last && md->en > 1) return launch_step(md, true);
+    AC4_HIP(hipGraphLaunch(md->gexec[0], md->stream));
+    return AC4_OK;
 }
 
 extern "C" int ac4_md_step_graph(ac4_md *md, int nsteps) {
     AC4_REQUIRE(md && nsteps >= 0, AC4_EARG, "bad arguments");
     TRY(ready_graphs(md));
     for (int k = 0; k < nsteps / GRAPH_CHUNK; k++) AC4_HIP(hipGraphLaunch(md->gexec[1], md->stream));
-    for (int k = 0; k < nsteps % GRAPH_CHUNK; k++) AC4_HIP(hipGraphLaunch(md->gexec[0], md->stream));
-    return nsteps > 0 ? launch_energy(md, true) : AC4_OK;
+    const int rest = nsteps % GRAPH_CHUNK;
+    for (int k = 0; k < rest; k++) TRY(launch_rest(md, k == rest - 1));
+    return rest == 0 && nsteps > 0 ? launch_energy(md) : AC4_OK;
 }
 
 // Several handles stepped together: each on its own stream, the graph
@@ -3488,9 +3502,10 @@ extern "C" int ac4_md_step_graph_multi(ac4_md *const *mds, int nh, int nsteps) {
     }
     for (int k = 0; k < nsteps / GRAPH_CHUNK; k++)
         for (int h = 0; h < nh; h++) AC4_HIP(hipGraphLaunch(mds[h]->gexec[1], mds[h]->stream));
-    for (int k = 0; k < nsteps % GRAPH_CHUNK; k++)
-        for (int h = 0; h < nh; h++) AC4_HIP(hipGraphLaunch(mds[h]->gexec[0], mds[h]->stream));
-    for (int h = 0; h < nh && nsteps > 0; h++) TRY(launch_energy(mds[h], true));
+    const int rest = nsteps % GRAPH_CHUNK;
+    for (int k = 0; k < rest; k++)
+        for (int h = 0; h < nh; h++) TRY(launch_rest(mds[h], k == rest - 1));
+    for (int h = 0; h < nh && rest == 0 && nsteps > 0; h++) TRY(launch_energy(mds[h]));
     return AC4_OK;
 }
 
@@ -3502,7 +3517,6 @@ extern "C" int ac4_md_relax(ac4_md *md, int nsteps, double f_start, double f_end
     for (auto &e : c) { e.mode = 1; e.ramp_n = nsteps; e.ramp_k = 0; e.ramp0 = f_start; e.ramp1 = f_end; }
     TRY(put_chains(md, c));
     for (int k = 0; k < nsteps; k++) TRY(launch_step(md, k == nsteps - 1));
-    TRY(launch_energy(md, true));
     return check_err(md);
 }
 
@@ -3537,7 +3551,6 @@ extern "C" int ac4_md_kernel_times(ac4_md *md, int nsteps, double *ms) {
     }
     for (auto &e : ev) (void)hipEventDestroy(e);
     for (int q = 0; q < 5; q++) ms[q] = acc[q] / nsteps;
-    TRY(launch_energy(md, true));
     return check_err(md);
 }
 

@@ -635,3 +635,75 @@ def test_slot_bytes_cover_the_handle(gpu):
     # arrays is rounded up to 2 MiB at most
     want = sum(gpu.slot_bytes(c) for c in caps) - 28 * sum(caps)
     assert used <= want + 70 * (2 << 20), (used, want)
+
+
+# FP32 pair energy of the automatic force team, formed in the order of the list
+# layout's team (8, 4, 2 lanes and one), against that team pinned: the same
+# FP32 partial sums, added up in FP64 in another order; several replicas, lists
+# of few and of many entries.
+@pytest.mark.parametrize("sizes,layout", [((5000,), 8), ((8192,), 8), ((3000, 700, 1500), 8), ((8193,), 4), ((14001,), 4),
+                                          ((16385,), 2), ((300, 20000, 5001), 2), ((32769,), 1), ((60001, 500), 1),
+                                          ((160001,), 1)])
+def test_fp32_energy_in_the_layouts_order(gpu, sizes, layout):
+    out = []
+    for tpp in (0, layout):
+        gpu.set_tuning(tpp)
+        try:
+            md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 200, 3 + r) for r, n in enumerate(sizes)], precision=gpu.FP32)
+        finally:
+            gpu.set_tuning()
+        for r, n in enumerate(sizes):
+            s = gpu.init_lattice(n, 0.5, n)
+            rng = np.random.default_rng(n)
+            x = [(s[k] + rng.normal(0, 0.02 / n ** (1 / 3), n)) % 1.0 for k in ("x", "y", "z")]
+            md.set_state(r, *x, *x, s["px"], s["py"], s["pz"], s["type"], s["act_tag"], s["kx"], s["ky"], s["kz"])
+        pv = np.array(md.calculate_forces())
+        md.step(1)
+        out.append((pv, [md.stats(r) for r in range(len(sizes))]))
+        md.close()
+    (pa, sa), (pb, sb) = out
+    # sums of n terms of both signs: a few roundings of the sum of their sizes, about 5 n
+    for r, n in enumerate(sizes):
+        assert np.abs(pa[r] - pb[r]).max() <= 2.0 ** -53 * 8 * 5 * n
+        # after a step the positions differ by the order of the force sums, which an FP32 term can round away from
+        assert np.isclose(sa[r]["pe"], sb[r]["pe"], rtol=1e-9) and np.isclose(sa[r]["Heff"], sb[r]["Heff"], rtol=1e-9)
+
+
+# Energy, virial and Heff after the same steps taken one by one, in calls of
+# several, from recorded chunks and from several handles together: bit for bit,
+# for every order of the energy and both modes of its last step.
+@pytest.mark.parametrize("prec,n", [(0, 700), (1, 700), (1, 5000), (1, 9001), (1, 20000), (1, 40000)])
+@pytest.mark.parametrize("nsteps", [1, 25, 26, 49, 50])
+def test_energy_after_every_kind_of_call(gpu, prec, n, nsteps):
+    mds = []
+    for k in range(4):
+        md = gpu.MD([gpu.ReplicaParams(n, 1.2, 0.5, 1.0, -1, 7, 3)], precision=prec)
+        s = gpu.init_lattice(n, 0.5, n)
+        md.set_state(0, *[s[q] for q in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], s["act_tag"],
+                     s["kx"], s["ky"], s["kz"])
+        md.relax(30)
+        md.init_chain(0)
+        mds.append(md)
+    a, b, c, d = mds
+    for rep in range(2):
+        for _ in range(nsteps):
+            a.step(1)
+        b.step(nsteps)
+        c.step(nsteps, graph=True)
+        gpu.step_multi([d], nsteps)
+        want = a.stats(0)
+        assert want["pe"] != 0.0
+        for md in (b, c, d):
+            assert md.stats(0) == want
+        x = a.get_state(0)
+        for md in (b, c, d):
+            y = md.get_state(0)
+            assert all(np.array_equal(x[k], y[k]) for k in x)
+            assert np.array_equal(np.stack(a.forces(0)), np.stack(md.forces(0)))
+    if n <= 32768:  # calls of whole chunks that the plain step replays
+        for _ in range(14):
+            b.step(25)
+            c.step(25, graph=True)
+            assert b.stats(0) == c.stats(0)
+    for md in mds:
+        md.close()
