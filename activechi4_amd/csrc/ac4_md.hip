@@ -2087,9 +2087,8 @@ struct ac4_md {
     OvCfg ov{0, 0, 0, 0, 0.0};
     double *ox = nullptr, *oy = nullptr, *oz = nullptr, *ov_q = nullptr, *ov_q2 = nullptr;
     long long *ov_step = nullptr;
-    // block tables of every slot, in slot order, with each slot's first
-    // entry: the launch grids cover only the occupied slots (refresh_tables)
-    std::vector<int> t_brep, t_bfirst, t_bidx, t_ffirst, t_lrep, t_lfirst, t_b0, t_f0, t_l0;
+    std::vector<char> tables;  // refresh_tables' copy of the block tables and reps
+    char *mem = nullptr;       // the arrays of each_array
     int *ov_list = nullptr;     // replica list of ac4_md_overlap_chi4
     double *ov_out = nullptr;   // its per-lag results
     // frame text (ac4_md_format_frame): a slot of 80 bytes per line in
@@ -2136,17 +2135,18 @@ static int each_part(PartArrays &a, size_t n, F get) {
 
 // What slots add up to, and the device arrays a handle of that many has: the
 // list creation allocates and ac4_md_slot_bytes adds up, get(&array, count).
+// First what refresh_tables writes, blk_rep to reps.
 struct SlotCounts {
     size_t slots, n, cells, nblk, fnblk, lnblk, ncb;  // particles, cells, blocks of each kind
     size_t shuf;                                      // swap blocks of the parallel shuffle, 0 without it
 };
 template <class F>
 static int each_array(ac4_md *md, const SlotCounts &k, F get) {
-    if (k.shuf) { TRY(get(&md->shuf_ent, k.shuf * 2 * SHUF_M)); TRY(get(&md->shuf_ent_n, k.shuf)); }
-    TRY(get(&md->reps, k.slots)); TRY(get(&md->chain, k.slots)); TRY(get(&md->mid, 6 * k.slots));
     TRY(get(&md->blk_rep, k.nblk)); TRY(get(&md->blk_first, k.nblk)); TRY(get(&md->blk_idx, k.nblk));
     TRY(get(&md->blkd, k.nblk)); TRY(get(&md->fblk, k.fnblk));
     TRY(get(&md->lblk_rep, k.lnblk)); TRY(get(&md->lblk_first, k.lnblk));
+    TRY(get(&md->reps, k.slots)); TRY(get(&md->chain, k.slots)); TRY(get(&md->mid, 6 * k.slots));
+    if (k.shuf) { TRY(get(&md->shuf_ent, k.shuf * 2 * SHUF_M)); TRY(get(&md->shuf_ent_n, k.shuf)); }
     TRY(get(&md->wl_item, k.nblk + k.lnblk + k.ncb)); TRY(get(&md->wl_n, (size_t)4));
     TRY(get(&md->ranges, k.cells * NRANGE)); TRY(get(&md->xmid, k.cells));
     TRY(get(&md->cblk_rep, k.cells)); TRY(get(&md->cblk_cell, k.cells));
@@ -2177,11 +2177,29 @@ static int each_overlap_array(ac4_md *md, size_t slots, size_t n, size_t n_origi
 }
 static const auto alloc_array = [](auto **p, size_t n) { return dalloc(p, n); };
 
-static void free_parts(PartArrays &a) {
-    void *q[] = {a.x, a.y, a.z, a.xu, a.yu, a.zu, a.px, a.py, a.pz, a.type, a.act, a.id, a.cell_ref, a.cell_of};
-    for (void *v : q)
-        if (v) (void)hipFree(v);
-    a = PartArrays{};
+// each_array's arrays in one allocation, zeroed: small ones at whole pages,
+// those of 2 MiB and more at multiples of that, as allocations of their own lie.
+// (An allocation and a fill for each of 65 arrays: 20 slots of 2000 particles
+// 1.57 ms to create and destroy, this 0.76.)
+static int alloc_arrays(ac4_md *md, const SlotCounts &k) {
+    size_t total = 0;
+    const auto place = [&](size_t bytes) {
+        const size_t to = bytes >= (2u << 20) ? 2u << 20 : 4096;
+        const size_t at = (total + to - 1) / to * to;
+        total = at + std::max<size_t>(bytes, 1);
+        return at;
+    };
+    TRY(each_array(md, k, [&](auto **p, size_t n) {
+        (void)place(sizeof(**p) * n);
+        return AC4_OK;
+    }));
+    AC4_HIP(hipMalloc((void **)&md->mem, total));
+    AC4_HIP(hipMemset(md->mem, 0, total));
+    total = 0;
+    return each_array(md, k, [&](auto **p, size_t n) {
+        *(void **)p = md->mem + place(sizeof(**p) * n);
+        return AC4_OK;
+    });
 }
 
 // Kernel shape of handles created afterwards.  tpp: lanes per particle in
@@ -2321,6 +2339,8 @@ static void fresh_chain(ChainS &c, const RepC &R) {
     c.force_rebuild = R.n > 0 ? 1 : 0;
 }
 
+static int refresh_tables(ac4_md *md);
+
 // cells a slot of capacity cn can hold: those of the least dense box (rho 0.5)
 static int slot_cells(int cn) { return (int)pow((int)(pow((double)cn / 0.5, 1.0 / 3.0) / K_CELL_CUT) + 1, 3); }
 
@@ -2343,9 +2363,8 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     md->R = nslots;
     md->prec = precision;
     md->nlist_mode = g_nlist_mode;
-    int off = 0, off_act = 0, off_cell = 0, blk_off = 0, fblk_off = 0;
-    std::vector<int> brep, bfirst, bidx, ffirst, crep, ccell, lrep, lfirst;
-    std::vector<BlkD> bd, fd;
+    int off = 0, off_act = 0, off_cell = 0, blk_off = 0, fblk_off = 0, lblk_off = 0;
+    std::vector<int> crep, ccell;
     int ncb = 0;
     AC4_REQUIRE(nslots < 32768, AC4_EARG, "at most 32767 slots");
     double cap_tot = 0.0;
@@ -2389,14 +2408,11 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         R.lc = tpp == 1 ? 3 : ltpp;
         R.nblk = (cn + BLK - 1) / BLK;
         R.blk_off = blk_off;
-        for (int k = 0; k < R.nblk; k++) { brep.push_back(r); bfirst.push_back(k * BLK); bidx.push_back(k); bd.push_back(BlkD{r, k * BLK, off, 0}); }
         const int ppb = BLK / W;  // particles per force block
         R.fnblk = (cn + ppb - 1) / ppb;
         R.fblk_off = fblk_off;
-        for (int k = 0; k < R.fnblk; k++) { ffirst.push_back(k * ppb); fd.push_back(BlkD{r, k * ppb, off, 0}); }
-        R.lblk_off = (int)lrep.size();
+        R.lblk_off = lblk_off;
         R.lnblk = (cn + LPB - 1) / LPB;
-        for (int k = 0; k < R.lnblk; k++) { lrep.push_back(r); lfirst.push_back(k * LPB); }
         if ((cap_cells + BLK / 64 - 1) / (BLK / 64) >= 65536) { delete md; ac4_set_error("slot %d: too many cells", r); return AC4_EARG; }
         ncb += (cap_cells + BLK / 64 - 1) / (BLK / 64);
         for (int c = 0; c < cap_cells; c++) { crep.push_back(r); ccell.push_back(c); }
@@ -2405,15 +2421,9 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         off_cell += cap_cells;
         blk_off += R.nblk;
         fblk_off += R.fnblk;
+        lblk_off += R.lnblk;
         md->max_ncell = std::max(md->max_ncell, cap_cells);
         md->reps_h.push_back(R);  // idle: n = 0
-    }
-    md->t_brep = brep; md->t_bfirst = bfirst; md->t_bidx = bidx;
-    md->t_ffirst = ffirst; md->t_lrep = lrep; md->t_lfirst = lfirst;
-    for (const RepC &R : md->reps_h) {
-        md->t_b0.push_back(R.blk_off);
-        md->t_f0.push_back(R.fblk_off);
-        md->t_l0.push_back(R.lblk_off);
     }
     md->ntot = off;
     md->nact_tot = off_act;
@@ -2421,7 +2431,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     md->nblk = blk_off;
     md->stride = off;
     md->fnblk = fblk_off;
-    md->lnblk = (int)lrep.size();
+    md->lnblk = lblk_off;
     md->ncb = ncb;
     {  // k_shuffle: the partner chunk plus one component in LDS when it fits
         int dev = 0, lds = 65536, cap_max = 0;
@@ -2445,7 +2455,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     int rc = AC4_OK;
     const SlotCounts counts{(size_t)nslots, (size_t)off, (size_t)off_cell, (size_t)md->nblk, (size_t)md->fnblk,
                             (size_t)md->lnblk, (size_t)md->ncb, (size_t)nslots * 3 * md->shuf_bmax};
-    if ((rc = each_array(md, counts, alloc_array)) != AC4_OK) { ac4_md_destroy(md); return rc; }
+    if ((rc = alloc_arrays(md, counts)) != AC4_OK) { ac4_md_destroy(md); return rc; }
     {
         void *tab[2 * PART_FIELDS];
         for (int k = 0; k < 2; k++) {
@@ -2465,14 +2475,6 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
         ac4_set_error("hipStreamCreate failed");
         return AC4_EHIP;
     }
-    AC4_HIP(hipMemcpy(md->reps, md->reps_h.data(), sizeof(RepC) * nslots, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->blk_rep, brep.data(), sizeof(int) * md->nblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->blk_first, bfirst.data(), sizeof(int) * md->nblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->blk_idx, bidx.data(), sizeof(int) * md->nblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->blkd, bd.data(), sizeof(BlkD) * md->nblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->fblk, fd.data(), sizeof(BlkD) * md->fnblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->lblk_rep, lrep.data(), sizeof(int) * md->lnblk, hipMemcpyHostToDevice));
-    AC4_HIP(hipMemcpy(md->lblk_first, lfirst.data(), sizeof(int) * md->lnblk, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->cblk_rep, crep.data(), sizeof(int) * off_cell, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->cblk_cell, ccell.data(), sizeof(int) * off_cell, hipMemcpyHostToDevice));
     std::vector<ChainS> ch(nslots);
@@ -2484,6 +2486,7 @@ extern "C" int ac4_md_create_slots_rule(int nslots, const int *cap_n, int precis
     AC4_HIP(hipMemcpy(md->P.act, neg.data(), sizeof(int) * off, hipMemcpyHostToDevice));
     AC4_HIP(hipMemcpy(md->P.id, ids.data(), sizeof(int) * off, hipMemcpyHostToDevice));
     md->have_forces = true;  // nothing loaded yet; set_state asks for a force evaluation
+    if ((rc = refresh_tables(md)) != AC4_OK) { ac4_md_destroy(md); return rc; }
     *out = md;
     return AC4_OK;
 }
@@ -2507,35 +2510,42 @@ static void drop_graphs(ac4_md *md) {
 static int refresh_tables(ac4_md *md) {
     bool any = false;
     for (const RepC &R : md->reps_h) any |= R.n > 0;
-    std::vector<int> br, bf, bi, lr, lf;
-    std::vector<BlkD> bd, fd;
+    // the tables as they lie on the device, in one copy
+    char *const first = (char *)md->blk_rep;
+    md->tables.resize((size_t)((char *)(md->reps + md->R) - first));
+    const auto host = [&](auto *dev) { return (decltype(dev))(md->tables.data() + ((char *)dev - first)); };
+    int *const br = host(md->blk_rep), *const bf = host(md->blk_first), *const bi = host(md->blk_idx),
+        *const lr = host(md->lblk_rep), *const lf = host(md->lblk_first);
+    BlkD *const bd = host(md->blkd), *const fd = host(md->fblk);
+    int nb = 0, nfb = 0, nlb = 0;
     for (int r = 0; r < md->R; r++) {
         RepC &R = md->reps_h[r];
         if (any && R.n == 0) continue;
-        R.blk_off = (int)br.size();
-        br.insert(br.end(), md->t_brep.begin() + md->t_b0[r], md->t_brep.begin() + md->t_b0[r] + R.nblk);
-        bf.insert(bf.end(), md->t_bfirst.begin() + md->t_b0[r], md->t_bfirst.begin() + md->t_b0[r] + R.nblk);
-        bi.insert(bi.end(), md->t_bidx.begin() + md->t_b0[r], md->t_bidx.begin() + md->t_b0[r] + R.nblk);
-        for (int k = 0; k < R.nblk; k++) bd.push_back(BlkD{r, md->t_bfirst[md->t_b0[r] + k], R.off, R.n});
-        R.fblk_off = (int)fd.size();
-        for (int k = 0; k < R.fnblk; k++) fd.push_back(BlkD{r, md->t_ffirst[md->t_f0[r] + k], R.off, R.n});
-        R.lblk_off = (int)lr.size();
-        lr.insert(lr.end(), md->t_lrep.begin() + md->t_l0[r], md->t_lrep.begin() + md->t_l0[r] + R.lnblk);
-        lf.insert(lf.end(), md->t_lfirst.begin() + md->t_l0[r], md->t_lfirst.begin() + md->t_l0[r] + R.lnblk);
+        R.blk_off = nb;
+        for (int k = 0; k < R.nblk; k++, nb++) {
+            br[nb] = r;
+            bf[nb] = k * BLK;
+            bi[nb] = k;
+            bd[nb] = BlkD{r, k * BLK, R.off, R.n};
+        }
+        R.fblk_off = nfb;
+        for (int k = 0; k < R.fnblk; k++) fd[nfb++] = BlkD{r, k * (BLK >> md->lw), R.off, R.n};
+        R.lblk_off = nlb;
+        for (int k = 0; k < R.lnblk; k++, nlb++) {
+            lr[nlb] = r;
+            lf[nlb] = k * LPB;
+        }
     }
+    memcpy(host(md->reps), md->reps_h.data(), sizeof(RepC) * md->R);
     hipStream_t s = md->stream;
     AC4_HIP(hipStreamSynchronize(s));
     drop_graphs(md);
     job_rules(md);
-    TRY(h2d(md->blk_rep, br.data(), br.size(), s)); TRY(h2d(md->blk_first, bf.data(), bf.size(), s));
-    TRY(h2d(md->blk_idx, bi.data(), bi.size(), s));
-    TRY(h2d(md->blkd, bd.data(), bd.size(), s)); TRY(h2d(md->fblk, fd.data(), fd.size(), s));
-    TRY(h2d(md->lblk_rep, lr.data(), lr.size(), s)); TRY(h2d(md->lblk_first, lf.data(), lf.size(), s));
-    TRY(h2d(md->reps, md->reps_h.data(), md->reps_h.size(), s));
+    AC4_HIP(hipMemcpyAsync(first, md->tables.data(), md->tables.size(), hipMemcpyHostToDevice, s));
     AC4_HIP(hipStreamSynchronize(s));
-    md->nblk = (int)br.size();
-    md->fnblk = (int)fd.size();
-    md->lnblk = (int)lr.size();
+    md->nblk = nb;
+    md->fnblk = nfb;
+    md->lnblk = nlb;
     return AC4_OK;
 }
 
@@ -2544,13 +2554,16 @@ extern "C" int ac4_md_assign(ac4_md *md, int slot, const ac4_replica_params *p) 
     RepC R = md->reps_h[slot];
     const char *why = configure_rep(R, *p);
     AC4_REQUIRE(!why, AC4_EARG, "slot %d: %s", slot, why ? why : "");
+    // the block tables hold the replica's n, the launch rules its n_act and cells
+    const RepC &old = md->reps_h[slot];
+    const bool same = old.n == R.n && old.nact == R.nact && old.ncell == R.ncell;
     md->reps_h[slot] = R;
     ChainS c;
     fresh_chain(c, R);
     AC4_HIP(hipMemcpyAsync(md->reps + slot, &md->reps_h[slot], sizeof(RepC), hipMemcpyHostToDevice, md->stream));
     AC4_HIP(hipMemcpyAsync(md->chain + slot, &c, sizeof(ChainS), hipMemcpyHostToDevice, md->stream));
     AC4_HIP(hipStreamSynchronize(md->stream));
-    return refresh_tables(md);  // the block tables hold the replica's n
+    return same ? AC4_OK : refresh_tables(md);
 }
 
 extern "C" int ac4_md_release(ac4_md *md, int slot) {
@@ -2604,19 +2617,11 @@ extern "C" int ac4_md_destroy(ac4_md *md) {
     if (!md) return AC4_OK;
     if (md->stream) (void)hipStreamSynchronize(md->stream);
     drop_graphs(md);
-    void *ptrs[] = {md->reps, md->chain, md->blk_rep, md->blk_first, md->blk_idx, md->blkd, md->fblk,
-                    md->lblk_rep, md->lblk_first, md->wl_item, md->wl_n, md->ranges, md->xmid,
-                    md->cblk_rep, md->cblk_cell, md->ox, md->oy, md->oz, md->ov_q, md->ov_q2,
-                    md->ov_step, md->ov_cnt, md->ov_n, md->ov_list, md->ov_out,
-                    md->partial, md->mid, md->gpart, md->gdone, md->rdone, md->bdone, md->fx, md->fy, md->fz, md->xo, md->yo, md->zo, md->pos4, md->posq, md->cell_mem, md->shuf_ent, md->shuf_ent_n, md->nn,
-                    md->nn_ref, md->nl,
-                    md->cnt, md->start, md->members, md->kx, md->ky, md->kz, md->ex, md->ey, md->ez, md->et};
+    void *ptrs[] = {md->mem, md->ox, md->oy, md->oz, md->ov_q, md->ov_q2, md->ov_step, md->ov_cnt, md->ov_n, md->ov_list,
+                    md->ov_out, md->ex, md->ey, md->ez, md->et};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     free_fmt(md);
-    free_parts(md->P);
-    free_parts(md->A);
-    if (md->ftab) (void)hipFree(md->ftab);
     if (md->stream) (void)hipStreamDestroy(md->stream);
     delete md;
     return AC4_OK;

@@ -707,3 +707,44 @@ def test_energy_after_every_kind_of_call(gpu, prec, n, nsteps):
             assert b.stats(0) == c.stats(0)
     for md in mds:
         md.close()
+
+
+# A slot assigned again while it is occupied, by a job of the same size, of
+# another number of active particles, denser and smaller, after steps from
+# recorded graphs: it runs as in a handle of its own assignment, and so does
+# its neighbour.
+def test_slots_assigned_again(gpu):
+    def fill(md, r, p):
+        md.params[r] = p
+        assert gpu.lib.ac4_md_assign(md.h, r, ctypes.byref(p)) == 0
+        s = gpu.init_lattice(p.n, 0.5, 5 + r)
+        act = s["act_tag"] if p.n_act < 0 else np.where(np.arange(p.n) < p.n_act, np.arange(p.n), -1).astype(np.int32)
+        k = [np.resize(s[c], max(p.n_act, 0)) if p.n_act >= 0 else s[c] for c in ("kx", "ky", "kz")]
+        md.set_state(r, *[s[c] for c in ("x", "y", "z", "xu", "yu", "zu", "px", "py", "pz")], s["type"], act, *k)
+        md.init_chain(r)
+
+    def handle():
+        h = ctypes.c_void_p()
+        assert gpu.lib.ac4_md_create_slots(2, (ctypes.c_int * 2)(900, 1200), 1, ctypes.byref(h)) == 0
+        md = gpu.MD.__new__(gpu.MD)
+        md.h, md.params = h, [None] * 2
+        return md
+
+    P = gpu.ReplicaParams
+    other = P(1100, 1.2, 0.5, 1.0, -1, 10, 4)
+    used = handle()
+    fill(used, 0, P(900, 1.2, 0.5, 1.0, -1, 10, 3))
+    fill(used, 1, other)
+    used.step(30, graph=True)
+    for p in (P(900, 1.2, 0.6, 1.5, -1, 7, 8), P(900, 1.2, 0.5, 1.0, 250, 10, 3), P(900, 0.9, 0.5, 1.0, -1, 10, 3),
+              P(640, 1.2, 0.5, 1.0, -1, 10, 3)):
+        fresh = handle()
+        for md in (used, fresh):
+            fill(md, 0, p)
+            fill(md, 1, other)
+            md.step(51, graph=True)
+        for r in range(2):
+            x, y = used.get_state(r), fresh.get_state(r)
+            assert all(np.array_equal(x[k], y[k]) for k in x) and used.stats(r) == fresh.stats(r)
+        fresh.close()
+    used.close()
