@@ -1922,10 +1922,10 @@ struct EndArgs {
 // FP32 handles whose team is 2 or 4 times the list layout's take EN = 2 or 4,
 // which sums the FP32 terms of eight entries as the layout's team does, so that
 // the partial sums, whose rounding shows in the seventh to ninth digit of the
-// energy, do not depend on the force team's width (walk_list): a third more of
-// the pass.  us of a call of one step, 8000, 160001 and 500000 particles: with
-// the energy in two kernels of its own after it 32.6, 156 and 292, this 27.6,
-// 140 and 254.
+// energy, do not depend on the force team's width (walk_list): four to five
+// tenths more of the pass (18.3 -> 25.1 us at 50000, 162 -> 239 at 1e6).  us of
+// a call of one step, 8000, 160001 and 500000 particles: with the energy in two
+// kernels of its own after it 32.6, 156 and 292, this 27.6, 140 and 254.
 template <bool FP32, bool KICK, int EN, int VEC>
 __global__ void __launch_bounds__(BLK) k_force(const RepC *__restrict__ reps, const BlkD *__restrict__ fblk,
                                                const double4 *__restrict__ pos4, const QPos *__restrict__ posq,
@@ -3316,8 +3316,8 @@ static int launch_force(ac4_md *md, bool energy, bool step = false) {
                          : launch_force_kernel<true, KICK, 4>(md, step);
 }
 // The energy after a call whose last step is the end of a recorded chunk, on
-// handles that form it in the layout's order (EN > 1: a third more of the
-// pass, so chunks leave it out): the forces once more, with it.
+// handles that form it in the layout's order (EN > 1: four to five tenths more
+// of the pass, so chunks leave it out): the forces once more, with it.
 static int launch_energy(ac4_md *md) { return md->en > 1 ? launch_force<false>(md, true, true) : AC4_OK; }
 
 static void launch_shuffle(ac4_md *md, int force) {

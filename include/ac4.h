@@ -436,7 +436,11 @@ typedef struct ac4_ana ac4_ana;
  * gap: origin spacing (0 -> detected as read_all_data.c:36-48);
  * factor: lag growth (1.4, Analysis/main.c:4); a: overlap length (0.3);
  * obs: AC4_OBS_* mask; type_flag: the reference's `flag` argument
- * (1 -> exclude type-1 particles, msd_pos.c:62, overlap.c:59, Fsqt.c:104). */
+ * (1 -> exclude type-1 particles, msd_pos.c:62, overlap.c:59, Fsqt.c:104).
+ * Device memory, allocated here: 24 bytes per particle of the origins resident
+ * together and of one more frame, and per (origin, lag) pair up to 256 blocks'
+ * sums (MSD 24 bytes a block, overlap and S4 4 each), S4's mask (a bit per
+ * particle) and 2.6 KB each for S4 and Fs. */
 int ac4_ana_create(int n, double L, int nframes, const int *fidx, int gap,
                    double factor, double a, int obs, int type_flag,
                    ac4_ana **out);
