@@ -989,7 +989,7 @@ static void build_slots(WalkInfo &W, int nslots) {
     for (int p = 0; p < W.w.np; p++) W.slot_pairs[fill[W.w.slot[p]]++] = p;  // walk order kept
 }
 
-// the permuted-vector columns of S4 and Fs
+// the permuted-vector columns of S4 and Fs, and the permutations of each vector
 static int set_columns(ac4_ana *an, const std::vector<int> &dg) {
     std::vector<int> pv(3 * S4_NCOL, 0), pcol(AC4_NQ, 0);
     int col = 0;
@@ -999,6 +999,7 @@ static int set_columns(ac4_ana *an, const std::vector<int> &dg) {
             perm_q(dg[q], s, an->vx[q], an->vy[q], an->vz[q], pv[3 * col], pv[3 * col + 1], pv[3 * col + 2]);
     }
     AC4_REQUIRE(col <= S4_NCOL, AC4_EARG, "S4: %d permuted vectors exceed %d columns", col, S4_NCOL);
+    AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_dg), dg.data(), sizeof(int) * AC4_NQ));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_pv), pv.data(), sizeof(int) * 3 * S4_NCOL));
     AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_pcol), pcol.data(), sizeof(int) * AC4_NQ));
     return AC4_OK;
@@ -1109,8 +1110,7 @@ extern "C" int ac4_ana_create(int n, double L, int nframes, const int *fidx, int
     int rc = AC4_OK;
     auto fail = [&](int e) { ac4_ana_destroy(an); return e; };
     if (hipGetDevice(&an->dev) != hipSuccess || hipStreamCreate(&an->stream) != hipSuccess) return fail(AC4_EHIP);
-    AC4_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_dg), dg.data(), sizeof(int) * AC4_NQ));
-    if ((rc = set_columns(an, dg)) != AC4_OK) return fail(rc);
+    if ((obs & (AC4_OBS_S4 | AC4_OBS_FS)) && (rc = set_columns(an, dg)) != AC4_OK) return fail(rc);
     // blocks of a frame row: one tile of the block's threads each up to 256 of them, then more tiles per block
     const int fb = obs & AC4_OBS_FS ? FS_T : ABLK;
     an->ppb = fb * ((n + 256 * fb - 1) / (256 * fb));
